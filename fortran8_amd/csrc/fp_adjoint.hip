@@ -738,7 +738,7 @@ void adjoint_step(Ctx& c, Adj& a, int t, int seg_len, int s, double wdrag) {
   f64_solve(c, 3, a.phib, a.bb);
   hipLaunchKernelGGL(k_adj_div, dim3(nb), dim3(256), 0, st, g, a.bb, a.ubs);
   // Helmholtz
-  for (int comp = 0; comp < 3; comp++) f64_solve(c, comp, a.ubs + comp * n, a.Rb + comp * n);
+  f64_helmholtz(c, a.ubs, a.Rb);
   hipLaunchKernelGGL(k_adj_helm_beta, dim3(nb), dim3(256), 0, st, g, a.Rb, Up, a.part);
   // immersed boundary
   const double* Qb = a.Rb;

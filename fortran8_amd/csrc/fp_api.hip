@@ -155,19 +155,23 @@ void fp::step_f64(Ctx& c) {
   { Timer t(c, "predictor"); f64_predictor(c); }
   if (c.p.method == FP_METHOD_FFT) {
     Timer t(c, "helmholtz");
-    for (int comp = 0; comp < 3; comp++) f64_solve(c, comp, c.Q + comp * g.n, c.Up + comp * g.n);
+    f64_helmholtz(c, c.Q, c.Up);
   } else if (c.p.method == FP_METHOD_EXPLICIT) {
     FP_HIP_CHECK(hipMemcpyAsync(c.Up, c.Q, sizeof(double) * 3 * g.n, hipMemcpyDeviceToDevice, c.stream));
   } else {
     { Timer t(c, "ibm"); f64_ibm(c); }
     Timer t(c, "helmholtz");
-    for (int comp = 0; comp < 3; comp++) f64_solve(c, comp, c.Up + comp * g.n, c.Up + comp * g.n);
+    f64_helmholtz(c, c.Up, c.Up);
   }
   {
     Timer t(c, "poisson");
-    f64_divergence(c, c.Up, c.Q);
-    if (c.p.poisson_variant == FP_POISSON_SOR) c.sor_itr = (double)f64_sor(c, c.Q, c.Phi);
-    else { f64_solve(c, 3, c.Q, c.Phi); c.sor_itr = -1.0; }
+    if (c.p.poisson_variant == FP_POISSON_SOR) {
+      f64_divergence(c, c.Up, c.Q);
+      c.sor_itr = (double)f64_sor(c, c.Q, c.Phi);
+    } else {
+      f64_poisson(c, c.Up, c.Phi);
+      c.sor_itr = -1.0;
+    }
   }
   { Timer t(c, "march"); f64_march(c); }
   c.has_history = 1;
@@ -224,8 +228,7 @@ int fp_create(const fp_params* p, void** out) {
     dalloc(&c->fC, n); dalloc(&c->sel, n); dalloc(&c->nitr, n);
     dalloc(&c->A0, 3 * n); dalloc(&c->T0, 3 * n); dalloc(&c->B0, 3 * n); dalloc(&c->B, 3 * n);
     dalloc(&c->Q, 3 * n); dalloc(&c->Up, 3 * n);
-    dalloc(&c->spec, (size_t)g.nxh * g.sy * g.nz);
-    if (g.walls) dalloc(&c->thp, (size_t)(g.ny + 2) * g.nxh * g.nz);
+    f64_spectral_create(*c);
     dalloc(&c->red, 64);
     dalloc(&c->part, (size_t)(g.n / 256 + 1024));
     auto up2 = [&](double2** d, const std::vector<double2>& h) {
@@ -263,7 +266,7 @@ int fp_destroy(void* vc) {
   dfree(c->U); dfree(c->V); dfree(c->W); dfree(c->P); dfree(c->Phi);
   dfree(c->C[0]); dfree(c->C[1]); dfree(c->fC); dfree(c->sel); dfree(c->nitr);
   dfree(c->A0); dfree(c->T0); dfree(c->B0); dfree(c->B); dfree(c->Q); dfree(c->Up); dfree(c->F);
-  dfree(c->spec); dfree(c->thp); dfree(c->red); dfree(c->part);
+  dfree(c->spec); dfree(c->piv); dfree(c->red); dfree(c->part);
   dfree(c->twx); dfree(c->twy); dfree(c->twz); dfree(c->kx2); dfree(c->ky2); dfree(c->kz2);
   dfree(c->mk); dfree(c->mf); dfree(c->mb); dfree(c->ftmp);
   dfree(c->mean_acc); dfree(c->mean_u);

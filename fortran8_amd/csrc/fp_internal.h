@@ -47,8 +47,11 @@ struct Ctx {
   double *Q = nullptr;                // 3 planes: predictor RHS / Ua
   double *Up = nullptr;               // 3 planes: u*
   double *F = nullptr;                // 3 planes body-force field (nullable)
-  double2* spec = nullptr;            // nxh*sy*nz complex
-  double* thp = nullptr;              // Thomas P scratch (ny+2)*nxh*nz
+  double2* spec = nullptr;            // half spectra [component][kx][z][y] (fp_spectral_f64.hip)
+  int nspec = 1;                      // components it holds
+  bool slab64 = false;                // a kx slab fits in LDS
+  double* piv = nullptr;              // walls: pivots of the y line solves (three kinds)
+  double piv_beta = 0.0;              // the beta they were built with
   double2 *twx = nullptr, *twy = nullptr, *twz = nullptr;
   double *kx2 = nullptr, *ky2 = nullptr, *kz2 = nullptr;
   double* red = nullptr;              // reduction scratch
@@ -93,7 +96,6 @@ struct Ctx {
 void f64_select(Ctx& c);
 void f64_cstar_newton(Ctx& c);
 void f64_predictor(Ctx& c);
-void f64_solve(Ctx& c, int kind, const double* q, double* x);   // kind 0..2 Helmholtz, 3 Poisson
 void f64_divergence(Ctx& c, const double* up, double* q);
 void f64_march(Ctx& c);
 void f64_ibm(Ctx& c);        // interp + forces + spread + predictor RHS into Q
@@ -110,7 +112,12 @@ void f64_mean_accumulate(Ctx& c, const float* u32, const float* v32, const float
 int f64_mean_apply(Ctx& c, int mode);
 void f64_fill_f(Ctx& c);     // Peterlin factor of the current C
 void f64_spread_markers(Ctx& c, const double* mfield, double* ftmp);  // spread + ghost folds
-int thomas_lines(int ny, int bytes_per_row);  // lines per block of the LDS line solve
+// ---- spectral solves (fp_spectral_f64.hip)
+void f64_spectral_create(Ctx& c);
+void f64_solve(Ctx& c, int kind, const double* q, double* x);   // kind 0..2 Helmholtz, 3 Poisson
+void f64_helmholtz(Ctx& c, const double* q, double* x);         // the three components
+void f64_poisson(Ctx& c, const double* up, double* x);          // lap x = div up / dt
+void f64_forward(Ctx& c, const double* q);                      // transform into c.spec
 void step_f64(Ctx& c);       // one FP64 time step (fp_api.hip)
 
 // ---- recording and discrete adjoint (fp_adjoint.hip)

@@ -250,277 +250,6 @@ __global__ __launch_bounds__(256) void k_predictor(Grid g, int method, int first
 #undef Wg
 }
 
-// ============================================================ FFT ==========
-// Stockham radix-2 autosort (forward e^{-2 pi i jk/n}, unnormalised; the
-// inverse uses the conjugate twiddles) over `nl` lines resident in LDS.
-// x and y are LDS buffers of nl*n complex; line l occupies [l*n, (l+1)*n).
-// Returns the buffer holding the result.
-__device__ double2* stockham_lds(double2* x, double2* y, int n, int logn, int nl, const double2* __restrict__ tw, bool inv) {
-  int len = n, s = 1, lgs = 0;
-  const int half = n >> 1;
-  while (len > 1) {
-    int m = len >> 1;
-    for (int b = threadIdx.x; b < nl * half; b += blockDim.x) {
-      int line = b >> (logn - 1);
-      int t = b & (half - 1);
-      int p = t >> lgs, q = t & (s - 1);
-      double2 w = tw[p * s];
-      double wr = w.x, wi = inv ? -w.y : w.y;
-      const double2* xl = x + line * n;
-      double2* yl = y + line * n;
-      double2 a = xl[q + s * p], bb = xl[q + s * (p + m)];
-      double2 y0, y1;
-      y0.x = a.x + bb.x;
-      y0.y = a.y + bb.y;
-      double dr = a.x - bb.x, di = a.y - bb.y;
-      y1.x = dr * wr - di * wi;
-      y1.y = dr * wi + di * wr;
-      yl[q + s * (2 * p)] = y0;
-      yl[q + s * (2 * p + 1)] = y1;
-    }
-    __syncthreads();
-    double2* tt = x; x = y; y = tt;
-    len = m; s <<= 1; lgs++;
-  }
-  return x;
-}
-
-__device__ __forceinline__ int ilog2(int n) { int l = 0; while ((1 << l) < n) l++; return l; }
-
-// real x-lines -> half spectrum rows (fftr2c along x)
-__global__ __launch_bounds__(256) void k_fft_x_fwd(Grid g, const double* __restrict__ q, double2* __restrict__ spec,
-                                                   const double2* __restrict__ tw, int lines_per_block) {
-  extern __shared__ double2 lds[];
-  const int n = g.nx, nl = lines_per_block;
-  double2* x = lds;
-  double2* y = lds + nl * n;
-  long nlines = (long)g.ny * g.nz;
-  long l0 = (long)blockIdx.x * nl;
-  for (int e = threadIdx.x; e < nl * n; e += blockDim.x) {
-    int l = e / n, i = e % n;
-    long L = l0 + l;
-    double v = L < nlines ? q[L * n + i] : 0.0;
-    x[e] = make_double2(v, 0.0);
-  }
-  __syncthreads();
-  double2* r = stockham_lds(x, y, n, ilog2(n), nl, tw, false);
-  const int nxh = g.nxh;
-  for (int e = threadIdx.x; e < nl * nxh; e += blockDim.x) {
-    int l = e / nxh, i = e % nxh;
-    long L = l0 + l;
-    if (L >= nlines) continue;
-    long j = L % g.ny, k = L / g.ny;
-    spec[i + (long)nxh * ((j + g.jo) + g.sy * k)] = r[l * n + i];
-  }
-}
-
-// half spectrum rows -> real x-lines (fftc2r along x)
-__global__ __launch_bounds__(256) void k_fft_x_inv(Grid g, const double2* __restrict__ spec, double* __restrict__ out,
-                                                   const double2* __restrict__ tw, int lines_per_block) {
-  extern __shared__ double2 lds[];
-  const int n = g.nx, nl = lines_per_block, h = n / 2, nxh = g.nxh;
-  double2* x = lds;
-  double2* y = lds + nl * n;
-  long nlines = (long)g.ny * g.nz;
-  long l0 = (long)blockIdx.x * nl;
-  for (int e = threadIdx.x; e < nl * nxh; e += blockDim.x) {
-    int l = e / nxh, i = e % nxh;
-    long L = l0 + l;
-    double2 v = make_double2(0.0, 0.0);
-    if (L < nlines) {
-      long j = L % g.ny, k = L / g.ny;
-      v = spec[i + (long)nxh * ((j + g.jo) + g.sy * k)];
-    }
-    if (i == 0 || i == h) v.y = 0.0;
-    x[l * n + i] = v;
-    if (i > 0 && i < h) x[l * n + (n - i)] = make_double2(v.x, -v.y);
-  }
-  __syncthreads();
-  double2* r = stockham_lds(x, y, n, ilog2(n), nl, tw, true);
-  for (int e = threadIdx.x; e < nl * n; e += blockDim.x) {
-    int l = e / n, i = e % n;
-    long L = l0 + l;
-    if (L < nlines) out[L * n + i] = r[e].x;
-  }
-}
-
-// complex lines along y (axis 1) or z (axis 2) of the spectrum.  mode 0:
-// forward, 1: inverse, 2: forward, divide by the periodic LHS of `kind`, then
-// inverse (fft_solve's divide fused between the z transforms).
-__global__ __launch_bounds__(256) void k_fft_yz(Grid g, double2* __restrict__ spec, const double2* __restrict__ tw,
-                                                int axis, int mode, int kind, int row0, int nrows, int ti,
-                                                const double* __restrict__ kx2, const double* __restrict__ ky2,
-                                                const double* __restrict__ kz2) {
-  extern __shared__ double2 lds[];
-  const int n = axis == 1 ? g.ny : g.nz;
-  const int nxh = g.nxh;
-  const long stride = axis == 1 ? (long)nxh : (long)nxh * g.sy;
-  const int ntile = (nxh + ti - 1) / ti;
-  int tile = blockIdx.x % ntile;
-  long other = blockIdx.x / ntile;  // k for axis 1, row for axis 2
-  int i0 = tile * ti;
-  double2* base;
-  if (axis == 1) base = spec + (long)nxh * (g.jo + g.sy * other);
-  else base = spec + (long)nxh * (row0 + other);
-  double2* x = lds;
-  double2* y = lds + ti * n;
-  // LDS layout: line l (i = i0+l) contiguous
-  for (int e = threadIdx.x; e < ti * n; e += blockDim.x) {
-    int l = e % ti, r = e / ti;
-    int i = i0 + l;
-    x[l * n + r] = i < nxh ? base[i + stride * r] : make_double2(0.0, 0.0);
-  }
-  __syncthreads();
-  int logn = ilog2(n);
-  double2* res = stockham_lds(x, y, n, logn, ti, tw, mode == 1);
-  if (mode == 2) {
-    double2* other_buf = res == x ? y : x;
-    const double ntot = (double)((long)g.nx * g.ny * g.nz);
-    const double coef = ((g.dt * g.beta) / g.re) / 2.0;
-    for (int e = threadIdx.x; e < ti * n; e += blockDim.x) {
-      int l = e / n, kk = e % n;
-      int i = i0 + l;
-      if (i >= nxh) continue;
-      long jj = other;  // axis 2: row index == j for periodic grids
-      double lhs;
-      if (kind == 3) lhs = -((kx2[i] + ky2[jj]) + kz2[kk]);
-      else lhs = 1.0 + coef * ((kx2[i] + ky2[jj]) + kz2[kk]);
-      double2 s = res[e];
-      double re = s.x / ntot, im = s.y / ntot;
-      if (fabs(lhs) < 1.0e-16) { s.x = 0.0; s.y = 0.0; }
-      else { s.x = re / lhs; s.y = im / lhs; }
-      res[e] = s;
-    }
-    __syncthreads();
-    res = stockham_lds(res, other_buf, n, logn, ti, tw, true);
-  }
-  for (int e = threadIdx.x; e < ti * n; e += blockDim.x) {
-    int l = e % ti, r = e / ti;
-    int i = i0 + l;
-    if (i < nxh) base[i + stride * r] = res[l * n + r];
-  }
-}
-
-// tridiagonal line solve along y with the wall rows of fenep_2d.f90:1222-1331
-// (tdma, fenep_2d.f90:1145-1177), one thread per (kx, kz) line.
-// Tridiagonal line solve along y of each (kx, kz) mode (tdma with the wall
-// rows of fft_*_kabe, fenep_2d.f90:1145-1177, 1222-1331).  One block of 256
-// threads solves `tl` consecutive kx lines of one kz plane: the rows are
-// staged through LDS with coalesced loads, one thread per line runs the
-// recurrence from LDS, and the rows are stored back.  The arithmetic is the
-// Thomas recurrence of the reference, in its order.
-__global__ __launch_bounds__(256) void k_thomas(Grid g, double2* __restrict__ spec, int kind, int tl,
-                                                const double* __restrict__ kx2, const double* __restrict__ kz2) {
-  extern __shared__ double2 tq[];                 // [size][tl] right-hand sides / Q
-  const int nxh = g.nxh, ny = g.ny, size = ny + 2;
-  double* tp = (double*)(tq + (long)size * tl);   // [size][tl] P
-  const int ngrp = (nxh + tl - 1) / tl;
-  const int i0 = (int)(blockIdx.x % ngrp) * tl;
-  const long k = blockIdx.x / ngrp;
-  const int nl = min(tl, nxh - i0);
-  double2* base = spec + (long)nxh * g.sy * k + i0;  // row r of line l at base[nxh*r + l]
-  for (int e = threadIdx.x; e < size * tl; e += blockDim.x) {
-    const int r = e / tl, l = e - r * tl;
-    if (l < nl) tq[e] = base[(long)nxh * r + l];
-  }
-  __syncthreads();
-  if (threadIdx.x < nl) {
-    const int l = threadIdx.x, i = i0 + l;
-    const double nxz = (double)((long)g.nx * g.nz);
-    const double coef = ((g.dt * g.beta) / g.re) / 2.0;
-    const double idy2 = g.dy * g.dy;
-    const double kk = kx2[i] + kz2[k];
-    auto coeffs = [&](int r, double& a, double& b, double& c, bool& rhs) {
-      rhs = false;
-      if (kind == 3) {
-        if (r == 0) { a = 1.0; b = -1.0; c = 0.0; }
-        else if (r == size - 1) { a = 1.0; b = 0.0; c = -1.0; }
-        else { a = -(kk + 2.0 / idy2); b = 1.0 / idy2; c = 1.0 / idy2; rhs = true; }
-      } else if (kind == 1) {
-        if (r == 0) { a = 1.0; b = 0.0; c = 0.0; }
-        else if (r >= ny) { a = 1.0; b = 0.0; c = 0.0; }
-        else { a = 1.0 + coef * (kk + 2.0 / idy2); b = -(coef / idy2); c = -(coef / idy2); rhs = true; }
-      } else {
-        if (r == 0) { a = 1.0; b = 1.0; c = 0.0; }
-        else if (r == size - 1) { a = 1.0; b = 0.0; c = 1.0; }
-        else { a = 1.0 + coef * (kk + 2.0 / idy2); b = -(coef / idy2); c = -(coef / idy2); rhs = true; }
-      }
-    };
-    double a, b, c; bool rhs;
-    coeffs(0, a, b, c, rhs);
-    double Pp = -b / a;
-    double Qr = 0.0 / a, Qi = 0.0 / a;
-    tp[l] = Pp;
-    tq[l] = make_double2(Qr, Qi);
-    // the next row's right-hand side is read before the current row's
-    // results are stored (the recurrence then waits on arithmetic only)
-    double2 nxt = tq[tl + l];
-    for (int r = 1; r < size; r++) {
-      coeffs(r, a, b, c, rhs);
-      const double2 sv = nxt;
-      if (r + 1 < size) nxt = tq[(r + 1) * tl + l];
-      double dr = 0.0, di = 0.0;
-      if (rhs) { dr = sv.x / nxz; di = sv.y / nxz; }
-      const double den = a + c * Pp;
-      double P, nQr, nQi;
-      if (fabs(den) < 1.0e-16) { P = 0.0; nQr = 0.0; nQi = 0.0; }
-      else { P = -b / den; nQr = (dr - c * Qr) / den; nQi = (di - c * Qi) / den; }
-      Pp = P; Qr = nQr; Qi = nQi;
-      tp[r * tl + l] = P;
-      tq[r * tl + l] = make_double2(Qr, Qi);
-    }
-    double xr = Qr, xi = Qi;
-    double Pn = tp[(size - 2) * tl + l];
-    double2 qn = tq[(size - 2) * tl + l];
-    for (int r = size - 2; r >= 0; r--) {
-      const double P = Pn;
-      const double2 q = qn;
-      if (r > 0) { Pn = tp[(r - 1) * tl + l]; qn = tq[(r - 1) * tl + l]; }
-      xr = P * xr + q.x;
-      xi = P * xi + q.y;
-      tq[r * tl + l] = make_double2(xr, xi);
-    }
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < size * tl; e += blockDim.x) {
-    const int r = e / tl, l = e - r * tl;
-    if (l < nl) base[(long)nxh * r + l] = tq[e];
-  }
-}
-
-// lines per block of the LDS line solve: 64 KiB of LDS at most
-int thomas_lines(int ny, int bytes_per_row) {
-  const int per_line = (ny + 2) * bytes_per_row;
-  return std::max(1, std::min(32, 65536 / per_line));
-}
-
-static int lines_for(int n) { return std::max(1, std::min(16, 2048 / n)); }
-
-void f64_solve(Ctx& c, int kind, const double* q, double* x) {
-  const Grid& g = c.g;
-  hipStream_t s = c.stream;
-  int lx = lines_for(g.nx);
-  long xlines = (long)g.ny * g.nz;
-  size_t shx = sizeof(double2) * 2 * lx * g.nx;
-  hipLaunchKernelGGL(k_fft_x_fwd, dim3(nblk(xlines, lx)), dim3(256), shx, s, g, q, c.spec, c.twx, lx);
-  int tiy = std::max(1, std::min(16, 2048 / g.ny)), tiz = std::max(1, std::min(16, 2048 / g.nz));
-  int nty = (g.nxh + tiy - 1) / tiy, ntz = (g.nxh + tiz - 1) / tiz;
-  size_t shy = sizeof(double2) * 2 * tiy * g.ny, shz = sizeof(double2) * 2 * tiz * g.nz;
-  if (!g.walls) {
-    hipLaunchKernelGGL(k_fft_yz, dim3(nty * g.nz), dim3(256), shy, s, g, c.spec, c.twy, 1, 0, kind, 0, 0, tiy, c.kx2, c.ky2, c.kz2);
-    hipLaunchKernelGGL(k_fft_yz, dim3(ntz * g.ny), dim3(256), shz, s, g, c.spec, c.twz, 2, 2, kind, 0, g.ny, tiz, c.kx2, c.ky2, c.kz2);
-    hipLaunchKernelGGL(k_fft_yz, dim3(nty * g.nz), dim3(256), shy, s, g, c.spec, c.twy, 1, 1, kind, 0, 0, tiy, c.kx2, c.ky2, c.kz2);
-  } else {
-    hipLaunchKernelGGL(k_fft_yz, dim3(ntz * g.ny), dim3(256), shz, s, g, c.spec, c.twz, 2, 0, kind, 1, g.ny, tiz, c.kx2, c.ky2, c.kz2);
-    const int tl = thomas_lines(g.ny, (int)(sizeof(double2) + sizeof(double)));
-    const int ngrp = (g.nxh + tl - 1) / tl;
-    hipLaunchKernelGGL(k_thomas, dim3(ngrp * g.nz), dim3(256), (size_t)(g.ny + 2) * tl * (sizeof(double2) + sizeof(double)),
-                       s, g, c.spec, kind, tl, c.kx2, c.kz2);
-    hipLaunchKernelGGL(k_fft_yz, dim3(ntz * g.ny), dim3(256), shz, s, g, c.spec, c.twz, 2, 1, kind, 1, g.ny, tiz, c.kx2, c.ky2, c.kz2);
-  }
-  hipLaunchKernelGGL(k_fft_x_inv, dim3(nblk(xlines, lx)), dim3(256), shx, s, g, c.spec, x, c.twx, lx);
-}
-
 // ======================================================= projection =======
 // fft_poisson right-hand side (fenep.f90:1550-1552)
 template <bool WL>
@@ -1338,9 +1067,11 @@ __global__ __launch_bounds__(256) void k_spec_shells(Grid g, const double2* __re
   const long total = (long)g.nxh * g.ny * g.nz;
   const double N = (double)g.n;
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
-    const int i = (int)(e % g.nxh);
-    const int j = (int)((e / g.nxh) % g.ny);
-    const int k = (int)(e / ((long)g.nxh * g.ny));
+    // [kx][z][y], the wavenumbers of y and z bit-reversed (f64_forward)
+    const int j = (int)(__brev((unsigned)e & (g.ny - 1)) >> (32 - g.lny));
+    const int lnz = __ffs(g.nz) - 1;
+    const int k = (int)(__brev((unsigned)(e >> g.lny) & (g.nz - 1)) >> (32 - lnz));
+    const int i = (int)(e >> (g.lny + lnz));
     const double kx = (double)i;
     const double ky = (double)(j <= g.ny / 2 ? j : j - g.ny);
     const double kz = (double)(k <= g.nz / 2 ? k : k - g.nz);
@@ -1363,20 +1094,10 @@ void f64_energy_spectrum(Ctx& c, double* E, int nbins) {
   try {
     zero_words(dE, 2L * nbins, s);
     hipLaunchKernelGGL(k_reg_velocity, dim3(nblk(g.n, 256)), dim3(256), 0, s, g, c.U, c.V, c.W, c.mean_u, c.Q);
-    const int lx = lines_for(g.nx);
-    const long xlines = (long)g.ny * g.nz;
-    const size_t shx = sizeof(double2) * 2 * lx * g.nx;
-    const int tiy = std::max(1, std::min(16, 2048 / g.ny)), tiz = std::max(1, std::min(16, 2048 / g.nz));
-    const int nty = (g.nxh + tiy - 1) / tiy, ntz = (g.nxh + tiz - 1) / tiz;
-    const size_t shy = sizeof(double2) * 2 * tiy * g.ny, shz = sizeof(double2) * 2 * tiz * g.nz;
     const long total = (long)g.nxh * g.ny * g.nz;
     const int sb = (int)std::min<long>(1024, (total + 255) / 256);
     for (int comp = 0; comp < 3; comp++) {
-      hipLaunchKernelGGL(k_fft_x_fwd, dim3(nblk(xlines, lx)), dim3(256), shx, s, g, c.Q + comp * g.n, c.spec, c.twx, lx);
-      hipLaunchKernelGGL(k_fft_yz, dim3(nty * g.nz), dim3(256), shy, s, g, c.spec, c.twy, 1, 0, 3, 0, 0, tiy, c.kx2, c.ky2,
-                         c.kz2);
-      hipLaunchKernelGGL(k_fft_yz, dim3(ntz * g.ny), dim3(256), shz, s, g, c.spec, c.twz, 2, 0, 3, 0, g.ny, tiz, c.kx2,
-                         c.ky2, c.kz2);
+      f64_forward(c, c.Q + comp * g.n);
       hipLaunchKernelGGL(k_spec_shells, dim3(sb), dim3(256), sizeof(double) * nbins, s, g, c.spec, nbins, dE);
     }
     FP_HIP_CHECK(hipMemcpyAsync(E, dE, sizeof(double) * nbins, hipMemcpyDeviceToHost, s));

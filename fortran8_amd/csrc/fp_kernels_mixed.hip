@@ -2063,6 +2063,11 @@ __global__ __launch_bounds__(256) void m_thomas(Grid g, float2* __restrict__ spe
 // real x-lines per block (even: the x transforms pack two real lines per
 // complex line); LDS 8 B * n * lines + n/2 twiddles.  A power of two for the
 // power-of-two n (4, 8 or 16): the spectrum stages index lines by shifts.
+// lines per block of the LDS line solve: 64 KiB of LDS at most
+static int thomas_lines(int ny, int bytes_per_row) {
+  const int per_line = (ny + 2) * bytes_per_row;
+  return std::max(1, std::min(32, 65536 / per_line));
+}
 static int lines_for32(int n) { return std::max(2, std::min(16, 4096 / n)) & ~1; }
 // kx columns per block of the y/z transforms (pitch n + 1)
 static int cols_for32(int n) { return std::max(1, std::min(16, 3968 / (n + 1))); }

@@ -1,0 +1,645 @@
+// FP64 spectral solves of the parity path: the Crank-Nicolson Helmholtz
+// problems of the three velocity components (fft_navier, fenep.f90:1430-1527;
+// fft_*_kabe, fenep_2d.f90:1179-1342) and the pressure Poisson equation
+// (fft_poisson, fenep.f90:1529-1560; fft_poisson_kabe and tdma,
+// fenep_2d.f90:1145-1342).  Compiled with -ffp-contract=off; fused
+// multiply-adds appear only where they are written out (quot, below).
+//
+// The transforms are radix-2 decimations in frequency: the butterflies, their
+// twiddles and their operand order are those of the CPU restatement's Stockham
+// form, so every spectrum value has its bits; only the places differ.  They
+// run in place in LDS, up to three radix-2 stages per pass with the eight
+// elements in registers, and leave their output bit-reversed; the inverse
+// reads the bit-reversed order back, so no pass permutes anything.
+//
+// The half spectrum is stored [component][kx][z][y] (y fastest): an x
+// transform of `nl` consecutive (y, z) lines stores runs of nl values, and a
+// kx slab is contiguous.  After the z (and y) transforms the row of
+// wavenumber m is row bitrev(m).
+//
+// Three launches serve the three Helmholtz problems and three the Poisson
+// equation (its right-hand side formed in the x transform) where a kx slab
+// fits in LDS, five otherwise.  Before: five per component (x, y, z with the
+// division, y, x), 24 of the step's launches.  Small grids are bound by those
+// launches: the Newtonian 32^3 step took 127 us and takes 49, the FENE-P step
+// at 64^3 340 and 228 us.  At 256 x 128 x 128 between walls the four solves
+// went from 1.16 to 0.46 ms; there the line solves' serial recurrence and the
+// LDS passes bound them.
+#include "fp_device.h"
+#include <algorithm>
+#include <cmath>
+
+namespace fp {
+
+namespace {
+
+// n / d correctly rounded, from y = 1/d correctly rounded: two residual
+// corrections (P. W. Markstein, "Computation of elementary functions on the
+// IBM RISC System/6000 processor", 1990: with q within an ulp of n/d and
+// y = RN(1/d), q + (n - d q) y rounds to RN(n/d)).  The first correction
+// brings n y, whose error can exceed an ulp, within one; the residuals are
+// exact unless |n| is below 2^-960.  Five dependent operations instead of about twelve with a
+// quarter-rate reciprocal among them.  y = 0 gives 0.
+__device__ __forceinline__ double quot(double n, double d, double y) {
+  double q = n * y;
+  q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
+  return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+
+__device__ __forceinline__ int brev(int v, int bits) { return bits ? (int)(__brev((unsigned)v) >> (32 - bits)) : 0; }
+
+// one radix-2 butterfly of the Stockham form: (a, b) -> (a + b, (a - b) w)
+template <bool CONJ>
+__device__ __forceinline__ void bfly(double2& a, double2& b, double2 w) {
+  const double wi = CONJ ? -w.y : w.y;
+  const double dr = a.x - b.x, di = a.y - b.y;
+  a.x = a.x + b.x;
+  a.y = a.y + b.y;
+  b.x = dr * w.x - di * wi;
+  b.y = dr * wi + di * w.x;
+}
+
+// LR radix-2 stages, spans len/2, len/4, ..., on the 2^LR elements p + c
+// len/2^LR of one block: p the first one's place in the block, sh = log2(n /
+// len)
+template <int LR, bool CONJ>
+__device__ __forceinline__ void stages(double2 (&v)[1 << LR], int p, int step, int sh, const double2* tws) {
+  constexpr int R = 1 << LR;
+#pragma unroll
+  for (int s = 0; s < LR; s++) {
+    const int half = R >> (s + 1);
+#pragma unroll
+    for (int c = 0; c < half; c++) {
+      const double2 w = tws[(p + c * step) << (sh + s)];
+#pragma unroll
+      for (int b = 0; b < R; b += 2 * half) bfly<CONJ>(v[b + c], v[b + c + half], w);
+    }
+  }
+}
+
+// A set of 2^lnl lines of n = 2^L points in LDS: point r of line l at
+// X[r rs + l ls].  Consecutive threads take consecutive lines, whose stride
+// (1, or an odd pitch) keeps the 16-byte accesses off each other's banks.
+struct Lines {
+  double2* X;
+  int rs, ls, lnl, L;
+};
+
+// the LR stages from blocks of 2^ll points on; REV: the points lie
+// bit-reversed
+template <int LR, bool CONJ, bool REV>
+__device__ __forceinline__ void dif_pass(const Lines& f, int ll, const double2* tws) {
+  constexpr int R = 1 << LR;
+  const int n = 1 << f.L, step = 1 << (ll - LR);
+  for (int e = threadIdx.x; e < (n >> LR) << f.lnl; e += blockDim.x) {
+    const int l = e & ((1 << f.lnl) - 1), t = e >> f.lnl;
+    const int p = t & (step - 1), base = ((t >> (ll - LR)) << ll) + p;
+    double2* x = f.X + l * f.ls;
+    double2 v[R];
+    int at[R];
+#pragma unroll
+    for (int c = 0; c < R; c++) {
+      const int o = base + c * step;
+      at[c] = (REV ? brev(o, f.L) : o) * f.rs;
+      v[c] = x[at[c]];
+    }
+    stages<LR, CONJ>(v, p, step, f.L - ll, tws);
+#pragma unroll
+    for (int c = 0; c < R; c++) x[at[c]] = v[c];
+  }
+  __syncthreads();
+}
+
+// The stages of a transform of 2^L points in passes of M (2 or 3): forward,
+// what is left over comes first, as one shorter pass (M = 3, L = 1 mod 3: two
+// of two stages); the inverse mirrors it.
+__device__ __forceinline__ int lead_stages(int M, int L) { return M == 2 ? (L & 1) : (L % 3 == 1 ? 4 : L % 3); }
+// stages of the last forward pass and of the first inverse one
+__device__ __forceinline__ int last_stages(int M, int L) { return M == 3 && L != 2 && L != 4 ? 3 : 2; }
+
+// natural order in, bit-reversed out; all passes, or all but the last one
+template <int M, bool CONJ>
+__device__ void dif_from_natural(const Lines& f, const double2* tws, bool all = true) {
+  const int stop = all ? 0 : last_stages(M, f.L);
+  const int rest = f.L - lead_stages(M, f.L);
+  int ll = f.L;
+  if constexpr (M == 2) {
+    if (ll > rest) { dif_pass<1, CONJ, false>(f, ll, tws); ll--; }
+  } else {
+    for (; ll > rest && ll > stop; ll -= 2) dif_pass<2, CONJ, false>(f, ll, tws);
+  }
+  for (; ll > stop; ll -= M) dif_pass<M, CONJ, false>(f, ll, tws);
+}
+// bit-reversed in, natural order out; all passes, or all but the first one
+template <int M>
+__device__ void dif_from_reversed(const Lines& f, const double2* tws, bool all = true) {
+  const int lead = lead_stages(M, f.L);
+  int ll = f.L - (all ? 0 : last_stages(M, f.L));
+  for (; ll > lead; ll -= M) dif_pass<M, true, true>(f, ll, tws);
+  if constexpr (M == 2) {
+    if (ll > 0) dif_pass<1, true, true>(f, ll, tws);
+  } else {
+    for (; ll > 0; ll -= 2) dif_pass<2, true, true>(f, ll, tws);
+  }
+}
+
+// The last forward pass, op on every spectrum value, the first inverse pass:
+// both work on the same 2^LR elements (places t R + c, wavenumbers bitrev(c)
+// n/R + bitrev(t)), which stay in registers between them.
+template <int LR, typename Op>
+__device__ __forceinline__ void turn_pass(const Lines& f, const double2* tws, Op op) {
+  constexpr int R = 1 << LR;
+  const int n = 1 << f.L;
+  for (int e = threadIdx.x; e < (n >> LR) << f.lnl; e += blockDim.x) {
+    const int l = e & ((1 << f.lnl) - 1), t = e >> f.lnl;
+    double2* x = f.X + l * f.ls + t * R * f.rs;
+    double2 v[R], u[R];
+#pragma unroll
+    for (int c = 0; c < R; c++) v[c] = x[c * f.rs];
+    stages<LR, false>(v, 0, 1, f.L - LR, tws);
+    const int p = brev(t, f.L - LR), step = n >> LR;
+#pragma unroll
+    for (int c = 0; c < R; c++) {
+      // static bit reversal of c in LR bits
+      const int rc = LR == 2 ? ((c & 1) << 1 | c >> 1) : ((c & 1) << 2 | (c & 2) | c >> 2);
+      u[rc] = op(l, p + rc * step, v[c]);
+    }
+    stages<LR, true>(u, p, step, 0, tws);
+#pragma unroll
+    for (int c = 0; c < R; c++) {
+      const int rc = LR == 2 ? ((c & 1) << 1 | c >> 1) : ((c & 1) << 2 | (c & 2) | c >> 2);
+      x[c * f.rs] = u[rc];
+    }
+  }
+  __syncthreads();
+}
+template <int M, typename Op>
+__device__ __forceinline__ void turn(const Lines& f, const double2* tws, Op op) {
+  if (M == 2 || last_stages(M, f.L) == 2) turn_pass<2>(f, tws, op);
+  else turn_pass<3>(f, tws, op);
+}
+
+__device__ __forceinline__ int log2i(int n) { return __ffs(n) - 1; }
+
+// twiddles exp(-2 pi i t/n), t < n/2, into LDS (no barrier)
+__device__ __forceinline__ void load_tw(double2* tws, const double2* __restrict__ tw, int n) {
+  for (int e = threadIdx.x; e < n / 2; e += blockDim.x) tws[e] = tw[e];
+}
+
+// divides a spectrum value by N and the operator of the periodic problem
+// (fenep.f90:1458-1462, 1540-1548): kinds 0-2 Helmholtz, 3 Poisson.  N is a
+// power of two: its reciprocal multiplies exactly.
+struct Divide {
+  int kind;
+  double coef, rn;
+  __device__ __forceinline__ double2 operator()(double k2, double2 s) const {
+    const double lhs = kind == 3 ? -k2 : 1.0 + coef * k2;
+    if (fabs(lhs) < 1.0e-16) return make_double2(0.0, 0.0);
+    const double y = 1.0 / lhs;
+    return make_double2(quot(s.x * rn, lhs, y), quot(s.y * rn, lhs, y));
+  }
+};
+
+}  // namespace
+
+// ------------------------------------------------------------- x transforms
+// Real x-lines -> half spectrum, 2^lnl consecutive (y, z) lines per block and
+// component blockIdx.y.  DIV: the line values are the divergence of u* / dt
+// (the Poisson right-hand side, fenep.f90:1550-1552), formed here from u* = q.
+template <int M, int DIV, bool WL>
+__global__ __launch_bounds__(256) void k_x_forward(Grid g, const double* __restrict__ q, double2* __restrict__ spec,
+                                                   const double2* __restrict__ tw, int lnl) {
+  extern __shared__ double2 lds[];
+  const int n = g.nx, L = g.lnx, nl = 1 << lnl, pitch = n + 1;
+  double2* tws = lds + nl * pitch;
+  const long plane = (long)g.ny * g.nz, l0 = (long)blockIdx.x << lnl;
+  load_tw(tws, tw, n);
+  const double* src = DIV ? q : q + blockIdx.y * g.n;
+  for (int e = threadIdx.x; e < nl << L; e += blockDim.x) {
+    const int l = e >> L, i = e & (n - 1);
+    const long m = (l0 + l) * n + i;
+    double v;
+    if (DIV) {
+      int ii, j, k;
+      cell_ijk(g, m, ii, j, k);
+      const double *U = q, *V = q + g.n, *W = q + 2 * g.n;
+      v = (((-ldbw<WL>(U, g, i - 1, j, k, BC_U) + ldbw<WL>(U, g, i, j, k, BC_U)) / g.dx
+            + (-ldbw<WL>(V, g, i, j - 1, k, BC_V) + ldbw<WL>(V, g, i, j, k, BC_V)) / g.dy)
+           + (-ldbw<WL>(W, g, i, j, k - 1, BC_W) + ldbw<WL>(W, g, i, j, k, BC_W)) / g.dz) / g.dt;
+    } else {
+      v = src[m];
+    }
+    lds[l * pitch + i] = make_double2(v, 0.0);
+  }
+  __syncthreads();
+  const Lines f{lds, 1, pitch, lnl, L};
+  dif_from_natural<M, false>(f, tws);
+  double2* out = spec + blockIdx.y * (plane * g.nxh) + l0;
+  for (int e = threadIdx.x; e < g.nxh << lnl; e += blockDim.x) {
+    const int l = e & (nl - 1), i = e >> lnl;
+    out[plane * i + l] = lds[l * pitch + brev(i, L)];
+  }
+}
+
+// half spectrum -> real x-lines
+template <int M>
+__global__ __launch_bounds__(256) void k_x_inverse(Grid g, const double2* __restrict__ spec, double* __restrict__ out,
+                                                   const double2* __restrict__ tw, int lnl) {
+  extern __shared__ double2 lds[];
+  const int n = g.nx, L = g.lnx, nl = 1 << lnl, pitch = n + 1, h = n / 2;
+  double2* tws = lds + nl * pitch;
+  const long plane = (long)g.ny * g.nz, l0 = (long)blockIdx.x << lnl;
+  load_tw(tws, tw, n);
+  const double2* in = spec + blockIdx.y * (plane * g.nxh) + l0;
+  for (int e = threadIdx.x; e < g.nxh << lnl; e += blockDim.x) {
+    const int l = e & (nl - 1), i = e >> lnl;
+    double2 v = in[plane * i + l];
+    if (i == 0 || i == h) v.y = 0.0;
+    lds[l * pitch + i] = v;
+    if (i > 0 && i < h) lds[l * pitch + (n - i)] = make_double2(v.x, -v.y);
+  }
+  __syncthreads();
+  const Lines f{lds, 1, pitch, lnl, L};
+  dif_from_natural<M, true>(f, tws);
+  double* o = out + blockIdx.y * g.n + l0 * n;
+  for (int e = threadIdx.x; e < nl << L; e += blockDim.x) o[e] = lds[(e >> L) * pitch + brev(e & (n - 1), L)].x;
+}
+
+// -------------------------------------------------------- line solve in y
+// Tridiagonal line solve along y of one (kx, kz) mode, between walls (tdma
+// with the wall rows of fft_*_kabe, fenep_2d.f90:1145-1177, 1222-1331), in the
+// reference's order.  Rows: 0 and ny+1 the ghosts, 1..ny the cells; the
+// right-hand side of the ghost rows is zero and their solution is not needed,
+// so only the cells are stored.  The pivots 1/den depend on the mode and the
+// kind alone and come from a table (k_line_pivots); the recurrence for P
+// follows from them with multiplies.  re and im are independent: one lane
+// each.
+struct LineRow {
+  int kind, ny;
+  double diag, off;   // the interior rows' coefficients
+  __device__ __forceinline__ LineRow(const Grid& g, int kd, double k2) : kind(kd), ny(g.ny) {
+    const double coef = ((g.dt * g.beta) / g.re) / 2.0, idy2 = g.dy * g.dy;
+    if (kd == 3) { diag = -(k2 + 2.0 / idy2); off = 1.0 / idy2; }
+    else { diag = 1.0 + coef * (k2 + 2.0 / idy2); off = -(coef / idy2); }
+  }
+  // P of the ghost row below; a, b, c of row r >= 1
+  __device__ __forceinline__ double first() const { return kind == 3 ? 1.0 : (kind == 1 ? -0.0 : -1.0); }
+  __device__ __forceinline__ void row(int r, double& a, double& b, double& c, bool& rhs) const {
+    const bool inner = r <= ny - (kind == 1 ? 1 : 0);
+    rhs = inner;
+    a = inner ? diag : 1.0;
+    b = inner ? off : 0.0;
+    c = inner ? off : (kind == 3 ? -1.0 : (kind == 1 ? 0.0 : 1.0));
+  }
+};
+
+// table[kx][r][row of kz], r = 0..ny (rows 1..ny+1 of the line): 1/den, 0 where the
+// reference takes the row for singular
+__global__ __launch_bounds__(256) void k_line_pivots(Grid g, int kind, const double* __restrict__ kx2,
+                                                     const double* __restrict__ kz2, double* __restrict__ table) {
+  const long t = blockIdx.x * 256L + threadIdx.x;
+  if (t >= (long)g.nxh * g.nz) return;
+  const int kr = (int)(t & (g.nz - 1)), i = (int)(t / g.nz);
+  const LineRow lr(g, kind, kx2[i] + kz2[brev(kr, log2i(g.nz))]);
+  double P = lr.first();
+  double* o = table + (long)i * (g.ny + 1) * g.nz + kr;
+  for (int r = 1; r <= g.ny + 1; r++) {
+    double a, b, c;
+    bool rhs;
+    lr.row(r, a, b, c, rhs);
+    const double den = a + c * P;
+    const bool zero = fabs(den) < 1.0e-16;
+    P = zero ? 0.0 : -b / den;
+    o[(long)(r - 1) * g.nz] = zero ? 0.0 : 1.0 / den;
+  }
+}
+
+// One lane's line: its values v[0..ny) (stride vs doubles) in LDS, its P in
+// lp[0..ny) (stride ps); y the pivots (stride ys), read LINE_AHEAD rows ahead.
+constexpr int LINE_AHEAD = 16;
+__device__ __forceinline__ void line_solve(const Grid& g, int kind, double k2, double rn, const double* __restrict__ y,
+                                           int ys, double* v, int vs, double* lp, int ps) {
+  const LineRow lr(g, kind, k2);
+  const int ny = g.ny;
+  double P = lr.first(), Q = 0.0;
+  double yn[LINE_AHEAD];
+#pragma unroll
+  for (int u = 0; u < LINE_AHEAD; u++) yn[u] = y[(long)min(u, ny) * ys];
+  double nxt = v[0];
+  for (int r0 = 1; r0 <= ny; r0 += LINE_AHEAD) {
+    double yc[LINE_AHEAD];
+#pragma unroll
+    for (int u = 0; u < LINE_AHEAD; u++) {
+      yc[u] = yn[u];
+      yn[u] = y[(long)min(r0 + LINE_AHEAD - 1 + u, ny) * ys];
+    }
+#pragma unroll
+    for (int u = 0; u < LINE_AHEAD; u++) {
+      const int r = r0 + u;
+      if (r <= ny) {
+        double a, b, c;
+        bool rhs;
+        lr.row(r, a, b, c, rhs);
+        const double d = rhs ? nxt * rn : 0.0;
+        if (r < ny) nxt = v[r * vs];
+        const double den = a + c * P;
+        Q = quot(d - c * Q, den, yc[u]);
+        P = quot(-b, den, yc[u]);
+        v[(r - 1) * vs] = Q;
+        lp[(r - 1) * ps] = P;   // both lanes of the line: the same value
+      }
+    }
+  }
+  {
+    double a, b, c;
+    bool rhs;
+    lr.row(ny + 1, a, b, c, rhs);
+    Q = quot(0.0 - c * Q, a + c * P, y[(long)ny * ys]);
+  }
+  double x = Q, Pn = lp[(ny - 1) * ps], qn = v[(ny - 1) * vs];
+  for (int r = ny; r >= 1; r--) {
+    const double p = Pn, q = qn;
+    if (r > 1) { Pn = lp[(r - 2) * ps]; qn = v[(r - 2) * vs]; }
+    x = p * x + q;
+    v[(r - 1) * vs] = x;
+  }
+}
+
+// Line solves of 2^ltl consecutive kz rows of one kx and component per block,
+// the lines staged through LDS with coalesced copies.  Bound by the serial
+// recurrence of a line: 16 lines per block keep three blocks on a CU.
+__global__ __launch_bounds__(128) void k_lines_y(Grid g, double2* __restrict__ spec, int kind0, double rn,
+                                                 const double* __restrict__ table, long tstride, const double* __restrict__ kx2,
+                                                 const double* __restrict__ kz2, int ltl) {
+  extern __shared__ double2 lds[];
+  const int ny = g.ny, tl = 1 << ltl, pitch = ny + 1;
+  double* lp = (double*)(lds + tl * pitch);   // [row][line]
+  const int kind = kind0 + blockIdx.y;
+  const long b0 = (long)blockIdx.x << ltl;    // first (kx, kz row) line
+  const int i = (int)(b0 / g.nz), kr0 = (int)(b0 & (g.nz - 1));
+  double2* base = spec + blockIdx.y * ((long)g.nxh * ny * g.nz) + b0 * ny;
+  for (int e = threadIdx.x; e < tl << g.lny; e += blockDim.x) lds[(e >> g.lny) * pitch + (e & (ny - 1))] = base[e];
+  __syncthreads();
+  if (threadIdx.x < 2 * tl) {
+    const int l = threadIdx.x >> 1, c = threadIdx.x & 1, kr = kr0 + l;
+    const double* y = table + (kind == 1 ? tstride : (kind == 3 ? 2 * tstride : 0)) + (long)i * (ny + 1) * g.nz + kr;
+    line_solve(g, kind, kx2[i] + kz2[brev(kr, log2i(g.nz))], rn, y, g.nz, (double*)(lds + l * pitch) + c, 2, lp + l, tl);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < tl << g.lny; e += blockDim.x) base[e] = lds[(e >> g.lny) * pitch + (e & (ny - 1))];
+}
+
+// ------------------------------------------------------------ one kx slab
+// Everything between the x transforms for one kx and component, the [z][y]
+// slab in LDS: periodic, the y and z transforms, the division and back;
+// between walls, the z transforms around the line solves.  Taken where the
+// slab fits in the LDS of a CU.
+template <int M, bool WL>
+__global__ __launch_bounds__(1024) void k_slab(Grid g, double2* __restrict__ spec, int kind0, double rn,
+                                               const double2* __restrict__ twy, const double2* __restrict__ twz,
+                                               const double* __restrict__ kx2, const double* __restrict__ ky2,
+                                               const double* __restrict__ kz2, const double* __restrict__ table,
+                                               long tstride) {
+  extern __shared__ double2 lds[];
+  const int ny = g.ny, nz = g.nz, pitch = ny + 1, lnz = log2i(nz);
+  double2* tz = lds + nz * pitch;
+  double2* ty = tz + nz / 2;                  // periodic
+  double* lp = (double*)ty;                   // between walls: P, [row][kz]
+  const int i = blockIdx.x, kind = kind0 + blockIdx.y;
+  double2* base = spec + (blockIdx.y * (long)g.nxh + i) * ((long)ny * nz);
+  load_tw(tz, twz, nz);
+  if (!WL) load_tw(ty, twy, ny);
+  for (int e = threadIdx.x; e < ny * nz; e += blockDim.x) lds[(e >> g.lny) * pitch + (e & (ny - 1))] = base[e];
+  __syncthreads();
+  const Lines fy{lds, 1, pitch, lnz, g.lny}, fz{lds, pitch, 1, g.lny, lnz};
+  if constexpr (!WL) {
+    dif_from_natural<M, false>(fy, ty);
+    dif_from_natural<M, false>(fz, tz, false);
+    const Divide dv{kind, ((g.dt * g.beta) / g.re) / 2.0, rn};
+    const double kx = kx2[i];
+    turn<M>(fz, tz, [&](int l, int kz, double2 s) { return dv((kx + ky2[brev(l, g.lny)]) + kz2[kz], s); });
+    dif_from_reversed<M>(fz, tz, false);
+    dif_from_reversed<M>(fy, ty);
+  } else {
+    dif_from_natural<M, false>(fz, tz);
+    for (int t = threadIdx.x; t < 2 * nz; t += blockDim.x) {
+      const int kr = t >> 1, c = t & 1;
+      const double* y = table + (kind == 1 ? tstride : (kind == 3 ? 2 * tstride : 0)) + (long)i * (ny + 1) * nz + kr;
+      line_solve(g, kind, kx2[i] + kz2[brev(kr, lnz)], rn, y, nz, (double*)(lds + kr * pitch) + c, 2, lp + kr, nz);
+    }
+    __syncthreads();
+    dif_from_reversed<M>(fz, tz);
+  }
+  for (int e = threadIdx.x; e < ny * nz; e += blockDim.x) base[e] = lds[(e >> g.lny) * pitch + (e & (ny - 1))];
+}
+
+// ---------------------------------------- y and z transforms of larger grids
+// y: 2^lnl consecutive contiguous lines per block (inv: bit-reversed in)
+template <int M>
+__global__ __launch_bounds__(256) void k_y_lines(Grid g, double2* __restrict__ spec, const double2* __restrict__ tw, int inv,
+                                                 int lnl) {
+  extern __shared__ double2 lds[];
+  const int n = g.ny, nl = 1 << lnl, pitch = n + 1;
+  double2* tws = lds + nl * pitch;
+  double2* base = spec + blockIdx.y * ((long)g.nxh * n * g.nz) + ((long)blockIdx.x << (lnl + g.lny));
+  load_tw(tws, tw, n);
+  for (int e = threadIdx.x; e < nl << g.lny; e += blockDim.x) lds[(e >> g.lny) * pitch + (e & (n - 1))] = base[e];
+  __syncthreads();
+  const Lines f{lds, 1, pitch, lnl, g.lny};
+  if (inv) dif_from_reversed<M>(f, tws);
+  else dif_from_natural<M, false>(f, tws);
+  for (int e = threadIdx.x; e < nl << g.lny; e += blockDim.x) base[e] = lds[(e >> g.lny) * pitch + (e & (n - 1))];
+}
+
+// z: 2^lnl consecutive y columns of one kx.  mode 0 forward, 1 inverse
+// (bit-reversed in), 2 forward, the periodic division, inverse
+template <int M>
+__global__ __launch_bounds__(256) void k_z_lines(Grid g, double2* __restrict__ spec, const double2* __restrict__ tw, int mode,
+                                                 int kind0, double rn, int lnl, const double* __restrict__ kx2,
+                                                 const double* __restrict__ ky2, const double* __restrict__ kz2) {
+  extern __shared__ double2 lds[];
+  const int n = g.nz, nl = 1 << lnl, L = log2i(n);
+  double2* tws = lds + (n << lnl);
+  const int lt = g.lny - lnl;                 // log2 of the tiles per kx
+  const int i = blockIdx.x >> lt, j0 = (blockIdx.x & ((1 << lt) - 1)) << lnl;
+  double2* base = spec + (blockIdx.y * (long)g.nxh + i) * ((long)g.ny * n) + j0;
+  load_tw(tws, tw, n);
+  for (int e = threadIdx.x; e < n << lnl; e += blockDim.x) lds[e] = base[((long)(e >> lnl) << g.lny) + (e & (nl - 1))];
+  __syncthreads();
+  const Lines f{lds, nl, 1, lnl, L};
+  if (mode == 0) {
+    dif_from_natural<M, false>(f, tws);
+  } else if (mode == 1) {
+    dif_from_reversed<M>(f, tws);
+  } else {
+    dif_from_natural<M, false>(f, tws, false);
+    const Divide dv{kind0 + (int)blockIdx.y, ((g.dt * g.beta) / g.re) / 2.0, rn};
+    const double kx = kx2[i];
+    turn<M>(f, tws, [&](int l, int kz, double2 s) { return dv((kx + ky2[brev(j0 + l, g.lny)]) + kz2[kz], s); });
+    dif_from_reversed<M>(f, tws, false);
+  }
+  for (int e = threadIdx.x; e < n << lnl; e += blockDim.x) base[((long)(e >> lnl) << g.lny) + (e & (nl - 1))] = lds[e];
+}
+
+// -------------------------------------------------------------------- host
+namespace {
+
+inline int lg(int n) { int l = 0; while ((1 << l) < n) l++; return l; }
+
+// log2 of the lines of n points a block holds: 16 where they take at most 33
+// KB of LDS (four blocks per CU), fewer for long lines, and fewer (4 at
+// least) while the launch would leave CUs without a block
+int lines_log2(int n, long lines, int comps) {
+  int l = std::max(2, std::min(4, 11 - lg(n)));
+  while (l > 2 && (lines >> l) * comps < 512) l--;
+  while (l > 0 && (1L << l) > lines) l--;
+  return l;
+}
+size_t lds_lines(int n, int lnl) { return sizeof(double2) * (((size_t)(n + 1) << lnl) + n / 2); }
+size_t lds_slab64(const Grid& g) {
+  size_t w = sizeof(double2) * ((size_t)g.nz * (g.ny + 1) + g.nz / 2);
+  return w + (g.walls ? sizeof(double) * (size_t)g.ny * g.nz : sizeof(double2) * (g.ny / 2));
+}
+constexpr int LNL_Y = 4;   // lines per block of k_lines_y (log2)
+size_t lds_lines_y(int ny, int ltl) { return (sizeof(double2) * (ny + 1) + sizeof(double) * ny) << ltl; }
+
+template <typename F>
+void allow_lds(F* f, int bytes) {
+  FP_HIP_CHECK(hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+}
+
+int lnl_lines_y(const Grid& g) {
+  int l = std::min(LNL_Y, lg(g.nz));
+  while (l > 0 && lds_lines_y(g.ny, l) > 64 * 1024) l--;
+  return l;
+}
+
+void line_pivots(Ctx& c) {
+  const Grid& g = c.g;
+  const long stride = (long)g.nxh * (g.ny + 1) * g.nz;
+  if (!c.piv) FP_HIP_CHECK(hipMalloc((void**)&c.piv, sizeof(double) * 3 * stride));
+  const int kinds[3] = {0, 1, 3};   // U and W share a table
+  for (int t = 0; t < 3; t++)
+    hipLaunchKernelGGL(k_line_pivots, dim3((unsigned)(((long)g.nxh * g.nz + 255) / 256)), dim3(256), 0, c.stream, g, kinds[t],
+                       c.kx2, c.kz2, c.piv + t * stride);
+  c.piv_beta = g.beta;
+}
+
+// Stages per pass: two where the launch has few points per CU (a pass of
+// three would leave SIMDs without a thread), three above.
+int stages_per_pass(const Grid& g, int comps) { return g.n * comps <= (1L << 20) ? 2 : 3; }
+int threads_for(long points, int M) { return (int)std::max(64L, std::min(256L, points >> M)); }
+
+// the transforms along one axis of `comps` components
+void x_forward(Ctx& c, int comps, const double* q, bool div) {
+  const Grid& g = c.g;
+  const long lines = (long)g.ny * g.nz;
+  const int lx = lines_log2(g.nx, lines, comps), M = stages_per_pass(g, comps);
+  auto k = M == 2 ? (div ? (g.walls ? k_x_forward<2, 1, true> : k_x_forward<2, 1, false>) : k_x_forward<2, 0, false>)
+                  : (div ? (g.walls ? k_x_forward<3, 1, true> : k_x_forward<3, 1, false>) : k_x_forward<3, 0, false>);
+  hipLaunchKernelGGL(k, dim3((unsigned)(lines >> lx), comps), dim3(threads_for((long)g.nx << lx, M)), lds_lines(g.nx, lx),
+                     c.stream, g, q, c.spec, c.twx, lx);
+}
+void x_inverse(Ctx& c, int comps, double* x) {
+  const Grid& g = c.g;
+  const long lines = (long)g.ny * g.nz;
+  const int lx = lines_log2(g.nx, lines, comps), M = stages_per_pass(g, comps);
+  hipLaunchKernelGGL(M == 2 ? k_x_inverse<2> : k_x_inverse<3>, dim3((unsigned)(lines >> lx), comps),
+                     dim3(threads_for((long)g.nx << lx, M)), lds_lines(g.nx, lx), c.stream, g, c.spec, x, c.twx, lx);
+}
+void y_lines(Ctx& c, int comps, int inv) {
+  const Grid& g = c.g;
+  // (the lines of a block share their kx)
+  const int l = std::min(lines_log2(g.ny, (long)g.nxh * g.nz, comps), lg(g.nz)), M = stages_per_pass(g, comps);
+  hipLaunchKernelGGL(M == 2 ? k_y_lines<2> : k_y_lines<3>, dim3((unsigned)((long)g.nxh * g.nz >> l), comps),
+                     dim3(threads_for((long)g.ny << l, M)), lds_lines(g.ny, l), c.stream, g, c.spec, c.twy, inv, l);
+}
+void z_lines(Ctx& c, int comps, int mode, int kind0, double rn) {
+  const Grid& g = c.g;
+  const int l = std::min(lines_log2(g.nz, (long)g.nxh * g.ny, comps), g.lny), M = stages_per_pass(g, comps);
+  hipLaunchKernelGGL(M == 2 ? k_z_lines<2> : k_z_lines<3>, dim3((unsigned)((long)g.nxh * g.ny >> l), comps),
+                     dim3(threads_for((long)g.nz << l, M)), sizeof(double2) * (((size_t)g.nz << l) + g.nz / 2), c.stream, g, c.spec,
+                     c.twz, mode, kind0, rn, l, c.kx2, c.ky2, c.kz2);
+}
+
+// the solves of `comps` components, kinds kind0, kind0 + 1, ..., at once
+void solve(Ctx& c, int kind0, int comps, const double* q, double* x, bool div) {
+  const Grid& g = c.g;
+  hipStream_t s = c.stream;
+  x_forward(c, comps, q, div);
+  const double rn = 1.0 / (double)(g.walls ? (long)g.nx * g.nz : g.n);
+  const long tstride = (long)g.nxh * (g.ny + 1) * g.nz;
+  if (g.walls && (!c.piv || c.piv_beta != g.beta)) line_pivots(c);
+  if (c.slab64) {
+    const int threads = std::max(64, std::min(1024, g.ny * g.nz / 4));
+    auto slab = g.walls ? k_slab<2, true> : k_slab<2, false>;
+    hipLaunchKernelGGL(slab, dim3(g.nxh, comps), dim3(threads), lds_slab64(g), s, g,
+                       c.spec, kind0, rn, c.twy, c.twz, c.kx2, c.ky2, c.kz2, c.piv, tstride);
+  } else if (!g.walls) {
+    y_lines(c, comps, 0);
+    z_lines(c, comps, 2, kind0, rn);
+    y_lines(c, comps, 1);
+  } else {
+    const int lt = lnl_lines_y(g);
+    z_lines(c, comps, 0, kind0, rn);
+    hipLaunchKernelGGL(k_lines_y, dim3((unsigned)((long)g.nxh * g.nz >> lt), comps), dim3(128), lds_lines_y(g.ny, lt), s, g,
+                       c.spec, kind0, rn, c.piv, tstride, c.kx2, c.kz2, lt);
+    z_lines(c, comps, 1, kind0, rn);
+  }
+  x_inverse(c, comps, x);
+}
+
+}  // namespace
+
+// The spectrum holds three components where that is small beside the state
+// (their solves then share launches); one above it, where a component alone
+// fills the device.
+void f64_spectral_create(Ctx& c) {
+  const Grid& g = c.g;
+  const size_t per = (size_t)g.nxh * g.ny * g.nz;
+  c.nspec = per <= ((size_t)1 << 24) ? 3 : 1;
+  FP_HIP_CHECK(hipMalloc((void**)&c.spec, sizeof(double2) * per * c.nspec));
+  int lds_max = 0, dev = 0;
+  FP_HIP_CHECK(hipGetDevice(&dev));
+  FP_HIP_CHECK(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  c.slab64 = lds_slab64(g) <= (size_t)lds_max;
+  allow_lds(k_slab<2, false>, lds_max);
+  allow_lds(k_slab<2, true>, lds_max);
+  allow_lds(k_x_forward<2, 0, false>, lds_max);
+  allow_lds(k_x_forward<2, 1, false>, lds_max);
+  allow_lds(k_x_forward<2, 1, true>, lds_max);
+  allow_lds(k_x_forward<3, 0, false>, lds_max);
+  allow_lds(k_x_forward<3, 1, false>, lds_max);
+  allow_lds(k_x_forward<3, 1, true>, lds_max);
+  allow_lds(k_x_inverse<2>, lds_max);
+  allow_lds(k_x_inverse<3>, lds_max);
+  allow_lds(k_y_lines<2>, lds_max);
+  allow_lds(k_y_lines<3>, lds_max);
+  allow_lds(k_z_lines<2>, lds_max);
+  allow_lds(k_z_lines<3>, lds_max);
+  allow_lds(k_lines_y, lds_max);
+}
+
+void f64_solve(Ctx& c, int kind, const double* q, double* x) { solve(c, kind, 1, q, x, false); }
+
+// the three components' Helmholtz problems: q and x of 3 planes
+void f64_helmholtz(Ctx& c, const double* q, double* x) {
+  if (c.nspec == 3) {
+    solve(c, 0, 3, q, x, false);
+    return;
+  }
+  for (int comp = 0; comp < 3; comp++) solve(c, comp, 1, q + comp * c.g.n, x + comp * c.g.n, false);
+}
+
+// the Poisson equation lap_h x = div_h up / dt
+void f64_poisson(Ctx& c, const double* up, double* x) { solve(c, 3, 1, up, x, true); }
+
+// forward transform of one periodic field into c.spec, wavenumbers m at
+// bitrev(m) in y and z (f64_energy_spectrum)
+void f64_forward(Ctx& c, const double* q) {
+  x_forward(c, 1, q, false);
+  y_lines(c, 1, 0);
+  z_lines(c, 1, 0, 3, 1.0);
+}
+
+}  // namespace fp
