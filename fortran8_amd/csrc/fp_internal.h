@@ -43,6 +43,7 @@ struct Ctx {
   int cur = 0;
   double *fC = nullptr;               // Peterlin factor of the current C
   uint8_t* sel = nullptr;
+  unsigned* sel_count = nullptr;      // FP64 step: selections left to FP64
   double *A0 = nullptr, *T0 = nullptr, *B0 = nullptr, *B = nullptr;  // 3 planes each
   double *Q = nullptr;                // 3 planes: predictor RHS / Ua
   double *Up = nullptr;               // 3 planes: u*
@@ -92,7 +93,7 @@ struct Ctx {
   long mean_count = 0;
 };
 
-// ---- launchers (fp_kernels_f64.hip)
+// ---- launchers (fp_kernels_f64.hip; f64_select: fp_kernels_mixed.hip)
 void f64_select(Ctx& c);
 void f64_cstar_newton(Ctx& c);
 void f64_predictor(Ctx& c);

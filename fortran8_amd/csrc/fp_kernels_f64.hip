@@ -11,32 +11,6 @@ namespace fp {
 static inline int nblk(long n, int t) { return (int)((n + t - 1) / t); }
 
 // ============================================================ FENE-P ======
-// CpxCnx/CpyCny/CpzCnz selection (fenep.f90:169-382) for all three axes of
-// one cell; the chosen candidate per axis is packed in 2 bits.
-template <bool WL>
-__global__ __launch_bounds__(256) void k_select(Grid g, const double* __restrict__ C, uint8_t* __restrict__ sel) {
-  const long L = xcd_cell();
-  if (L >= g.n) return;
-  long m;
-  int i, j, k;
-  band_cell(g, L, m, i, j, k);
-  uint8_t s = 0;
-#pragma unroll 1
-  for (int d = 0; d < 3; d++) {
-    double cm[6], c[6], cp[6];
-    int di = d == 0, dj = d == 1, dk = d == 2;
-#pragma unroll
-    for (int q = 0; q < 6; q++) {
-      const double* Cq = C + q * g.n;
-      cm[q] = ldbw<WL>(Cq, g, i - di, j - dj, k - dk, BC_C);
-      c[q] = Cq[m];
-      cp[q] = ldbw<WL>(Cq, g, i + di, j + dj, k + dk, BC_C);
-    }
-    s |= (uint8_t)(select_d(cm, c, cp) << (2 * d));
-  }
-  sel[m] = s;
-}
-
 // face value of cell a (wrapped) along axis d with its own selection:
 // left (Cp) when left=true, right (Cn) otherwise, component q.
 template <bool WL>
@@ -63,8 +37,9 @@ __global__ __launch_bounds__(128) void k_cstar_newton(Grid g, const double* __re
                                                       const double* __restrict__ U, const double* __restrict__ V,
                                                       const double* __restrict__ W, double* __restrict__ Cn,
                                                       double* __restrict__ fC, int* __restrict__ nitr,
-                                                      double dc, double eps, int itrmax) {
+                                                      unsigned* __restrict__ sel_count, double dc, double eps, int itrmax) {
   const long L = xcd_cell();
+  if (L == 0) *sel_count = 0u;   // for the next step's selection
   if (L >= g.n) return;
   long m;
   int i, j, k;
@@ -612,13 +587,9 @@ int f64_sor(Ctx& c, const double* q, double* phi) {
 }
 
 // ======================================================= per step =========
-void f64_select(Ctx& c) {
-  hipLaunchKernelGGL(c.g.walls ? k_select<true> : k_select<false>, dim3(nblk(c.g.n, 256)), dim3(256), 0, c.stream, c.g, c.C[c.cur], c.sel);
-}
-
 void f64_cstar_newton(Ctx& c) {
   hipLaunchKernelGGL(c.g.walls ? k_cstar_newton<true> : k_cstar_newton<false>, dim3(nblk(c.g.n, 128)), dim3(128), 0, c.stream, c.g, c.C[c.cur], c.sel, c.U, c.V, c.W,
-                     c.C[1 - c.cur], c.fC, c.nitr, c.p.newton_dc, c.p.newton_eps, c.p.newton_itrmax);
+                     c.C[1 - c.cur], c.fC, c.nitr, c.sel_count, c.p.newton_dc, c.p.newton_eps, c.p.newton_itrmax);
   c.cur = 1 - c.cur;
 }
 
