@@ -102,6 +102,19 @@ __device__ __forceinline__ void band_cell(const Grid& g, long L, long& m, int& i
 }
 
 
+// n / d correctly rounded, from y = 1/d correctly rounded: two residual
+// corrections (P. W. Markstein, "Computation of elementary functions on the
+// IBM RISC System/6000 processor", 1990: with q within an ulp of n/d and
+// y = RN(1/d), q + (n - d q) y rounds to RN(n/d)).  The first correction
+// brings n y, whose error can exceed an ulp, within one; the residuals are
+// exact unless |n| is below 2^-960.  Five dependent operations instead of about twelve with a
+// quarter-rate reciprocal among them.  y = 0 gives 0.
+__device__ __forceinline__ double quot(double n, double d, double y) {
+  double q = n * y;
+  q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
+  return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+
 // ---- FENE-P algebra (FP64) ------------------------------------------------
 // Vieta, fenep.f90:425-444
 // The reference formulas below are evaluated exactly as written, also in
@@ -168,11 +181,24 @@ __device__ __forceinline__ int select_d(const double* cm, const double* c, const
   return idx;
 }
 
-// Lyapunov_func, fenep.f90:588-605 (A column-major, already transposed)
-__device__ __forceinline__ void lyap_func_d(const double* A0, const double* b, const double* x, double dt,
-                                            double wi, double lp, double* l) {
-  double f = (lp * lp - 3.0) / (((lp * lp - x[0]) - x[3]) - x[5]);
-  double dg = (1.0 + (f * dt) / wi) / 2.0;
+// Constants of the conformation update: spacings and divisors with their
+// correctly rounded reciprocals (quot), made on the host.
+struct CstarConst {
+  double h[3], ih[3], h2[3], ih2[3], h4[3], ih4[3];   // h, 2h, 4h per axis
+  double wi, iwi, dtwi;                               // dt / wi
+  double L2, L2m3;
+  double dc, dc2, idc2;                               // Jacobian step, 2 dc
+  double eps;
+  int itrmax;
+};
+
+// Lyapunov_func, fenep.f90:588-605 (A column-major, already transposed), for
+// the diagonal shift dg = (1 + f dt / wi) / 2
+__device__ __forceinline__ double lyap_shift_d(const CstarConst& K, double dt, double x0, double x3, double x5) {
+  const double f = K.L2m3 / (((K.L2 - x0) - x3) - x5);
+  return (1.0 + quot(f * dt, K.wi, K.iwi)) / 2.0;
+}
+__device__ __forceinline__ void lyap_func_d(const double* A0, const double* b, const double* x, double dg, double* l) {
   double a11 = A0[0] + dg, a22 = A0[4] + dg, a33 = A0[8] + dg;
   double a21 = A0[1], a31 = A0[2], a12 = A0[3], a32 = A0[5], a13 = A0[6], a23 = A0[7];
   l[0] = ((((a11 + a11) * x[0] + a12 * x[1]) + a13 * x[2]) + a12 * x[1]) + a13 * x[2] - b[0];
@@ -183,12 +209,18 @@ __device__ __forceinline__ void lyap_func_d(const double* A0, const double* b, c
   l[5] = ((((a31 * x[2] + a32 * x[4]) + a31 * x[2]) + a32 * x[4]) + (a33 + a33) * x[5]) - b[5];
 }
 
-// gauss, fenep.f90:608-643, fully unrolled so that row swaps are selects.
+// gauss, fenep.f90:608-643, fully unrolled.  The row swaps are selects, made
+// only where a lane of the wavefront has a larger entry below its diagonal
+// (the shifted operator is diagonally dominant: hardly ever).  A zero pivot
+// makes the solution zero; what is computed past it is discarded.
 __device__ __forceinline__ void gauss6_d(double (&Ah)[6][7], double* x) {
   bool zero = false;
 #pragma unroll
   for (int k = 0; k < 6; k++) {
-    if (!zero) {
+    bool swap = false;
+#pragma unroll
+    for (int r = k + 1; r < 6; r++) swap = swap || fabs(Ah[r][k]) > fabs(Ah[k][k]);
+    if (__any(swap)) {
       int mi = k;
       double ma = fabs(Ah[k][k]);
 #pragma unroll
@@ -196,29 +228,27 @@ __device__ __forceinline__ void gauss6_d(double (&Ah)[6][7], double* x) {
         double v = fabs(Ah[r][k]);
         if (v > ma) { ma = v; mi = r; }
       }
-      if (ma == 0.0) {
-        zero = true;
-      } else {
 #pragma unroll
-        for (int r = k + 1; r < 6; r++) {
-          if (r == mi) {
+      for (int r = k + 1; r < 6; r++) {
+        const bool here = r == mi;
 #pragma unroll
-            for (int c = k; c < 7; c++) { double t = Ah[k][c]; Ah[k][c] = Ah[r][c]; Ah[r][c] = t; }
-          }
+        for (int c = k; c < 7; c++) {
+          const double t = Ah[k][c], u = Ah[r][c];
+          Ah[k][c] = here ? u : t;
+          Ah[r][c] = here ? t : u;
         }
-        double piv = Ah[k][k];
+      }
+    }
+    const double piv = Ah[k][k], y = 1.0 / piv;
+    zero = zero || piv == 0.0;
 #pragma unroll
-        for (int c = k + 1; c < 7; c++) Ah[k][c] = Ah[k][c] / piv;
-        Ah[k][k] = 1.0;
+    for (int c = k + 1; c < 7; c++) Ah[k][c] = quot(Ah[k][c], piv, y);
 #pragma unroll
-        for (int r = 0; r < 6; r++) {
-          if (r != k) {
-            double f = Ah[r][k];
+    for (int r = 0; r < 6; r++) {
+      if (r != k) {
+        double f = Ah[r][k];
 #pragma unroll
-            for (int c = k + 1; c < 7; c++) Ah[r][c] = Ah[r][c] - f * Ah[k][c];
-            Ah[r][k] = 0.0;
-          }
-        }
+        for (int c = k + 1; c < 7; c++) Ah[r][c] = Ah[r][c] - f * Ah[k][c];
       }
     }
   }
@@ -227,26 +257,33 @@ __device__ __forceinline__ void gauss6_d(double (&Ah)[6][7], double* x) {
 }
 
 // Newton of Lyapunov (fenep.f90:554-578) with the central-difference Jacobian.
+// Only the diagonal entries of the iterate move the shift: 7 values of it per
+// iteration, not 13; the entries of the Jacobian that no term of a row makes
+// are the zero differences they were.
 // Returns the iterations taken, itrmax + 1 when the tolerance was not met.
-__device__ __forceinline__ int newton_d(const double* A0, const double* b, double* x, double dt, double wi,
-                                        double lp, double dc, double eps, int itrmax) {
+__device__ __forceinline__ int newton_d(const CstarConst& K, const double* A0, const double* b, double* x, double dt) {
   int itr;
-  for (itr = 1; itr <= itrmax; itr++) {
+  for (itr = 1; itr <= K.itrmax; itr++) {
     double Ah[6][7];
+    const double dg = lyap_shift_d(K, dt, x[0], x[3], x[5]);
 #pragma unroll
     for (int col = 0; col < 6; col++) {
       double x1[6], x2[6], l1[6], l2[6];
 #pragma unroll
       for (int m = 0; m < 6; m++) { x1[m] = x[m]; x2[m] = x[m]; }
-      x1[col] = x1[col] + dc;
-      x2[col] = x2[col] - dc;
-      lyap_func_d(A0, b, x1, dt, wi, lp, l1);
-      lyap_func_d(A0, b, x2, dt, wi, lp, l2);
+      x1[col] = x1[col] + K.dc;
+      x2[col] = x2[col] - K.dc;
+      const bool trace = col == 0 || col == 3 || col == 5;
+      lyap_func_d(A0, b, x1, trace ? lyap_shift_d(K, dt, x1[0], x1[3], x1[5]) : dg, l1);
+      lyap_func_d(A0, b, x2, trace ? lyap_shift_d(K, dt, x2[0], x2[3], x2[5]) : dg, l2);
 #pragma unroll
-      for (int row = 0; row < 6; row++) Ah[row][col] = (l1[row] - l2[row]) / (2.0 * dc);
+      for (int row = 0; row < 6; row++) {
+        const bool none = (col == 1 && row == 5) || (col == 2 && row == 3) || (col == 4 && row == 0);
+        Ah[row][col] = none ? 0.0 : quot(l1[row] - l2[row], K.dc2, K.idc2);
+      }
     }
     double l[6], r[6];
-    lyap_func_d(A0, b, x, dt, wi, lp, l);
+    lyap_func_d(A0, b, x, dg, l);
 #pragma unroll
     for (int m = 0; m < 6; m++) Ah[m][6] = l[m];
     gauss6_d(Ah, r);
@@ -257,7 +294,7 @@ __device__ __forceinline__ int newton_d(const double* A0, const double* b, doubl
     for (int m = 0; m < 6; m++) sr = sr + r[m] * r[m];
 #pragma unroll
     for (int m = 0; m < 6; m++) sx = sx + x[m] * x[m];
-    if (sqrt(sr / sx) < eps) break;
+    if (sqrt(sr / sx) < K.eps) break;
   }
   return itr;
 }

@@ -11,33 +11,53 @@ namespace fp {
 static inline int nblk(long n, int t) { return (int)((n + t - 1) / t); }
 
 // ============================================================ FENE-P ======
-// face value of cell a (wrapped) along axis d with its own selection:
-// left (Cp) when left=true, right (Cn) otherwise, component q.
-template <bool WL>
-__device__ __forceinline__ void face_vals(const Grid& g, const double* __restrict__ C, const uint8_t* __restrict__ sel,
-                                          int d, int i, int j, int k, bool left, double* out) {
-  i = wrapi(i, g.nx); j = wrapi(j, g.ny); k = wrapi(k, g.nz);
-  long m = cidx(g, i, j, k);
-  int l = (sel[m] >> (2 * d)) & 3;
-  int di = d == 0, dj = d == 1, dk = d == 2;
-#pragma unroll
-  for (int q = 0; q < 6; q++) {
-    const double* Cq = C + q * g.n;
-    double c = Cq[m];
-    double cm = l == 3 ? 0.0 : ldbw<WL>(Cq, g, i - di, j - dj, k - dk, BC_C);
-    double cp = l == 3 ? 0.0 : ldbw<WL>(Cq, g, i + di, j + dj, k + dk, BC_C);
-    out[q] = left ? cand_p(l, cm, c, cp) : cand_n(l, cm, c, cp);
+// Value e of an FP64 plane of n values.  Below 2^29 cells through a raw
+// buffer resource (base and size in scalar registers, one 32-bit byte offset
+// per lane); BIG: through 64-bit addresses.
+template <bool BIG>
+__device__ __forceinline__ double ldv(const double* __restrict__ base, long n, unsigned e) {
+  if constexpr (BIG) {
+    return base[e];
+  } else {
+    typedef unsigned v2u __attribute__((ext_vector_type(2)));
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)((unsigned)n * 8u), 0x00020000);
+    return __builtin_bit_cast(double, (v2u)__builtin_amdgcn_raw_buffer_load_b64(r, (int)(e * 8u), 0, 0));
   }
+}
+// offset, in cells, of the neighbour at distance d along an axis of n cells
+// whose stride is 2^ls (periodic)
+__device__ __forceinline__ int wrapped(int a, int d, int n, int ls) { return (int)((unsigned)(((a + d) & (n - 1)) - a) << ls); }
+
+// Coefficients of the candidate faces (cand_p, cand_n) as fma(cp, c, fma(cm,
+// a, z b)): halves and quarters multiply exactly, (3 z)/2 rounds as 1.5 z, and a
+// term that a candidate lacks adds zero, so the value is cand_p's, bit for bit.
+struct FaceCoef {
+  double a, b, c;
+  __device__ __forceinline__ double operator()(double cm, double z, double cp) const {
+    return __builtin_fma(cp, c, __builtin_fma(cm, a, z * b));
+  }
+};
+__device__ __forceinline__ FaceCoef face_p(int l) {
+  return {l == 1 ? 0.5 : (l == 2 ? 0.25 : 0.0), l == 0 ? 1.5 : (l == 1 ? 0.5 : 1.0), l == 0 ? -0.5 : (l == 2 ? -0.25 : 0.0)};
+}
+__device__ __forceinline__ FaceCoef face_n(int l) {
+  return {l == 1 ? -0.5 : (l == 2 ? -0.25 : 0.0), l == 0 ? 0.5 : (l == 1 ? 1.5 : 1.0), l == 0 ? 0.5 : (l == 2 ? 0.25 : 0.0)};
 }
 
 // Cstar (fenep.f90:464-507) + Lyapunov Newton (fenep.f90:518-585) + the
 // Peterlin factor of the new C (f, fenep.f90:510-515, used by polymer_stress).
-template <bool WL>
-__global__ __launch_bounds__(128) void k_cstar_newton(Grid g, const double* __restrict__ C, const uint8_t* __restrict__ sel,
-                                                      const double* __restrict__ U, const double* __restrict__ V,
-                                                      const double* __restrict__ W, double* __restrict__ Cn,
-                                                      double* __restrict__ fC, int* __restrict__ nitr,
-                                                      unsigned* __restrict__ sel_count, double dc, double eps, int itrmax) {
+// The four faces of a cell and axis come from one line of five cells (30 loads an
+// axis; each face with its own loads took 72).  Bound by FP64 issue: the
+// Newton's 6 x 6 elimination and its central-difference Jacobian.  256x128x128
+// between walls: 1420 -> 549 us (quotients by a shared divisor through its
+// reciprocal, row swaps only where a wavefront needs one, 7 shifts a Newton
+// iteration instead of 13, the shared line); 64^3: 85 -> 42 us.
+template <bool WL, bool BIG>
+__global__ __launch_bounds__(128) void k_cstar_newton(Grid g, CstarConst K, const double* __restrict__ C,
+                                                      const uint8_t* __restrict__ sel, const double* __restrict__ U,
+                                                      const double* __restrict__ V, const double* __restrict__ W,
+                                                      double* __restrict__ Cn, double* __restrict__ fC, int* __restrict__ nitr,
+                                                      unsigned* __restrict__ sel_count) {
   const long L = xcd_cell();
   if (L == 0) *sel_count = 0u;   // for the next step's selection
   if (L >= g.n) return;
@@ -45,30 +65,56 @@ __global__ __launch_bounds__(128) void k_cstar_newton(Grid g, const double* __re
   int i, j, k;
   band_cell(g, L, m, i, j, k);
   const double dt = g.dt;
-  double cx[6];
+  const unsigned mu = (unsigned)m;
+  const int lz = g.lnx + g.lny;
+  const int xm = wrapped(i, -1, g.nx, 0), xp = wrapped(i, 1, g.nx, 0);
+  const int ym = wrapped(j, -1, g.ny, g.lnx), yp = wrapped(j, 1, g.ny, g.lnx);
+  const int zm = wrapped(k, -1, g.nz, lz), zp = wrapped(k, 1, g.nz, lz);
+  const bool wlo = WL && j == 0, whi = WL && j == g.ny - 1;
+#define LD(F, o) ldv<BIG>(F, g.n, mu + (unsigned)(o))
+  double cx[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll 1
   for (int d = 0; d < 3; d++) {
-    double h = d == 0 ? g.dx : (d == 1 ? g.dy : g.dz);
     double v1, v2;
-    if (d == 0) { v1 = ldbw<WL>(U, g, i - 1, j, k, BC_U); v2 = U[m]; }
-    else if (d == 1) { v1 = ldbw<WL>(V, g, i, j - 1, k, BC_V); v2 = ldbw<WL>(V, g, i, j, k, BC_V); }
-    else { v1 = ldbw<WL>(W, g, i, j, k - 1, BC_W); v2 = W[m]; }
-    double s1 = ((-v2 + fabs(v2)) * dt) / (2.0 * h);
-    double s2 = 1.0 / 6.0 + ((-v2 - fabs(v2)) * dt) / (2.0 * h);
-    double s3 = 1.0 / 6.0 + ((v1 - fabs(v1)) * dt) / (2.0 * h);
-    double s4 = ((v1 + fabs(v1)) * dt) / (2.0 * h);
-    int di = d == 0, dj = d == 1, dk = d == 2;
-    double pl[6], pr[6], nl[6], nr[6];
-    face_vals<WL>(g, C, sel, d, i, j, k, true, pl);                    // Cp(a-1): own left face
-    face_vals<WL>(g, C, sel, d, i + di, j + dj, k + dk, true, pr);     // Cp(a): left face of a+1
-    face_vals<WL>(g, C, sel, d, i - di, j - dj, k - dk, false, nl);    // Cn(a-1): right face of a-1
-    face_vals<WL>(g, C, sel, d, i, j, k, false, nr);                   // Cn(a): own right face
+    if (d == 0) { v1 = LD(U, xm); v2 = LD(U, 0); }
+    else if (d == 1) { v1 = wlo ? 0.0 : LD(V, ym); v2 = whi ? 0.0 : LD(V, 0); }   // V_kabe
+    else { v1 = LD(W, zm); v2 = LD(W, 0); }
+    const double h2 = K.h2[d], ih2 = K.ih2[d];
+    const double s1 = quot((-v2 + fabs(v2)) * dt, h2, ih2);
+    const double s2 = 1.0 / 6.0 + quot((-v2 - fabs(v2)) * dt, h2, ih2);
+    const double s3 = 1.0 / 6.0 + quot((v1 - fabs(v1)) * dt, h2, ih2);
+    const double s4 = quot((v1 + fabs(v1)) * dt, h2, ih2);
+    const int a = d == 0 ? i : (d == 1 ? j : k), na = d == 0 ? g.nx : (d == 1 ? g.ny : g.nz);
+    const int ls = d == 0 ? 0 : (d == 1 ? g.lnx : lz);
+    const int om = wrapped(a, -1, na, ls), op = wrapped(a, 1, na, ls);
+    const unsigned e[5] = {mu + (unsigned)wrapped(a, -2, na, ls), mu + (unsigned)om, mu, mu + (unsigned)op,
+                           mu + (unsigned)wrapped(a, 2, na, ls)};
+    const int lm = (sel[mu + (unsigned)om] >> (2 * d)) & 3, l0 = (sel[mu] >> (2 * d)) & 3,
+              lp = (sel[mu + (unsigned)op] >> (2 * d)) & 3;
+    const FaceCoef pl = face_p(l0), pr = face_p(lp), nl = face_n(lm), nr = face_n(l0);
+    double v[6][5];
+#pragma unroll
+    for (int q = 0; q < 6; q++)
+#pragma unroll
+      for (int o = 0; o < 5; o++) v[q][o] = ldv<BIG>(C + q * g.n, g.n, e[o]);
+    // the ghost rows (C_kabe): 2 C_0 - C_1; a point beyond them only feeds
+    // faces whose weight is zero (a wavefront shares its row where nx >= 64)
+    if (WL && d == 1 && (j < 2 || j >= g.ny - 2)) {
+      const bool i0 = j == 0, i1 = j == 1, h1 = j == g.ny - 2, h0 = j == g.ny - 1;
+#pragma unroll
+      for (int q = 0; q < 6; q++) {
+        v[q][1] = i0 ? 2.0 * v[q][2] - v[q][3] : v[q][1];
+        v[q][0] = i0 ? v[q][2] : (i1 ? 2.0 * v[q][1] - v[q][2] : v[q][0]);
+        v[q][3] = h0 ? 2.0 * v[q][2] - v[q][1] : v[q][3];
+        v[q][4] = h0 ? v[q][2] : (h1 ? 2.0 * v[q][3] - v[q][2] : v[q][4]);
+      }
+    }
 #pragma unroll
     for (int q = 0; q < 6; q++) {
-      double acc = d == 0 ? s3 * pl[q] : cx[q] + s3 * pl[q];
-      acc = acc + s1 * pr[q];
-      acc = acc + s4 * nl[q];
-      acc = acc + s2 * nr[q];
+      double acc = cx[q] + s3 * pl(v[q][1], v[q][2], v[q][3]);   // Cp(a-1): own left face
+      acc = acc + s1 * pr(v[q][2], v[q][3], v[q][4]);            // Cp(a): left face of a+1
+      acc = acc + s4 * nl(v[q][0], v[q][1], v[q][2]);            // Cn(a-1): right face of a-1
+      acc = acc + s2 * nr(v[q][1], v[q][2], v[q][3]);            // Cn(a): own right face
       cx[q] = acc;
     }
   }
@@ -76,34 +122,45 @@ __global__ __launch_bounds__(128) void k_cstar_newton(Grid g, const double* __re
   double b[6];
 #pragma unroll
   for (int q = 0; q < 6; q++) b[q] = cx[q];
-  b[0] = b[0] + dt / g.wi;
-  b[3] = b[3] + dt / g.wi;
-  b[5] = b[5] + dt / g.wi;
-  const double dx = g.dx, dy = g.dy, dz = g.dz;
-#define UL(a, bb, c) ldbw<WL>(U, g, a, bb, c, BC_U)
-#define VL(a, bb, c) ldbw<WL>(V, g, a, bb, c, BC_V)
-#define WL(a, bb, c) ldbw<WL>(W, g, a, bb, c, BC_W)
-  double a11 = -((dt * (-UL(i - 1, j, k) + UL(i, j, k))) / dx);
-  double a12 = -((dt * (((-VL(i - 1, j - 1, k) + VL(i + 1, j - 1, k)) - VL(i - 1, j, k)) + VL(i + 1, j, k))) / (4.0 * dx));
-  double a13 = -((dt * (((-WL(i - 1, j, k - 1) + WL(i + 1, j, k - 1)) - WL(i - 1, j, k)) + WL(i + 1, j, k))) / (4.0 * dx));
-  double a21 = -((dt * (((-UL(i - 1, j - 1, k) - UL(i, j - 1, k)) + UL(i - 1, j + 1, k)) + UL(i, j + 1, k))) / (4.0 * dy));
-  double a22 = -((dt * (-VL(i, j - 1, k) + VL(i, j, k))) / dy);
-  double a23 = -((dt * (((-WL(i, j - 1, k - 1) + WL(i, j + 1, k - 1)) - WL(i, j - 1, k)) + WL(i, j + 1, k))) / (4.0 * dy));
-  double a31 = -((dt * (((-UL(i - 1, j, k - 1) - UL(i, j, k - 1)) + UL(i - 1, j, k + 1)) + UL(i, j, k + 1))) / (4.0 * dz));
-  double a32 = -((dt * (((-VL(i, j - 1, k - 1) - VL(i, j, k - 1)) + VL(i, j - 1, k + 1)) + VL(i, j, k + 1))) / (4.0 * dz));
-  double a33 = -((dt * (-WL(i, j, k - 1) + WL(i, j, k))) / dz);
+  b[0] = b[0] + K.dtwi;
+  b[3] = b[3] + K.dtwi;
+  b[5] = b[5] + K.dtwi;
+  // the boundary rules (U_kabe, V_kabe, W_kabe) at the reads that reach a ghost
+  // row or the wall face of V; B the row -1, 0, 1 of the read
+#define UL(a, B, c) uw(U, a, B, c)
+#define VL(a, B, c) vw(a, B, c)
+#define WV(a, B, c) uw(W, a, B, c)
+  auto row = [&](int B) { return B < 0 ? ym : (B > 0 ? yp : 0); };
+  auto uw = [&](const double* F, int a, int B, int c) {
+    const double x = LD(F, a + ((B < 0 && wlo) || (B > 0 && whi) ? 0 : row(B)) + c);
+    return B < 0 && wlo ? -x : (B > 0 && whi ? 2.0 * 0.0 - x : x);
+  };
+  auto vw = [&](int a, int B, int c) {
+    const double x = LD(V, a + row(B) + c);
+    return (B < 0 && wlo) || (B == 0 && whi) ? 0.0 : x;
+  };
+  double a11 = -quot(dt * (-UL(xm, 0, 0) + UL(0, 0, 0)), K.h[0], K.ih[0]);
+  double a12 = -quot(dt * (((-VL(xm, -1, 0) + VL(xp, -1, 0)) - VL(xm, 0, 0)) + VL(xp, 0, 0)), K.h4[0], K.ih4[0]);
+  double a13 = -quot(dt * (((-WV(xm, 0, zm) + WV(xp, 0, zm)) - WV(xm, 0, 0)) + WV(xp, 0, 0)), K.h4[0], K.ih4[0]);
+  double a21 = -quot(dt * (((-UL(xm, -1, 0) - UL(0, -1, 0)) + UL(xm, 1, 0)) + UL(0, 1, 0)), K.h4[1], K.ih4[1]);
+  double a22 = -quot(dt * (-VL(0, -1, 0) + VL(0, 0, 0)), K.h[1], K.ih[1]);
+  double a23 = -quot(dt * (((-WV(0, -1, zm) + WV(0, 1, zm)) - WV(0, -1, 0)) + WV(0, 1, 0)), K.h4[1], K.ih4[1]);
+  double a31 = -quot(dt * (((-UL(xm, 0, zm) - UL(0, 0, zm)) + UL(xm, 0, zp)) + UL(0, 0, zp)), K.h4[2], K.ih4[2]);
+  double a32 = -quot(dt * (((-VL(0, -1, zm) - VL(0, 0, zm)) + VL(0, -1, zp)) + VL(0, 0, zp)), K.h4[2], K.ih4[2]);
+  double a33 = -quot(dt * (-WV(0, 0, zm) + WV(0, 0, 0)), K.h[2], K.ih[2]);
 #undef UL
 #undef VL
-#undef WL
+#undef WV
   double A[9] = {a11, a12, a13, a21, a22, a23, a31, a32, a33};  // transpose(A0), column-major
   double x[6];
 #pragma unroll
-  for (int q = 0; q < 6; q++) x[q] = C[q * g.n + m];
-  const int it = newton_d(A, b, x, dt, g.wi, g.lp, dc, eps, itrmax);
+  for (int q = 0; q < 6; q++) x[q] = ldv<BIG>(C + q * g.n, g.n, mu);
+#undef LD
+  const int it = newton_d(K, A, b, x, dt);
 #pragma unroll
   for (int q = 0; q < 6; q++) Cn[q * g.n + m] = x[q];
   fC[m] = peterlin_d(g.lp, x[0], x[3], x[5]);
-  nitr[m] = it > itrmax ? -itrmax : it;   // negative: stopped at the cap
+  nitr[m] = it > K.itrmax ? -K.itrmax : it;   // negative: stopped at the cap
 }
 
 // ========================================================= predictor ======
@@ -588,8 +645,23 @@ int f64_sor(Ctx& c, const double* q, double* phi) {
 
 // ======================================================= per step =========
 void f64_cstar_newton(Ctx& c) {
-  hipLaunchKernelGGL(c.g.walls ? k_cstar_newton<true> : k_cstar_newton<false>, dim3(nblk(c.g.n, 128)), dim3(128), 0, c.stream, c.g, c.C[c.cur], c.sel, c.U, c.V, c.W,
-                     c.C[1 - c.cur], c.fC, c.nitr, c.sel_count, c.p.newton_dc, c.p.newton_eps, c.p.newton_itrmax);
+  const Grid& g = c.g;
+  CstarConst K{};
+  const double h[3] = {g.dx, g.dy, g.dz};
+  for (int d = 0; d < 3; d++) {
+    K.h[d] = h[d]; K.ih[d] = 1.0 / K.h[d];
+    K.h2[d] = 2.0 * h[d]; K.ih2[d] = 1.0 / K.h2[d];
+    K.h4[d] = 4.0 * h[d]; K.ih4[d] = 1.0 / K.h4[d];
+  }
+  K.wi = g.wi; K.iwi = 1.0 / g.wi; K.dtwi = g.dt / g.wi;
+  K.L2 = g.lp * g.lp; K.L2m3 = K.L2 - 3.0;
+  K.dc = c.p.newton_dc; K.dc2 = 2.0 * K.dc; K.idc2 = 1.0 / K.dc2;
+  K.eps = c.p.newton_eps; K.itrmax = c.p.newton_itrmax;
+  const bool big = g.n >= (1L << 29);
+  auto kern = g.walls ? (big ? k_cstar_newton<true, true> : k_cstar_newton<true, false>)
+                      : (big ? k_cstar_newton<false, true> : k_cstar_newton<false, false>);
+  hipLaunchKernelGGL(kern, dim3(nblk(g.n, 128)), dim3(128), 0, c.stream, g, K, c.C[c.cur], c.sel, c.U, c.V, c.W,
+                     c.C[1 - c.cur], c.fC, c.nitr, c.sel_count);
   c.cur = 1 - c.cur;
 }
 

@@ -33,19 +33,6 @@ namespace fp {
 
 namespace {
 
-// n / d correctly rounded, from y = 1/d correctly rounded: two residual
-// corrections (P. W. Markstein, "Computation of elementary functions on the
-// IBM RISC System/6000 processor", 1990: with q within an ulp of n/d and
-// y = RN(1/d), q + (n - d q) y rounds to RN(n/d)).  The first correction
-// brings n y, whose error can exceed an ulp, within one; the residuals are
-// exact unless |n| is below 2^-960.  Five dependent operations instead of about twelve with a
-// quarter-rate reciprocal among them.  y = 0 gives 0.
-__device__ __forceinline__ double quot(double n, double d, double y) {
-  double q = n * y;
-  q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
-  return __builtin_fma(__builtin_fma(-d, q, n), y, q);
-}
-
 __device__ __forceinline__ int brev(int v, int bits) { return bits ? (int)(__brev((unsigned)v) >> (32 - bits)) : 0; }
 
 // one radix-2 butterfly of the Stockham form: (a, b) -> (a + b, (a - b) w)
