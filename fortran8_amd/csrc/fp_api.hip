@@ -245,6 +245,7 @@ int fp_create(const fp_params* p, void** out) {
     up1(&c->kx2, modwav(g.nx, g.dx, g.nxh)); up1(&c->ky2, modwav(g.ny, g.dy, g.ny)); up1(&c->kz2, modwav(g.nz, g.dz, g.nz));
     c->gn = (long)(g.nx + 2) * (g.ny + 2) * (g.nz + 2);
     if (p->precision == FP_PREC_MIXED) mixed_create(*c);
+    else if (p->poisson_variant == FP_POISSON_SOR) f64_sor_create(*c);
     FP_HIP_CHECK(hipDeviceSynchronize());
   } catch (const std::string& e) {
     fp_destroy(c);
@@ -265,6 +266,7 @@ int fp_destroy(void* vc) {
   for (auto e : c->evpool) (void)hipEventDestroy(e);
   if (c->mixed) mixed_destroy(*c);
   adj_free(*c);
+  f64_sor_destroy(*c);
   dfree(c->U); dfree(c->V); dfree(c->W); dfree(c->P); dfree(c->Phi);
   dfree(c->C[0]); dfree(c->C[1]); dfree(c->fC); dfree(c->sel); dfree(c->sel_count); dfree(c->nitr);
   dfree(c->A0); dfree(c->T0); dfree(c->B0); dfree(c->B); dfree(c->Q); dfree(c->Up); dfree(c->F);

@@ -74,6 +74,10 @@ struct Ctx {
   double* ib_w = nullptr;             // interpolation weights, (3 nmk) x 27 stencil points
   // SOR
   double sor_itr = -1.0;
+  double* sor_part = nullptr;         // sums of E^2 per sweep of a batch and block
+  int* sor_flag = nullptr;
+  int* sor_host = nullptr;            // pinned copy of the flags
+  hipEvent_t sor_ev[2] = {nullptr, nullptr};
   // timing: recorded (name, event) pairs and a pool of created events, so
   // that timed steps do not create or destroy events
   std::vector<std::pair<std::string, hipEvent_t>> ev;
@@ -101,6 +105,8 @@ void f64_divergence(Ctx& c, const double* up, double* q);
 void f64_march(Ctx& c);
 void f64_ibm(Ctx& c);        // interp + forces + spread + predictor RHS into Q
 void f64_ibm_setup(Ctx& c);  // CSR build (host) after markers are set
+void f64_sor_create(Ctx& c);
+void f64_sor_destroy(Ctx& c);
 int  f64_sor(Ctx& c, const double* q, double* phi);
 void f64_zero_c(Ctx& c);
 void f64_diag(Ctx& c, fp_diag* d, double* scratch, const double* mf);  // scratch: diag_scratch_words

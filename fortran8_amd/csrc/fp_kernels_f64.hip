@@ -2,6 +2,7 @@
 // Compiled with -ffp-contract=off: every expression is evaluated in the
 // order written, which is the order of the reference statement it restates.
 #include "fp_device.h"
+#include "fp_sor.h"
 #include <algorithm>
 #include <map>
 #include <cmath>
@@ -571,7 +572,9 @@ void f64_ibm_setup(Ctx& c) {
 // converged solution is the same to the solver tolerance).  Residuals are
 // taken before each update, as E in the reference.
 __global__ __launch_bounds__(256) void k_sor_color(Grid g, int color, double om, const double* __restrict__ q,
-                                                   double* __restrict__ phi, double* __restrict__ e2) {
+                                                   double* __restrict__ phi, double* __restrict__ e2,
+                                                   const int* __restrict__ stop) {
+  if (*stop) return;
   long h = blockIdx.x * (long)blockDim.x + threadIdx.x;
   long half = g.n / 2;
   double e = 0.0;
@@ -604,43 +607,99 @@ __global__ __launch_bounds__(256) void k_sumsq(long n, const double* __restrict_
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-__global__ void k_zero_n(double* p, int n) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = 0.0;
+constexpr int SOR_CHECK = 10;   // the residuals are looked at every so many sweeps
+
+// flag[0] stop, [1] sweeps up to the first that met the test, [2] batches of
+// SOR_CHECK sweeps made; host: their copy in pinned memory, once stopped.
+// mode 0: er0 = sum Q^2, flags cleared (stop at once when Q = 0); mode 1: the
+// residual sums of a batch of `rows` sweeps, `nb` partials each
+__global__ __launch_bounds__(1024) void k_sor_decide(const double* __restrict__ part, int nb, int rows, double* __restrict__ er0,
+                                                     double eps, int mode, int* __restrict__ flag, volatile int* host) {
+  if (mode == 1 && flag[0]) return;
+  __shared__ double res[SOR_CHECK];
+  sor_row_sums(part, nb, rows, res);
+  if (threadIdx.x != 0) return;
+  if (mode == 0) {
+    *er0 = res[0];
+    flag[0] = res[0] == 0.0 ? 1 : 0;
+    flag[1] = flag[2] = 0;
+  } else {
+    flag[2]++;
+    for (int r = 0; r < rows && !flag[0]; r++) {
+      flag[1]++;
+      if (sqrt(res[r] / *er0) < eps) flag[0] = 1;
+    }
+  }
+  // (a store across the bus costs microseconds: only what the host waits for)
+  if (mode == 0 || flag[0]) {
+    host[1] = flag[1];
+    host[2] = flag[2];
+    __threadfence_system();
+    host[0] = flag[0];
+  }
 }
 
+void f64_sor_create(Ctx& c) {
+  const SorPlan<double> p = sor_plan<double>(c.g);
+  const long nb = std::max(p.blocks, (long)nblk(c.g.n / 2, 256));
+  FP_HIP_CHECK(hipMalloc((void**)&c.sor_part, sizeof(double) * SOR_CHECK * nb));
+  FP_HIP_CHECK(hipMalloc((void**)&c.sor_flag, sizeof(int) * 4));
+  FP_HIP_CHECK(hipHostMalloc((void**)&c.sor_host, 4 * sizeof(int), hipHostMallocDefault));
+  for (int e = 0; e < 2; e++) FP_HIP_CHECK(hipEventCreateWithFlags(&c.sor_ev[e], hipEventDisableTiming));
+}
+void f64_sor_destroy(Ctx& c) {
+  (void)hipFree(c.sor_part); (void)hipFree(c.sor_flag);
+  if (c.sor_host) (void)hipHostFree(c.sor_host);
+  for (int e = 0; e < 2; e++)
+    if (c.sor_ev[e]) (void)hipEventDestroy(c.sor_ev[e]);
+}
+
+// Sweeps in batches of SOR_CHECK; every batch is enqueued before the host waits
+// for the flags of the one before it (its launches end at once if that one
+// stopped), so the device does not wait for the host.  The second array of the
+// tiles is the previous C, which nothing reads after CStar.
 int f64_sor(Ctx& c, const double* q, double* phi) {
   const Grid& g = c.g;
   hipStream_t s = c.stream;
-  double om = c.p.sor_omega > 0.0 ? c.p.sor_omega : 2.0 / (1.0 + sin(3.14159265358979323846 * g.dx));
-  const int check = 10;  // residual read back every `check` sweeps
-  double* red = c.red;   // [0] = er0, [1 + s] = residual of sweep s
-  double* part = c.part; // per-block partial sums
-  hipLaunchKernelGGL(k_sumsq, dim3(nblk(g.n, 256)), dim3(256), 0, s, g.n, q, part);
-  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, part, nblk(g.n, 256), red, 0);
-  double er0 = 0.0;
-  FP_HIP_CHECK(hipMemcpyAsync(&er0, red, sizeof(double), hipMemcpyDeviceToHost, s));
-  FP_HIP_CHECK(hipStreamSynchronize(s));
-  if (er0 == 0.0) return 0;
-  long half = g.n / 2;
-  const int nbh = nblk(half, 256);
-  int itr = 0;
-  std::vector<double> res(check);
-  while (itr < c.p.sor_itrmax) {
-    int batch = std::min(check, c.p.sor_itrmax - itr);
-    for (int b = 0; b < batch; b++) {
-      hipLaunchKernelGGL(k_sor_color, dim3(nbh), dim3(256), 0, s, g, 0, om, q, phi, part);
-      hipLaunchKernelGGL(k_sor_color, dim3(nbh), dim3(256), 0, s, g, 1, om, q, phi, part);
-      hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, part, nbh, red + 1 + b, 0);
+  const double om = c.p.sor_omega > 0.0 ? c.p.sor_omega : 2.0 / (1.0 + sin(3.14159265358979323846 * g.dx));
+  const SorPlan<double> plan = sor_plan<double>(g);
+  const int nbh = nblk(g.n / 2, 256), nb = plan.k ? (int)plan.blocks : nbh;
+  double* const buf[2] = {phi, c.C[1 - c.cur]};
+  SorCoef<double> co;
+  co.bx = 1.0 / (g.dx * g.dx); co.by = 1.0 / (g.dy * g.dy); co.bz = 1.0 / (g.dz * g.dz);
+  co.b0 = ((((co.bx + co.bx) + co.by) + co.by) + co.bz) + co.bz;
+  co.om = om; co.ib0 = 1.0 / co.b0;
+  volatile int* h = c.sor_host;
+  hipLaunchKernelGGL(k_sumsq, dim3(nblk(g.n, 256)), dim3(256), 0, s, g.n, q, c.part);
+  hipLaunchKernelGGL(k_sor_decide, dim3(1), dim3(1024), 0, s, c.part, nblk(g.n, 256), 1, c.red, c.p.sor_eps, 0, c.sor_flag,
+                     c.sor_host);
+  std::vector<int> launches;   // made up to the end of each batch
+  int at = 0, sweeps = 0;
+  while (sweeps < c.p.sor_itrmax) {
+    const int b = (int)launches.size(), batch = std::min(SOR_CHECK, c.p.sor_itrmax - sweeps);
+    if (plan.k) {
+      double* const from[2] = {buf[at & 1], buf[(at + 1) & 1]};
+      at += sor_launch<double>(g, plan, co, q, from, c.sor_part, batch, false, c.sor_flag, s);
+    } else {
+      for (int r = 0; r < batch; r++)
+        for (int color = 0; color < 2; color++)
+          hipLaunchKernelGGL(k_sor_color, dim3(nbh), dim3(256), 0, s, g, color, om, q, phi, c.sor_part + (long)r * nbh, c.sor_flag);
     }
-    FP_HIP_CHECK(hipMemcpyAsync(res.data(), red + 1, sizeof(double) * batch, hipMemcpyDeviceToHost, s));
-    FP_HIP_CHECK(hipStreamSynchronize(s));
-    for (int b = 0; b < batch; b++) {
-      itr++;
-      if (std::sqrt(res[b] / er0) < c.p.sor_eps) return itr;
-    }
+    sweeps += batch;
+    launches.push_back(at);
+    hipLaunchKernelGGL(k_sor_decide, dim3(1), dim3(1024), 0, s, c.sor_part, nb, batch, c.red, c.p.sor_eps, 1, c.sor_flag,
+                       c.sor_host);
+    FP_HIP_CHECK(hipEventRecord(c.sor_ev[b & 1], s));
+    if (b > 0) FP_HIP_CHECK(hipEventSynchronize(c.sor_ev[(b - 1) & 1]));
+    if (b > 0 && h[0]) break;
   }
-  return itr;
+  if (launches.empty()) return 0;
+  FP_HIP_CHECK(hipEventSynchronize(c.sor_ev[(launches.size() - 1) & 1]));
+  // the batches that ran: up to the stop, or all
+  const int ran = h[0] ? h[2] : (int)launches.size();
+  if (ran > 0 && (launches[ran - 1] & 1))
+    FP_HIP_CHECK(hipMemcpyAsync(phi, buf[1], sizeof(double) * g.n, hipMemcpyDeviceToDevice, s));
+  return h[0] ? h[1] : sweeps;
 }
 
 // ======================================================= per step =========

@@ -14,6 +14,7 @@
 // carry no information in FP32 (fenep.f90:558-568 uses dc = 1e-5).
 #include "fp_mixed.h"
 #include "fp_device.h"
+#include "fp_sor.h"
 #include <algorithm>
 #include <cmath>
 #include <map>
@@ -47,8 +48,10 @@ struct Mixed {
   float* r32 = nullptr;
   float* e32 = nullptr;           // SOR: the FP32 correction e
   double* sor_pb = nullptr;       // SOR: per-block |b|^2
-  int* sor_flag = nullptr;        // SOR: converged, sweeps, FP64 check (m_sor_decide)
+  double* sor_part = nullptr;     // SOR: sums of E^2 per sweep of a batch and block
+  int* sor_flag = nullptr;        // SOR: m_sor_decide
   int* sor_host = nullptr;        // pinned copy of sor_flag
+  hipEvent_t sor_ev[2] = {nullptr, nullptr};
   double* red = nullptr;          // [0]=|b|^2, [1]=|r|^2 of the last sweep
   double* part = nullptr;         // per-block partial sums
   int* skip = nullptr;            // defect correction converged: skip the sweep
@@ -2233,16 +2236,25 @@ __global__ __launch_bounds__(1024) void m_sum_decide(const double* __restrict__ 
 // the defect is taken again; once the sweeps stop, the FP64 residual of the
 // new phi is held to the same tolerance, and sweeps go on if it is not met.
 //
-// flag[0]: converged (sweeps return at once), flag[1]: sweeps counted as the
-// reference counts them, flag[2]: the FP64 check passed.
+// Sweeps are made in batches, one to a launch (fp_sor.h), and their residuals
+// looked at after the batch.  A batch that met the test before its end is made
+// again up to that sweep: it starts from e = 0 and r, which it does not
+// change.
+//
+// flag[0]: stop, what is enqueued returns at once; [1]: sweeps counted as the
+// reference counts them; [2]: the FP64 check passed; [3]: sweeps of the batch
+// to make again (0: none); [4]: the last sweep met the test, the FP64 check is
+// due; [5]: batches whose correction went into phi; [6]: sweeps made.  The copy
+// in pinned host memory is written at a stop and at the end, the stop last.
+constexpr int SOR_FLAGS = 7;
 
-// b (FP64), r = b - L_h phi (FP64, stored in FP32), e = 0, per-block |b|^2
+// b (FP64), r = b - L_h phi (FP64, stored in FP32), per-block |b|^2
 template <bool WL>
 __global__ __launch_bounds__(256) void m_sor_start(Grid g, const float* __restrict__ U, const float* __restrict__ V,
                                                    const float* __restrict__ W, const float* __restrict__ up,
                                                    const double* __restrict__ phi,
                                                    double* __restrict__ b, float* __restrict__ r32,
-                                                   float* __restrict__ e, double* __restrict__ pb) {
+                                                   double* __restrict__ pb) {
   const long m = xcd_cell();
   double bb = 0.0;
   if (m < g.n) {
@@ -2258,7 +2270,6 @@ __global__ __launch_bounds__(256) void m_sor_start(Grid g, const float* __restri
 #undef PH
     b[m] = bb;
     r32[m] = (float)(bb - lap);
-    e[m] = 0.0f;
   }
   __shared__ double sh[256];
   const double sum = block_sum256(bb * bb, sh);
@@ -2305,42 +2316,92 @@ __device__ __forceinline__ double sum_partials1024(const double* __restrict__ p,
   return sh[0];
 }
 
-// mode 0 (after m_sor_start): red[0] = sum Q^2, flags cleared (converged at
-// once when Q = 0).  mode 1 (after a sweep): count the sweep and test it.
-// mode 2 (after the FP64 residual of phi + e, only once the sweeps have met
-// the test): red[1] = |b - L_h phi|^2, flag[2] = the FP64 test; the sweeps
-// resume when it fails.
-__global__ __launch_bounds__(1024) void m_sor_decide(const double* __restrict__ part, int nb, double* __restrict__ red,
-                                                     double eps, int mode, int* __restrict__ flag) {
-  if (mode == 2 && !flag[0]) return;   // the same for every thread
+// mode 0 (after m_sor_start): red[0] = sum Q^2, flags cleared (stop at once
+// when Q = 0).  mode 1 (after a batch of `rows` sweeps): the FP64 check of the
+// batch before, if due (|b - L_h phi|^2 from the `nr` partials `pr` of the
+// defect; the batch just made is dropped when it passes); else count the
+// sweeps and find the first that met the test.  mode 2: the FP64 check alone.
+constexpr int SOR_BATCH = 10;
+__global__ __launch_bounds__(1024) void m_sor_decide(const double* __restrict__ part, int nb, int rows,
+                                                     const double* __restrict__ pr, int nr, double* __restrict__ red,
+                                                     double eps, int mode, int* __restrict__ flag, volatile int* host) {
+  // (the same for every thread)
+  if (mode != 0 && flag[0]) return;
   __shared__ double sh[1024];
-  const double sum = sum_partials1024(part, nb, sh);
+  __shared__ double res[SOR_BATCH];
+  const bool check = mode != 0 && flag[4];
+  double defect = 0.0;
+  if (check) {
+    defect = sum_partials1024(pr, nr, sh);
+    __syncthreads();
+  }
+  if (mode != 2) sor_row_sums(part, nb, rows, res);
   if (threadIdx.x != 0) return;
   if (mode == 0) {
-    red[0] = sum;
-    flag[0] = sum == 0.0 ? 1 : 0;
-    flag[1] = 0;
-    flag[2] = 0;
-  } else if (mode == 1) {
-    if (!flag[0]) {
-      flag[1] += 1;
-      if (sqrt(sum / red[0]) < eps) flag[0] = 1;
-    }
+    red[0] = res[0];
+    for (int f = 1; f < SOR_FLAGS; f++) flag[f] = 0;
+    flag[0] = res[0] == 0.0 ? 1 : 0;
   } else {
-    red[1] = sum;
-    const int ok = red[0] == 0.0 || sqrt(sum / red[0]) < eps;
-    flag[2] = ok;
-    flag[0] = ok;
+    if (check) {
+      red[1] = defect;
+      flag[2] = sqrt(defect / red[0]) < eps;
+      flag[0] = flag[2];
+      flag[4] = 0;
+    }
+    if (mode == 1 && !flag[0]) {
+      flag[6] += rows;
+      for (int r = 0; r < rows; r++) {
+        flag[1] += 1;
+        if (sqrt(res[r] / red[0]) < eps) {
+          if (r == rows - 1) flag[4] = 1;
+          else flag[0] = 1, flag[3] = r + 1;
+          break;
+        }
+      }
+      if (!flag[0]) flag[5] += 1;
+    }
+  }
+  // (a store across the bus costs microseconds: only what the host waits for)
+  if (mode != 1 || flag[0]) {
+    for (int f = 1; f < SOR_FLAGS; f++) host[f] = flag[f];
+    __threadfence_system();
+    host[0] = flag[0];
   }
 }
+// the batch that stopped is made again: its sweeps, already counted, end at
+// the one that met the test
+__global__ void m_sor_again(int* __restrict__ flag) {
+  flag[0] = flag[3] = 0;
+  flag[4] = 1;
+  flag[5] += 1;
+}
 
-// phi += e (FP64), e = 0
-__global__ __launch_bounds__(256) void m_sor_accum(long n, double* __restrict__ phi, float* __restrict__ e) {
-  const long m = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (m < n) {
-    phi[m] += (double)e[m];
-    e[m] = 0.0f;
+// phi_out = phi + e and its defect r = b - L_h phi_out (FP64, stored in FP32),
+// per-block |r|^2: m_residual on the new phi, formed here from phi and e
+template <bool WL>
+__global__ __launch_bounds__(256) void m_sor_settle(Grid g, const double* __restrict__ b, const double* __restrict__ phi,
+                                                    const float* __restrict__ e, double* __restrict__ phi_out,
+                                                    float* __restrict__ r32, double* __restrict__ nrm,
+                                                    const int* __restrict__ stop) {
+  if (*stop) return;
+  const long m = xcd_cell();
+  double r = 0.0;
+  if (m < g.n) {
+    int i, j, k;
+    cell_ijk(g, m, i, j, k);
+    const double p = phi[m] + (double)e[m];
+#define PH(a, bb, c) (ldbw<WL>(phi, g, a, bb, c, BC_P) + (double)ldbw<WL>(e, g, a, bb, c, BC_P))
+    const double lap = (PH(i - 1, j, k) - 2.0 * p + PH(i + 1, j, k)) / (g.dx * g.dx) +
+                       (PH(i, j - 1, k) - 2.0 * p + PH(i, j + 1, k)) / (g.dy * g.dy) +
+                       (PH(i, j, k - 1) - 2.0 * p + PH(i, j, k + 1)) / (g.dz * g.dz);
+#undef PH
+    r = b[m] - lap;
+    phi_out[m] = p;
+    r32[m] = (float)r;
   }
+  __shared__ double sh[256];
+  const double sum = block_sum256(r * r, sh);
+  if (threadIdx.x == 0) nrm[blockIdx.x] = sum;
 }
 
 // One fixed-point sweep of the Crank-Nicolson Helmholtz problem
@@ -2997,8 +3058,11 @@ void mixed_create(Ctx& c) {
   if (g.walls) dalloc(&X->thp, (size_t)(g.ny + 2) * g.nxh * g.nz);
   dalloc(&X->phi, n); dalloc(&X->b, n); dalloc(&X->r32, n);
   if (c.p.poisson_variant == FP_POISSON_SOR) {
-    dalloc(&X->e32, n); dalloc(&X->sor_pb, (size_t)nblk(n, 256)); dalloc(&X->sor_flag, 4);
-    FP_HIP_CHECK(hipHostMalloc((void**)&X->sor_host, 4 * sizeof(int), hipHostMallocDefault));
+    const SorPlan<float> p = sor_plan<float>(g);
+    dalloc(&X->e32, n); dalloc(&X->sor_pb, (size_t)nblk(n, 256)); dalloc(&X->sor_flag, 8);
+    dalloc(&X->sor_part, (size_t)SOR_BATCH * std::max(p.blocks, (long)nblk(n / 2, 256)));
+    FP_HIP_CHECK(hipHostMalloc((void**)&X->sor_host, 8 * sizeof(int), hipHostMallocDefault));
+    for (int e = 0; e < 2; e++) FP_HIP_CHECK(hipEventCreateWithFlags(&X->sor_ev[e], hipEventDisableTiming));
   }
   dalloc(&X->red, 8);
   dalloc(&X->part, (size_t)(n / 256 + 1024));
@@ -3064,7 +3128,9 @@ void mixed_destroy(Ctx& c) {
   dfree(X->spec); dfree(X->thp); dfree(X->twx); dfree(X->twy); dfree(X->twz);
   dfree(X->kx2); dfree(X->ky2); dfree(X->kz2);
   dfree(X->phi); dfree(X->b); dfree(X->r32); dfree(X->red); dfree(X->part); dfree(X->skip);
-  dfree(X->e32); dfree(X->sor_pb); dfree(X->sor_flag);
+  dfree(X->e32); dfree(X->sor_pb); dfree(X->sor_flag); dfree(X->sor_part);
+  for (int e = 0; e < 2; e++)
+    if (X->sor_ev[e]) (void)hipEventDestroy(X->sor_ev[e]);
   if (X->sor_host) (void)hipHostFree(X->sor_host);
   dfree(X->partb);
   dfree(X->pbuf);
@@ -3586,43 +3652,87 @@ static void select_ahead(Ctx& c) {
 // the last few sweeps: a smooth correction that grew over many sweeps would
 // make L_h e cancel in FP32 down to the size of E and stall the stopping test.
 // (SOR is affine in its iterate: the restarted sweeps are the same iteration.)
-// The host reads the flags back after each batch, as the FP64 path reads its
-// residuals; sweeps launched after convergence return at once.
+// The host enqueues batches ahead of the flags it reads, so that the device
+// does not wait for it; what is enqueued after a stop returns at once.
 static void mixed_sor(Ctx& c) {
   Mixed& X = MX(c);
   const Grid& g = c.g;
   hipStream_t s = c.stream;
   const long n = g.n;
-  const int nb = nblk(n, 256), nbh = nblk(n / 2, 256);
   const double om = c.p.sor_omega > 0.0 ? c.p.sor_omega : 2.0 / (1.0 + sin(3.14159265358979323846 * g.dx));
   const double BX = 1.0 / (g.dx * g.dx), BY = 1.0 / (g.dy * g.dy), BZ = 1.0 / (g.dz * g.dz);
   const double B0 = ((((BX + BX) + BY) + BY) + BZ) + BZ;
-  const float om_b0 = (float)(om / B0);
-  const int SOR_BATCH = 10;
-  hipLaunchKernelGGL(g.walls ? m_sor_start<true> : m_sor_start<false>, dim3(nb), dim3(256), 0, s, g, X.U, X.V, X.W, X.Up, X.phi, X.b,
-                     X.r32, X.e32, X.sor_pb);
-  hipLaunchKernelGGL(m_sor_decide, dim3(1), dim3(1024), 0, s, X.sor_pb, nb, X.red, c.p.sor_eps, 0, X.sor_flag);
-  int launched = 0;
-  while (launched < c.p.sor_itrmax) {
-    const int batch = std::min(SOR_BATCH, c.p.sor_itrmax - launched);
-    for (int b = 0; b < batch; b++) {
-      for (int color = 0; color < 2; color++)
-        hipLaunchKernelGGL(g.walls ? m_sor_sweep<true> : m_sor_sweep<false>, dim3(nbh), dim3(256), 0, s, g, color, om_b0,
-                           (float)BX, (float)BY, (float)BZ, (float)B0, X.r32, X.e32, X.part, X.sor_flag);
-      hipLaunchKernelGGL(m_sor_decide, dim3(1), dim3(1024), 0, s, X.part, nbh, X.red, c.p.sor_eps, 1, X.sor_flag);
+  const SorCoef<float> co{(float)BX, (float)BY, (float)BZ, (float)B0, (float)(om / B0), 0.0f};
+  const SorPlan<float> plan = sor_plan<float>(g);
+  const int nb = nblk(n, 256), nbh = nblk(n / 2, 256), nbs = plan.k ? (int)plan.blocks : nbh;
+  float* const buf[2] = {X.e32, X.X2};         // (the Helmholtz iterate is free here)
+  double* const phi[2] = {X.phi, c.Phi};       // (as is the FP64 path's Phi)
+  const int itrmax = c.p.sor_itrmax;
+  volatile int* h = X.sor_host;
+  int settled = 0;                             // corrections enqueued into phi
+  auto sweeps = [&](int count) {
+    float* e = X.e32;
+    if (plan.k) {
+      e = buf[sor_launch<float>(g, plan, co, X.r32, buf, X.sor_part, count, true, X.sor_flag, s) & 1];
+    } else {
+      zero_words(e, n, s);
+      for (int r = 0; r < count; r++)
+        for (int color = 0; color < 2; color++)
+          hipLaunchKernelGGL(g.walls ? m_sor_sweep<true> : m_sor_sweep<false>, dim3(nbh), dim3(256), 0, s, g, color, co.om,
+                             co.bx, co.by, co.bz, co.b0, X.r32, e, X.sor_part + (long)r * nbh, X.sor_flag);
     }
-    launched += batch;
-    // phi += e, e = 0, the FP64 defect of the new phi; once the sweeps have
-    // met the test, the same test on the FP64 residual (else they go on)
-    hipLaunchKernelGGL(m_sor_accum, dim3(nb), dim3(256), 0, s, n, X.phi, X.e32);
-    hipLaunchKernelGGL(g.walls ? m_residual<true> : m_residual<false>, dim3(nb), dim3(256), 0, s, g, X.b, X.phi, X.r32,
-                       X.part);
-    hipLaunchKernelGGL(m_sor_decide, dim3(1), dim3(1024), 0, s, X.part, nb, X.red, c.p.sor_eps, 2, X.sor_flag);
-    FP_HIP_CHECK(hipMemcpyAsync(X.sor_host, X.sor_flag, 3 * sizeof(int), hipMemcpyDeviceToHost, s));
-    FP_HIP_CHECK(hipStreamSynchronize(s));
-    if (X.sor_host[0]) break;
+    return e;
+  };
+  auto decide = [&](const double* part, int np, int rows, int mode) {
+    hipLaunchKernelGGL(m_sor_decide, dim3(1), dim3(1024), 0, s, part, np, rows, X.part, nb, X.red, c.p.sor_eps, mode,
+                       X.sor_flag, X.sor_host);
+  };
+  // phi += e and the FP64 defect of the new phi
+  auto settle = [&](const float* e) {
+    hipLaunchKernelGGL(g.walls ? m_sor_settle<true> : m_sor_settle<false>, dim3(nb), dim3(256), 0, s, g, X.b,
+                       phi[settled & 1], e, phi[(settled + 1) & 1], X.r32, X.part, X.sor_flag);
+    settled++;
+  };
+  hipLaunchKernelGGL(g.walls ? m_sor_start<true> : m_sor_start<false>, dim3(nb), dim3(256), 0, s, g, X.U, X.V, X.W, X.Up, X.phi, X.b,
+                     X.r32, X.sor_pb);
+  decide(X.sor_pb, nb, 1, 0);
+  int ahead = 0, group = 0;    // sweeps enqueued, groups of batches recorded
+  while (true) {
+    // two batches a group once the solve is long: an event costs a few
+    // microseconds, a group too many a few more
+    for (int q = 0; q < (ahead < 100 ? 1 : 2) && ahead < itrmax; q++) {
+      const int batch = std::min(SOR_BATCH, itrmax - ahead);
+      const float* e = sweeps(batch);
+      decide(X.sor_part, nbs, batch, 1);
+      settle(e);
+      ahead += batch;
+    }
+    if (ahead >= itrmax) decide(nullptr, 0, 0, 2);
+    FP_HIP_CHECK(hipEventRecord(X.sor_ev[group & 1], s));
+    if (ahead >= itrmax) FP_HIP_CHECK(hipEventSynchronize(X.sor_ev[group & 1]));
+    else if (group > 0) FP_HIP_CHECK(hipEventSynchronize(X.sor_ev[(group - 1) & 1]));
+    else { group++; continue; }
+    group++;
+    const bool stop = h[0] != 0;
+    if (stop && h[3]) {
+      // met before the end of a batch: what was enqueued since did nothing
+      settled = h[5];
+      const int again = h[3];
+      hipLaunchKernelGGL(m_sor_again, dim3(1), dim3(1), 0, s, X.sor_flag);
+      settle(sweeps(again));
+      decide(nullptr, 0, 0, 2);
+      FP_HIP_CHECK(hipStreamSynchronize(s));
+      ahead = h[6];
+      group = 0;
+      if (h[0] || ahead >= itrmax) break;
+    } else if (stop || ahead >= itrmax) {
+      break;
+    }
   }
-  c.sor_itr = (double)X.sor_host[1];
+  // (after a stop what is still enqueued changes nothing)
+  if (h[5] & 1)
+    FP_HIP_CHECK(hipMemcpyAsync(X.phi, phi[1], sizeof(double) * n, hipMemcpyDeviceToDevice, s));
+  c.sor_itr = (double)h[1];
 }
 
 void mixed_step(Ctx& c) {
