@@ -500,7 +500,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select(Grid g, const T* __restric
 }
 
 // The selection streamed along z, for nx = 64, 128 or 256 and nz a multiple
-// of kc: a block of 256 threads holds 256/nx whole x-rows and walks kc planes
+// of KC: a block of 256 threads holds 256/nx whole x-rows and walks KC planes
 // (select_planes).  The midpoint candidate of a face, C_a/2 + C_{a+1}/2, is the right
 // face's candidate of level 0 for cell a and the left face's of level 1 for
 // cell a+1 (fenep.f90:179-184), bit for bit.  Along x a thread evaluates it
@@ -509,8 +509,8 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select(Grid g, const T* __restric
 // to the next plane in registers.  16 of the 18 eigenvalue evaluations of a
 // cell remain, plus one per column for its first plane, and the z line is
 // loaded one plane per step.
-template <typename T>
-__global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, int kc, const T* __restrict__ C, uint8_t* __restrict__ sel,
+template <typename T, int KC>
+__global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const T* __restrict__ C, uint8_t* __restrict__ sel,
                                                         unsigned* __restrict__ total, unsigned* __restrict__ amb_idx,
                                                         unsigned* __restrict__ amb_list, float* __restrict__ amb_data) {
   constexpr bool F64 = sizeof(T) == 8;
@@ -520,14 +520,14 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, int kc, const T*
   const int t = threadIdx.x;
   if (t == 0) s_cnt = 0u;
   const long xb = xcd_block();
-  const int nkg = g.nz / kc;
+  const int nkg = g.nz / KC;
   const int kg = (int)(xb % nkg), jg = (int)(xb / nkg);
   const int i = t & (g.nx - 1);
   const int j = (jg << (8 - g.lnx)) + (t >> g.lnx);
   const int tl = (t & ~(g.nx - 1)) | ((i - 1) & (g.nx - 1));   // the x neighbour on the left
-  const int k0 = kg * kc;
-  const unsigned cap = SEL_STAGE * kc;
-  unsigned* region = amb_list + (size_t)blockIdx.x * (SEL_REGION * kc);
+  const int k0 = kg * KC;
+  const unsigned cap = SEL_STAGE * KC;
+  unsigned* region = amb_list + (size_t)blockIdx.x * (SEL_REGION * KC);
   float* stage = amb_data + (size_t)blockIdx.x * 18 * cap;
   const long n = g.n;
   const int sz = g.nx * g.ny;
@@ -549,7 +549,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, int kc, const T*
   // Cp_1 along z of the first plane; later planes take the previous Cn_0
   Lmin zl = cand_lmin<F64>(false, 1, z, entry_term<T>(ebm, ebc, 0.0f));
   __syncthreads();
-  for (int kk = 0; kk < kc; kk++) {
+  for (int kk = 0; kk < KC; kk++) {
     const int par = kk & 1;
     {
       const unsigned e = m + (unsigned)woff32(k0 + kk, 1, g.nz, sz);
@@ -604,11 +604,16 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, int kc, const T*
       if (ylo || yhi) {   // a wavefront holds one row: interior rows skip this
 #pragma unroll
         for (int q = 0; q < 6; q++) {
-          // (in the stored type: the ghost is what the reference holds)
-          const T yc = ldu(C + q * n, n, m), yn = ldu(C + q * n, n, m + (unsigned)(ylo ? eyp : eym));
-          const float gh = (float)(T(2) * yc - yn);
-          y[0][q] = ylo ? gh : y[0][q];
-          y[2][q] = yhi ? gh : y[2][q];
+          if constexpr (F64) {
+            // (in the stored type: the ghost is what the reference holds)
+            const T yc = ldu(C + q * n, n, m), yn = ldu(C + q * n, n, m + (unsigned)(ylo ? eyp : eym));
+            const float gh = (float)(T(2) * yc - yn);
+            y[0][q] = ylo ? gh : y[0][q];
+            y[2][q] = yhi ? gh : y[2][q];
+          } else {
+            y[0][q] = ylo ? 2.0f * y[1][q] - y[2][q] : y[0][q];
+            y[2][q] = yhi ? 2.0f * y[1][q] - y[0][q] : y[2][q];
+          }
         }
       }
       const float einy = entry_term<T>(entry_bound(y[0]), ebc, entry_bound(y[2]));
@@ -640,7 +645,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, int kc, const T*
     ebc = ebp;
     m += (unsigned)sz;
   }
-  sel_publish(&s_cnt, &s_base, blockIdx.x, SEL_REGION * kc, total, amb_idx);
+  sel_publish(&s_cnt, &s_base, blockIdx.x, SEL_REGION * KC, total, amb_idx);
 }
 
 // the reference's selection (select_d, evaluated as written) of one (cell,
@@ -2703,9 +2708,9 @@ __device__ __forceinline__ void mz_put(const double (&r)[MZ_PER], double* __rest
   }
 }
 
-// grid: (nx / MZ_TX) (ny / MZ_TY) ceil(nz / MZ_KC) blocks of MZ_THREADS
+// grid: (nx / MZ_TX) (ny / MZ_TY) ceil(nz / kc) blocks of MZ_THREADS
 template <bool WL>
-__global__ __launch_bounds__(MZ_THREADS) void m_march_z(Grid g, const float* __restrict__ up,
+__global__ __launch_bounds__(MZ_THREADS) void m_march_z(Grid g, int kc, const float* __restrict__ up,
                                                         const double* __restrict__ phi, float* __restrict__ U,
                                                         float* __restrict__ V, float* __restrict__ W,
                                                         float* __restrict__ P) {
@@ -2713,8 +2718,8 @@ __global__ __launch_bounds__(MZ_THREADS) void m_march_z(Grid g, const float* __r
   const int ntx = g.nx / MZ_TX, nty = g.ny / MZ_TY;
   const long b = xcd_block();
   const int bx = (int)(b % ntx), by = (int)((b / ntx) % nty), bz = (int)(b / ((long)ntx * nty));
-  const int i0 = bx * MZ_TX, j0 = by * MZ_TY, k0 = bz * MZ_KC;
-  const int k1 = min(k0 + MZ_KC, g.nz);
+  const int i0 = bx * MZ_TX, j0 = by * MZ_TY, k0 = bz * kc;
+  const int k1 = min(k0 + kc, g.nz);
   const int tx = threadIdx.x % MZ_TX, ty = threadIdx.x / MZ_TX;
   const int i = i0 + tx, j = j0 + ty;
   const double dt = g.dt;
@@ -3600,10 +3605,10 @@ static void select_launch(Ctx& c, const T* C, unsigned* total, unsigned* idx, un
   const unsigned region = SEL_REGION * std::max(1, kc), cap = SEL_STAGE * std::max(1, kc);
   {
     MTimer t(c, tm ? "fenep_select" : nullptr, s);
-    if (kc)
-      hipLaunchKernelGGL(m_select_z<T>, dim3(g.n / (SEL_BLOCK * kc)), dim3(SEL_BLOCK), 0, s, g, kc, C, c.sel, total, idx, list,
-                         data);
-    else
+    if (kc) {
+      auto streamed = kc == 4 ? m_select_z<T, 4> : (kc == 2 ? m_select_z<T, 2> : m_select_z<T, 1>);
+      hipLaunchKernelGGL(streamed, dim3(g.n / (SEL_BLOCK * kc)), dim3(SEL_BLOCK), 0, s, g, C, c.sel, total, idx, list, data);
+    } else
       hipLaunchKernelGGL(m_select<T>, dim3(nb), dim3(SEL_BLOCK), 0, s, g, C, c.sel, total, idx, list, data);
   }
   {
@@ -3735,6 +3740,17 @@ static void mixed_sor(Ctx& c) {
   c.sor_itr = (double)h[1];
 }
 
+// Planes a block of a z-streamed kernel walks: `most` (or the axis) where
+// that leaves a block per CU, fewer on smaller grids, whose tiles would leave
+// most of the CUs idle: at 64^3, 16 planes a block made 16 blocks of the
+// predictor, 45 us, one plane 256 blocks, 9 us (the correction 13 and 7 us); at
+// 128x64x64 two planes instead of 16, 53 and 15 us (14.6 and 8.8).
+static int planes_per_block(const Grid& g, int tile, int most) {
+  int kc = std::min(most, g.nz);   // (powers of two)
+  while (kc > 1 && g.n / ((long)tile * kc) < 256) kc >>= 1;
+  return kc;
+}
+
 void mixed_step(Ctx& c) {
   Mixed& X = MX(c);
   const Grid& g = c.g;
@@ -3758,9 +3774,9 @@ void mixed_step(Ctx& c) {
   if (g.nx % PZ_TX == 0 && g.ny % PZ_TY == 0) {
     // streamed along z, wall rows included
     MTimer t(c, "predictor");
-    const long nbk = (g.nz + PZ_KC - 1) / PZ_KC;
-    const long grid = (long)(g.nx / PZ_TX) * (g.ny / PZ_TY) * nbk;
-    hipLaunchKernelGGL(g.walls ? m_predictor_z<true> : m_predictor_z<false>, dim3(grid), dim3(PZ_THREADS), 0, s, g, PZ_KC,
+    const int kc = planes_per_block(g, PZ_TX * PZ_TY, PZ_KC);
+    const long grid = g.n / (PZ_TX * PZ_TY * kc);
+    hipLaunchKernelGGL(g.walls ? m_predictor_z<true> : m_predictor_z<false>, dim3(grid), dim3(PZ_THREADS), 0, s, g, kc,
                        c.p.method, c.has_history ? 0 : 1, polymer, X.U, X.V, X.W, X.P, X.C[X.cur], X.f, X.A0, X.T0,
                        X.F, (float)c.p.body_force[0], (float)c.p.body_force[1], (float)c.p.body_force[2], X.Q);
   } else {
@@ -3843,8 +3859,9 @@ void mixed_step(Ctx& c) {
   {
     MTimer t(c, "march");
     if (g.nx % MZ_TX == 0 && g.ny % MZ_TY == 0) {
-      const long grid = (long)(g.nx / MZ_TX) * (g.ny / MZ_TY) * ((g.nz + MZ_KC - 1) / MZ_KC);
-      hipLaunchKernelGGL(g.walls ? m_march_z<true> : m_march_z<false>, dim3(grid), dim3(MZ_THREADS), 0, s, g, X.Up,
+      const int kc = planes_per_block(g, MZ_TX * MZ_TY, MZ_KC);
+      const long grid = g.n / (MZ_TX * MZ_TY * kc);
+      hipLaunchKernelGGL(g.walls ? m_march_z<true> : m_march_z<false>, dim3(grid), dim3(MZ_THREADS), 0, s, g, kc, X.Up,
                          X.phi, X.U, X.V, X.W, X.P);
     } else {
       hipLaunchKernelGGL(g.walls ? m_march<true> : m_march<false>, dim3(nblk(n, 256)), dim3(256), 0, s, g, X.Up, X.phi,
