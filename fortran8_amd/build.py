@@ -24,6 +24,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", "--offload-arch=" + ARCH,
 UNITS = [
     ("fp_kernels_f64.hip", ["-ffp-contract=off"]),
     ("fp_spectral_f64.hip", ["-ffp-contract=off"]),
+    ("fp_stats.hip", ["-ffp-contract=off"]),
     ("fp_kernels_mixed.hip", ["-ffp-contract=fast-honor-pragmas"]),
     ("fp_api.hip", ["-ffp-contract=off"]),
     ("fp_adjoint.hip", ["-ffp-contract=fast-honor-pragmas"]),

@@ -273,7 +273,7 @@ int fp_destroy(void* vc) {
   dfree(c->spec); dfree(c->piv); dfree(c->red); dfree(c->part);
   dfree(c->twx); dfree(c->twy); dfree(c->twz); dfree(c->kx2); dfree(c->ky2); dfree(c->kz2);
   dfree(c->mk); dfree(c->mf); dfree(c->mb); dfree(c->ftmp);
-  dfree(c->mean_acc); dfree(c->mean_u);
+  dfree(c->mean_acc); dfree(c->mean_u); dfree(c->stat);
   for (int k = 0; k < 3; k++) { dfree(c->sp_row[k]); dfree(c->sp_tgt[k]); dfree(c->sp_ent[k]); dfree(c->sp_w[k]); }
   dfree(c->ib_w);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -468,9 +468,7 @@ int fp_step(void* vc, int nsteps, int sync) {
 // `scratch` (diag_scratch_words(c.g) doubles of device memory).
 static void diagnostics_into(Ctx& c, fp_diag* d, double* scratch) {
   std::memset(d, 0, sizeof(*d));
-  if (c.mixed) mixed_store_to_f64(c);
-  const double* mf = c.nmk ? (c.mixed ? mixed_marker_forces(c) : c.mf) : nullptr;
-  f64_diag(c, d, scratch, mf);
+  f64_diag(c, d, scratch);
   d->sor_itr = c.sor_itr;
   d->n_dc = c.mixed ? mixed_last_ndc(c) : 0.0;
   if (c.mixed) {
@@ -646,7 +644,6 @@ int fp_time_stats(void* vc, double* out) {
   if (!c || !out) return FP_E_ARG;
   if (!c->state_set) return fail(c, FP_E_STATE, "state not set");
   try {
-    if (c->mixed) mixed_store_to_f64(*c);
     f64_time_stats(*c, out);
   } catch (const std::string& e) {
     return fail(c, FP_E_HIP, e);
@@ -660,7 +657,6 @@ int fp_energy_spectrum(void* vc, double* E, int nbins) {
   if (c->g.walls) return fail(c, FP_E_ARG, "the shell spectrum needs a periodic grid");
   if (!c->state_set) return fail(c, FP_E_STATE, "state not set");
   try {
-    if (c->mixed) mixed_store_to_f64(*c);
     f64_energy_spectrum(*c, E, nbins);
   } catch (const std::string& e) {
     return fail(c, FP_E_HIP, e);
@@ -673,7 +669,6 @@ int fp_time_stats_map(void* vc, int ncyl, const double* xy, double diameter, dou
   if (!c || ncyl < 0 || (ncyl > 0 && !xy) || !(diameter >= 0.0) || (!map18 && !out13)) return fail(c, FP_E_ARG, "bad arguments");
   if (!c->state_set) return fail(c, FP_E_STATE, "state not set");
   try {
-    if (c->mixed) mixed_store_to_f64(*c);
     if (f64_time_stats_map(*c, ncyl, xy, diameter, map18, out13)) return fail(c, FP_E_ARG, "the mask covers the whole plane");
   } catch (const std::string& e) {
     return fail(c, FP_E_HIP, e);
@@ -686,7 +681,6 @@ int fp_energy_spectrum_z(void* vc, int ncyl, const double* xy, double diameter, 
   if (!c || ncyl < 0 || (ncyl > 0 && !xy) || !(diameter >= 0.0) || (!Emask && !Efirst)) return fail(c, FP_E_ARG, "bad arguments");
   if (!c->state_set) return fail(c, FP_E_STATE, "state not set");
   try {
-    if (c->mixed) mixed_store_to_f64(*c);
     if (f64_energy_spectrum_z(*c, ncyl, xy, diameter, Emask, Efirst)) return fail(c, FP_E_ARG, "the mask covers the whole plane");
   } catch (const std::string& e) {
     return fail(c, FP_E_HIP, e);

@@ -95,6 +95,8 @@ struct Ctx {
   double* mean_acc = nullptr;
   double* mean_u = nullptr;
   long mean_count = 0;
+  double* stat = nullptr;             // workspace of the statistics
+  size_t stat_words = 0;
 };
 
 // ---- launchers (fp_kernels_f64.hip; f64_select: fp_kernels_mixed.hip)
@@ -109,7 +111,8 @@ void f64_sor_create(Ctx& c);
 void f64_sor_destroy(Ctx& c);
 int  f64_sor(Ctx& c, const double* q, double* phi);
 void f64_zero_c(Ctx& c);
-void f64_diag(Ctx& c, fp_diag* d, double* scratch, const double* mf);  // scratch: diag_scratch_words
+// ---- statistics (fp_stats.hip)
+void f64_diag(Ctx& c, fp_diag* d, double* scratch);  // scratch: diag_scratch_words
 size_t diag_scratch_words(const Grid& g);
 void f64_time_stats(Ctx& c, double* out13);  // all_time_dif statistics
 void f64_energy_spectrum(Ctx& c, double* E, int nbins);  // shell spectrum (periodic)
@@ -124,7 +127,9 @@ void f64_spectral_create(Ctx& c);
 void f64_solve(Ctx& c, int kind, const double* q, double* x);   // kind 0..2 Helmholtz, 3 Poisson
 void f64_helmholtz(Ctx& c, const double* q, double* x);         // the three components
 void f64_poisson(Ctx& c, const double* up, double* x);          // lap x = div up / dt
-void f64_forward(Ctx& c, const double* q);                      // transform into c.spec
+// transforms of `comps` components of the regular-grid velocity, from component `comp` on, into c.spec
+void f64_forward_regular(Ctx& c, const double* U, const double* V, const double* W, int comp, int comps);
+void f64_forward_regular(Ctx& c, const float* U, const float* V, const float* W, int comp, int comps);
 void step_f64(Ctx& c);       // one FP64 time step (fp_api.hip)
 
 // ---- recording and discrete adjoint (fp_adjoint.hip)

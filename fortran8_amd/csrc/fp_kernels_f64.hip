@@ -742,591 +742,4 @@ void f64_zero_c(Ctx& c) {
   zero_words(c.C[c.cur], 12 * c.g.n, c.stream);
 }
 
-// =============================================== time-series statistics ===
-// Per-cell terms of all_time_dif / all_time_dif_map (fenep_mpi.f90:2200-2564)
-// for the velocity fluctuation u' = u - u_mean (u_mean = nullptr: none, the
-// 'same' records; otherwise the 'diff' records): 0-2 regular-grid u'^2,
-// 3-5 squared staggered gradients of u', 6 S:S with S = D + D^T of the
-// 4-point gradient of u', 7 |u|^2 on the staggered grid (raw u, the
-// K_staggered term), 8 log f(C), 9 tr C.  The ghosts of u' are those of u
-// minus those of the mean, each by the boundary rules.
-constexpr int TS_N = 10;
-__device__ __forceinline__ void stat_cell(const Grid& g, const double* __restrict__ U, const double* __restrict__ V,
-                                          const double* __restrict__ W, const double* __restrict__ Um,
-                                          const double* __restrict__ C, int i, int j, int k, long m, double* s) {
-  const double dx = g.dx, dy = g.dy, dz = g.dz;
-  const double* Vm = Um ? Um + g.n : nullptr;
-  const double* Wm = Um ? Um + 2 * g.n : nullptr;
-  auto UG = [&](int a, int b, int c) {
-    return ldb(U, g, i + a, j + b, k + c, BC_U) - (Um ? ldb(Um, g, i + a, j + b, k + c, BC_U) : 0.0);
-  };
-  auto VG = [&](int a, int b, int c) {
-    return ldb(V, g, i + a, j + b, k + c, BC_V) - (Vm ? ldb(Vm, g, i + a, j + b, k + c, BC_V) : 0.0);
-  };
-  auto WG = [&](int a, int b, int c) {
-    return ldb(W, g, i + a, j + b, k + c, BC_W) - (Wm ? ldb(Wm, g, i + a, j + b, k + c, BC_W) : 0.0);
-  };
-  const double u0 = UG(0, 0, 0), v0 = VG(0, 0, 0), w0 = WG(0, 0, 0);
-  const double ur = (u0 + UG(-1, 0, 0)) / 2.0, vr = (v0 + VG(0, -1, 0)) / 2.0, wr = (w0 + WG(0, 0, -1)) / 2.0;
-  s[0] = ur * ur; s[1] = vr * vr; s[2] = wr * wr;
-  double D[3][3];
-  D[0][0] = (u0 - UG(-1, 0, 0)) / dx;
-  D[0][1] = (UG(0, 1, 0) - UG(0, -1, 0) + UG(-1, 1, 0) - UG(-1, -1, 0)) / (4 * dy);
-  D[0][2] = (UG(0, 0, 1) - UG(0, 0, -1) + UG(-1, 0, 1) - UG(-1, 0, -1)) / (4 * dz);
-  D[1][0] = (VG(1, 0, 0) - VG(-1, 0, 0) + VG(1, -1, 0) - VG(-1, -1, 0)) / (4 * dx);
-  D[1][1] = (v0 - VG(0, -1, 0)) / dy;
-  D[1][2] = (VG(0, 0, 1) - VG(0, 0, -1) + VG(0, -1, 1) - VG(0, -1, -1)) / (4 * dz);
-  D[2][0] = (WG(1, 0, 0) - WG(-1, 0, 0) + WG(1, 0, -1) - WG(-1, 0, -1)) / (4 * dx);
-  D[2][1] = (WG(0, 1, 0) - WG(0, -1, 0) + WG(0, 1, -1) - WG(0, -1, -1)) / (4 * dy);
-  D[2][2] = (w0 - WG(0, 0, -1)) / dz;
-  s[3] = D[0][0] * D[0][0]; s[4] = D[1][1] * D[1][1]; s[5] = D[2][2] * D[2][2];
-  s[6] = 0.0;
-  for (int a = 0; a < 3; a++)
-    for (int b = 0; b < 3; b++) { const double sab = D[a][b] + D[b][a]; s[6] += sab * sab; }
-  s[7] = U[m] * U[m] + V[m] * V[m] + W[m] * W[m];
-  const double t = (C[m] + C[3 * g.n + m]) + C[5 * g.n + m];
-  const double L2 = g.lp * g.lp;
-  s[8] = log((L2 - 3.0) / (L2 - t));
-  s[9] = t;
-}
-
-__global__ __launch_bounds__(256) void k_time_stats(Grid g, const double* __restrict__ U, const double* __restrict__ V,
-                                                    const double* __restrict__ W, const double* __restrict__ Um,
-                                                    const double* __restrict__ C, double* __restrict__ part, int nb) {
-  const long m = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  double s[TS_N];
-  for (int q = 0; q < TS_N; q++) s[q] = 0.0;
-  if (m < g.n) {
-    int i, j, k;
-    cell_ijk(g, m, i, j, k);
-    stat_cell(g, U, V, W, Um, C, i, j, k, m, s);
-  }
-  __shared__ double sh[256];
-  for (int q = 0; q < TS_N; q++) {
-    const double v = block_sum256(s[q], sh);
-    if (threadIdx.x == 0) part[(long)q * nb + blockIdx.x] = v;
-    __syncthreads();
-  }
-}
-
-// all_time_dif_map (fenep_mpi.f90:2350-2500): the per-cell terms summed over
-// z for each (i, j) column, in k order, then the z variance of tr C about the
-// column mean.  col[q * nx*ny + i + nx*j]: q = 0..9 as stat_cell (7 unused),
-// q = 10 the sum of (tr C - column mean)^2.
-constexpr int COL_N = 11;
-__global__ __launch_bounds__(256) void k_column_stats(Grid g, const double* __restrict__ U, const double* __restrict__ V,
-                                                      const double* __restrict__ W, const double* __restrict__ Um,
-                                                      const double* __restrict__ C, double* __restrict__ col) {
-  const long ij = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  const long nxy = (long)g.nx * g.ny;
-  if (ij >= nxy) return;
-  const int i = (int)(ij & (g.nx - 1)), j = (int)(ij >> g.lnx);
-  double acc[TS_N], s[TS_N];
-  for (int q = 0; q < TS_N; q++) acc[q] = 0.0;
-  for (int k = 0; k < g.nz; k++) {
-    const long m = ij + nxy * k;
-    stat_cell(g, U, V, W, Um, C, i, j, k, m, s);
-    for (int q = 0; q < TS_N; q++) acc[q] += s[q];
-  }
-  const double mean = acc[9] / (double)g.nz;
-  double var = 0.0;
-  for (int k = 0; k < g.nz; k++) {
-    const long m = ij + nxy * k;
-    const double t = (C[m] + C[3 * g.n + m]) + C[5 * g.n + m] - mean;
-    var += t * t;
-  }
-  for (int q = 0; q < TS_N; q++) col[q * nxy + ij] = acc[q];
-  col[TS_N * nxy + ij] = var;
-}
-
-// fft_energy_dif_map (fenep_mpi.f90:2670-2797): the z transform of the
-// regular-grid fluctuation velocity of every (i, j) column, normalised by
-// 1/NZ (fft_z, fenep_mpi.f90:1442-1463), as a direct sum over z; energy
-// (|u^|^2 + |v^|^2 + |w^|^2)/2 per |kz| = 0..NZ/2, doubled for 0 < kz < NZ/2
-// (the +-kz pair).  E[kz * nx*ny + i + nx*j].
-__global__ __launch_bounds__(256) void k_zspec_columns(Grid g, const double* __restrict__ U, const double* __restrict__ V,
-                                                       const double* __restrict__ W, const double* __restrict__ Um,
-                                                       double* __restrict__ E) {
-  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  const long nxy = (long)g.nx * g.ny;
-  const int nk = g.nz / 2 + 1;
-  if (t >= nxy * nk) return;
-  const long ij = t % nxy;
-  const int kz = (int)(t / nxy);
-  const int i = (int)(ij & (g.nx - 1)), j = (int)(ij >> g.lnx);
-  const double* Vm = Um ? Um + g.n : nullptr;
-  const double* Wm = Um ? Um + 2 * g.n : nullptr;
-  double re[3] = {0, 0, 0}, im[3] = {0, 0, 0};
-  for (int k = 0; k < g.nz; k++) {
-    const double ur = ((ldb(U, g, i, j, k, BC_U) - (Um ? ldb(Um, g, i, j, k, BC_U) : 0.0))
-                       + (ldb(U, g, i - 1, j, k, BC_U) - (Um ? ldb(Um, g, i - 1, j, k, BC_U) : 0.0))) / 2.0;
-    const double vr = ((ldb(V, g, i, j, k, BC_V) - (Vm ? ldb(Vm, g, i, j, k, BC_V) : 0.0))
-                       + (ldb(V, g, i, j - 1, k, BC_V) - (Vm ? ldb(Vm, g, i, j - 1, k, BC_V) : 0.0))) / 2.0;
-    const double wr = ((ldb(W, g, i, j, k, BC_W) - (Wm ? ldb(Wm, g, i, j, k, BC_W) : 0.0))
-                       + (ldb(W, g, i, j, k - 1, BC_W) - (Wm ? ldb(Wm, g, i, j, k - 1, BC_W) : 0.0))) / 2.0;
-    // e^{-2 pi i kz k / NZ}; the product kz*k is reduced mod NZ first
-    const double a = 2.0 * (double)((long)kz * k & (g.nz - 1)) / (double)g.nz;
-    double sn, cs;
-    sincospi(a, &sn, &cs);
-    re[0] += ur * cs; im[0] -= ur * sn;
-    re[1] += vr * cs; im[1] -= vr * sn;
-    re[2] += wr * cs; im[2] -= wr * sn;
-  }
-  const double nz = (double)g.nz;
-  double e = 0.0;
-  for (int q = 0; q < 3; q++) e += (re[q] / nz) * (re[q] / nz) + (im[q] / nz) * (im[q] / nz);
-  E[t] = (kz == 0 || kz == g.nz / 2) ? e / 2.0 : e;
-}
-
-// masked average over the (i, j) plane of each kz row: sum(E * mask)/sum(mask)
-__global__ __launch_bounds__(256) void k_masked_rows(long nxy, const double* __restrict__ E,
-                                                     const double* __restrict__ mask, double msum,
-                                                     double* __restrict__ out) {
-  const double* row = E + nxy * blockIdx.x;
-  double v = 0.0;
-  for (long ij = threadIdx.x; ij < nxy; ij += blockDim.x) v += row[ij] * mask[ij];
-  __shared__ double sh[256];
-  v = block_sum256(v, sh);
-  if (threadIdx.x == 0) out[blockIdx.x] = v / msum;
-}
-
-// time-mean accumulation of the velocity (fenep_mpi.f90:2969-2971)
-template <typename T>
-__global__ __launch_bounds__(256) void k_mean_acc(long n, const T* __restrict__ U, const T* __restrict__ V,
-                                                  const T* __restrict__ W, double* __restrict__ acc) {
-  const long m = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (m >= n) return;
-  acc[m] += (double)U[m];
-  acc[n + m] += (double)V[m];
-  acc[2 * n + m] += (double)W[m];
-}
-
-// mean = acc / count, then (zavg) its z average for every (i, j) (ave_mean,
-// fenep_mpi.f90:2010-2033), in k order
-__global__ __launch_bounds__(256) void k_mean_finish(Grid g, const double* __restrict__ acc, double count, int zavg,
-                                                     double* __restrict__ mean) {
-  const long nxy = (long)g.nx * g.ny;
-  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (t >= 3 * nxy) return;
-  const int comp = (int)(t / nxy);
-  const long ij = t % nxy;
-  const double* a = acc + comp * g.n;
-  double* o = mean + comp * g.n;
-  if (!zavg) {
-    for (int k = 0; k < g.nz; k++) o[ij + nxy * k] = a[ij + nxy * k] / count;
-    return;
-  }
-  double s = 0.0;
-  for (int k = 0; k < g.nz; k++) s += a[ij + nxy * k] / count;
-  s = s / (double)g.nz;
-  for (int k = 0; k < g.nz; k++) o[ij + nxy * k] = s;
-}
-
-// sum of (tr C - mean)^2, per block
-__global__ __launch_bounds__(256) void k_trc_var(Grid g, const double* __restrict__ C, const double* __restrict__ mean,
-                                                 double* __restrict__ part) {
-  const long m = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  double v = 0.0;
-  if (m < g.n) {
-    const double t = (C[m] + C[3 * g.n + m]) + C[5 * g.n + m] - mean[0];
-    v = t * t;
-  }
-  __shared__ double sh[256];
-  const double s = block_sum256(v, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
-void f64_time_stats(Ctx& c, double* out) {
-  const Grid& g = c.g;
-  hipStream_t s = c.stream;
-  const int nb = nblk(g.n, 256);
-  double* part = nullptr;
-  double* red = nullptr;
-  FP_HIP_CHECK(hipMalloc((void**)&part, sizeof(double) * (size_t)(TS_N + 1) * nb));
-  FP_HIP_CHECK(hipMalloc((void**)&red, sizeof(double) * (TS_N + 2)));
-  double r[TS_N + 2];
-  try {
-    hipLaunchKernelGGL(k_time_stats, dim3(nb), dim3(256), 0, s, g, c.U, c.V, c.W, c.mean_u, c.C[c.cur], part, nb);
-    for (int q = 0; q < TS_N; q++)
-      hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, part + (long)q * nb, nb, red + q, 0);
-    FP_HIP_CHECK(hipMemcpyAsync(r, red, sizeof(double) * TS_N, hipMemcpyDeviceToHost, s));
-    FP_HIP_CHECK(hipStreamSynchronize(s));
-    const double mean = r[9] / (double)g.n;
-    FP_HIP_CHECK(hipMemcpyAsync(red + TS_N, &mean, sizeof(double), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_trc_var, dim3(nb), dim3(256), 0, s, g, c.C[c.cur], red + TS_N, part + (long)TS_N * nb);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, part + (long)TS_N * nb, nb, red + TS_N + 1, 0);
-    FP_HIP_CHECK(hipMemcpyAsync(r + TS_N + 1, red + TS_N + 1, sizeof(double), hipMemcpyDeviceToHost, s));
-    FP_HIP_CHECK(hipStreamSynchronize(s));
-  } catch (...) {
-    (void)hipFree(part); (void)hipFree(red);
-    throw;
-  }
-  (void)hipFree(part);
-  (void)hipFree(red);
-  const double N = (double)g.n, nu = 1.0 / c.p.re, L2 = c.p.lp * c.p.lp;
-  const double urms = r[0] / N, vrms = r[1] / N, wrms = r[2] / N;
-  const double all_rms = (urms + vrms + wrms) / 3.0, all_grad = (r[3] / N + r[4] / N + r[5] / N) / 3.0;
-  const double eps = nu / 2.0 * r[6] / N;
-  const double lambda = std::sqrt(all_rms / all_grad);
-  out[0] = (double)c.step;
-  out[1] = c.step * c.p.dt;
-  out[2] = (urms + vrms + wrms) / 2.0;
-  out[3] = r[7] / (2.0 * N);
-  out[4] = lambda;
-  out[5] = std::sqrt(all_rms) * lambda / nu;
-  out[6] = eps;
-  out[7] = std::pow(nu * nu * nu / eps, 0.25);
-  out[8] = std::sqrt(nu / eps);
-  out[9] = std::pow(nu * eps, 0.25);
-  out[10] = 0.5 * (1.0 - c.p.beta) / c.p.re / c.p.wi * (L2 - 3.0) * r[8] / N;
-  out[11] = r[9] / N;
-  out[12] = std::sqrt(r[TS_N + 1] / N);
-}
-
-// all_time_dif_map (fenep_mpi.f90:2350-2564): column sums on the device, the
-// per-(i, j) statistics and their masked plane averages here.  mask(i, j) = 0
-// within 1.5 radii of a cylinder centre (fenep_mpi.f90:2530-2537, with the
-// centres given instead of the reference's four fixed ones, and dY for y).
-static std::vector<double> plane_mask(const Grid& g, int ncyl, const double* xy, double diameter) {
-  std::vector<double> mask((size_t)g.nx * g.ny, 1.0);
-  const double r = diameter * 1.5 / 2.0;
-  for (int j = 0; j < g.ny; j++)
-    for (int i = 0; i < g.nx; i++)
-      for (int c = 0; c < ncyl; c++) {
-        const double dxc = (i + 0.5) * g.dx - xy[2 * c], dyc = (j + 0.5) * g.dy - xy[2 * c + 1];
-        if (dxc * dxc + dyc * dyc < r * r) mask[i + (size_t)g.nx * j] = 0.0;
-      }
-  return mask;
-}
-
-int f64_time_stats_map(Ctx& c, int ncyl, const double* xy, double diameter, double* map18, double* out13) {
-  const Grid& g = c.g;
-  hipStream_t s = c.stream;
-  const long nxy = (long)g.nx * g.ny;
-  std::vector<double> col((size_t)COL_N * nxy);
-  double* dcol = nullptr;
-  FP_HIP_CHECK(hipMalloc((void**)&dcol, sizeof(double) * col.size()));
-  try {
-    hipLaunchKernelGGL(k_column_stats, dim3(nblk(nxy, 256)), dim3(256), 0, s, g, c.U, c.V, c.W, c.mean_u, c.C[c.cur], dcol);
-    FP_HIP_CHECK(hipMemcpyAsync(col.data(), dcol, sizeof(double) * col.size(), hipMemcpyDeviceToHost, s));
-    FP_HIP_CHECK(hipStreamSynchronize(s));
-  } catch (...) {
-    (void)hipFree(dcol);
-    throw;
-  }
-  (void)hipFree(dcol);
-  const std::vector<double> mask = plane_mask(g, ncyl, xy, diameter);
-  double msum = 0.0;
-  for (double m : mask) msum += m;
-  if (msum == 0.0) return 1;
-  const double NZ = (double)g.nz, nu = 1.0 / c.p.re, L2 = c.p.lp * c.p.lp;
-  const double epc = 0.5 * (1.0 - c.p.beta) / c.p.re / c.p.wi * (L2 - 3.0);
-  double acc[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  for (long ij = 0; ij < nxy; ij++) {
-    auto C_ = [&](int q) { return col[(size_t)q * nxy + ij]; };
-    const double urms = C_(0) / NZ, vrms = C_(1) / NZ, wrms = C_(2) / NZ;
-    const double all_rms = (urms + vrms + wrms) / 3.0;
-    const double all_grad = (C_(3) / NZ + C_(4) / NZ + C_(5) / NZ) / 3.0;
-    const double eps = nu / 2.0 * C_(6) / NZ;
-    const double Lk = std::pow(nu * nu * nu / eps, 0.25), Tk = std::sqrt(nu / eps), Uk = std::pow(nu * eps, 0.25);
-    const double lam = std::sqrt(all_rms / all_grad);
-    const double relam = std::sqrt(all_rms) * lam / nu;
-    const double K = (urms + vrms + wrms) / 2.0;
-    const double Ep = epc * (C_(8) / NZ);
-    const double trm = C_(9) / NZ, trs = std::sqrt(C_(10) / NZ);
-    const double vals[11] = {K, lam, relam, eps, Lk, Tk, Uk, Ep, trm, trs, mask[ij]};
-    const int i = (int)(ij % g.nx), j = (int)(ij / g.nx);
-    double* row = map18 ? map18 + 18 * ij : nullptr;
-    if (row) {
-      row[0] = (i + 0.5) * g.dx;
-      row[1] = (j + 0.5) * g.dy;
-      for (int q = 0; q < 11; q++) row[2 + q] = vals[q];
-      for (int q = 13; q < 18; q++) row[q] = 0.0;
-    }
-    for (int q = 0; q < 10; q++) acc[q] += vals[q] * mask[ij];
-  }
-  if (out13) {
-    out13[0] = (double)c.step;
-    out13[1] = c.step * c.p.dt;
-    out13[2] = acc[0] / msum;   // K
-    out13[3] = 0.0;             // no K_staggered in the masked record
-    out13[4] = acc[1] / msum;   // lambda
-    out13[5] = acc[2] / msum;   // Re_lambda
-    out13[6] = acc[3] / msum;   // epsilon
-    out13[7] = acc[4] / msum;   // Kolmogorov length, time, velocity
-    out13[8] = acc[5] / msum;
-    out13[9] = acc[6] / msum;
-    out13[10] = acc[7] / msum;  // Ep
-    out13[11] = acc[8] / msum;  // tr C mean
-    out13[12] = acc[9] / msum;  // tr C std
-  }
-  return 0;
-}
-
-// fft_energy_dif_map (fenep_mpi.f90:2670-2797) of the current state:
-// Emask[kz] = masked plane average of the column z spectra, Efirst[kz] = the
-// spectrum of column (1, 1); kz = 0..NZ-1 (zero above NZ/2).
-int f64_energy_spectrum_z(Ctx& c, int ncyl, const double* xy, double diameter, double* Emask, double* Efirst) {
-  const Grid& g = c.g;
-  hipStream_t s = c.stream;
-  const long nxy = (long)g.nx * g.ny;
-  const int nk = g.nz / 2 + 1;
-  const std::vector<double> mask = plane_mask(g, ncyl, xy, diameter);
-  double msum = 0.0;
-  for (double m : mask) msum += m;
-  if (msum == 0.0) return 1;
-  double *dE = nullptr, *dmask = nullptr, *dout = nullptr;
-  std::vector<double> em(nk), ef(nk);
-  try {
-    FP_HIP_CHECK(hipMalloc((void**)&dE, sizeof(double) * nxy * nk));
-    FP_HIP_CHECK(hipMalloc((void**)&dmask, sizeof(double) * nxy));
-    FP_HIP_CHECK(hipMalloc((void**)&dout, sizeof(double) * nk));
-    FP_HIP_CHECK(hipMemcpyAsync(dmask, mask.data(), sizeof(double) * nxy, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_zspec_columns, dim3(nblk(nxy * nk, 256)), dim3(256), 0, s, g, c.U, c.V, c.W, c.mean_u, dE);
-    hipLaunchKernelGGL(k_masked_rows, dim3(nk), dim3(256), 0, s, nxy, dE, dmask, msum, dout);
-    FP_HIP_CHECK(hipMemcpyAsync(em.data(), dout, sizeof(double) * nk, hipMemcpyDeviceToHost, s));
-    FP_HIP_CHECK(hipMemcpy2DAsync(ef.data(), sizeof(double), dE, sizeof(double) * nxy, sizeof(double), nk,
-                                  hipMemcpyDeviceToHost, s));
-    FP_HIP_CHECK(hipStreamSynchronize(s));
-  } catch (...) {
-    (void)hipFree(dE); (void)hipFree(dmask); (void)hipFree(dout);
-    throw;
-  }
-  (void)hipFree(dE); (void)hipFree(dmask); (void)hipFree(dout);
-  for (int k = 0; k < g.nz; k++) {
-    if (Emask) Emask[k] = k < nk ? em[k] : 0.0;
-    if (Efirst) Efirst[k] = k < nk ? ef[k] : 0.0;
-  }
-  return 0;
-}
-
-// time mean of the velocity for the mean-subtracted statistics
-void f64_mean_accumulate(Ctx& c, const float* u32, const float* v32, const float* w32) {
-  const Grid& g = c.g;
-  if (!c.mean_acc) {
-    FP_HIP_CHECK(hipMalloc((void**)&c.mean_acc, sizeof(double) * 3 * g.n));
-    zero_words(c.mean_acc, 6 * g.n, c.stream);
-    c.mean_count = 0;
-  }
-  if (u32)
-    hipLaunchKernelGGL(k_mean_acc<float>, dim3(nblk(g.n, 256)), dim3(256), 0, c.stream, g.n, u32, v32, w32, c.mean_acc);
-  else
-    hipLaunchKernelGGL(k_mean_acc<double>, dim3(nblk(g.n, 256)), dim3(256), 0, c.stream, g.n, (const double*)c.U,
-                       (const double*)c.V, (const double*)c.W, c.mean_acc);
-  c.mean_count++;
-}
-
-int f64_mean_apply(Ctx& c, int mode) {
-  const Grid& g = c.g;
-  if (mode == 0) {
-    if (c.mean_u) (void)hipFree(c.mean_u);
-    c.mean_u = nullptr;
-  } else {
-    if (!c.mean_acc || c.mean_count == 0) return 1;
-    if (!c.mean_u) FP_HIP_CHECK(hipMalloc((void**)&c.mean_u, sizeof(double) * 3 * g.n));
-    const long nxy = (long)g.nx * g.ny;
-    hipLaunchKernelGGL(k_mean_finish, dim3(nblk(3 * nxy, 256)), dim3(256), 0, c.stream, g, c.mean_acc,
-                       (double)c.mean_count, mode == 1 ? 1 : 0, c.mean_u);
-  }
-  if (c.mean_acc) {
-    FP_HIP_CHECK(hipStreamSynchronize(c.stream));
-    (void)hipFree(c.mean_acc);
-    c.mean_acc = nullptr;
-  }
-  c.mean_count = 0;
-  FP_HIP_CHECK(hipStreamSynchronize(c.stream));
-  return 0;
-}
-
-// ===================================================== energy spectrum =====
-// fft_energy_dif (fenep_mpi.f90:2566-2665) without a subtracted mean: the
-// regular-grid velocity, its forward transform / N, |u^|^2 summed over the
-// three components into integer shells nint(|k|), half weight on the kx = 0
-// and Nyquist planes of the half spectrum.
-__global__ __launch_bounds__(256) void k_reg_velocity(Grid g, const double* __restrict__ U, const double* __restrict__ V,
-                                                      const double* __restrict__ W, const double* __restrict__ Um,
-                                                      double* __restrict__ out) {
-  const long m = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (m >= g.n) return;
-  int i, j, k;
-  cell_ijk(g, m, i, j, k);
-  out[m] = (U[m] + ldb(U, g, i - 1, j, k, BC_U)) / 2.0;
-  out[g.n + m] = (V[m] + ldb(V, g, i, j - 1, k, BC_V)) / 2.0;
-  out[2 * g.n + m] = (W[m] + ldb(W, g, i, j, k - 1, BC_W)) / 2.0;
-  if (Um) {  // the fluctuation about the subtracted mean
-    const double *Vm = Um + g.n, *Wm = Um + 2 * g.n;
-    out[m] = ((U[m] - Um[m]) + (ldb(U, g, i - 1, j, k, BC_U) - ldb(Um, g, i - 1, j, k, BC_U))) / 2.0;
-    out[g.n + m] = ((V[m] - Vm[m]) + (ldb(V, g, i, j - 1, k, BC_V) - ldb(Vm, g, i, j - 1, k, BC_V))) / 2.0;
-    out[2 * g.n + m] = ((W[m] - Wm[m]) + (ldb(W, g, i, j, k - 1, BC_W) - ldb(Wm, g, i, j, k - 1, BC_W))) / 2.0;
-  }
-}
-
-__global__ __launch_bounds__(256) void k_spec_shells(Grid g, const double2* __restrict__ spec, int nbins,
-                                                     double* __restrict__ E) {
-  extern __shared__ double bins[];
-  for (int b = threadIdx.x; b < nbins; b += blockDim.x) bins[b] = 0.0;
-  __syncthreads();
-  const long total = (long)g.nxh * g.ny * g.nz;
-  const double N = (double)g.n;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
-    // [kx][z][y], the wavenumbers of y and z bit-reversed (f64_forward)
-    const int j = (int)(__brev((unsigned)e & (g.ny - 1)) >> (32 - g.lny));
-    const int lnz = __ffs(g.nz) - 1;
-    const int k = (int)(__brev((unsigned)(e >> g.lny) & (g.nz - 1)) >> (32 - lnz));
-    const int i = (int)(e >> (g.lny + lnz));
-    const double kx = (double)i;
-    const double ky = (double)(j <= g.ny / 2 ? j : j - g.ny);
-    const double kz = (double)(k <= g.nz / 2 ? k : k - g.nz);
-    const int idx = (int)floor(sqrt(kx * kx + ky * ky + kz * kz) + 0.5);
-    const double2 s = spec[e];
-    const double a = (s.x / N) * (s.x / N) + (s.y / N) * (s.y / N);
-    const double w = (i == 0 || i == g.nxh - 1) ? 0.5 : 1.0;
-    if (idx < nbins) atomicAdd(&bins[idx], a * w);
-  }
-  __syncthreads();
-  for (int b = threadIdx.x; b < nbins; b += blockDim.x)
-    if (bins[b] != 0.0) atomicAdd(&E[b], bins[b]);
-}
-
-void f64_energy_spectrum(Ctx& c, double* E, int nbins) {
-  const Grid& g = c.g;
-  hipStream_t s = c.stream;
-  double* dE = nullptr;
-  FP_HIP_CHECK(hipMalloc((void**)&dE, sizeof(double) * nbins));
-  try {
-    zero_words(dE, 2L * nbins, s);
-    hipLaunchKernelGGL(k_reg_velocity, dim3(nblk(g.n, 256)), dim3(256), 0, s, g, c.U, c.V, c.W, c.mean_u, c.Q);
-    const long total = (long)g.nxh * g.ny * g.nz;
-    const int sb = (int)std::min<long>(1024, (total + 255) / 256);
-    for (int comp = 0; comp < 3; comp++) {
-      f64_forward(c, c.Q + comp * g.n);
-      hipLaunchKernelGGL(k_spec_shells, dim3(sb), dim3(256), sizeof(double) * nbins, s, g, c.spec, nbins, dE);
-    }
-    FP_HIP_CHECK(hipMemcpyAsync(E, dE, sizeof(double) * nbins, hipMemcpyDeviceToHost, s));
-    FP_HIP_CHECK(hipStreamSynchronize(s));
-  } catch (...) {
-    (void)hipFree(dE);
-    throw;
-  }
-  (void)hipFree(dE);
-}
-
-// ===================================================== diagnostics ========
-__global__ __launch_bounds__(256) void k_diag(Grid g, const double* __restrict__ U, const double* __restrict__ V,
-                                              const double* __restrict__ W, const double* __restrict__ C,
-                                              const int* __restrict__ nitr, int polymer, double* __restrict__ red) {
-  long m = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  double s[6] = {0, 0, 0, 0, 0, 0};  // ke, trsum, trsq, nitr, nan, Newton stopped at the cap
-  double mx[6] = {-1e300, -1e300, -1e300, -1e300, 1e300, 0.0};  // umax vmax wmax trmax -trmin divmax
-  if (m < g.n) {
-    int i, j, k;
-  cell_ijk(g, m, i, j, k);
-    double u = ldb(U, g, i, j, k, BC_U), v = ldb(V, g, i, j, k, BC_V), w = ldb(W, g, i, j, k, BC_W);
-    double ur = (u + ldb(U, g, i - 1, j, k, BC_U)) / 2.0;
-    double vr = (v + ldb(V, g, i, j - 1, k, BC_V)) / 2.0;
-    double wr = (w + ldb(W, g, i, j, k - 1, BC_W)) / 2.0;
-    s[0] = ur * ur + vr * vr + wr * wr;
-    double tr = (C[m] + C[3 * g.n + m]) + C[5 * g.n + m];
-    s[1] = tr; s[2] = tr * tr;
-    s[3] = polymer ? (double)abs(nitr[m]) : 0.0;
-    s[5] = (polymer && nitr[m] < 0) ? 1.0 : 0.0;
-    s[4] = isnan(U[m]) ? 1.0 : 0.0;
-    mx[0] = u; mx[1] = v; mx[2] = w; mx[3] = tr; mx[4] = tr;
-    double dv = ((u - ldb(U, g, i - 1, j, k, BC_U)) / g.dx + (v - ldb(V, g, i, j - 1, k, BC_V)) / g.dy)
-                + (w - ldb(W, g, i, j, k - 1, BC_W)) / g.dz;
-    mx[5] = fabs(dv);
-  }
-  __shared__ double sh[256];
-  for (int a = 0; a < 12; a++) {
-    double v = a < 6 ? s[a] : mx[a - 6];
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-      if (threadIdx.x < o) {
-        double x = sh[threadIdx.x], y = sh[threadIdx.x + o];
-        if (a < 6) sh[threadIdx.x] = x + y;
-        else if (a == 10) sh[threadIdx.x] = fmin(x, y);
-        else sh[threadIdx.x] = fmax(x, y);
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) red[a * gridDim.x + blockIdx.x] = sh[0];
-    __syncthreads();
-  }
-}
-
-// the 12 per-block partials of k_diag reduced to one value each: sums for
-// a < 6, the minimum of tr C for a = 10, maxima otherwise (one block per a)
-__global__ __launch_bounds__(1024) void k_diag_reduce(const double* __restrict__ part, int nb, double* __restrict__ out) {
-  const int a = blockIdx.x;
-  const double* row = part + (long)a * nb;
-  __shared__ double sh[1024];
-  const double init = a < 6 ? 0.0 : (a == 10 ? 1e300 : -1e300);
-  double v = init;
-  for (int b = threadIdx.x; b < nb; b += 1024) {
-    const double x = row[b];
-    v = a < 6 ? v + x : (a == 10 ? fmin(v, x) : fmax(v, x));
-  }
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  for (int o = 512; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      const double x = sh[threadIdx.x], y = sh[threadIdx.x + o];
-      sh[threadIdx.x] = a < 6 ? x + y : (a == 10 ? fmin(x, y) : fmax(x, y));
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[a] = sh[0];
-}
-
-// sums of the x and y marker forces (drag and lift before the -dX^3 factor)
-__global__ __launch_bounds__(1024) void k_marker_sums(const double* __restrict__ mf, long nmk, double* __restrict__ out) {
-  __shared__ double sh[1024];
-  for (int comp = 0; comp < 2; comp++) {
-    double v = 0.0;
-    for (long id = threadIdx.x; id < nmk; id += 1024) v += mf[comp * nmk + id];
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = 512; o > 0; o >>= 1) {
-      if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[comp] = sh[0];
-    __syncthreads();
-  }
-}
-
-size_t diag_scratch_words(const Grid& g) { return (size_t)12 * nblk(g.n, 256) + 16; }
-
-// log_progress quantities (fenep.f90:2279-2311) and the drag and lift of the
-// marker forces mf (nullptr: none), reduced on the device in `scratch`
-// (diag_scratch_words doubles, owned by the caller); 14 doubles come back.
-void f64_diag(Ctx& c, fp_diag* d, double* scratch, const double* mf) {
-  const Grid& g = c.g;
-  const int nb = nblk(g.n, 256);
-  double* out = scratch + (size_t)12 * nb;
-  hipLaunchKernelGGL(k_diag, dim3(nb), dim3(256), 0, c.stream, g, c.U, c.V, c.W, c.C[c.cur], c.nitr,
-                     c.p.beta != 1.0 ? 1 : 0, scratch);
-  hipLaunchKernelGGL(k_diag_reduce, dim3(12), dim3(1024), 0, c.stream, scratch, nb, out);
-  if (mf && c.nmk) hipLaunchKernelGGL(k_marker_sums, dim3(1), dim3(1024), 0, c.stream, mf, c.nmk, out + 12);
-  double h[14] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  FP_HIP_CHECK(hipMemcpyAsync(h, out, sizeof(double) * ((mf && c.nmk) ? 14 : 12), hipMemcpyDeviceToHost, c.stream));
-  FP_HIP_CHECK(hipStreamSynchronize(c.stream));
-  const double N = (double)g.n;
-  d->ke = (h[0] / 2.0) / N;
-  d->cfl = std::max(h[6] * g.dt / g.dx, std::max(h[7] * g.dt / g.dy, h[8] * g.dt / g.dz)) * 6.0;
-  d->trc_mean = h[1] / N;
-  d->trc_std = std::sqrt(std::max(0.0, h[2] / N - d->trc_mean * d->trc_mean));
-  d->trc_max = h[9];
-  d->trc_min = h[10];
-  d->div_max = h[11];
-  d->newton_itr_mean = h[3] / N;
-  d->newton_unconverged = h[5];
-  d->nan_flag = h[4] > 0 ? 1 : 0;
-  if (mf && c.nmk) {
-    d->drag = -(h[12] * g.sw);
-    d->lift = -(h[13] * g.sw);
-  }
-}
-
 }  // namespace fp

@@ -3515,6 +3515,12 @@ void mixed_velocity(Ctx& c, const float** u, const float** v, const float** w) {
   *u = X.U; *v = X.V; *w = X.W;
 }
 
+void mixed_fields(Ctx& c, const float** u, const float** v, const float** w, const float** C) {
+  mixed_velocity(c, u, v, w);
+  *C = MX(c).C[MX(c).cur];
+}
+const float* mixed_marker_forces32(Ctx& c) { return MX(c).mf; }
+
 void mixed_join(Ctx& c) {
   Mixed& X = MX(c);
   if (X.sel_ready) FP_HIP_CHECK(hipStreamWaitEvent(c.stream, X.sel_done, 0));

@@ -25,4 +25,6 @@ void mixed_step(Ctx& c);
 void mixed_join(Ctx& c);
 void mixed_physics(Ctx& c);   // after Wi, beta or Lp changed
 void mixed_velocity(Ctx& c, const float** u, const float** v, const float** w);  // FP32 state
+void mixed_fields(Ctx& c, const float** u, const float** v, const float** w, const float** C);
+const float* mixed_marker_forces32(Ctx& c);
 }  // namespace fp

@@ -25,153 +25,13 @@
 // at 64^3 340 and 228 us.  At 256 x 128 x 128 between walls the four solves
 // went from 1.16 to 0.46 ms; there the line solves' serial recurrence and the
 // LDS passes bound them.
-#include "fp_device.h"
+#include "fp_fft.h"
 #include <algorithm>
 #include <cmath>
 
 namespace fp {
 
 namespace {
-
-__device__ __forceinline__ int brev(int v, int bits) { return bits ? (int)(__brev((unsigned)v) >> (32 - bits)) : 0; }
-
-// one radix-2 butterfly of the Stockham form: (a, b) -> (a + b, (a - b) w)
-template <bool CONJ>
-__device__ __forceinline__ void bfly(double2& a, double2& b, double2 w) {
-  const double wi = CONJ ? -w.y : w.y;
-  const double dr = a.x - b.x, di = a.y - b.y;
-  a.x = a.x + b.x;
-  a.y = a.y + b.y;
-  b.x = dr * w.x - di * wi;
-  b.y = dr * wi + di * w.x;
-}
-
-// LR radix-2 stages, spans len/2, len/4, ..., on the 2^LR elements p + c
-// len/2^LR of one block: p the first one's place in the block, sh = log2(n /
-// len)
-template <int LR, bool CONJ>
-__device__ __forceinline__ void stages(double2 (&v)[1 << LR], int p, int step, int sh, const double2* tws) {
-  constexpr int R = 1 << LR;
-#pragma unroll
-  for (int s = 0; s < LR; s++) {
-    const int half = R >> (s + 1);
-#pragma unroll
-    for (int c = 0; c < half; c++) {
-      const double2 w = tws[(p + c * step) << (sh + s)];
-#pragma unroll
-      for (int b = 0; b < R; b += 2 * half) bfly<CONJ>(v[b + c], v[b + c + half], w);
-    }
-  }
-}
-
-// A set of 2^lnl lines of n = 2^L points in LDS: point r of line l at
-// X[r rs + l ls].  Consecutive threads take consecutive lines, whose stride
-// (1, or an odd pitch) keeps the 16-byte accesses off each other's banks.
-struct Lines {
-  double2* X;
-  int rs, ls, lnl, L;
-};
-
-// the LR stages from blocks of 2^ll points on; REV: the points lie
-// bit-reversed
-template <int LR, bool CONJ, bool REV>
-__device__ __forceinline__ void dif_pass(const Lines& f, int ll, const double2* tws) {
-  constexpr int R = 1 << LR;
-  const int n = 1 << f.L, step = 1 << (ll - LR);
-  for (int e = threadIdx.x; e < (n >> LR) << f.lnl; e += blockDim.x) {
-    const int l = e & ((1 << f.lnl) - 1), t = e >> f.lnl;
-    const int p = t & (step - 1), base = ((t >> (ll - LR)) << ll) + p;
-    double2* x = f.X + l * f.ls;
-    double2 v[R];
-    int at[R];
-#pragma unroll
-    for (int c = 0; c < R; c++) {
-      const int o = base + c * step;
-      at[c] = (REV ? brev(o, f.L) : o) * f.rs;
-      v[c] = x[at[c]];
-    }
-    stages<LR, CONJ>(v, p, step, f.L - ll, tws);
-#pragma unroll
-    for (int c = 0; c < R; c++) x[at[c]] = v[c];
-  }
-  __syncthreads();
-}
-
-// The stages of a transform of 2^L points in passes of M (2 or 3): forward,
-// what is left over comes first, as one shorter pass (M = 3, L = 1 mod 3: two
-// of two stages); the inverse mirrors it.
-__device__ __forceinline__ int lead_stages(int M, int L) { return M == 2 ? (L & 1) : (L % 3 == 1 ? 4 : L % 3); }
-// stages of the last forward pass and of the first inverse one
-__device__ __forceinline__ int last_stages(int M, int L) { return M == 3 && L != 2 && L != 4 ? 3 : 2; }
-
-// natural order in, bit-reversed out; all passes, or all but the last one
-template <int M, bool CONJ>
-__device__ void dif_from_natural(const Lines& f, const double2* tws, bool all = true) {
-  const int stop = all ? 0 : last_stages(M, f.L);
-  const int rest = f.L - lead_stages(M, f.L);
-  int ll = f.L;
-  if constexpr (M == 2) {
-    if (ll > rest) { dif_pass<1, CONJ, false>(f, ll, tws); ll--; }
-  } else {
-    for (; ll > rest && ll > stop; ll -= 2) dif_pass<2, CONJ, false>(f, ll, tws);
-  }
-  for (; ll > stop; ll -= M) dif_pass<M, CONJ, false>(f, ll, tws);
-}
-// bit-reversed in, natural order out; all passes, or all but the first one
-template <int M>
-__device__ void dif_from_reversed(const Lines& f, const double2* tws, bool all = true) {
-  const int lead = lead_stages(M, f.L);
-  int ll = f.L - (all ? 0 : last_stages(M, f.L));
-  for (; ll > lead; ll -= M) dif_pass<M, true, true>(f, ll, tws);
-  if constexpr (M == 2) {
-    if (ll > 0) dif_pass<1, true, true>(f, ll, tws);
-  } else {
-    for (; ll > 0; ll -= 2) dif_pass<2, true, true>(f, ll, tws);
-  }
-}
-
-// The last forward pass, op on every spectrum value, the first inverse pass:
-// both work on the same 2^LR elements (places t R + c, wavenumbers bitrev(c)
-// n/R + bitrev(t)), which stay in registers between them.
-template <int LR, typename Op>
-__device__ __forceinline__ void turn_pass(const Lines& f, const double2* tws, Op op) {
-  constexpr int R = 1 << LR;
-  const int n = 1 << f.L;
-  for (int e = threadIdx.x; e < (n >> LR) << f.lnl; e += blockDim.x) {
-    const int l = e & ((1 << f.lnl) - 1), t = e >> f.lnl;
-    double2* x = f.X + l * f.ls + t * R * f.rs;
-    double2 v[R], u[R];
-#pragma unroll
-    for (int c = 0; c < R; c++) v[c] = x[c * f.rs];
-    stages<LR, false>(v, 0, 1, f.L - LR, tws);
-    const int p = brev(t, f.L - LR), step = n >> LR;
-#pragma unroll
-    for (int c = 0; c < R; c++) {
-      // static bit reversal of c in LR bits
-      const int rc = LR == 2 ? ((c & 1) << 1 | c >> 1) : ((c & 1) << 2 | (c & 2) | c >> 2);
-      u[rc] = op(l, p + rc * step, v[c]);
-    }
-    stages<LR, true>(u, p, step, 0, tws);
-#pragma unroll
-    for (int c = 0; c < R; c++) {
-      const int rc = LR == 2 ? ((c & 1) << 1 | c >> 1) : ((c & 1) << 2 | (c & 2) | c >> 2);
-      x[c * f.rs] = u[rc];
-    }
-  }
-  __syncthreads();
-}
-template <int M, typename Op>
-__device__ __forceinline__ void turn(const Lines& f, const double2* tws, Op op) {
-  if (M == 2 || last_stages(M, f.L) == 2) turn_pass<2>(f, tws, op);
-  else turn_pass<3>(f, tws, op);
-}
-
-__device__ __forceinline__ int log2i(int n) { return __ffs(n) - 1; }
-
-// twiddles exp(-2 pi i t/n), t < n/2, into LDS (no barrier)
-__device__ __forceinline__ void load_tw(double2* tws, const double2* __restrict__ tw, int n) {
-  for (int e = threadIdx.x; e < n / 2; e += blockDim.x) tws[e] = tw[e];
-}
 
 // divides a spectrum value by N and the operator of the periodic problem
 // (fenep.f90:1458-1462, 1540-1548): kinds 0-2 Helmholtz, 3 Poisson.  N is a
@@ -191,35 +51,52 @@ struct Divide {
 
 // ------------------------------------------------------------- x transforms
 // Real x-lines -> half spectrum, 2^lnl consecutive (y, z) lines per block and
-// component blockIdx.y.  DIV: the line values are the divergence of u* / dt
-// (the Poisson right-hand side, fenep.f90:1550-1552), formed here from u* = q.
-template <int M, int DIV, bool WL>
-__global__ __launch_bounds__(256) void k_x_forward(Grid g, const double* __restrict__ q, double2* __restrict__ spec,
+// component comp + blockIdx.y.  The line values: Plain: q, one plane per
+// component; Div: the divergence of u* / dt (the Poisson right-hand side,
+// fenep.f90:1550-1552) of the planes u, v, w; Regular: the velocity u, v, w less
+// the mean um (nullptr: none) at the cell centres.
+enum class Line { Plain, Div, Regular };
+template <typename T>
+struct LineSrc {
+  const T *u, *v, *w;
+  const double* um;
+};
+template <int M, Line S, bool WL, typename T>
+__global__ __launch_bounds__(256) void k_x_forward(Grid g, LineSrc<T> q, int comp, double2* __restrict__ spec,
                                                    const double2* __restrict__ tw, int lnl) {
   extern __shared__ double2 lds[];
   const int n = g.nx, L = g.lnx, nl = 1 << lnl, pitch = n + 1;
   double2* tws = lds + nl * pitch;
   const long plane = (long)g.ny * g.nz, l0 = (long)blockIdx.x << lnl;
+  comp += blockIdx.y;
   load_tw(tws, tw, n);
-  const double* src = DIV ? q : q + blockIdx.y * g.n;
   for (int e = threadIdx.x; e < nl << L; e += blockDim.x) {
     const int l = e >> L, i = e & (n - 1);
     const long m = (l0 + l) * n + i;
     double v;
-    if (DIV) {
-      int ii, j, k;
-      cell_ijk(g, m, ii, j, k);
-      const double *U = q, *V = q + g.n, *W = q + 2 * g.n;
-      v = (((-ldbw<WL>(U, g, i - 1, j, k, BC_U) + ldbw<WL>(U, g, i, j, k, BC_U)) / g.dx
-            + (-ldbw<WL>(V, g, i, j - 1, k, BC_V) + ldbw<WL>(V, g, i, j, k, BC_V)) / g.dy)
-           + (-ldbw<WL>(W, g, i, j, k - 1, BC_W) + ldbw<WL>(W, g, i, j, k, BC_W)) / g.dz) / g.dt;
+    int ii, j, k;
+    cell_ijk(g, m, ii, j, k);
+    if constexpr (S == Line::Plain) {
+      v = q.u[comp * g.n + m];
+    } else if constexpr (S == Line::Div) {
+      v = (((-ldbw<WL>(q.u, g, i - 1, j, k, BC_U) + ldbw<WL>(q.u, g, i, j, k, BC_U)) / g.dx
+            + (-ldbw<WL>(q.v, g, i, j - 1, k, BC_V) + ldbw<WL>(q.v, g, i, j, k, BC_V)) / g.dy)
+           + (-ldbw<WL>(q.w, g, i, j, k - 1, BC_W) + ldbw<WL>(q.w, g, i, j, k, BC_W)) / g.dz) / g.dt;
     } else {
-      v = src[m];
+      const T* f = comp == 0 ? q.u : (comp == 1 ? q.v : q.w);
+      const int a = comp == 0, b = comp == 1, c = comp == 2;
+      double x = (double)f[m], y = (double)ldbw<WL>(f, g, i - a, j - b, k - c, BC_U + comp);
+      if (q.um) {
+        const double* mean = q.um + comp * g.n;
+        x = x - mean[m];
+        y = y - ldbw<WL>(mean, g, i - a, j - b, k - c, BC_U + comp);
+      }
+      v = (x + y) / 2.0;
     }
     lds[l * pitch + i] = make_double2(v, 0.0);
   }
   __syncthreads();
-  const Lines f{lds, 1, pitch, lnl, L};
+  const Lines<double2> f{lds, 1, pitch, lnl, L};
   dif_from_natural<M, false>(f, tws);
   double2* out = spec + blockIdx.y * (plane * g.nxh) + l0;
   for (int e = threadIdx.x; e < g.nxh << lnl; e += blockDim.x) {
@@ -246,7 +123,7 @@ __global__ __launch_bounds__(256) void k_x_inverse(Grid g, const double2* __rest
     if (i > 0 && i < h) lds[l * pitch + (n - i)] = make_double2(v.x, -v.y);
   }
   __syncthreads();
-  const Lines f{lds, 1, pitch, lnl, L};
+  const Lines<double2> f{lds, 1, pitch, lnl, L};
   dif_from_natural<M, true>(f, tws);
   double* o = out + blockIdx.y * g.n + l0 * n;
   for (int e = threadIdx.x; e < nl << L; e += blockDim.x) o[e] = lds[(e >> L) * pitch + brev(e & (n - 1), L)].x;
@@ -398,7 +275,7 @@ __global__ __launch_bounds__(1024) void k_slab(Grid g, double2* __restrict__ spe
   if (!WL) load_tw(ty, twy, ny);
   for (int e = threadIdx.x; e < ny * nz; e += blockDim.x) lds[(e >> g.lny) * pitch + (e & (ny - 1))] = base[e];
   __syncthreads();
-  const Lines fy{lds, 1, pitch, lnz, g.lny}, fz{lds, pitch, 1, g.lny, lnz};
+  const Lines<double2> fy{lds, 1, pitch, lnz, g.lny}, fz{lds, pitch, 1, g.lny, lnz};
   if constexpr (!WL) {
     dif_from_natural<M, false>(fy, ty);
     dif_from_natural<M, false>(fz, tz, false);
@@ -432,7 +309,7 @@ __global__ __launch_bounds__(256) void k_y_lines(Grid g, double2* __restrict__ s
   load_tw(tws, tw, n);
   for (int e = threadIdx.x; e < nl << g.lny; e += blockDim.x) lds[(e >> g.lny) * pitch + (e & (n - 1))] = base[e];
   __syncthreads();
-  const Lines f{lds, 1, pitch, lnl, g.lny};
+  const Lines<double2> f{lds, 1, pitch, lnl, g.lny};
   if (inv) dif_from_reversed<M>(f, tws);
   else dif_from_natural<M, false>(f, tws);
   for (int e = threadIdx.x; e < nl << g.lny; e += blockDim.x) base[e] = lds[(e >> g.lny) * pitch + (e & (n - 1))];
@@ -453,7 +330,7 @@ __global__ __launch_bounds__(256) void k_z_lines(Grid g, double2* __restrict__ s
   load_tw(tws, tw, n);
   for (int e = threadIdx.x; e < n << lnl; e += blockDim.x) lds[e] = base[((long)(e >> lnl) << g.lny) + (e & (nl - 1))];
   __syncthreads();
-  const Lines f{lds, nl, 1, lnl, L};
+  const Lines<double2> f{lds, nl, 1, lnl, L};
   if (mode == 0) {
     dif_from_natural<M, false>(f, tws);
   } else if (mode == 1) {
@@ -471,18 +348,6 @@ __global__ __launch_bounds__(256) void k_z_lines(Grid g, double2* __restrict__ s
 // -------------------------------------------------------------------- host
 namespace {
 
-inline int lg(int n) { int l = 0; while ((1 << l) < n) l++; return l; }
-
-// log2 of the lines of n points a block holds: 16 where they take at most 33
-// KB of LDS (four blocks per CU), fewer for long lines, and fewer (4 at
-// least) while the launch would leave CUs without a block
-int lines_log2(int n, long lines, int comps) {
-  int l = std::max(2, std::min(4, 11 - lg(n)));
-  while (l > 2 && (lines >> l) * comps < 512) l--;
-  while (l > 0 && (1L << l) > lines) l--;
-  return l;
-}
-size_t lds_lines(int n, int lnl) { return sizeof(double2) * (((size_t)(n + 1) << lnl) + n / 2); }
 size_t lds_slab64(const Grid& g) {
   size_t w = sizeof(double2) * ((size_t)g.nz * (g.ny + 1) + g.nz / 2);
   return w + (g.walls ? sizeof(double) * (size_t)g.ny * g.nz : sizeof(double2) * (g.ny / 2));
@@ -518,14 +383,15 @@ int stages_per_pass(const Grid& g, int comps) { return g.n * comps <= (1L << 20)
 int threads_for(long points, int M) { return (int)std::max(64L, std::min(256L, points >> M)); }
 
 // the transforms along one axis of `comps` components
-void x_forward(Ctx& c, int comps, const double* q, bool div) {
+template <Line S, bool WL, typename T>
+void x_forward(Ctx& c, int comp, int comps, const LineSrc<T>& q) {
   const Grid& g = c.g;
   const long lines = (long)g.ny * g.nz;
   const int lx = lines_log2(g.nx, lines, comps), M = stages_per_pass(g, comps);
-  auto k = M == 2 ? (div ? (g.walls ? k_x_forward<2, 1, true> : k_x_forward<2, 1, false>) : k_x_forward<2, 0, false>)
-                  : (div ? (g.walls ? k_x_forward<3, 1, true> : k_x_forward<3, 1, false>) : k_x_forward<3, 0, false>);
+  auto k = M == 2 ? k_x_forward<2, S, WL, T> : k_x_forward<3, S, WL, T>;
+  if (lds_lines(g.nx, lx) > 65536) allow_lds(k, (int)lds_lines(g.nx, lx));
   hipLaunchKernelGGL(k, dim3((unsigned)(lines >> lx), comps), dim3(threads_for((long)g.nx << lx, M)), lds_lines(g.nx, lx),
-                     c.stream, g, q, c.spec, c.twx, lx);
+                     c.stream, g, q, comp, c.spec, c.twx, lx);
 }
 void x_inverse(Ctx& c, int comps, double* x) {
   const Grid& g = c.g;
@@ -553,7 +419,10 @@ void z_lines(Ctx& c, int comps, int mode, int kind0, double rn) {
 void solve(Ctx& c, int kind0, int comps, const double* q, double* x, bool div) {
   const Grid& g = c.g;
   hipStream_t s = c.stream;
-  x_forward(c, comps, q, div);
+  const LineSrc<double> src{q, q + g.n, q + 2 * g.n, nullptr};
+  if (!div) x_forward<Line::Plain, false>(c, 0, comps, src);
+  else if (g.walls) x_forward<Line::Div, true>(c, 0, comps, src);
+  else x_forward<Line::Div, false>(c, 0, comps, src);
   const double rn = 1.0 / (double)(g.walls ? (long)g.nx * g.nz : g.n);
   const long tstride = (long)g.nxh * (g.ny + 1) * g.nz;
   if (g.walls && (!c.piv || c.piv_beta != g.beta)) line_pivots(c);
@@ -592,12 +461,6 @@ void f64_spectral_create(Ctx& c) {
   c.slab64 = lds_slab64(g) <= (size_t)lds_max;
   allow_lds(k_slab<2, false>, lds_max);
   allow_lds(k_slab<2, true>, lds_max);
-  allow_lds(k_x_forward<2, 0, false>, lds_max);
-  allow_lds(k_x_forward<2, 1, false>, lds_max);
-  allow_lds(k_x_forward<2, 1, true>, lds_max);
-  allow_lds(k_x_forward<3, 0, false>, lds_max);
-  allow_lds(k_x_forward<3, 1, false>, lds_max);
-  allow_lds(k_x_forward<3, 1, true>, lds_max);
   allow_lds(k_x_inverse<2>, lds_max);
   allow_lds(k_x_inverse<3>, lds_max);
   allow_lds(k_y_lines<2>, lds_max);
@@ -621,12 +484,19 @@ void f64_helmholtz(Ctx& c, const double* q, double* x) {
 // the Poisson equation lap_h x = div_h up / dt
 void f64_poisson(Ctx& c, const double* up, double* x) { solve(c, 3, 1, up, x, true); }
 
-// forward transform of one periodic field into c.spec, wavenumbers m at
-// bitrev(m) in y and z (f64_energy_spectrum)
-void f64_forward(Ctx& c, const double* q) {
-  x_forward(c, 1, q, false);
-  y_lines(c, 1, 0);
-  z_lines(c, 1, 0, 3, 1.0);
+// forward transforms of the regular-grid velocity (periodic grids; the
+// wavenumbers m of y and z at bitrev(m))
+template <typename T>
+static void forward_regular(Ctx& c, const T* U, const T* V, const T* W, int comp, int comps) {
+  x_forward<Line::Regular, false>(c, comp, comps, LineSrc<T>{U, V, W, c.mean_u});
+  y_lines(c, comps, 0);
+  z_lines(c, comps, 0, 3, 1.0);
+}
+void f64_forward_regular(Ctx& c, const double* U, const double* V, const double* W, int comp, int comps) {
+  forward_regular(c, U, V, W, comp, comps);
+}
+void f64_forward_regular(Ctx& c, const float* U, const float* V, const float* W, int comp, int comps) {
+  forward_regular(c, U, V, W, comp, comps);
 }
 
 }  // namespace fp
