@@ -95,9 +95,9 @@ __global__ __launch_bounds__(256) void k_adj_div(Grid g, const double* __restric
 }
 
 // d/dbeta through the Helmholtz operator H = 1 - (dt beta/2Re) lap:
-// (dt/2Re) <Rbar_c, lap u*_c>
+// (dt/2Re) <Rbar_c, lap u*_c>.  Qb, if given, receives a copy of Rbar.
 __global__ __launch_bounds__(256) void k_adj_helm_beta(Grid g, const double* __restrict__ Rb, const double* __restrict__ up,
-                                                       double* __restrict__ part) {
+                                                       double* __restrict__ part, double* __restrict__ Qb) {
   const long m = blockIdx.x * (long)blockDim.x + threadIdx.x;
   double sb = 0.0;
   if (m < g.n) {
@@ -112,6 +112,7 @@ __global__ __launch_bounds__(256) void k_adj_helm_beta(Grid g, const double* __r
       const double lap = (X[mx] - 2.0 * X[m] + X[px]) * ix2 + (X[my] - 2.0 * X[m] + X[py]) * iy2 +
                          (X[mz] - 2.0 * X[m] + X[pz]) * iz2;
       sb += Rb[c * n + m] * lap;
+      if (Qb) Qb[c * n + m] = Rb[c * n + m];
     }
     sb *= g.dt / (2.0 * g.re);
   }
@@ -125,41 +126,33 @@ __global__ __launch_bounds__(256) void k_adj_helm_beta(Grid g, const double* __r
 // R = Ua + dt f - dt B/2; D = -sum Fcx W (W the spreading weight g.sw, dX^3
 // by default).  With Rbar given: Fcbar = dt spread^T(Rbar) - w W e_x and
 // Uabar = Rbar + interp^T(-Fcbar/dt).
-// This kernel writes gm = -Fcbar/dt (times dX^3 / W) per marker and component.
-__global__ __launch_bounds__(256) void k_adj_ibm_markers(Grid g, long nmk, int nc, int nl, const double* __restrict__ mk,
-                                                         const double* __restrict__ w, const double* __restrict__ Rb,
-                                                         double wdrag, double* __restrict__ gm) {
+// This kernel writes gm = -Fcbar/dt (times dX^3 / W) per marker and component
+// (a thread each, its 27 loads ahead of the ordered sum: latency, as in the
+// forward step); interp^T is then added to the copy of Rbar that
+// k_adj_helm_beta makes, at the forced cells only.
+__global__ __launch_bounds__(64) void k_adj_ibm_markers(Grid g, long nmk, int nc, int nl, const double* __restrict__ mk,
+                                                        const double* __restrict__ w, const double* __restrict__ Rb,
+                                                        double wdrag, double* __restrict__ gm) {
   const long id = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (id >= nmk) return;
+  const int c = blockIdx.y;
   const int n = (int)(id / ((long)nc * nl)) + 1;
-  const double xc = mk[id], yc = mk[nmk + id];
-  for (int c = 0; c < 3; c++) {
-    int i0, j0;
-    ibm_origin_d(g, c, xc, yc, i0, j0);
-    const double* X = Rb + c * g.n;
-    const double* wm = w + (c * nmk + id) * 27;   // the interpolation weights
-    double acc = 0.0;
-    int slot = 0;
-    for (int kk = n - 1; kk <= n + 1; kk++)
-      for (int jj = j0; jj <= j0 + 2; jj++)
-        for (int ii = i0; ii <= i0 + 2; ii++, slot++)
-          acc += X[pidx(g, ii - 1, jj - 1, kk - 1)] * wm[slot] * g.sw;
-    const double fbar = g.dt * acc - (c == 0 ? g.sw * wdrag : 0.0);
-    // interp^T(x) = spread(x) dX^3 / W: the spread kernels apply W
-    gm[c * nmk + id] = (-fbar / g.dt) * (((g.dx * g.dx) * g.dx) / g.sw);
+  int i0, j0;
+  ibm_origin_d(g, c, mk[id], mk[nmk + id], i0, j0);
+  const double* X = Rb + c * g.n;
+  const double* wm = w + (long)c * 27 * nmk + id;   // the interpolation weights
+  double v[27], wv[27];
+#pragma unroll
+  for (int q = 0; q < 27; q++) {
+    v[q] = X[pidx(g, i0 - 1 + q % 3, j0 - 1 + q / 3 % 3, n - 2 + q / 9)];
+    wv[q] = wm[q * nmk];
   }
-}
-
-__global__ __launch_bounds__(256) void k_adj_ibm_q(Grid g, const double* __restrict__ Rb, const double* __restrict__ ft,
-                                                   double* __restrict__ Qb) {
-  const long e = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (e >= 3 * g.n) return;
-  const int c = (int)(e / g.n);
-  const long m = e % g.n;
-  int i, j, k;
-  cell_ijk(g, m, i, j, k);
-  const long gx = g.nx + 2, gy = g.ny + 2, gn = gx * gy * (g.nz + 2);
-  Qb[e] = Rb[e] + ft[c * gn + (i + 1) + gx * ((j + 1) + gy * (long)(k + 1))];
+  double acc = 0.0;
+#pragma unroll
+  for (int q = 0; q < 27; q++) acc += v[q] * wv[q] * g.sw;
+  const double fbar = g.dt * acc - (c == 0 ? g.sw * wdrag : 0.0);
+  // interp^T(x) = spread(x) dX^3 / W: the spread kernel applies W
+  gm[c * nmk + id] = (-fbar / g.dt) * (((g.dx * g.dx) * g.dx) / g.sw);
 }
 
 // ------------------------------------------------------- predictor^T
@@ -739,14 +732,14 @@ void adjoint_step(Ctx& c, Adj& a, int t, int seg_len, int s, double wdrag) {
   hipLaunchKernelGGL(k_adj_div, dim3(nb), dim3(256), 0, st, g, a.bb, a.ubs);
   // Helmholtz
   f64_helmholtz(c, a.ubs, a.Rb);
-  hipLaunchKernelGGL(k_adj_helm_beta, dim3(nb), dim3(256), 0, st, g, a.Rb, Up, a.part);
+  const bool ibm = c.p.method == FP_METHOD_IBM;
+  hipLaunchKernelGGL(k_adj_helm_beta, dim3(nb), dim3(256), 0, st, g, a.Rb, Up, a.part, ibm ? a.Qb : nullptr);
   // immersed boundary
   const double* Qb = a.Rb;
-  if (c.p.method == FP_METHOD_IBM) {
-    hipLaunchKernelGGL(k_adj_ibm_markers, dim3(nblk(c.nmk, 256)), dim3(256), 0, st, g, c.nmk, c.nc, c.nl, c.mk, c.ib_w,
+  if (ibm) {
+    hipLaunchKernelGGL(k_adj_ibm_markers, dim3(nblk(c.nmk, 64), 3), dim3(64), 0, st, g, c.nmk, c.nc, c.nl, c.mk, c.ib_w,
                        a.Rb, wdrag, a.gm);
-    f64_spread_markers(c, a.gm, c.ftmp);
-    hipLaunchKernelGGL(k_adj_ibm_q, dim3(nblk(3 * n, 256)), dim3(256), 0, st, g, a.Rb, c.ftmp, a.Qb);
+    f64_spread_add(c, a.gm, a.Qb);
     Qb = a.Qb;
   }
   // predictor

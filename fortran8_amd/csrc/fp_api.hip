@@ -226,7 +226,7 @@ int fp_create(const fp_params* p, void** out) {
     dalloc(&c->U, n); dalloc(&c->V, n); dalloc(&c->W, n); dalloc(&c->P, n); dalloc(&c->Phi, n);
     dalloc(&c->C[0], 6 * n); dalloc(&c->C[1], 6 * n);
     dalloc(&c->fC, n); dalloc(&c->sel, n); dalloc(&c->nitr, n);
-    dalloc(&c->A0, 3 * n); dalloc(&c->T0, 3 * n); dalloc(&c->B0, 3 * n); dalloc(&c->B, 3 * n);
+    dalloc(&c->A0, 3 * n); dalloc(&c->T0, 3 * n); dalloc(&c->B0, 3 * n);
     // (Q also holds the lists of the selection: 1536 words per 256 cells)
     dalloc(&c->Q, std::max<long>(3 * n, 768)); dalloc(&c->Up, 3 * n);
     dalloc(&c->sel_count, 1);
@@ -269,12 +269,13 @@ int fp_destroy(void* vc) {
   f64_sor_destroy(*c);
   dfree(c->U); dfree(c->V); dfree(c->W); dfree(c->P); dfree(c->Phi);
   dfree(c->C[0]); dfree(c->C[1]); dfree(c->fC); dfree(c->sel); dfree(c->sel_count); dfree(c->nitr);
-  dfree(c->A0); dfree(c->T0); dfree(c->B0); dfree(c->B); dfree(c->Q); dfree(c->Up); dfree(c->F);
+  dfree(c->A0); dfree(c->T0); dfree(c->B0); dfree(c->Q); dfree(c->Up); dfree(c->F);
   dfree(c->spec); dfree(c->piv); dfree(c->red); dfree(c->part);
   dfree(c->twx); dfree(c->twy); dfree(c->twz); dfree(c->kx2); dfree(c->ky2); dfree(c->kz2);
-  dfree(c->mk); dfree(c->mf); dfree(c->mb); dfree(c->ftmp);
+  dfree(c->mk); dfree(c->mf);
   dfree(c->mean_acc); dfree(c->mean_u); dfree(c->stat);
   for (int k = 0; k < 3; k++) { dfree(c->sp_row[k]); dfree(c->sp_tgt[k]); dfree(c->sp_ent[k]); dfree(c->sp_w[k]); }
+  for (int k = 0; k < 3; k++) { dfree(c->fc_cell[k]); dfree(c->fc_row[k]); dfree(c->fc_img[k]); }
   dfree(c->ib_w);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -416,10 +417,9 @@ int fp_set_markers(void* vc, int nc, int nl, const double* xc, const double* yc,
       if (!(x >= 0.5 * g.dx && x <= (g.nx - 0.5) * g.dx && y >= 1.5 * g.dy && y <= (g.ny - 1.5) * g.dy))
         return fail(c, FP_E_ARG, "marker too close to the domain boundary");
     }
-    dfree(c->mk); dfree(c->mf); dfree(c->mb); dfree(c->ftmp);
+    dfree(c->mk); dfree(c->mf);
     c->nc = nc; c->nl = nl; c->nmk = nmk;
-    dalloc(&c->mk, 6 * nmk); dalloc(&c->mf, 3 * nmk); dalloc(&c->mb, 3 * nmk);
-    dalloc(&c->ftmp, 3 * c->gn);
+    dalloc(&c->mk, 6 * nmk); dalloc(&c->mf, 3 * nmk);
     const double* src[6] = {xc, yc, zc, uc, vc_, wc};
     for (int a = 0; a < 6; a++) FP_HIP_CHECK(hipMemcpy(c->mk + a * nmk, src[a], sizeof(double) * nmk, hipMemcpyHostToDevice));
     f64_ibm_setup(*c);

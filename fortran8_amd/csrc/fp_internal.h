@@ -44,7 +44,7 @@ struct Ctx {
   double *fC = nullptr;               // Peterlin factor of the current C
   uint8_t* sel = nullptr;
   unsigned* sel_count = nullptr;      // FP64 step: selections left to FP64
-  double *A0 = nullptr, *T0 = nullptr, *B0 = nullptr, *B = nullptr;  // 3 planes each
+  double *A0 = nullptr, *T0 = nullptr, *B0 = nullptr;  // 3 planes each
   double *Q = nullptr;                // 3 planes: predictor RHS / Ua
   double *Up = nullptr;               // 3 planes: u*
   double *F = nullptr;                // 3 planes body-force field (nullable)
@@ -63,15 +63,17 @@ struct Ctx {
   long nmk = 0;
   double* mk = nullptr;               // 6 planes: xc,yc,zc,uc,vc,wc
   double* mf = nullptr;               // 3 planes: Fxc,Fyc,Fzc
-  double* mb = nullptr;               // 3 planes: Ub,Vb,Wb
-  double* ftmp = nullptr;             // 3 ghosted raw spread arrays
   long gn = 0;
   int* sp_row[3] = {nullptr, nullptr, nullptr};   // CSR row pointers
   long* sp_tgt[3] = {nullptr, nullptr, nullptr};  // ghosted target index
   int* sp_ent[3] = {nullptr, nullptr, nullptr};   // marker of each entry
   int sp_rows[3] = {0, 0, 0};
   double* sp_w[3] = {nullptr, nullptr, nullptr};  // weight of each entry (ibm_weight)
-  double* ib_w = nullptr;             // interpolation weights, (3 nmk) x 27 stencil points
+  long* fc_cell[3] = {nullptr, nullptr, nullptr}; // forced cells
+  int* fc_row[3] = {nullptr, nullptr, nullptr};   // their CSR row, or -1 - index into fc_img
+  int* fc_img[3] = {nullptr, nullptr, nullptr};   // rows of the cells with ghost images (-1: none)
+  int fc_cells[3] = {0, 0, 0};
+  double* ib_w = nullptr;             // interpolation weights, 3 x 27 stencil points x nmk
   // SOR
   double sor_itr = -1.0;
   double* sor_part = nullptr;         // sums of E^2 per sweep of a batch and block
@@ -105,7 +107,7 @@ void f64_cstar_newton(Ctx& c);
 void f64_predictor(Ctx& c);
 void f64_divergence(Ctx& c, const double* up, double* q);
 void f64_march(Ctx& c);
-void f64_ibm(Ctx& c);        // interp + forces + spread + predictor RHS into Q
+void f64_ibm(Ctx& c);        // marker forces, and the forced cells of the right-hand side Up
 void f64_ibm_setup(Ctx& c);  // CSR build (host) after markers are set
 void f64_sor_create(Ctx& c);
 void f64_sor_destroy(Ctx& c);
@@ -121,7 +123,7 @@ int f64_energy_spectrum_z(Ctx& c, int ncyl, const double* xy, double diameter, d
 void f64_mean_accumulate(Ctx& c, const float* u32, const float* v32, const float* w32);
 int f64_mean_apply(Ctx& c, int mode);
 void f64_fill_f(Ctx& c);     // Peterlin factor of the current C
-void f64_spread_markers(Ctx& c, const double* mfield, double* ftmp);  // spread + ghost folds
+void f64_spread_add(Ctx& c, const double* mfield, double* out);  // out += spread of marker values
 // ---- spectral solves (fp_spectral_f64.hip)
 void f64_spectral_create(Ctx& c);
 void f64_solve(Ctx& c, int kind, const double* q, double* x);   // kind 0..2 Helmholtz, 3 Poisson

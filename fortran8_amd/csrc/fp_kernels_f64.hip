@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256) void k_predictor(Grid g, int method, int first
                                                    const double* __restrict__ W, const double* __restrict__ P,
                                                    const double* __restrict__ C, const double* __restrict__ fC,
                                                    double* __restrict__ A0, double* __restrict__ T0, double* __restrict__ B0,
-                                                   double* __restrict__ Bout, const double* __restrict__ F,
+                                                   double* __restrict__ Rout, const double* __restrict__ F,
                                                    double bf0, double bf1, double bf2, double* __restrict__ Q) {
   const long L = xcd_cell();
   if (L >= g.n) return;
@@ -276,7 +276,12 @@ __global__ __launch_bounds__(256) void k_predictor(Grid g, int method, int first
     A0[o] = a[c];
     T0[o] = t[c];
     B0[o] = bv[c];
-    if (Bout) Bout[o] = bv[c];
+    // ibm_predict's right-hand side where no marker reaches (f = 0): the wall
+    // row of V counts as 0 there
+    if (Rout) {
+      const bool wall = WL && c == 1 && j == g.ny - 1;
+      Rout[o] = ((wall ? 0.0 : r) + 0.0) - (dt * bv[c]) / 2.0;
+    }
   }
 #undef Ug
 #undef Vg
@@ -332,59 +337,119 @@ __global__ __launch_bounds__(256) void k_march(Grid g, int explicit_p, const dou
 }
 
 // ============================================================ IBM ==========
+// A step's IBM work is two launches: marker forces from Ua (k_ibm_forces), and
+// the forced cells of the Helmholtz right-hand side (k_ibm_spread<true>), whose
+// other cells the predictor has written.  Both are latency: short chains of
+// dependent loads, so every thread has one sum only and its loads are issued
+// ahead of the ordered additions.  256x128x128 between walls, 8 cylinders:
+// 300 -> 82 us a step with the ghosted array, its folds and its pass gone.
+
 // interpolation and marker forces of ibm_Helmholtz (fenep.f90:2076-2119,
-// forces kept as in fenep_mpi.f90:1845-1853)
+// forces kept as in fenep_mpi.f90:1845-1853), one thread per marker and
+// component: a marker per thread left 64^3 with 4 blocks (22 us).
 // w: the 27 weights ibm_weight of each marker and component (k_ibm_interp_w).
-__global__ __launch_bounds__(256) void k_ibm_interp(Grid g, long nmk, int nc, int nl, const double* __restrict__ mk,
-                                                    const double* __restrict__ w, const double* __restrict__ ua,
-                                                    double* __restrict__ mb, double* __restrict__ mf) {
-  long id = blockIdx.x * (long)blockDim.x + threadIdx.x;
+template <bool WL>
+__global__ __launch_bounds__(64) void k_ibm_forces(Grid g, long nmk, int nc, int nl, const double* __restrict__ mk,
+                                                   const double* __restrict__ w, const double* __restrict__ ua,
+                                                   double* __restrict__ mf) {
+  const long id = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (id >= nmk) return;
-  int n = (int)(id / ((long)nc * nl)) + 1;
-  double xc = mk[id], yc = mk[nmk + id];
+  const int c = blockIdx.y;
+  const int n = (int)(id / ((long)nc * nl)) + 1;
   const double dx3 = (g.dx * g.dx) * g.dx;
-  for (int c = 0; c < 3; c++) {
-    int i0, j0; ibm_origin_d(g, c, xc, yc, i0, j0);
-    const double* X = ua + c * g.n;
-    const double* wm = w + (c * nmk + id) * 27;
-    int kind = c == 0 ? BC_U : (c == 1 ? BC_V : BC_W);
-    double acc = 0.0;
-    int slot = 0;
-    for (int kk = n - 1; kk <= n + 1; kk++)
-      for (int jj = j0; jj <= j0 + 2; jj++)
-        for (int ii = i0; ii <= i0 + 2; ii++, slot++) {
-          double v = ldb(X, g, ii - 1, jj - 1, kk - 1, kind);
-          acc = acc + (v * wm[slot]) * dx3;
-        }
-    mb[c * nmk + id] = acc;
-    double uc = mk[(3 + c) * nmk + id];
-    mf[c * nmk + id] = 0.0 + (uc - acc) / g.dt;
+  int i0, j0; ibm_origin_d(g, c, mk[id], mk[nmk + id], i0, j0);
+  const double* X = ua + c * g.n;
+  const double* wm = w + (long)c * 27 * nmk + id;
+  const int kind = c == 0 ? BC_U : (c == 1 ? BC_V : BC_W);
+  double v[27], wv[27];
+#pragma unroll
+  for (int q = 0; q < 27; q++) {
+    v[q] = ldbw<WL>(X, g, i0 - 1 + q % 3, j0 - 1 + q / 3 % 3, n - 2 + q / 9, kind);
+    wv[q] = wm[q * nmk];
   }
+  double acc = 0.0;
+#pragma unroll
+  for (int q = 0; q < 27; q++) acc = acc + (v[q] * wv[q]) * dx3;
+  mf[c * nmk + id] = 0.0 + (mk[(3 + c) * nmk + id] - acc) / g.dt;
 }
 
 // spreading (fenep.f90:2125-2162) as a gather over the CSR of contributions
-// of each ghosted target, in the reference's marker loop order.
-// (w: each entry's weight, k_ibm_spread_w).  The three components in one
-// launch: component blockIdx.y, its CSR and its ghosted array ft0 + comp gn.
+// of each ghosted target, in the reference's marker loop order
+// (w: each entry's weight, k_ibm_spread_w), and the folds of ibm_PBM
+// (fenep.f90:2195-2205) over each cell's ghost images.  A row that no marker
+// reaches, and an image that does not exist, is the +0 of the cleared array;
+// a sum begun at +0 is never -0, so adding it changes no bit.
+// Three components: grid row blockIdx.y.
 struct SpreadCsr {
   const int* rowp[3];
-  const long* tgt[3];
   const int* ent[3];
   const double* w[3];
-  int rows[3];
+  const long* cell[3];   // forced cells
+  const int* row[3];     // their row; -1 - q: the 8 rows img[8q ..] (-1: none)
+  const int* img[3];
+  int cells[3];
 };
-__global__ __launch_bounds__(256) void k_ibm_spread(Grid g, SpreadCsr cs, long nmk, const double* __restrict__ mf,
-                                                    double* __restrict__ ft0, long gn) {
-  const int comp = blockIdx.y;
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= cs.rows[comp]) return;
-  const int* __restrict__ rowp = cs.rowp[comp];
-  const int* __restrict__ ent = cs.ent[comp];
-  const double* __restrict__ w = cs.w[comp];
-  long t = cs.tgt[comp][r];
+__device__ __forceinline__ double spread_row(int r, const int* __restrict__ rowp, const int* __restrict__ ent,
+                                             const double* __restrict__ w, const double* __restrict__ mf, double sw) {
   double acc = 0.0;
-  for (int e = rowp[r]; e < rowp[r + 1]; e++) acc = acc + (mf[comp * nmk + ent[e]] * w[e]) * g.sw;
-  ft0[comp * gn + t] = acc;
+  if (r < 0) return acc;
+  const int e1 = rowp[r + 1];
+  for (int e = rowp[r]; e < e1; e += 8) {
+    double f[8], x[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int p = e + q < e1 ? e + q : e1 - 1;
+      f[q] = mf[ent[p]];
+      x[q] = w[p];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (e + q < e1) acc = acc + (f[q] * x[q]) * sw;
+  }
+  return acc;
+}
+// RHS: out = Ua + dt f - dt B/2, the right-hand side of ibm_predict
+// (fenep.f90:2229), with in = Ua and B this step's viscous term.
+// Otherwise out = in + f.
+template <bool RHS, bool WL>
+__global__ __launch_bounds__(64) void k_ibm_spread(Grid g, SpreadCsr cs, long nmk, const double* __restrict__ mf,
+                                                   const double* in, const double* __restrict__ B, double* out) {
+  const int c = blockIdx.y;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= cs.cells[c]) return;
+  const int* rowp = cs.rowp[c];
+  const int* ent = cs.ent[c];
+  const double* w = cs.w[c];
+  const double* mc = mf + c * nmk;
+  const long m = cs.cell[c][t], o = c * g.n + m;
+  const int r = cs.row[c][t];
+  double f;
+  if (r >= 0) {
+    f = spread_row(r, rowp, ent, w, mc, g.sw);
+  } else {
+    const int* im = cs.img[c] + 8L * (-1 - r);   // x fastest: the folds go x, y, z
+    f = 0.0;
+    for (int kk = 0; kk < 2; kk++) {
+      double z = 0.0;
+      for (int jj = 0; jj < 2; jj++) {
+        double y = 0.0;
+        for (int ii = 0; ii < 2; ii++) y = y + spread_row(*im++, rowp, ent, w, mc, g.sw);
+        z = z + y;
+      }
+      f = f + z;
+    }
+  }
+  if (RHS) {
+    double u = in[o];
+    if (WL && c == 1) {
+      int i, j, k;
+      cell_ijk(g, m, i, j, k);
+      u = ldbw<WL>(in + c * g.n, g, i, j, k, BC_V);
+    }
+    out[o] = (u + g.dt * f) - (g.dt * B[o]) / 2.0;
+  } else {
+    out[o] = in[o] + f;
+  }
 }
 
 // The weights depend only on the markers and the grid: ibm_weight of every
@@ -411,87 +476,49 @@ __global__ __launch_bounds__(256) void k_ibm_interp_w(Grid g, long nmk, int nc, 
   double xc = mk[id], yc = mk[nmk + id], zc = mk[2 * nmk + id];
   for (int c = 0; c < 3; c++) {
     int i0, j0; ibm_origin_d(g, c, xc, yc, i0, j0);
-    double* wm = w + (c * nmk + id) * 27;
-    int slot = 0;
+    double* wm = w + (long)c * 27 * nmk + id;   // point-major: the markers of a wavefront side by side
     for (int kk = n - 1; kk <= n + 1; kk++)
       for (int jj = j0; jj <= j0 + 2; jj++)
-        for (int ii = i0; ii <= i0 + 2; ii++, slot++) wm[slot] = ibm_weight(g, c, ii, jj, kk, xc, yc, zc);
+        for (int ii = i0; ii <= i0 + 2; ii++, wm += nmk) *wm = ibm_weight(g, c, ii, jj, kk, xc, yc, zc);
   }
 }
 
-// ibm_PBM fold (fenep.f90:2195-2205), one axis per launch, the component
-// (ghosted array ft + blockIdx.y gn) per grid row
-__global__ __launch_bounds__(256) void k_ibm_fold(Grid g, int axis, double* __restrict__ ft0, long gn) {
-  const long gx = g.nx + 2, gy = g.ny + 2, gz = g.nz + 2;
-  double* __restrict__ ft = ft0 + blockIdx.y * gn;
-  long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  auto G = [&](long i, long j, long k) { return i + gx * (j + gy * k); };
-  if (axis == 0) {
-    if (t >= gy * gz) return;
-    long j = t % gy, k = t / gy;
-    ft[G(1, j, k)] = ft[G(1, j, k)] + ft[G(g.nx + 1, j, k)];
-    ft[G(g.nx, j, k)] = ft[G(g.nx, j, k)] + ft[G(0, j, k)];
-  } else if (axis == 1) {
-    if (t >= gx * gz) return;
-    long i = t % gx, k = t / gx;
-    ft[G(i, 1, k)] = ft[G(i, 1, k)] + ft[G(i, g.ny + 1, k)];
-    ft[G(i, g.ny, k)] = ft[G(i, g.ny, k)] + ft[G(i, 0, k)];
-  } else {
-    if (t >= gx * gy) return;
-    long i = t % gx, j = t / gx;
-    ft[G(i, j, 1)] = ft[G(i, j, 1)] + ft[G(i, j, g.nz + 1)];
-    ft[G(i, j, g.nz)] = ft[G(i, j, g.nz)] + ft[G(i, j, 0)];
-  }
-}
-
-// ibm_predict right-hand side (fenep.f90:2229): Ua + dt f - dt B/2
-__global__ __launch_bounds__(256) void k_ibm_rhs(Grid g, const double* __restrict__ ua, const double* __restrict__ ft,
-                                                 const double* __restrict__ B, double* __restrict__ q) {
-  long m = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (m >= 3 * g.n) return;
-  int c = (int)(m / g.n);
-  long mm = m % g.n;
-  int i, j, k;
-  cell_ijk(g, mm, i, j, k);
-  const long gx = g.nx + 2, gy = g.ny + 2, gn = gx * gy * (g.nz + 2);
-  double f = ft[c * gn + (i + 1) + gx * ((j + 1) + gy * (long)(k + 1))];
-  int kind = c == 0 ? BC_U : (c == 1 ? BC_V : BC_W);
-  double u = ldb(ua + c * g.n, g, i, j, k, kind);
-  q[m] = (u + g.dt * f) - (g.dt * B[m]) / 2.0;
-}
-
-// spread of the marker values mfield (3 x nmk) onto the ghosted arrays ft
-// (3 x gn) followed by the ghost folds; rows of the CSR that no marker
-// reaches keep their previous (zero) value.
-void f64_spread_markers(Ctx& c, const double* mfield, double* ftmp) {
-  const Grid& g = c.g;
-  hipStream_t s = c.stream;
-  const long gx = g.nx + 2, gy = g.ny + 2, gz = g.nz + 2;
+static SpreadCsr spread_csr(Ctx& c, int& cmax) {
   SpreadCsr cs{};
-  int rmax = 0;
-  for (int comp = 0; comp < 3; comp++) {
-    cs.rowp[comp] = c.sp_row[comp];
-    cs.tgt[comp] = c.sp_tgt[comp];
-    cs.ent[comp] = c.sp_ent[comp];
-    cs.w[comp] = c.sp_w[comp];
-    cs.rows[comp] = c.sp_rows[comp];
-    rmax = std::max(rmax, c.sp_rows[comp]);
+  cmax = 0;
+  for (int k = 0; k < 3; k++) {
+    cs.rowp[k] = c.sp_row[k];
+    cs.ent[k] = c.sp_ent[k];
+    cs.w[k] = c.sp_w[k];
+    cs.cell[k] = c.fc_cell[k];
+    cs.row[k] = c.fc_row[k];
+    cs.img[k] = c.fc_img[k];
+    cs.cells[k] = c.fc_cells[k];
+    cmax = std::max(cmax, c.fc_cells[k]);
   }
-  if (rmax > 0)
-    hipLaunchKernelGGL(k_ibm_spread, dim3(nblk(rmax, 256), 3), dim3(256), 0, s, g, cs, c.nmk, mfield, ftmp, c.gn);
-  // the folds of the three components, x, then y, then z
-  hipLaunchKernelGGL(k_ibm_fold, dim3(nblk(gy * gz, 256), 3), dim3(256), 0, s, g, 0, ftmp, c.gn);
-  hipLaunchKernelGGL(k_ibm_fold, dim3(nblk(gx * gz, 256), 3), dim3(256), 0, s, g, 1, ftmp, c.gn);
-  hipLaunchKernelGGL(k_ibm_fold, dim3(nblk(gx * gy, 256), 3), dim3(256), 0, s, g, 2, ftmp, c.gn);
+  return cs;
 }
 
+// out += spread of the marker values mfield (3 x nmk), over the forced cells
+void f64_spread_add(Ctx& c, const double* mfield, double* out) {
+  int cmax;
+  const SpreadCsr cs = spread_csr(c, cmax);
+  if (cmax > 0)
+    hipLaunchKernelGGL((k_ibm_spread<false, false>), dim3(nblk(cmax, 64), 3), dim3(64), 0, c.stream, c.g, cs, c.nmk, mfield,
+                       out, (const double*)nullptr, out);
+}
+
+// the marker forces of Ua = c.Q and the forced cells of c.Up; B0 is this
+// step's B once the predictor has run
 void f64_ibm(Ctx& c) {
   const Grid& g = c.g;
   hipStream_t s = c.stream;
-  hipLaunchKernelGGL(k_ibm_interp, dim3(nblk(c.nmk, 256)), dim3(256), 0, s, g, c.nmk, c.nc, c.nl, c.mk, c.ib_w, c.Q, c.mb,
-                     c.mf);
-  f64_spread_markers(c, c.mf, c.ftmp);
-  hipLaunchKernelGGL(k_ibm_rhs, dim3(nblk(3 * g.n, 256)), dim3(256), 0, s, g, c.Q, c.ftmp, c.B, c.Up);
+  hipLaunchKernelGGL(g.walls ? k_ibm_forces<true> : k_ibm_forces<false>, dim3(nblk(c.nmk, 64), 3), dim3(64), 0, s, g, c.nmk,
+                     c.nc, c.nl, c.mk, c.ib_w, c.Q, c.mf);
+  int cmax;
+  const SpreadCsr cs = spread_csr(c, cmax);
+  auto k = g.walls ? k_ibm_spread<true, true> : k_ibm_spread<true, false>;
+  if (cmax > 0) hipLaunchKernelGGL(k, dim3(nblk(cmax, 64), 3), dim3(64), 0, s, g, cs, c.nmk, c.mf, c.Q, c.B0, c.Up);
 }
 
 // Host-side construction of the spreading CSR: for each ghosted target the
@@ -543,9 +570,42 @@ void f64_ibm_setup(Ctx& c) {
       tgt.push_back(t);
       rowp.push_back((int)ent.size());
     }
-    if (c.sp_row[comp]) {
-      (void)hipFree(c.sp_row[comp]); (void)hipFree(c.sp_tgt[comp]); (void)hipFree(c.sp_ent[comp]); (void)hipFree(c.sp_w[comp]);
+    // the forced cells and the rows each one gathers: its own, and where it
+    // borders a periodic axis those of its ghost images
+    auto row_of = [&](long t) {
+      const auto it = std::lower_bound(tgt.begin(), tgt.end(), t);
+      return it != tgt.end() && *it == t ? (int)(it - tgt.begin()) : -1;
+    };
+    auto image = [](long i, int nn, int b) {   // a cell and its ghost image along an axis (-1: none)
+      return !b ? i : (i == 1 ? (long)nn + 1 : (i == nn ? 0L : -1L));
+    };
+    std::vector<long> cell;
+    std::vector<int> crow, img;
+    for (size_t r = 0; r < tgt.size(); r++) {
+      const long i = tgt[r] % gx, j = (tgt[r] / gx) % gy, k = tgt[r] / (gx * gy);
+      if (i < 1 || i > g.nx || j < 1 || j > g.ny || k < 1 || k > g.nz) continue;
+      int rr[8], ghosts = 0;
+      for (int b = 0; b < 8; b++) {
+        const long ii = image(i, g.nx, b & 1), jj = image(j, g.ny, b >> 1 & 1), kk = image(k, g.nz, b >> 2);
+        rr[b] = b == 0 ? (int)r : (ii < 0 || jj < 0 || kk < 0 ? -1 : row_of(G(ii, jj, kk)));
+        ghosts += b > 0 && rr[b] >= 0;
+      }
+      cell.push_back((i - 1) + g.nx * ((j - 1) + (long)g.ny * (k - 1)));
+      crow.push_back(ghosts ? -1 - (int)(img.size() / 8) : (int)r);
+      if (ghosts) img.insert(img.end(), rr, rr + 8);
     }
+    for (void* q : {(void*)c.sp_row[comp], (void*)c.sp_tgt[comp], (void*)c.sp_ent[comp], (void*)c.sp_w[comp],
+                    (void*)c.fc_cell[comp], (void*)c.fc_row[comp], (void*)c.fc_img[comp]})
+      if (q) (void)hipFree(q);
+    c.fc_cells[comp] = (int)cell.size();
+    FP_HIP_CHECK(hipMalloc(&c.fc_cell[comp], sizeof(long) * std::max<size_t>(1, cell.size())));
+    FP_HIP_CHECK(hipMalloc(&c.fc_row[comp], sizeof(int) * std::max<size_t>(1, crow.size())));
+    FP_HIP_CHECK(hipMalloc(&c.fc_img[comp], sizeof(int) * std::max<size_t>(1, img.size())));
+    if (!cell.empty()) {
+      FP_HIP_CHECK(hipMemcpy(c.fc_cell[comp], cell.data(), sizeof(long) * cell.size(), hipMemcpyHostToDevice));
+      FP_HIP_CHECK(hipMemcpy(c.fc_row[comp], crow.data(), sizeof(int) * crow.size(), hipMemcpyHostToDevice));
+    }
+    if (!img.empty()) FP_HIP_CHECK(hipMemcpy(c.fc_img[comp], img.data(), sizeof(int) * img.size(), hipMemcpyHostToDevice));
     c.sp_rows[comp] = (int)tgt.size();
     FP_HIP_CHECK(hipMalloc(&c.sp_row[comp], sizeof(int) * rowp.size()));
     FP_HIP_CHECK(hipMalloc(&c.sp_tgt[comp], sizeof(long) * std::max<size_t>(1, tgt.size())));
@@ -727,9 +787,9 @@ void f64_cstar_newton(Ctx& c) {
 void f64_predictor(Ctx& c) {
   const Grid& g = c.g;
   int polymer = c.p.beta != 1.0;
-  double* Bout = c.p.method == FP_METHOD_IBM ? c.B : nullptr;
+  double* Rout = c.p.method == FP_METHOD_IBM ? c.Up : nullptr;
   hipLaunchKernelGGL(c.g.walls ? k_predictor<true> : k_predictor<false>, dim3(nblk(g.n, 256)), dim3(256), 0, c.stream, g, c.p.method, c.has_history ? 0 : 1,
-                     polymer, c.U, c.V, c.W, c.P, c.C[c.cur], c.fC, c.A0, c.T0, c.B0, Bout, c.F,
+                     polymer, c.U, c.V, c.W, c.P, c.C[c.cur], c.fC, c.A0, c.T0, c.B0, Rout, c.F,
                      c.p.body_force[0], c.p.body_force[1], c.p.body_force[2], c.Q);
 }
 
