@@ -688,6 +688,7 @@ void save_state(Ctx& c, double* dst) {
 
 void load_state(Ctx& c, const double* src) {
   const long n = c.g.n;
+  if (c.mixed) mixed_settle_history(c);
   d2d(c, c.U, src, sizeof(double) * n);
   d2d(c, c.V, src + n, sizeof(double) * n);
   d2d(c, c.W, src + 2 * n, sizeof(double) * n);

@@ -59,6 +59,23 @@ void drain(Ctx& c) {
   FP_HIP_CHECK(hipStreamSynchronize(c.stream));
 }
 
+// whether kernels of the current device may follow these pointers (nullptr
+// counts as yes): memory of another device or of the host takes copies
+bool on_this_device(const void* const* p, int count) {
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  for (int q = 0; q < count; q++) {
+    if (!p[q]) continue;
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p[q]) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    if (a.type != hipMemoryTypeDevice || a.device != dev) return false;
+  }
+  return true;
+}
+
 int fail(Ctx* c, int code, const std::string& msg) {
   if (c) c->err = msg;
   return code;
@@ -310,6 +327,10 @@ int fp_set_state(void* vc, const double* U, const double* V, const double* W, co
     for (int q = 0; q < 6; q++) ghosted_to_interior(g, C6, 6, q, buf.data() + q * n);
     c->cur = 0;
     FP_HIP_CHECK(hipMemcpy(c->C[0], buf.data(), sizeof(double) * 6 * n, hipMemcpyHostToDevice));
+    if (c->mixed) {
+      mixed_settle_history(*c);
+      FP_HIP_CHECK(hipStreamSynchronize(c->stream));
+    }
     if (hist) {
       FP_HIP_CHECK(hipMemcpy(c->A0, hist, sizeof(double) * 3 * n, hipMemcpyHostToDevice));
       FP_HIP_CHECK(hipMemcpy(c->T0, hist + 3 * n, sizeof(double) * 3 * n, hipMemcpyHostToDevice));
@@ -552,6 +573,15 @@ int fp_set_state_device(void* vc, const double* U, const double* V, const double
     drain(*c);
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const long n = c->g.n;
+    const double* src[5] = {U, V, W, P, C6};
+    if (c->mixed && on_this_device((const void* const*)src, 5)) {
+      c->cur = 0;
+      mixed_set_from_device(*c, src, has_history == 2, s);
+      FP_HIP_CHECK(hipStreamSynchronize(s));
+      c->has_history = has_history ? 1 : 0;
+      c->state_set = 1;
+      return FP_OK;
+    }
     FP_HIP_CHECK(hipMemcpyAsync(c->U, U, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     FP_HIP_CHECK(hipMemcpyAsync(c->V, V, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     FP_HIP_CHECK(hipMemcpyAsync(c->W, W, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
@@ -579,9 +609,16 @@ int fp_get_state_device(void* vc, double* U, double* V, double* W, double* P, do
   Ctx* c = (Ctx*)vc;
   if (!c) return FP_E_ARG;
   try {
-    if (c->mixed) mixed_store_to_f64(*c);
-    FP_HIP_CHECK(hipStreamSynchronize(c->stream));
+    double* dst[5] = {U, V, W, P, C6};
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+    const bool direct = c->mixed && on_this_device((const void* const*)dst, 5);
+    if (c->mixed && !direct) mixed_store_to_f64(*c);
+    FP_HIP_CHECK(hipStreamSynchronize(c->stream));
+    if (direct) {
+      mixed_get_to_device(*c, dst, s);
+      FP_HIP_CHECK(hipStreamSynchronize(s));
+      return FP_OK;
+    }
     const long n = c->g.n;
     if (U) FP_HIP_CHECK(hipMemcpyAsync(U, c->U, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     if (V) FP_HIP_CHECK(hipMemcpyAsync(V, c->V, sizeof(double) * n, hipMemcpyDeviceToDevice, s));

@@ -36,7 +36,12 @@ struct Mixed {
   float* C[2] = {nullptr, nullptr};
   int cur = 0;
   float* f = nullptr;
-  float *A0 = nullptr, *T0 = nullptr, *B = nullptr;
+  // histories A0 (3 planes) and T0 (3 planes): AT[h] holds the context's, and
+  // AT[hs] those of the last copy-out (hs < 0: c.A0 and c.T0 do).  A step
+  // whose histories are both writes the other buffer, so a copy-out of the
+  // state moves no history.
+  float* AT[2] = {nullptr, nullptr};
+  int h = 0, hs = -1;
   float* Q = nullptr;             // predictor increment d_q (+ dt f of the IBM spread)
   float* Up = nullptr;            // Helmholtz increment d: u* = u^n + d
   float* F = nullptr;
@@ -1190,15 +1195,16 @@ struct PredWalls {
 struct PredCell {
   float a0[3], t0[3], fv[3];
 };
-__device__ __forceinline__ void pred_cell_load(const Grid& g, long m, int first, const float* __restrict__ A0,
-                                               const float* __restrict__ T0, const float* __restrict__ F, float bf0,
-                                               float bf1, float bf2, PredCell& in) {
+// AT: A0 in planes 0 to 2, T0 in planes 3 to 5
+__device__ __forceinline__ void pred_cell_load(const Grid& g, long m, int first, const float* AT,
+                                               const float* __restrict__ F, float bf0, float bf1, float bf2,
+                                               PredCell& in) {
   const float bfs[3] = {bf0, bf1, bf2};
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     const long oo = c * g.n + m;
-    in.a0[c] = first ? 0.0f : A0[oo];
-    in.t0[c] = first ? 0.0f : T0[oo];
+    in.a0[c] = first ? 0.0f : AT[oo];
+    in.t0[c] = first ? 0.0f : AT[3 * g.n + oo];
     in.fv[c] = (F ? F[oo] : 0.0f) + bfs[c];
   }
 }
@@ -1220,8 +1226,7 @@ __device__ __forceinline__ void pred_cell_load(const Grid& g, long m, int first,
 // d_q = r + dt B for both methods; the IBM spread adds dt f to it.
 template <class S_t>
 __device__ __forceinline__ void predictor_body(const Grid& g, const S_t& S, const PredCell& in, long m, int j,
-                                               int method, int first, int polymer, float* __restrict__ A0,
-                                               float* __restrict__ T0, float* __restrict__ Q) {
+                                               int method, int first, int polymer, float* AT, float* __restrict__ Q) {
   const float dx = (float)g.dx, dy = (float)g.dy, dz = (float)g.dz, dt = (float)g.dt;
   const float idx_ = 1.0f / dx, idy = 1.0f / dy, idz = 1.0f / dz;
 #define Ug(a, b, c) S.u(a, b, c)
@@ -1285,8 +1290,8 @@ __device__ __forceinline__ void predictor_body(const Grid& g, const S_t& S, cons
                      0.5f * dt * (t[c] + t0) + dt * in.fv[c];
     // the wall face of V stays 0 (V_kabe)
     Q[oo] = (c == 1 && g.walls && j == g.ny - 1) ? 0.0f : dq;
-    A0[oo] = a[c];
-    T0[oo] = t[c];
+    AT[oo] = a[c];
+    AT[3 * g.n + oo] = t[c];
   }
 #undef Ug
 #undef Vg
@@ -1302,20 +1307,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
                                                    const float* __restrict__ U, const float* __restrict__ V,
                                                    const float* __restrict__ W, const float* __restrict__ P,
                                                    const float* __restrict__ C, const float* __restrict__ fC,
-                                                   float* __restrict__ A0, float* __restrict__ T0,
-                                                   const float* __restrict__ F,
+                                                   const float* ATi, float* ATo, const float* __restrict__ F,
                                                    float bf0, float bf1, float bf2, float* __restrict__ Q) {
   long m;
   int i, j, k;
   if (!row_cell<GEN, 1>(g, m, i, j, k)) return;
   PredCell in;
-  pred_cell_load(g, m, first, A0, T0, F, bf0, bf1, bf2, in);
+  pred_cell_load(g, m, first, ATi, F, bf0, bf1, bf2, in);
   if (GEN) {
     const PredWalls S{g, i, j, k, U, V, W, P, C, fC};
-    predictor_body(g, S, in, m, j, method, first, polymer, A0, T0, Q);
+    predictor_body(g, S, in, m, j, method, first, polymer, ATo, Q);
   } else {
     const PredFast S{g, m, nbr(g, i, j, k), U, V, W, P, C, fC};
-    predictor_body(g, S, in, m, j, method, first, polymer, A0, T0, Q);
+    predictor_body(g, S, in, m, j, method, first, polymer, ATo, Q);
   }
 }
 
@@ -1445,8 +1449,7 @@ __global__ __launch_bounds__(PZ_THREADS) void m_predictor_z(Grid g, int kc, int 
                                                             const float* __restrict__ U, const float* __restrict__ V,
                                                             const float* __restrict__ W, const float* __restrict__ P,
                                                             const float* __restrict__ C, const float* __restrict__ fC,
-                                                            float* __restrict__ A0, float* __restrict__ T0,
-                                                            const float* __restrict__ F,
+                                                            const float* ATi, float* ATo, const float* __restrict__ F,
                                                             float bf0, float bf1, float bf2, float* __restrict__ Q) {
   __shared__ float lds[3][PZ_NF * PZ_PTS];
   const int ntx = g.nx / PZ_TX, nty = g.ny / PZ_TY;
@@ -1471,9 +1474,9 @@ __global__ __launch_bounds__(PZ_THREADS) void m_predictor_z(Grid g, int kc, int 
     __syncthreads();
     const long m = cidx(g, i, j, kk);
     PredCell in;
-    pred_cell_load(g, m, first, A0, T0, F, bf0, bf1, bf2, in);
+    pred_cell_load(g, m, first, ATi, F, bf0, bf1, bf2, in);
     const PredLds S{lds[sm], lds[s0], lds[sp], (ty + 1) * PZ_HX + tx + 1};
-    predictor_body(g, S, in, m, j, method, first, polymer, A0, T0, Q);
+    predictor_body(g, S, in, m, j, method, first, polymer, ATo, Q);
     __syncthreads();
     // plane kk+2 replaces plane kk-1; fetch plane kk+3
     if (kk + 2 <= k1) pz_put<WL>(g, j0, r, lds[sm]);
@@ -3027,6 +3030,45 @@ __global__ void m_to64(long n, const float* __restrict__ a, double* __restrict__
   if (m < n) b[m] = (double)a[m];
 }
 
+// The state between a caller's FP64 planes and the FP32 fields, plane
+// blockIdx.y, four cells a thread: 12 bytes a value once, at the rate of a
+// copy.  The caller's planes are aligned to 8 bytes only; n is a multiple of 64.
+struct StateIn {
+  const double* src[10];
+  float* dst[10];
+};
+struct StateOut {
+  const float* src[10];
+  double* dst[10];
+};
+__global__ __launch_bounds__(256) void m_state_in(long n, StateIn p) {
+  const long m = (blockIdx.x * 256L + threadIdx.x) * 4;
+  if (m >= n) return;
+  const double* a = p.src[blockIdx.y] + m;
+  double2 v0, v1;
+  if (((size_t)p.src[blockIdx.y] & 15) == 0) {
+    v0 = *(const double2*)a;
+    v1 = *(const double2*)(a + 2);
+  } else {
+    v0 = make_double2(a[0], a[1]);
+    v1 = make_double2(a[2], a[3]);
+  }
+  *(float4*)(p.dst[blockIdx.y] + m) = make_float4((float)v0.x, (float)v0.y, (float)v1.x, (float)v1.y);
+}
+__global__ __launch_bounds__(256) void m_state_out(long n, StateOut p) {
+  const long m = (blockIdx.x * 256L + threadIdx.x) * 4;
+  double* base = p.dst[blockIdx.y];
+  if (m >= n || !base) return;
+  const float4 v = *(const float4*)(p.src[blockIdx.y] + m);
+  double* a = base + m;
+  if (((size_t)base & 15) == 0) {
+    *(double2*)a = make_double2(v.x, v.y);
+    *(double2*)(a + 2) = make_double2(v.z, v.w);
+  } else {
+    a[0] = v.x; a[1] = v.y; a[2] = v.z; a[3] = v.w;
+  }
+}
+
 // ================================================================= host ===
 // Fixed-point Helmholtz sweeps x <- q + eps Lap x from x = q: the error
 // starts at eps Lap x* (<= rho |x*|, rho = eps lambda_max) and contracts by
@@ -3057,7 +3099,7 @@ void mixed_create(Ctx& c) {
   FP_HIP_CHECK(hipEventCreateWithFlags(&X->sel_done, hipEventDisableTiming | hipEventReleaseToDevice));
   dalloc(&X->U, n); dalloc(&X->V, n); dalloc(&X->W, n); dalloc(&X->P, n);
   dalloc(&X->C[0], 6 * n); dalloc(&X->C[1], 6 * n); dalloc(&X->f, n);
-  dalloc(&X->A0, 3 * n); dalloc(&X->T0, 3 * n); dalloc(&X->B, 3 * n);
+  dalloc(&X->AT[0], 6 * n); dalloc(&X->AT[1], 6 * n);
   dalloc(&X->Q, 3 * n); dalloc(&X->Up, 3 * n);
   dalloc(&X->spec, (size_t)g.nxh * g.sy * g.nz);
   if (g.walls) dalloc(&X->thp, (size_t)(g.ny + 2) * g.nxh * g.nz);
@@ -3129,7 +3171,7 @@ void mixed_destroy(Ctx& c) {
   if (X->sel_done) (void)hipEventDestroy(X->sel_done);
   if (X->side) (void)hipStreamDestroy(X->side);
   dfree(X->U); dfree(X->V); dfree(X->W); dfree(X->P); dfree(X->C[0]); dfree(X->C[1]); dfree(X->f);
-  dfree(X->A0); dfree(X->T0); dfree(X->B); dfree(X->Q); dfree(X->Up); dfree(X->F);
+  dfree(X->AT[0]); dfree(X->AT[1]); dfree(X->Q); dfree(X->Up); dfree(X->F);
   dfree(X->spec); dfree(X->thp); dfree(X->twx); dfree(X->twy); dfree(X->twz);
   dfree(X->kx2); dfree(X->ky2); dfree(X->kz2);
   dfree(X->phi); dfree(X->b); dfree(X->r32); dfree(X->red); dfree(X->part); dfree(X->skip);
@@ -3152,24 +3194,81 @@ void mixed_destroy(Ctx& c) {
   c.mixed = nullptr;
 }
 
+static void history_to_f64(Ctx& c, const float* AT) {
+  const long n3 = 3 * c.g.n;
+  hipLaunchKernelGGL(m_to64, dim3(nblk(n3, 256)), dim3(256), 0, c.stream, n3, AT, c.A0);
+  hipLaunchKernelGGL(m_to64, dim3(nblk(n3, 256)), dim3(256), 0, c.stream, n3, AT + n3, c.T0);
+}
+static void history_from_f64(Ctx& c, float* AT) {
+  const long n3 = 3 * c.g.n;
+  hipLaunchKernelGGL(m_to32, dim3(nblk(n3, 256)), dim3(256), 0, c.stream, n3, c.A0, AT);
+  hipLaunchKernelGGL(m_to32, dim3(nblk(n3, 256)), dim3(256), 0, c.stream, n3, c.T0, AT + n3);
+}
+
+void mixed_settle_history(Ctx& c) {
+  Mixed& X = MX(c);
+  if (X.hs >= 0) history_to_f64(c, X.AT[X.hs]);
+  X.hs = -1;
+}
+
+// a selection made ahead still reads the old C; it no longer applies
+static void drop_selection(Mixed& X, hipStream_t s) {
+  if (X.sel_ready) FP_HIP_CHECK(hipStreamWaitEvent(s, X.sel_done, 0));
+  X.sel_ready = 0;
+}
+
 void mixed_load_from_f64(Ctx& c) {
   Mixed& X = MX(c);
   const long n = c.g.n;
   hipStream_t s = c.stream;
-  // a selection made ahead still reads the old C; it no longer applies
-  if (X.sel_ready) FP_HIP_CHECK(hipStreamWaitEvent(s, X.sel_done, 0));
-  X.sel_ready = 0;
+  drop_selection(X, s);
+  mixed_settle_history(c);
   hipLaunchKernelGGL(m_to32, dim3(nblk(n, 256)), dim3(256), 0, s, n, c.U, X.U);
   hipLaunchKernelGGL(m_to32, dim3(nblk(n, 256)), dim3(256), 0, s, n, c.V, X.V);
   hipLaunchKernelGGL(m_to32, dim3(nblk(n, 256)), dim3(256), 0, s, n, c.W, X.W);
   hipLaunchKernelGGL(m_to32, dim3(nblk(n, 256)), dim3(256), 0, s, n, c.P, X.P);
   X.cur = 0;
   hipLaunchKernelGGL(m_to32, dim3(nblk(6 * n, 256)), dim3(256), 0, s, 6 * n, c.C[c.cur], X.C[0]);
-  hipLaunchKernelGGL(m_to32, dim3(nblk(3 * n, 256)), dim3(256), 0, s, 3 * n, c.A0, X.A0);
-  hipLaunchKernelGGL(m_to32, dim3(nblk(3 * n, 256)), dim3(256), 0, s, 3 * n, c.T0, X.T0);
+  history_from_f64(c, X.AT[X.h]);
   // the potential: the SOR variant starts its sweeps from it
   FP_HIP_CHECK(hipMemcpyAsync(X.phi, c.Phi, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   FP_HIP_CHECK(hipStreamSynchronize(s));
+}
+
+// The state of the caller's FP64 device arrays (U, V, W, P, 6 planes C),
+// straight into the FP32 fields; the histories of the last copy-out and, with
+// keep_phi, the potential stay.  256^3: 1230 -> 357 us against a copy into
+// the FP64 arrays and a conversion of those.
+void mixed_set_from_device(Ctx& c, const double* const* src, int keep_phi, hipStream_t s) {
+  Mixed& X = MX(c);
+  const long n = c.g.n;
+  drop_selection(X, s);
+  X.cur = 0;
+  if (X.hs >= 0) {
+    X.h = X.hs;
+  } else {
+    history_from_f64(c, X.AT[X.h]);
+    FP_HIP_CHECK(hipStreamSynchronize(c.stream));
+  }
+  StateIn in{};
+  for (int q = 0; q < 10; q++) in.src[q] = q < 4 ? src[q] : src[4] + (q - 4) * n;
+  float* dst[4] = {X.U, X.V, X.W, X.P};
+  for (int q = 0; q < 10; q++) in.dst[q] = q < 4 ? dst[q] : X.C[0] + (q - 4) * n;
+  hipLaunchKernelGGL(m_state_in, dim3(nblk(n, 1024), 10), dim3(256), 0, s, n, in);
+  if (!keep_phi) FP_HIP_CHECK(hipMemsetAsync(X.phi, 0, sizeof(double) * n, s));
+}
+
+// the state widened into the caller's FP64 device arrays (nullptr: not
+// wanted); 256^3: 1300 -> 482 us
+void mixed_get_to_device(Ctx& c, double* const* dst, hipStream_t s) {
+  Mixed& X = MX(c);
+  const long n = c.g.n;
+  StateOut out{};
+  for (int q = 0; q < 10; q++) out.dst[q] = q < 4 ? dst[q] : (dst[4] ? dst[4] + (q - 4) * n : nullptr);
+  const float* src[4] = {X.U, X.V, X.W, X.P};
+  for (int q = 0; q < 10; q++) out.src[q] = q < 4 ? src[q] : X.C[X.cur] + (q - 4) * n;
+  hipLaunchKernelGGL(m_state_out, dim3(nblk(n, 1024), 10), dim3(256), 0, s, n, out);
+  X.hs = X.h;
 }
 
 void mixed_phi_to_f64(Ctx& c) {
@@ -3185,8 +3284,8 @@ void mixed_store_to_f64(Ctx& c) {
   hipLaunchKernelGGL(m_to64, dim3(nblk(n, 256)), dim3(256), 0, s, n, X.W, c.W);
   hipLaunchKernelGGL(m_to64, dim3(nblk(n, 256)), dim3(256), 0, s, n, X.P, c.P);
   hipLaunchKernelGGL(m_to64, dim3(nblk(6 * n, 256)), dim3(256), 0, s, 6 * n, X.C[X.cur], c.C[c.cur]);
-  hipLaunchKernelGGL(m_to64, dim3(nblk(3 * n, 256)), dim3(256), 0, s, 3 * n, X.A0, c.A0);
-  hipLaunchKernelGGL(m_to64, dim3(nblk(3 * n, 256)), dim3(256), 0, s, 3 * n, X.T0, c.T0);
+  history_to_f64(c, X.AT[X.h]);
+  X.hs = -1;
   FP_HIP_CHECK(hipMemcpyAsync(c.Phi, X.phi, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   if (c.nmk) hipLaunchKernelGGL(m_to64, dim3(nblk(3 * c.nmk, 256)), dim3(256), 0, s, 3 * c.nmk, X.mf, X.mf64);
   FP_HIP_CHECK(hipStreamSynchronize(s));
@@ -3777,26 +3876,29 @@ void mixed_step(Ctx& c) {
     }
     X.cur = 1 - X.cur;
   }
+  const int ho = X.h == X.hs ? 1 - X.h : X.h;
+  float* ATo = X.AT[ho];
   if (g.nx % PZ_TX == 0 && g.ny % PZ_TY == 0) {
     // streamed along z, wall rows included
     MTimer t(c, "predictor");
     const int kc = planes_per_block(g, PZ_TX * PZ_TY, PZ_KC);
     const long grid = g.n / (PZ_TX * PZ_TY * kc);
     hipLaunchKernelGGL(g.walls ? m_predictor_z<true> : m_predictor_z<false>, dim3(grid), dim3(PZ_THREADS), 0, s, g, kc,
-                       c.p.method, c.has_history ? 0 : 1, polymer, X.U, X.V, X.W, X.P, X.C[X.cur], X.f, X.A0, X.T0,
+                       c.p.method, c.has_history ? 0 : 1, polymer, X.U, X.V, X.W, X.P, X.C[X.cur], X.f, X.AT[X.h], ATo,
                        X.F, (float)c.p.body_force[0], (float)c.p.body_force[1], (float)c.p.body_force[2], X.Q);
   } else {
     MTimer t(c, "predictor");
     hipLaunchKernelGGL(m_predictor<false>, dim3(nblk(n, 256)), dim3(256), 0, s, g, c.p.method, c.has_history ? 0 : 1, polymer,
-                       X.U, X.V, X.W, X.P, X.C[X.cur], X.f, X.A0, X.T0, X.F, (float)c.p.body_force[0],
+                       X.U, X.V, X.W, X.P, X.C[X.cur], X.f, X.AT[X.h], ATo, X.F, (float)c.p.body_force[0],
                        (float)c.p.body_force[1], (float)c.p.body_force[2], X.Q);
   }
   if (g.walls && !(g.nx % PZ_TX == 0 && g.ny % PZ_TY == 0)) {
     MTimer t(c, "predictor_walls");
     hipLaunchKernelGGL(m_predictor<true>, dim3(nblk(wall_rows(g, 1), 256)), dim3(256), 0, s, g, c.p.method, c.has_history ? 0 : 1, polymer,
-                       X.U, X.V, X.W, X.P, X.C[X.cur], X.f, X.A0, X.T0, X.F, (float)c.p.body_force[0],
+                       X.U, X.V, X.W, X.P, X.C[X.cur], X.f, X.AT[X.h], ATo, X.F, (float)c.p.body_force[0],
                        (float)c.p.body_force[1], (float)c.p.body_force[2], X.Q);
   }
+  X.h = ho;
   // The next step's selection (it reads only the new C) forks onto the second
   // stream here, beside the Helmholtz sweeps and the Poisson solve.  Forking
   // before the IBM phase measured slower, forking after the sweeps leaves the
