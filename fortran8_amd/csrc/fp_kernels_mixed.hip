@@ -16,6 +16,7 @@
 #include "fp_device.h"
 #include "fp_sor.h"
 #include <algorithm>
+#include <type_traits>
 #include <cmath>
 #include <map>
 #include <unordered_map>
@@ -1825,6 +1826,150 @@ __global__ __launch_bounds__(256) void m_fft_yz(Grid g, float2* __restrict__ spe
   }
 }
 
+// The same transforms for lines of 16 to 256 points, with the line in
+// registers: 16 points a thread, 2^(M-4) threads a line.  The stages of the
+// upper index bits run on points u + (N/16) r, those of the lower four on
+// points 16 u + r, with one exchange through the LDS between them; every
+// butterfly is stockham_f's, in place (decimation in frequency), so the values
+// are the same.  What the forward transform leaves in a thread's registers is
+// what the inverse starts from (the digit-reversed place of point 16 u + r has
+// its upper four bits in r), so mode 2 needs two exchanges in all.  Lines are
+// numbered along kx and on through the rows (axis 2) or planes (axis 1), 16 to
+// a block: a load takes 128 consecutive bytes, and no block is cut off at the
+// odd nx / 2 + 1.
+// The kernel moves its spectrum once, 16 B a point; m_fft_yz, a barrier and two
+// LDS passes a stage and its index arithmetic: the three launches of 64^3 23 us
+// there and 17 here, a step of 256^3 240 us less.
+// cmul_f with the fusions that m_fft_yz is compiled to written out (after the
+// divide the other product of each pair is rounded first); the functions below
+// contract nothing else, so that no product joins a sum of the next stage
+enum { FL_FWD = 0, FL_INV = 1, FL_BACK = 2 };   // BACK: inverse after the divide
+__device__ __forceinline__ float2 cmul_l(float2 a, float2 w, int dir) {
+#pragma clang fp contract(off)
+  if (dir == FL_BACK) return make_float2(fmaf(a.y, -w.y, a.x * w.x), fmaf(a.y, w.x, a.x * w.y));
+  return make_float2(fmaf(a.x, w.x, -(a.y * w.y)), fmaf(a.x, w.y, a.y * w.x));
+}
+template <int M>
+__device__ __forceinline__ void fft_bfly4(float2& a0, float2& a1, float2& a2, float2& a3, const float2* tws, int j1,
+                                          int dir) {
+#pragma clang fp contract(off)
+  constexpr int half = 1 << (M - 1);
+  const float2 b0 = make_float2(a0.x + a2.x, a0.y + a2.y), b1 = make_float2(a0.x - a2.x, a0.y - a2.y);
+  const float2 b2 = make_float2(a1.x + a3.x, a1.y + a3.y), d = make_float2(a1.x - a3.x, a1.y - a3.y);
+  const float2 b3 = dir != FL_FWD ? make_float2(-d.y, d.x) : make_float2(d.y, -d.x);
+  a0 = make_float2(b0.x + b2.x, b0.y + b2.y);
+  a1 = cmul_l(make_float2(b1.x + b3.x, b1.y + b3.y), tw_at(tws, half, j1, dir != FL_FWD), dir);
+  a2 = cmul_l(make_float2(b0.x - b2.x, b0.y - b2.y), tw_at(tws, half, 2 * j1, dir != FL_FWD), dir);
+  a3 = cmul_l(make_float2(b1.x - b3.x, b1.y - b3.y), tw_at(tws, half, 3 * j1, dir != FL_FWD), dir);
+}
+// the stages of the upper bits on points u + (N/16) r: two of radix 4, or one
+// of radix 2 and one of radix 4 where M is odd
+template <int M>
+__device__ __forceinline__ void fft_upper(float2 (&v)[16], int u, const float2* tws, int dir) {
+#pragma clang fp contract(off)
+  if (M & 1) {
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+      const float2 a = v[r], b = v[8 + r];
+      const float2 w = tw_at(tws, 1 << (M - 1), (r << (M - 4)) | u, dir != FL_FWD);
+      v[r] = make_float2(a.x + b.x, a.y + b.y);
+      const float2 d = make_float2(a.x - b.x, a.y - b.y), t = cmul_l(d, w, dir);
+      v[8 + r] = dir == FL_BACK ? make_float2(cmul_l(d, w, FL_INV).x, t.y) : t;   // (as compiled there)
+    }
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+      for (int e = 0; e < 2; e++)
+        fft_bfly4<M>(v[8 * e + f], v[8 * e + 2 + f], v[8 * e + 4 + f], v[8 * e + 6 + f], tws, 2 * ((f << (M - 4)) | u), dir);
+  } else {
+#pragma unroll
+    for (int b = 0; b < 4; b++) fft_bfly4<M>(v[b], v[4 + b], v[8 + b], v[12 + b], tws, (b << (M - 4)) | u, dir);
+#pragma unroll
+    for (int a = 0; a < 4; a++) fft_bfly4<M>(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3], tws, 4 * u, dir);
+  }
+}
+// the others, on points 16 u + r
+template <int M>
+__device__ __forceinline__ void fft_lower(float2 (&v)[16], const float2* tws, int dir) {
+  if (M >= 7) {
+#pragma unroll
+    for (int d = 0; d < 4; d++) fft_bfly4<M>(v[d], v[4 + d], v[8 + d], v[12 + d], tws, d << (M - 4), dir);
+  }
+  if (M >= 5) {
+#pragma unroll
+    for (int a = 0; a < 4; a++) fft_bfly4<M>(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3], tws, 0, dir);
+  }
+}
+__device__ __forceinline__ float2 scaled(float2 a, float s) {
+#pragma clang fp contract(off)
+  return make_float2(a.x * s, a.y * s);
+}
+constexpr int fl_lines(int M) { return M >= 6 ? 16 : 64 >> (M - 4); }
+constexpr int fl_threads(int M) { return fl_lines(M) << (M - 4); }
+
+// grid: nlines / fl_lines(M) blocks, rounded up
+template <int M, int MODE>
+__global__ __launch_bounds__(fl_threads(M)) void m_fft_lines(Grid g, float2* __restrict__ spec,
+                                                             const float2* __restrict__ tw, int axis, int kind, int row0,
+                                                             long nlines, const float* __restrict__ kx2,
+                                                             const float* __restrict__ ky2, const float* __restrict__ kz2,
+                                                             const int* __restrict__ skip) {
+  if (skip && *skip) return;
+  constexpr int N = 1 << M, TI = fl_lines(M);
+  __shared__ float2 lds[N * TI];
+  __shared__ float2 tws[N / 2];
+  const int l = threadIdx.x % TI, u = threadIdx.x / TI;
+  const long L = blockIdx.x * (long)TI + l;
+  const bool on = L < nlines;
+  const unsigned Lc = (unsigned)(on ? L : nlines - 1);
+  const int nxh = g.nxh;
+  const unsigned other = Lc / (unsigned)nxh, kx = Lc - other * (unsigned)nxh;
+  const long stride = axis == 1 ? (long)nxh : (long)nxh * g.sy;
+  float2* base = axis == 1 ? spec + (long)nxh * (g.jo + (long)g.sy * other) + kx : spec + (long)nxh * row0 + Lc;
+  load_twiddles(tws, tw, N);
+  float2 v[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) v[r] = base[stride * ((r << (M - 4)) | u)];
+  __syncthreads();
+  // the line's place (r, u) of points 16 u + r in digit-reversed order
+  const int ku = M == 8 ? (u >> 2) | (u & 3) << 2 : (M == 7 ? (u >> 2) | (u & 3) << 1 : u);
+  auto turn = [&](int w) {
+    if (M == 4) return;
+#pragma unroll
+    for (int r = 0; r < 16; r++) lds[((r << (M - 4)) | w) * TI + l] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = lds[(u << 4 | r) * TI + l];
+  };
+  constexpr int dir = MODE == 1 ? FL_INV : FL_FWD;
+  fft_upper<M>(v, u, tws, dir);
+  turn(u);
+  fft_lower<M>(v, tws, dir);
+  if (MODE == 2) {
+    const float intot = (float)(1.0 / ((double)g.nx * g.ny * g.nz));
+    const float coef = (float)(((g.dt * g.beta) / g.re) / 2.0);
+    const float kxy = kx2[kx] + ky2[other];
+    float2 w[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int rk = (r & 3) << 2 | r >> 2, kk = (rk << (M - 4)) | ku;
+      const float lhs = kind == 3 ? -(kxy + kz2[kk]) : 1.0f + coef * (kxy + kz2[kk]);
+      const float sc = fabsf(lhs) < 1.0e-16f ? 0.0f : intot / lhs;
+      w[rk] = scaled(v[r], sc);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = w[r];
+    fft_upper<M>(v, ku, tws, FL_BACK);
+    __syncthreads();   // (the first exchange is read)
+    turn(ku);
+    fft_lower<M>(v, tws, FL_BACK);
+  }
+  if (on) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) base[stride * ((((r & 3) << 2 | r >> 2) << (M - 4)) | ku)] = v[r];
+  }
+}
+
 // In-place radix-2 transforms along the slow index of an LDS array held
 // [point][row] (rows contiguous, point pitch P), for nr rows (a power of two,
 // lnr = log2 nr) of n points.  Consecutive threads take consecutive rows of
@@ -2129,6 +2274,33 @@ static int lines_for32(int n) { return std::max(2, std::min(16, 4096 / n)) & ~1;
 // kx columns per block of the y/z transforms (pitch n + 1)
 static int cols_for32(int n) { return std::max(1, std::min(16, 3968 / (n + 1))); }
 
+// transforms of all y (axis 1) or z (axis 2) lines of the half spectrum; mode
+// and kind as in m_fft_yz, the z lines of ny rows from row0 on
+static void fft_lines(Ctx& c, int axis, int mode, int kind, int row0, const int* skip) {
+  Mixed& X = MX(c);
+  const Grid& g = c.g;
+  const int n = axis == 1 ? g.ny : g.nz;
+  const long others = axis == 1 ? g.nz : g.ny;
+  const float2* tw = axis == 1 ? X.twy : X.twz;
+  auto lines = [&](auto m) {
+    constexpr int M = decltype(m)::value;
+    auto k = mode == 0 ? m_fft_lines<M, 0> : (mode == 1 ? m_fft_lines<M, 1> : m_fft_lines<M, 2>);
+    const long nl = g.nxh * others;
+    hipLaunchKernelGGL(k, dim3(nblk(nl, fl_lines(M))), dim3(fl_threads(M)), 0, c.stream, g, X.spec, tw, axis, kind, row0, nl,
+                       X.kx2, X.ky2, X.kz2, skip);
+  };
+  switch (n) {
+    case 16: return lines(std::integral_constant<int, 4>{});
+    case 32: return lines(std::integral_constant<int, 5>{});
+    case 64: return lines(std::integral_constant<int, 6>{});
+    case 128: return lines(std::integral_constant<int, 7>{});
+    case 256: return lines(std::integral_constant<int, 8>{});
+  }
+  const int ti = cols_for32(n), nt = (g.nxh + ti - 1) / ti;
+  hipLaunchKernelGGL(m_fft_yz, dim3(nt * others), dim3(256), sizeof(float2) * (2 * (size_t)ti * (n + 1) + n / 2), c.stream, g,
+                     X.spec, tw, axis, mode, kind, row0, ti, X.kx2, X.ky2, X.kz2, skip);
+}
+
 // y and z transforms (periodic y) or z transforms and the y line solve
 // (walls) of the half spectrum, with the spectral divide of the solve kind
 static void solve32_yz(Ctx& c, int kind, const int* skip, int tr = 0) {
@@ -2141,21 +2313,17 @@ static void solve32_yz(Ctx& c, int kind, const int* skip, int tr = 0) {
                        skip);
     return;
   }
-  int tiy = cols_for32(g.ny), tiz = cols_for32(g.nz);
-  int nty = (g.nxh + tiy - 1) / tiy, ntz = (g.nxh + tiz - 1) / tiz;
-  size_t shy = sizeof(float2) * (2 * (size_t)tiy * (g.ny + 1) + g.ny / 2);
-  size_t shz = sizeof(float2) * (2 * (size_t)tiz * (g.nz + 1) + g.nz / 2);
   if (!g.walls) {
-    hipLaunchKernelGGL(m_fft_yz, dim3(nty * g.nz), dim3(256), shy, s, g, X.spec, X.twy, 1, 0, kind, 0, tiy, X.kx2, X.ky2, X.kz2, skip);
-    hipLaunchKernelGGL(m_fft_yz, dim3(ntz * g.ny), dim3(256), shz, s, g, X.spec, X.twz, 2, 2, kind, 0, tiz, X.kx2, X.ky2, X.kz2, skip);
-    hipLaunchKernelGGL(m_fft_yz, dim3(nty * g.nz), dim3(256), shy, s, g, X.spec, X.twy, 1, 1, kind, 0, tiy, X.kx2, X.ky2, X.kz2, skip);
+    fft_lines(c, 1, 0, kind, 0, skip);
+    fft_lines(c, 2, 2, kind, 0, skip);
+    fft_lines(c, 1, 1, kind, 0, skip);
   } else {
-    hipLaunchKernelGGL(m_fft_yz, dim3(ntz * g.ny), dim3(256), shz, s, g, X.spec, X.twz, 2, 0, kind, 1, tiz, X.kx2, X.ky2, X.kz2, skip);
+    fft_lines(c, 2, 0, kind, 1, skip);
     const int tl = thomas_lines(g.ny, (int)(sizeof(float2) + sizeof(float)));
     const int ngrp = (g.nxh + tl - 1) / tl;
     hipLaunchKernelGGL(m_thomas, dim3(ngrp * g.nz), dim3(256), (size_t)(g.ny + 2) * tl * (sizeof(float2) + sizeof(float)),
                        s, g, X.spec, kind, tl, X.kx2, X.kz2, skip);
-    hipLaunchKernelGGL(m_fft_yz, dim3(ntz * g.ny), dim3(256), shz, s, g, X.spec, X.twz, 2, 1, kind, 1, tiz, X.kx2, X.ky2, X.kz2, skip);
+    fft_lines(c, 2, 1, kind, 1, skip);
   }
 }
 
