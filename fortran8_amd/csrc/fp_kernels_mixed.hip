@@ -1138,7 +1138,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
                                                       const float* __restrict__ U, const float* __restrict__ V,
                                                       const float* __restrict__ W, float* __restrict__ Cn,
                                                       float* __restrict__ fC, int* __restrict__ nitr, float eps,
-                                                      int itrmax) {
+                                                      int itrmax, unsigned* __restrict__ amb) {
+  // the count of the selection that the step starts after this kernel
+  if (blockIdx.x == 0 && threadIdx.x == 0) *amb = 0u;
   long m;
   int i, j, k;
   if (!row_cell<false, 0>(g, m, i, j, k)) return;
@@ -1849,18 +1851,22 @@ __device__ __forceinline__ float2 cmul_l(float2 a, float2 w, int dir) {
   if (dir == FL_BACK) return make_float2(fmaf(a.y, -w.y, a.x * w.x), fmaf(a.y, w.x, a.x * w.y));
   return make_float2(fmaf(a.x, w.x, -(a.y * w.y)), fmaf(a.x, w.y, a.y * w.x));
 }
+// tws: the whole circle, without tw_at's branch
+__device__ __forceinline__ float2 fl_tw(const float2* tws, int j, int dir) {
+  const float2 w = tws[j];
+  return dir == FL_FWD ? w : make_float2(w.x, -w.y);
+}
 template <int M>
 __device__ __forceinline__ void fft_bfly4(float2& a0, float2& a1, float2& a2, float2& a3, const float2* tws, int j1,
                                           int dir) {
 #pragma clang fp contract(off)
-  constexpr int half = 1 << (M - 1);
   const float2 b0 = make_float2(a0.x + a2.x, a0.y + a2.y), b1 = make_float2(a0.x - a2.x, a0.y - a2.y);
   const float2 b2 = make_float2(a1.x + a3.x, a1.y + a3.y), d = make_float2(a1.x - a3.x, a1.y - a3.y);
   const float2 b3 = dir != FL_FWD ? make_float2(-d.y, d.x) : make_float2(d.y, -d.x);
   a0 = make_float2(b0.x + b2.x, b0.y + b2.y);
-  a1 = cmul_l(make_float2(b1.x + b3.x, b1.y + b3.y), tw_at(tws, half, j1, dir != FL_FWD), dir);
-  a2 = cmul_l(make_float2(b0.x - b2.x, b0.y - b2.y), tw_at(tws, half, 2 * j1, dir != FL_FWD), dir);
-  a3 = cmul_l(make_float2(b1.x - b3.x, b1.y - b3.y), tw_at(tws, half, 3 * j1, dir != FL_FWD), dir);
+  a1 = cmul_l(make_float2(b1.x + b3.x, b1.y + b3.y), fl_tw(tws, j1, dir), dir);
+  a2 = cmul_l(make_float2(b0.x - b2.x, b0.y - b2.y), fl_tw(tws, 2 * j1, dir), dir);
+  a3 = cmul_l(make_float2(b1.x - b3.x, b1.y - b3.y), fl_tw(tws, 3 * j1, dir), dir);
 }
 // the stages of the upper bits on points u + (N/16) r: two of radix 4, or one
 // of radix 2 and one of radix 4 where M is odd
@@ -1871,7 +1877,7 @@ __device__ __forceinline__ void fft_upper(float2 (&v)[16], int u, const float2* 
 #pragma unroll
     for (int r = 0; r < 8; r++) {
       const float2 a = v[r], b = v[8 + r];
-      const float2 w = tw_at(tws, 1 << (M - 1), (r << (M - 4)) | u, dir != FL_FWD);
+      const float2 w = fl_tw(tws, (r << (M - 4)) | u, dir);
       v[r] = make_float2(a.x + b.x, a.y + b.y);
       const float2 d = make_float2(a.x - b.x, a.y - b.y), t = cmul_l(d, w, dir);
       v[8 + r] = dir == FL_BACK ? make_float2(cmul_l(d, w, FL_INV).x, t.y) : t;   // (as compiled there)
@@ -1917,7 +1923,7 @@ __global__ __launch_bounds__(fl_threads(M)) void m_fft_lines(Grid g, float2* __r
   if (skip && *skip) return;
   constexpr int N = 1 << M, TI = fl_lines(M);
   __shared__ float2 lds[N * TI];
-  __shared__ float2 tws[N / 2];
+  __shared__ float2 tws[N];
   const int l = threadIdx.x % TI, u = threadIdx.x / TI;
   const long L = blockIdx.x * (long)TI + l;
   const bool on = L < nlines;
@@ -1926,7 +1932,11 @@ __global__ __launch_bounds__(fl_threads(M)) void m_fft_lines(Grid g, float2* __r
   const unsigned other = Lc / (unsigned)nxh, kx = Lc - other * (unsigned)nxh;
   const long stride = axis == 1 ? (long)nxh : (long)nxh * g.sy;
   float2* base = axis == 1 ? spec + (long)nxh * (g.jo + (long)g.sy * other) + kx : spec + (long)nxh * row0 + Lc;
-  load_twiddles(tws, tw, N);
+  for (int e = threadIdx.x; e < N / 2; e += fl_threads(M)) {
+    const float2 w = tw[e];
+    tws[e] = w;
+    tws[e + N / 2] = make_float2(-w.x, -w.y);
+  }
   float2 v[16];
 #pragma unroll
   for (int r = 0; r < 16; r++) v[r] = base[stride * ((r << (M - 4)) | u)];
@@ -2051,6 +2061,109 @@ __device__ void fft_cols_inplace(float2* S, int P, int nr, int lnr, int n, int l
   }
 }
 
+// 1 / (a_r + c_r P_{r-1}) of every (kx, kz) line's rows 1 to ny + 1 of the slab
+// solve, P_r = -b_r times that, for pbuf ([kx][row][kz]): they depend on the
+// grid only.  0 where the pivot vanishes (the mean mode's last row).
+__global__ __launch_bounds__(256) void m_slab_pivots(Grid g, const float* __restrict__ kx2, const float* __restrict__ kz2,
+                                                     float* __restrict__ pbuf) {
+  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  if (t >= (long)g.nxh * g.nz) return;
+  const int kk = (int)(t % g.nz);
+  const long kx = t / g.nz;
+  float* I = pbuf + (size_t)g.sy * g.nz * kx + kk;
+  const float idy2 = (float)(1.0 / (g.dy * g.dy));
+  const float kq = kx2[kx] + kz2[kk];
+  const float ai = -(kq + 2.0f * idy2);
+  float Pp = 1.0f;   // row 0: a = 1, b = -1
+  for (int r = 1; r < g.sy; r++) {
+    const bool last = r == g.sy - 1;
+    const float a = last ? 1.0f : ai, cc = last ? -1.0f : idy2;
+    const float den = fmaf(cc, Pp, a);
+    const float id = fabsf(den) < 1.0e-16f * fabsf(a) + 1.0e-30f ? 0.0f : __builtin_amdgcn_rcpf(den);
+    I[(size_t)r * g.nz] = id;
+    Pp = -idy2 * id;
+  }
+}
+
+// The line solve of a slab [kz][row] in the LDS along y, one thread per kz, in
+// batches of TB rows (ny is a multiple) with the next batch's operands loaded
+// while the current one is computed.  The recurrence is the kernel's longest
+// chain: two dependent operations a row each way, the pivots' reciprocals
+// from pbuf.  Rows 0 and ny + 1 carry the boundary rule only and stay unset.
+template <int TB>
+__device__ __forceinline__ void slab_line_solve_by(const Grid& g, float2* S, int pitch, long kx,
+                                                   const float* __restrict__ pbuf) {
+#pragma clang fp contract(off)
+  const int nz = g.nz, ny = g.ny;
+  if ((int)threadIdx.x >= nz) return;
+  const int kk = threadIdx.x;
+  float2* L = S + (size_t)kk * pitch;
+  const float* I = pbuf + (size_t)g.sy * nz * kx + kk;   // [row][kz]
+  const float inxz = (float)(1.0 / ((double)g.nx * g.nz));
+  const float idy2 = (float)(1.0 / (g.dy * g.dy));
+  float Qr = 0.0f, Qi = 0.0f;
+  float2 cur[TB], nxt[TB];
+  float ic[TB], in[TB];
+#pragma unroll
+  for (int t = 0; t < TB; t++) {
+    cur[t] = L[1 + t];
+    ic[t] = I[(1 + t) * nz];
+  }
+  for (int r0 = 1; r0 <= ny; r0 += TB) {
+    if (r0 + TB <= ny) {
+#pragma unroll
+      for (int t = 0; t < TB; t++) {
+        nxt[t] = L[r0 + TB + t];
+        in[t] = I[(r0 + TB + t) * nz];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TB; t++) {
+      Qr = fmaf(-idy2, Qr, cur[t].x * inxz) * ic[t];
+      Qi = fmaf(-idy2, Qi, cur[t].y * inxz) * ic[t];
+      L[r0 + t] = make_float2(Qr, Qi);
+    }
+#pragma unroll
+    for (int t = 0; t < TB; t++) {
+      cur[t] = nxt[t];
+      ic[t] = in[t];
+    }
+  }
+  // row ny + 1: x_{ny+1} = x_ny; then x_r = P_r x_{r+1} + Q_r, r = ny .. 1
+  const float il = I[(ny + 1) * nz];
+  float xr = Qr * il, xi = Qi * il;
+#pragma unroll
+  for (int t = 0; t < TB; t++) {
+    cur[t] = L[ny - t];
+    ic[t] = I[(ny - t) * nz];
+  }
+  for (int r0 = ny; r0 >= 1; r0 -= TB) {
+    if (r0 > TB) {
+#pragma unroll
+      for (int t = 0; t < TB; t++) {
+        nxt[t] = L[r0 - TB - t];
+        in[t] = I[(r0 - TB - t) * nz];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TB; t++) {
+      const float P = -idy2 * ic[t];
+      xr = fmaf(P, xr, cur[t].x);
+      xi = fmaf(P, xi, cur[t].y);
+      L[r0 - t] = make_float2(xr, xi);
+    }
+#pragma unroll
+    for (int t = 0; t < TB; t++) {
+      cur[t] = nxt[t];
+      ic[t] = in[t];
+    }
+  }
+}
+__device__ __forceinline__ void slab_line_solve(const Grid& g, float2* S, int pitch, long kx, const float* __restrict__ pbuf) {
+  if (g.ny >= 8) slab_line_solve_by<8>(g, S, pitch, kx, pbuf);
+  else slab_line_solve_by<4>(g, S, pitch, kx, pbuf);
+}
+
 // Pressure Poisson solve of one kx slab with y-walls (fft_poisson_kabe and
 // tdma, fenep_2d.f90:1145-1177, 1179-1342): forward z transforms of the
 // interior rows, the line solve along y of every kz (boundary rows x_0 = x_1,
@@ -2061,12 +2174,11 @@ __device__ void fft_cols_inplace(float2* S, int P, int nr, int lnr, int n, int l
 // reversals are folded into the copies: the load puts kz at its bit-reversed
 // place for the decimation-in-time forward transform, and the store reads
 // the decimation-in-frequency inverse's bit-reversed output.  The line solve
-// keeps its P coefficients in pbuf (L2).
+// takes its pivots from pbuf (m_slab_pivots).
 static int slab_pitch(const Grid& g) { return g.sy | 1; }
 static size_t lds_slab(const Grid& g) { return sizeof(float2) * ((size_t)g.nz * slab_pitch(g) + g.nz / 2); }
 __global__ __launch_bounds__(1024) void m_poisson_slab(Grid g, float2* __restrict__ spec, const float2* __restrict__ tw,
-                                                      const float* __restrict__ kx2, const float* __restrict__ kz2,
-                                                      float* __restrict__ pbuf, const int* __restrict__ skip) {
+                                                      const float* __restrict__ pbuf, const int* __restrict__ skip) {
   if (skip && *skip) return;
   extern __shared__ float2 lds[];
   const int nz = g.nz, sy = g.sy, ny = g.ny, pitch = g.sy | 1;
@@ -2100,79 +2212,7 @@ __global__ __launch_bounds__(1024) void m_poisson_slab(Grid g, float2* __restric
   }
   __syncthreads();
   fft_cols_inplace(S + 1, pitch, ny, g.lny, nz, logn, tws, false, false);
-  // line solve along y, one thread per kz; rows go in batches of TB with the
-  // next batch's operands loaded while the current one is computed (the back
-  // substitution reads P from L2)
-  if ((int)threadIdx.x < nz) {
-    constexpr int TB = 8;
-    const int kk = threadIdx.x;
-    float2* L = S + (size_t)kk * pitch;
-    float* P = pbuf + (size_t)sy * nz * kx;   // [row][kz]
-    const float inxz = (float)(1.0 / ((double)g.nx * g.nz));
-    const float idy2 = (float)(1.0 / (g.dy * g.dy));
-    const float kq = kx2[kx] + kz2[kk];
-    const float ai = -(kq + 2.0f * idy2);
-    float Pp = 1.0f, Qr = 0.0f, Qi = 0.0f;   // row 0: a = 1, b = -1
-    P[kk] = Pp;
-    L[0] = make_float2(0.0f, 0.0f);
-    float2 cur[TB];
-#pragma unroll
-    for (int t = 0; t < TB; t++) cur[t] = 1 + t < sy ? L[1 + t] : make_float2(0.0f, 0.0f);
-    for (int r0 = 1; r0 < sy; r0 += TB) {
-      float2 nxt[TB];
-#pragma unroll
-      for (int t = 0; t < TB; t++) nxt[t] = r0 + TB + t < sy ? L[r0 + TB + t] : make_float2(0.0f, 0.0f);
-#pragma unroll
-      for (int t = 0; t < TB; t++) {
-        const int r = r0 + t;
-        if (r < sy) {
-          const bool last = r == sy - 1;
-          const float a = last ? 1.0f : ai;
-          const float bb = last ? 0.0f : idy2;
-          const float cc = last ? -1.0f : idy2;
-          const float dr = last ? 0.0f : cur[t].x * inxz, di = last ? 0.0f : cur[t].y * inxz;
-          const float den = a + cc * Pp;
-          if (fabsf(den) < 1.0e-16f * fabsf(a) + 1.0e-30f) { Pp = 0.0f; Qr = 0.0f; Qi = 0.0f; }
-          else { const float id = __builtin_amdgcn_rcpf(den); Pp = -bb * id; Qr = (dr - cc * Qr) * id; Qi = (di - cc * Qi) * id; }
-          P[r * nz + kk] = Pp;
-          L[r] = make_float2(Qr, Qi);
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < TB; t++) cur[t] = nxt[t];
-    }
-    // back substitution x_r = P_r x_{r+1} + Q_r, r = sy-2 .. 0
-    float xr = Qr, xi = Qi;
-    float pc[TB];
-    float2 qc[TB];
-#pragma unroll
-    for (int t = 0; t < TB; t++) {
-      const int r = sy - 2 - t;
-      pc[t] = r >= 0 ? P[r * nz + kk] : 0.0f;
-      qc[t] = r >= 0 ? L[r] : make_float2(0.0f, 0.0f);
-    }
-    for (int r0 = sy - 2; r0 >= 0; r0 -= TB) {
-      float pn[TB];
-      float2 qn[TB];
-#pragma unroll
-      for (int t = 0; t < TB; t++) {
-        const int r = r0 - TB - t;
-        pn[t] = r >= 0 ? P[r * nz + kk] : 0.0f;
-        qn[t] = r >= 0 ? L[r] : make_float2(0.0f, 0.0f);
-      }
-#pragma unroll
-      for (int t = 0; t < TB; t++) {
-        const int r = r0 - t;
-        if (r >= 0) {
-          xr = pc[t] * xr + qc[t].x;
-          xi = pc[t] * xi + qc[t].y;
-          L[r] = make_float2(xr, xi);
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < TB; t++) { pc[t] = pn[t]; qc[t] = qn[t]; }
-    }
-  }
+  slab_line_solve(g, S, pitch, kx, pbuf);
   __syncthreads();
   fft_cols_inplace(S + 1, pitch, ny, g.lny, nz, logn, tws, true, true);
   for (int e = threadIdx.x; e < ny * nz; e += blockDim.x) {
@@ -2180,6 +2220,145 @@ __global__ __launch_bounds__(1024) void m_poisson_slab(Grid g, float2* __restric
     const int rk = (int)(__brev((unsigned)kk) >> (32 - logn));
     slab[(size_t)sy * kk + j + 1] = S[(size_t)rk * pitch + j + 1];
   }
+}
+
+// The same solve for 16 to 256 planes with the z transforms in registers, 16
+// points of a row's line to a thread: the stages of the lower four index bits
+// on points 16 u + r, the others on points u + (N/16) r, one exchange through
+// the slab between them, and the loads and stores of the spectrum straight from
+// and to registers.  The radix-2 butterflies are fft_cols_inplace's, with the
+// fusions that it is compiled to written out, so the values are the same.
+// A slab is one block on one CU, so what counts is the length of its chain: a
+// barrier and an LDS pass for every two stages, 53 us at 256x128x128 (20 at
+// 128x64x64), are now one barrier a transform: 30 and 13 us, the line solve with
+// its reciprocals taken once included.
+template <int M>
+__device__ __forceinline__ void slab_dit(float2 (&v)[16], int lh, int r, int k, const float2* tws, int bit) {
+#pragma clang fp contract(off)
+  const float2 a = v[r], t = cmul_l(v[r | bit], tws[k << (M - 1 - lh)], FL_FWD);
+  v[r | bit] = make_float2(a.x - t.x, a.y - t.y);
+  v[r] = make_float2(a.x + t.x, a.y + t.y);
+}
+// inv: conjugate twiddles.  The second stage of a pair rounds one product of
+// its upper butterflies (`upper`) in the other order.
+template <int M>
+__device__ __forceinline__ void slab_dif(float2 (&v)[16], int lh, int r, int k, const float2* tws, int bit, bool upper) {
+#pragma clang fp contract(off)
+  const float2 a = v[r], b = v[r | bit];
+  const float2 d = make_float2(a.x - b.x, a.y - b.y), w0 = tws[k << (M - 1 - lh)], w = make_float2(w0.x, -w0.y);
+  const float2 t = cmul_l(d, w, FL_BACK);
+  v[r] = make_float2(a.x + b.x, a.y + b.y);
+  v[r | bit] = upper && lh % 2 == 0 && lh <= M - 2 ? make_float2(cmul_l(d, w, FL_INV).x, t.y) : t;
+}
+template <int M>
+__global__ __launch_bounds__(1024) void m_poisson_slab_lines(Grid g, float2* __restrict__ spec, const float2* __restrict__ tw,
+                                                            const float* __restrict__ pbuf, const int* __restrict__ skip) {
+  if (skip && *skip) return;
+  extern __shared__ float2 lds[];
+  const int nz = 1 << M, sy = g.sy, ny = g.ny, pitch = g.sy | 1;
+  const long kx = blockIdx.x;
+  float2* S = lds;                              // [kz][pitch]
+  float2* tws = lds + (size_t)nz * pitch;
+  load_twiddles(tws, tw, nz);
+  float2* slab = spec + (size_t)sy * nz * kx;   // [kz][row]
+  const int rows = (int)blockDim.x >> (M - 4);  // (a power of two)
+  const int l = threadIdx.x & (rows - 1), u = threadIdx.x / rows;
+  const int ru = M > 4 ? (int)(__brev((unsigned)u) >> (32 - (M > 4 ? M - 4 : 1))) : 0;
+  constexpr int brev4[16] = {0, 8, 4, 12, 2, 10, 6, 14, 1, 9, 5, 13, 3, 11, 7, 15};
+  __syncthreads();
+  // a row's points p = 16 u + r from A, p = u + (N/16) r from B, of the line in
+  // bit-reversed order from G (what depends on the thread's place is taken
+  // anew in every turn: kept in registers it spills)
+  for (int c0 = 0; c0 < ny; c0 += rows) {
+    int uu = u, rr = ru;
+    asm volatile("" : "+v"(uu), "+v"(rr));
+    const bool on = c0 + l < ny;
+    const int row = on ? c0 + l + 1 : ny;       // (idle threads repeat the last row)
+    const float2* G = slab + (unsigned)(sy * rr + row);
+    float2 *A = S + (uu * 16) * pitch + row, *B = S + uu * pitch + row;
+    float2 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = G[sy * (brev4[r] << (M - 4))];
+#pragma unroll
+    for (int lh = 0; lh < 4; lh++)
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+        if (!(r >> lh & 1)) slab_dit<M>(v, lh, r, r & ((1 << lh) - 1), tws, 1 << lh);
+    if (M > 4) {
+      if (on) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) A[r * pitch] = v[r];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 16; r++) v[r] = B[(r << (M - 4)) * pitch];
+#pragma unroll
+      for (int lh = 4; lh < M; lh++)
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          if (!(r >> (lh - M + 4) & 1))
+            slab_dit<M>(v, lh, r, ((r << (M - 4)) | uu) & ((1 << lh) - 1), tws, 1 << (lh - M + 4));
+    }
+    if (on) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) B[(r << (M - 4)) * pitch] = v[r];
+    }
+  }
+  __syncthreads();
+  slab_line_solve(g, S, pitch, kx, pbuf);
+  __syncthreads();
+  for (int c0 = 0; c0 < ny; c0 += rows) {
+    int uu = u, rr = ru;
+    asm volatile("" : "+v"(uu), "+v"(rr));
+    const bool on = c0 + l < ny;
+    const int row = on ? c0 + l + 1 : ny;
+    float2* G = slab + (unsigned)(sy * rr + row);
+    float2 *A = S + (uu * 16) * pitch + row, *B = S + uu * pitch + row;
+    float2 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = B[(r << (M - 4)) * pitch];
+    if (M > 4) {
+#pragma unroll
+      for (int lh = M - 1; lh >= 4; lh--)
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          if (!(r >> (lh - M + 4) & 1))
+            slab_dif<M>(v, lh, r, ((r << (M - 4)) | uu) & ((1 << lh) - 1), tws, 1 << (lh - M + 4),
+                        lh < M - 1 && (r >> (lh - M + 5) & 1));
+      if (on) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) B[(r << (M - 4)) * pitch] = v[r];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 16; r++) v[r] = A[r * pitch];
+    }
+#pragma unroll
+    for (int lh = 3; lh >= 0; lh--)
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+        if (!(r >> lh & 1)) slab_dif<M>(v, lh, r, r & ((1 << lh) - 1), tws, 1 << lh, r >> (lh + 1) & 1);
+    if (on) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) G[sy * (brev4[r] << (M - 4))] = v[r];
+    }
+  }
+}
+
+using SlabKernel = void (*)(Grid, float2*, const float2*, const float*, const int*);
+static SlabKernel slab_kernel(const Grid& g) {
+  switch (g.nz) {
+    case 16: return m_poisson_slab_lines<4>;
+    case 32: return m_poisson_slab_lines<5>;
+    case 64: return m_poisson_slab_lines<6>;
+    case 128: return m_poisson_slab_lines<7>;
+    case 256: return m_poisson_slab_lines<8>;
+  }
+  return m_poisson_slab;
+}
+// threads of a block: nz / 16 for every row, and one for every kz
+static int slab_threads(const Grid& g) {
+  return g.nz < 16 || g.nz > 256 ? 1024 : std::min(1024, std::max(std::max(g.nz, 64), g.ny * (g.nz / 16)));
 }
 
 // Line solve along y of each (kx, kz) mode (FP32), staged through LDS like
@@ -2309,8 +2488,7 @@ static void solve32_yz(Ctx& c, int kind, const int* skip, int tr = 0) {
   hipStream_t s = c.stream;
   if (tr) {
     // transposed half spectrum, walls, pressure Poisson
-    hipLaunchKernelGGL(m_poisson_slab, dim3(g.nxh), dim3(1024), lds_slab(g), s, g, X.spec, X.twz, X.kx2, X.kz2, X.pbuf,
-                       skip);
+    hipLaunchKernelGGL(slab_kernel(g), dim3(g.nxh), dim3(slab_threads(g)), lds_slab(g), s, g, X.spec, X.twz, X.pbuf, skip);
     return;
   }
   if (!g.walls) {
@@ -3243,7 +3421,7 @@ void mixed_create(Ctx& c) {
     FP_HIP_CHECK(hipGetDevice(&dev));
     FP_HIP_CHECK(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     if (lds_slab(g) <= (size_t)lds_max && g.nz <= 1024) {
-      FP_HIP_CHECK(hipFuncSetAttribute((const void*)m_poisson_slab, hipFuncAttributeMaxDynamicSharedMemorySize,
+      FP_HIP_CHECK(hipFuncSetAttribute((const void*)slab_kernel(g), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)lds_slab(g)));
       X->slab = 1;
       dalloc(&X->pbuf, (size_t)g.nxh * g.sy * g.nz);
@@ -3283,6 +3461,10 @@ void mixed_create(Ctx& c) {
   };
   tw32(c.twx, g.nx, &X->twx); tw32(c.twy, g.ny, &X->twy); tw32(c.twz, g.nz, &X->twz);
   k32(c.kx2, g.nxh, &X->kx2); k32(c.ky2, g.ny, &X->ky2); k32(c.kz2, g.nz, &X->kz2);
+  if (X->slab) {
+    hipLaunchKernelGGL(m_slab_pivots, dim3(nblk((long)g.nxh * g.nz, 256)), dim3(256), 0, c.stream, g, X->kx2, X->kz2, X->pbuf);
+    FP_HIP_CHECK(hipStreamSynchronize(c.stream));
+  }
 }
 
 void mixed_destroy(Ctx& c) {
@@ -3637,7 +3819,7 @@ double mixed_last_ndc(Ctx& c) {
 // C+- selection of the current stored field: certified FP32 decisions, the
 // per-block list counts scanned, the rest re-decided in FP64.  tm != 0 times
 // the two phases.
-static void select_fenep(Ctx& c, int tm, hipStream_t s);
+static void select_fenep(Ctx& c, int tm, hipStream_t s, bool cleared = false);
 
 // Selection of the current stored field as the step makes it (certified FP32
 // decisions, FP64 re-decision of the rest), compared with the reference's
@@ -3847,9 +4029,10 @@ static void select_launch(Ctx& c, const T* C, unsigned* total, unsigned* idx, un
   }
 }
 
-static void select_fenep(Ctx& c, int tm, hipStream_t s) {
+// cleared: X.amb is zero
+static void select_fenep(Ctx& c, int tm, hipStream_t s, bool cleared) {
   Mixed& X = MX(c);
-  zero_words(X.amb, 1, s);
+  if (!cleared) zero_words(X.amb, 1, s);
   select_launch<float>(c, X.C[X.cur], X.amb, X.amb_idx, X.amb_list, X.amb_data, tm, s);
 }
 
@@ -3873,7 +4056,7 @@ static void select_ahead(Ctx& c) {
   Mixed& X = MX(c);
   FP_HIP_CHECK(hipEventRecord(X.ev_cstar, c.stream));
   FP_HIP_CHECK(hipStreamWaitEvent(X.side, X.ev_cstar, 0));
-  select_fenep(c, 1, X.side);
+  select_fenep(c, 1, X.side, true);   // (m_cstar_newton has cleared the count)
   FP_HIP_CHECK(hipEventRecord(X.sel_done, X.side));
   X.sel_ready = 1;
 }
@@ -3994,7 +4177,7 @@ void mixed_step(Ctx& c) {
     {
       MTimer t(c, "fenep_cstar_newton");
       hipLaunchKernelGGL(m_cstar_newton, dim3(nblk(n, 256)), dim3(256), 0, s, g, X.C[X.cur], c.sel, X.U, X.V, X.W,
-                         X.C[1 - X.cur], X.f, c.nitr, (float)c.p.newton_eps, itmax);
+                         X.C[1 - X.cur], X.f, c.nitr, (float)c.p.newton_eps, itmax, X.amb);
     }
     X.cur = 1 - X.cur;
   }
