@@ -179,71 +179,107 @@ __device__ __forceinline__ double c0_at(const Grid& g, const double* __restrict_
   return fC[m] * C[q * g.n + m] - E;
 }
 
-// convection (fenep.f90:694-734), viscous (736-770), polymer_stress
+// One cell of the predictor over a stencil accessor S (v(c, ..): velocity
+// component c, c0(q, ..): C0, at an offset from the cell): convection (fenep.f90:694-734), viscous (736-770), polymer_stress
 // (645-691) and the predictor right-hand side of navier (803-826),
 // fft_navier (1466-1511) or ibm_preliminary (1994-2013), with the history
 // updates A0=A, T0=T, B0=B done in place.
+// the cell's own inputs, read where they are used
 template <bool WL>
-__global__ __launch_bounds__(256) void k_predictor(Grid g, int method, int first, int polymer,
-                                                   const double* __restrict__ U, const double* __restrict__ V,
-                                                   const double* __restrict__ W, const double* __restrict__ P,
-                                                   const double* __restrict__ C, const double* __restrict__ fC,
-                                                   double* __restrict__ A0, double* __restrict__ T0, double* __restrict__ B0,
-                                                   double* __restrict__ Rout, const double* __restrict__ F,
-                                                   double bf0, double bf1, double bf2, double* __restrict__ Q) {
-  const long L = xcd_cell();
-  if (L >= g.n) return;
-  long m;
+struct PredAt {
+  const Grid& g;
+  const double *A0, *T0, *B0, *F, *P;
   int i, j, k;
-  band_cell(g, L, m, i, j, k);
-  const double dx = g.dx, dy = g.dy, dz = g.dz, dt = g.dt;
-#define Ug(a, b, c) ldbw<WL>(U, g, a, b, c, BC_U)
-#define Vg(a, b, c) ldbw<WL>(V, g, a, b, c, BC_V)
-#define Wg(a, b, c) ldbw<WL>(W, g, a, b, c, BC_W)
+  long m;
+  __device__ __forceinline__ double a0(int c) const { return A0[c * g.n + m]; }
+  __device__ __forceinline__ double t0(int c) const { return T0[c * g.n + m]; }
+  __device__ __forceinline__ double b0(int c) const { return B0[c * g.n + m]; }
+  __device__ __forceinline__ double f(int c) const { return F ? F[c * g.n + m] : 0.0; }
+  __device__ __forceinline__ double p() const { return P[m]; }
+  __device__ __forceinline__ double p1(int c) const {
+    return ldbw<WL>(P, g, i + (c == 0), j + (c == 1), k + (c == 2), BC_P);
+  }
+};
+// the same, all loaded ahead
+struct PredIn {
+  double a[3], t[3], b[3], fv[3], pm, pp[3];
+  template <bool WL>
+  __device__ __forceinline__ void load(const PredAt<WL>& s, int first) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      a[c] = first ? 0.0 : s.a0(c);
+      t[c] = first ? 0.0 : s.t0(c);
+      b[c] = first ? 0.0 : s.b0(c);
+      fv[c] = s.f(c);
+      pp[c] = s.p1(c);
+    }
+    pm = s.p();
+  }
+  __device__ __forceinline__ double a0(int c) const { return a[c]; }
+  __device__ __forceinline__ double t0(int c) const { return t[c]; }
+  __device__ __forceinline__ double b0(int c) const { return b[c]; }
+  __device__ __forceinline__ double f(int c) const { return fv[c]; }
+  __device__ __forceinline__ double p() const { return pm; }
+  __device__ __forceinline__ double p1(int c) const { return pp[c]; }
+};
+
+// divisors of the predictor with their correctly rounded reciprocals (quot)
+struct PredConst {
+  double dx, dy, dz, dxx, dyy, dzz, dx4, dy4, dz4;
+  double idx, idy, idz, idxx, idyy, idzz, idx4, idy4, idz4;
+};
+template <bool WL, class Acc, class In>
+__device__ __forceinline__ void pred_cell(const Grid& g, const PredConst& K, const Acc& S, const In& in, int method,
+                                          int first, int polymer, int i, int j, int k, long m, double* A0, double* T0,
+                                          double* B0, double* __restrict__ Rout, double bf0, double bf1, double bf2,
+                                          double* __restrict__ Q) {
+  const double dt = g.dt;
+#define DIV(n, d) quot(n, K.d, K.i##d)
+#define Ug(a, b, c) S.v(0, (a) - i, (b) - j, (c) - k)
+#define Vg(a, b, c) S.v(1, (a) - i, (b) - j, (c) - k)
+#define Wg(a, b, c) S.v(2, (a) - i, (b) - j, (c) - k)
   double a[3], bv[3], t[3];
   {
     double h1 = (Ug(i - 1, j, k) + Ug(i, j, k)) / 2.0, h2 = (Ug(i, j, k) + Ug(i + 1, j, k)) / 2.0;
-    double ax = ((-(h1 * h1) + h2 * h2) / dx
-                 + (-((((Vg(i, j - 1, k) + Vg(i + 1, j - 1, k)) / 2.0) * (Ug(i, j - 1, k) + Ug(i, j, k))) / 2.0)
-                    + (((Vg(i, j, k) + Vg(i + 1, j, k)) / 2.0) * (Ug(i, j, k) + Ug(i, j + 1, k))) / 2.0) / dy)
-                + (-((((Wg(i, j, k - 1) + Wg(i + 1, j, k - 1)) / 2.0) * (Ug(i, j, k - 1) + Ug(i, j, k))) / 2.0)
-                   + (((Wg(i, j, k) + Wg(i + 1, j, k)) / 2.0) * (Ug(i, j, k) + Ug(i, j, k + 1))) / 2.0) / dz;
+    double ax = (DIV(-(h1 * h1) + h2 * h2, dx)
+                 + DIV(-((((Vg(i, j - 1, k) + Vg(i + 1, j - 1, k)) / 2.0) * (Ug(i, j - 1, k) + Ug(i, j, k))) / 2.0)
+                    + (((Vg(i, j, k) + Vg(i + 1, j, k)) / 2.0) * (Ug(i, j, k) + Ug(i, j + 1, k))) / 2.0, dy))
+                + DIV(-((((Wg(i, j, k - 1) + Wg(i + 1, j, k - 1)) / 2.0) * (Ug(i, j, k - 1) + Ug(i, j, k))) / 2.0)
+                   + (((Wg(i, j, k) + Wg(i + 1, j, k)) / 2.0) * (Ug(i, j, k) + Ug(i, j, k + 1))) / 2.0, dz);
     double g1 = (Vg(i, j - 1, k) + Vg(i, j, k)) / 2.0, g2 = (Vg(i, j, k) + Vg(i, j + 1, k)) / 2.0;
-    double ay = ((-((((Ug(i - 1, j, k) + Ug(i - 1, j + 1, k)) / 2.0) * (Vg(i - 1, j, k) + Vg(i, j, k))) / 2.0)
-                  + (((Ug(i, j, k) + Ug(i, j + 1, k)) / 2.0) * (Vg(i, j, k) + Vg(i + 1, j, k))) / 2.0) / dx
-                 + (-(g1 * g1) + g2 * g2) / dy)
-                + (-((((Wg(i, j, k - 1) + Wg(i, j + 1, k - 1)) / 2.0) * (Vg(i, j, k - 1) + Vg(i, j, k))) / 2.0)
-                   + (((Wg(i, j, k) + Wg(i, j + 1, k)) / 2.0) * (Vg(i, j, k) + Vg(i, j, k + 1))) / 2.0) / dz;
+    double ay = (DIV(-((((Ug(i - 1, j, k) + Ug(i - 1, j + 1, k)) / 2.0) * (Vg(i - 1, j, k) + Vg(i, j, k))) / 2.0)
+                  + (((Ug(i, j, k) + Ug(i, j + 1, k)) / 2.0) * (Vg(i, j, k) + Vg(i + 1, j, k))) / 2.0, dx)
+                 + DIV(-(g1 * g1) + g2 * g2, dy))
+                + DIV(-((((Wg(i, j, k - 1) + Wg(i, j + 1, k - 1)) / 2.0) * (Vg(i, j, k - 1) + Vg(i, j, k))) / 2.0)
+                   + (((Wg(i, j, k) + Wg(i, j + 1, k)) / 2.0) * (Vg(i, j, k) + Vg(i, j, k + 1))) / 2.0, dz);
     double e1 = (Wg(i, j, k - 1) + Wg(i, j, k)) / 2.0, e2 = (Wg(i, j, k) + Wg(i, j, k + 1)) / 2.0;
-    double az = ((-((((Ug(i - 1, j, k) + Ug(i - 1, j, k + 1)) / 2.0) * (Wg(i - 1, j, k) + Wg(i, j, k))) / 2.0)
-                  + (((Ug(i, j, k) + Ug(i, j, k + 1)) / 2.0) * (Wg(i, j, k) + Wg(i + 1, j, k))) / 2.0) / dx
-                 + (-((((Vg(i, j - 1, k) + Vg(i, j - 1, k + 1)) / 2.0) * (Wg(i, j - 1, k) + Wg(i, j, k))) / 2.0)
-                    + (((Vg(i, j, k) + Vg(i, j, k + 1)) / 2.0) * (Wg(i, j, k) + Wg(i, j + 1, k))) / 2.0) / dy)
-                + (-(e1 * e1) + e2 * e2) / dz;
+    double az = (DIV(-((((Ug(i - 1, j, k) + Ug(i - 1, j, k + 1)) / 2.0) * (Wg(i - 1, j, k) + Wg(i, j, k))) / 2.0)
+                  + (((Ug(i, j, k) + Ug(i, j, k + 1)) / 2.0) * (Wg(i, j, k) + Wg(i + 1, j, k))) / 2.0, dx)
+                 + DIV(-((((Vg(i, j - 1, k) + Vg(i, j - 1, k + 1)) / 2.0) * (Wg(i, j - 1, k) + Wg(i, j, k))) / 2.0)
+                    + (((Vg(i, j, k) + Vg(i, j, k + 1)) / 2.0) * (Wg(i, j, k) + Wg(i, j + 1, k))) / 2.0, dy))
+                + DIV(-(e1 * e1) + e2 * e2, dz);
     a[0] = -ax; a[1] = -ay; a[2] = -az;
   }
   const double cb = g.beta / g.re;
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    const double* X = c == 0 ? U : (c == 1 ? V : W);
-    int kind = c == 0 ? BC_U : (c == 1 ? BC_V : BC_W);
-    double x0 = ldbw<WL>(X, g, i, j, k, kind);
-    double bb = (((ldbw<WL>(X, g, i - 1, j, k, kind) - 2.0 * x0) + ldbw<WL>(X, g, i + 1, j, k, kind)) / (dx * dx)
-                 + ((ldbw<WL>(X, g, i, j - 1, k, kind) - 2.0 * x0) + ldbw<WL>(X, g, i, j + 1, k, kind)) / (dy * dy))
-                + ((ldbw<WL>(X, g, i, j, k - 1, kind) - 2.0 * x0) + ldbw<WL>(X, g, i, j, k + 1, kind)) / (dz * dz);
+    double x0 = S.v(c, (i) - i, (j) - j, (k) - k);
+    double bb = (DIV((S.v(c, (i - 1) - i, (j) - j, (k) - k) - 2.0 * x0) + S.v(c, (i + 1) - i, (j) - j, (k) - k), dxx)
+                 + DIV((S.v(c, (i) - i, (j - 1) - j, (k) - k) - 2.0 * x0) + S.v(c, (i) - i, (j + 1) - j, (k) - k), dyy))
+                + DIV((S.v(c, (i) - i, (j) - j, (k - 1) - k) - 2.0 * x0) + S.v(c, (i) - i, (j) - j, (k + 1) - k), dzz);
     bv[c] = cb * bb;
   }
   if (polymer) {
-#define C0g(q, aa, bb, cc) c0_at<WL>(g, C, fC, q, aa, bb, cc)
-    double tx = ((-C0g(0, i, j, k) + C0g(0, i + 1, j, k)) / dx
-                 + (((-C0g(1, i, j - 1, k) - C0g(1, i + 1, j - 1, k)) + C0g(1, i, j + 1, k)) + C0g(1, i + 1, j + 1, k)) / (4.0 * dy))
-                + (((-C0g(2, i, j, k - 1) - C0g(2, i + 1, j, k - 1)) + C0g(2, i, j, k + 1)) + C0g(2, i + 1, j, k + 1)) / (4.0 * dz);
-    double ty = ((((-C0g(1, i - 1, j, k) + C0g(1, i + 1, j, k)) - C0g(1, i - 1, j + 1, k)) + C0g(1, i + 1, j + 1, k)) / (4.0 * dx)
-                 + (-C0g(3, i, j, k) + C0g(3, i, j + 1, k)) / dy)
-                + (((-C0g(4, i, j, k - 1) - C0g(4, i, j + 1, k - 1)) + C0g(4, i, j, k + 1)) + C0g(4, i, j + 1, k + 1)) / (4.0 * dz);
-    double tz = ((((-C0g(2, i - 1, j, k) + C0g(2, i + 1, j, k)) - C0g(2, i - 1, j, k + 1)) + C0g(2, i + 1, j, k + 1)) / (4.0 * dx)
-                 + (((-C0g(4, i, j - 1, k) + C0g(4, i, j + 1, k)) - C0g(4, i, j - 1, k + 1)) + C0g(4, i, j + 1, k + 1)) / (4.0 * dy))
-                + (-C0g(5, i, j, k) + C0g(5, i, j, k + 1)) / dz;
+#define C0g(q, aa, bb, cc) S.c0(q, (aa) - i, (bb) - j, (cc) - k)
+    double tx = (DIV(-C0g(0, i, j, k) + C0g(0, i + 1, j, k), dx)
+                 + DIV(((-C0g(1, i, j - 1, k) - C0g(1, i + 1, j - 1, k)) + C0g(1, i, j + 1, k)) + C0g(1, i + 1, j + 1, k), dy4))
+                + DIV(((-C0g(2, i, j, k - 1) - C0g(2, i + 1, j, k - 1)) + C0g(2, i, j, k + 1)) + C0g(2, i + 1, j, k + 1), dz4);
+    double ty = (DIV(((-C0g(1, i - 1, j, k) + C0g(1, i + 1, j, k)) - C0g(1, i - 1, j + 1, k)) + C0g(1, i + 1, j + 1, k), dx4)
+                 + DIV(-C0g(3, i, j, k) + C0g(3, i, j + 1, k), dy))
+                + DIV(((-C0g(4, i, j, k - 1) - C0g(4, i, j + 1, k - 1)) + C0g(4, i, j, k + 1)) + C0g(4, i, j + 1, k + 1), dz4);
+    double tz = (DIV(((-C0g(2, i - 1, j, k) + C0g(2, i + 1, j, k)) - C0g(2, i - 1, j, k + 1)) + C0g(2, i + 1, j, k + 1), dx4)
+                 + DIV(((-C0g(4, i, j - 1, k) + C0g(4, i, j + 1, k)) - C0g(4, i, j - 1, k + 1)) + C0g(4, i, j + 1, k + 1), dy4))
+                + DIV(-C0g(5, i, j, k) + C0g(5, i, j, k + 1), dz);
 #undef C0g
     const double coef = (1.0 - g.beta) / (g.re * g.wi);
     t[0] = coef * tx; t[1] = coef * ty; t[2] = coef * tz;
@@ -253,17 +289,14 @@ __global__ __launch_bounds__(256) void k_predictor(Grid g, int method, int first
   const double bfs[3] = {bf0, bf1, bf2};
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    const double* X = c == 0 ? U : (c == 1 ? V : W);
-    int kind = c == 0 ? BC_U : (c == 1 ? BC_V : BC_W);
     long o = c * g.n + m;
-    double a0 = first ? a[c] : A0[o];
-    double t0 = first ? t[c] : T0[o];
-    double b0 = first ? bv[c] : B0[o];
-    double u = ldbw<WL>(X, g, i, j, k, kind);
-    double p1 = c == 0 ? ldbw<WL>(P, g, i + 1, j, k, BC_P) : (c == 1 ? ldbw<WL>(P, g, i, j + 1, k, BC_P) : ldbw<WL>(P, g, i, j, k + 1, BC_P));
-    double h = c == 0 ? dx : (c == 1 ? dy : dz);
-    double dp = (dt * (-P[m] + p1)) / h;
-    double fv = (F ? F[o] : 0.0) + bfs[c];
+    double a0 = first ? a[c] : in.a0(c);
+    double t0 = first ? t[c] : in.t0(c);
+    double b0 = first ? bv[c] : in.b0(c);
+    double u = S.v(c, (i) - i, (j) - j, (k) - k);
+    const double dpn = dt * (-in.p() + in.p1(c));
+    double dp = c == 0 ? DIV(dpn, dx) : (c == 1 ? DIV(dpn, dy) : DIV(dpn, dz));
+    double fv = in.f(c) + bfs[c];
     double r;
     if (method == FP_METHOD_EXPLICIT) {
       r = (((u - dp) + (dt * (3.0 * (a[c] + bv[c]) - (a0 + b0))) / 2.0) + (dt * (t[c] + t0)) / 2.0) + dt * fv;
@@ -283,9 +316,156 @@ __global__ __launch_bounds__(256) void k_predictor(Grid g, int method, int first
       Rout[o] = ((wall ? 0.0 : r) + 0.0) - (dt * bv[c]) / 2.0;
     }
   }
+#undef DIV
 #undef Ug
 #undef Vg
 #undef Wg
+}
+
+// any grid: the stencil through the boundary-rule accessor
+template <bool WL>
+struct PredGlobal {
+  const Grid& g;
+  const double *U, *V, *W, *C, *fC;
+  int i, j, k;
+  __device__ __forceinline__ double v(int c, int a, int b, int d) const {
+    return ldbw<WL>(c == 0 ? U : (c == 1 ? V : W), g, i + a, j + b, k + d, c == 0 ? BC_U : (c == 1 ? BC_V : BC_W));
+  }
+  __device__ __forceinline__ double c0(int q, int a, int b, int d) const {
+    return c0_at<WL>(g, C, fC, q, i + a, j + b, k + d);
+  }
+};
+template <bool WL>
+__global__ __launch_bounds__(256) void k_predictor(Grid g, PredConst K, int method, int first, int polymer,
+                                                   const double* __restrict__ U, const double* __restrict__ V,
+                                                   const double* __restrict__ W, const double* __restrict__ P,
+                                                   const double* __restrict__ C, const double* __restrict__ fC,
+                                                   double* __restrict__ A0, double* __restrict__ T0, double* __restrict__ B0,
+                                                   double* __restrict__ Rout, const double* __restrict__ F, double bf0,
+                                                   double bf1, double bf2, double* __restrict__ Q) {
+  const long L = xcd_cell();
+  if (L >= g.n) return;
+  long m;
+  int i, j, k;
+  band_cell(g, L, m, i, j, k);
+  const PredAt<WL> in{g, A0, T0, B0, F, P, i, j, k, m};
+  const PredGlobal<WL> S{g, U, V, W, C, fC, i, j, k};
+  pred_cell<WL>(g, K, S, in, method, first, polymer, i, j, k, m, A0, T0, B0, Rout, bf0, bf1, bf2, Q);
+}
+
+// Streamed along z: a block walks kc planes of a 32 by 8 tile with U, V, W and
+// C0 of three planes and a one-cell halo in the LDS, C0 = f C - E formed once a
+// point instead of at each of its 22 uses, the next plane's loads in flight
+// in registers.  k_predictor's wavefronts wait on some 120 loads each from
+// the caches: 541 us at 256x128x128 there (with divisions; 520 without) and 289
+// here, 64^3 27 and 18, 64x64x32 16 and 12.4.
+#define PD_TX 32
+#define PD_TY 8
+#define PD_HX (PD_TX + 2)
+#define PD_PTS (PD_HX * (PD_TY + 2))
+struct PredLds64 {
+  const double *m, *z, *p;   // planes k-1, k, k+1: nine fields of PD_PTS points
+  int at;
+  __device__ __forceinline__ double v(int c, int a, int b, int d) const {
+    return (d < 0 ? m : (d > 0 ? p : z))[c * PD_PTS + at + a + PD_HX * b];
+  }
+  __device__ __forceinline__ double c0(int q, int a, int b, int d) const { return v(3 + q, a, b, d); }
+};
+struct PdRegs {
+  double v[2][10];   // two points a thread: U, V, W, f, C
+};
+template <bool WL>
+__device__ __forceinline__ void pd_fetch(const Grid& g, int i0, int j0, int k, int polymer, const double* __restrict__ U,
+                                         const double* __restrict__ V, const double* __restrict__ W,
+                                         const double* __restrict__ C, const double* __restrict__ fC, PdRegs& r) {
+#pragma unroll
+  for (int e = 0; e < 2; e++) {
+    const int pt = threadIdx.x + 256 * e;
+    if (pt >= PD_PTS) break;
+    const int i = wrapi(i0 + pt % PD_HX - 1, g.nx);
+    int j = j0 + pt / PD_HX - 1;
+    j = WL ? min(max(j, 0), g.ny - 1) : wrapi(j, g.ny);
+    const long m = cidx(g, i, j, wrapi(k, g.nz));
+    r.v[e][0] = U[m];
+    r.v[e][1] = V[m];
+    r.v[e][2] = W[m];
+    if (polymer) {
+      r.v[e][3] = fC[m];
+#pragma unroll
+      for (int q = 0; q < 6; q++) r.v[e][4 + q] = C[q * g.n + m];
+    }
+  }
+}
+template <bool WL>
+__device__ __forceinline__ void pd_put(const Grid& g, int i0, int j0, int k, int polymer, const double* __restrict__ C,
+                                       const double* __restrict__ fC, const PdRegs& r, double* __restrict__ slot) {
+#pragma unroll
+  for (int e = 0; e < 2; e++) {
+    const int pt = threadIdx.x + 256 * e;
+    if (pt >= PD_PTS) break;
+    const int j = j0 + pt / PD_HX - 1;
+    const bool lo = WL && j < 0, hi = WL && j >= g.ny;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      double v = r.v[e][c];
+      if (WL) {   // U_kabe, V_kabe, W_kabe
+        if (c == 1) v = lo || j >= g.ny - 1 ? 0.0 : v;
+        else v = lo ? -v : (hi ? 2.0 * 0.0 - v : v);
+      }
+      slot[c * PD_PTS + pt] = v;
+    }
+    if (!polymer) continue;
+    if (lo || hi) {
+      const int i = wrapi(i0 + pt % PD_HX - 1, g.nx), kz = wrapi(k, g.nz);
+      for (int q = 0; q < 6; q++) slot[(3 + q) * PD_PTS + pt] = c0_at<WL>(g, C, fC, q, i, j, kz);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 6; q++) {
+        const double E = (q == 0 || q == 3 || q == 5) ? 1.0 : 0.0;
+        slot[(3 + q) * PD_PTS + pt] = r.v[e][3] * r.v[e][4 + q] - E;
+      }
+    }
+  }
+}
+// grid: (nx / PD_TX) (ny / PD_TY) (nz / kc) blocks
+template <bool WL>
+__global__ __launch_bounds__(256, 2) void k_predictor_z(Grid g, PredConst K, int kc, int method, int first, int polymer,
+                                                     const double* __restrict__ U, const double* __restrict__ V,
+                                                     const double* __restrict__ W, const double* __restrict__ P,
+                                                     const double* __restrict__ C, const double* __restrict__ fC, double* A0,
+                                                     double* T0, double* B0, double* __restrict__ Rout,
+                                                     const double* __restrict__ F, double bf0, double bf1, double bf2,
+                                                     double* __restrict__ Q) {
+  __shared__ double lds[3][9 * PD_PTS];
+  const int ntx = g.nx / PD_TX, nty = g.ny / PD_TY;
+  unsigned b = (unsigned)xcd_block();
+  const int i0 = (int)(b % ntx) * PD_TX; b /= ntx;
+  const int j0 = (int)(b % nty) * PD_TY;
+  const int k0 = (int)(b / nty) * kc, k1 = k0 + kc;
+  const int tx = threadIdx.x % PD_TX, ty = threadIdx.x / PD_TX;
+  const int i = i0 + tx, j = j0 + ty;
+  PdRegs r;
+#pragma unroll 1
+  for (int s = 0; s < 3; s++) {
+    pd_fetch<WL>(g, i0, j0, k0 - 1 + s, polymer, U, V, W, C, fC, r);
+    pd_put<WL>(g, i0, j0, k0 - 1 + s, polymer, C, fC, r, lds[s]);
+  }
+  int sm = 0, s0 = 1, sp = 2;
+#pragma unroll 1
+  for (int k = k0; k < k1; k++) {
+    __syncthreads();
+    const bool more = k + 1 < k1;
+    if (more) pd_fetch<WL>(g, i0, j0, k + 2, polymer, U, V, W, C, fC, r);
+    const long m = cidx(g, i, j, k);
+    PredIn in;
+    in.load(PredAt<WL>{g, A0, T0, B0, F, P, i, j, k, m}, first);
+    const PredLds64 S{lds[sm], lds[s0], lds[sp], (ty + 1) * PD_HX + tx + 1};
+    pred_cell<WL>(g, K, S, in, method, first, polymer, i, j, k, m, A0, T0, B0, Rout, bf0, bf1, bf2, Q);
+    if (!more) break;
+    __syncthreads();
+    pd_put<WL>(g, i0, j0, k + 2, polymer, C, fC, r, lds[sm]);
+    const int t = sm; sm = s0; s0 = sp; sp = t;
+  }
 }
 
 // ======================================================= projection =======
@@ -788,9 +968,24 @@ void f64_predictor(Ctx& c) {
   const Grid& g = c.g;
   int polymer = c.p.beta != 1.0;
   double* Rout = c.p.method == FP_METHOD_IBM ? c.Up : nullptr;
-  hipLaunchKernelGGL(c.g.walls ? k_predictor<true> : k_predictor<false>, dim3(nblk(g.n, 256)), dim3(256), 0, c.stream, g, c.p.method, c.has_history ? 0 : 1,
-                     polymer, c.U, c.V, c.W, c.P, c.C[c.cur], c.fC, c.A0, c.T0, c.B0, Rout, c.F,
-                     c.p.body_force[0], c.p.body_force[1], c.p.body_force[2], c.Q);
+  PredConst K{g.dx, g.dy, g.dz, g.dx * g.dx, g.dy * g.dy, g.dz * g.dz, 4.0 * g.dx, 4.0 * g.dy, 4.0 * g.dz};
+  for (int q = 0; q < 9; q++) (&K.idx)[q] = 1.0 / (&K.dx)[q];
+  const int first = c.has_history ? 0 : 1;
+  const double* bf = c.p.body_force;
+  // streamed where there are tiles for two blocks a CU: 32^3 has 128 (its step 10 us
+  // a pass of 20 slower so); as many planes a block as leave 512 blocks
+  const long tiles = g.nx % PD_TX || g.ny % PD_TY ? 0 : (g.nx / PD_TX) * (long)(g.ny / PD_TY);
+  if (tiles * g.nz >= 512) {
+    int kc = std::min(32, g.nz);
+    while (tiles * (g.nz / kc) < 512) kc >>= 1;
+    auto k = g.walls ? k_predictor_z<true> : k_predictor_z<false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)(tiles * (g.nz / kc))), dim3(256), 0, c.stream, g, K, kc, c.p.method, first, polymer,
+                       c.U, c.V, c.W, c.P, c.C[c.cur], c.fC, c.A0, c.T0, c.B0, Rout, c.F, bf[0], bf[1], bf[2], c.Q);
+    return;
+  }
+  hipLaunchKernelGGL(g.walls ? k_predictor<true> : k_predictor<false>, dim3(nblk(g.n, 256)), dim3(256), 0, c.stream, g, K,
+                     c.p.method, first, polymer, c.U, c.V, c.W, c.P, c.C[c.cur], c.fC, c.A0, c.T0, c.B0, Rout, c.F, bf[0],
+                     bf[1], bf[2], c.Q);
 }
 
 void f64_march(Ctx& c) {
