@@ -144,6 +144,22 @@ __device__ __forceinline__ void turn(const Lines<V>& f, const V* tws, Op op) {
 
 __device__ __forceinline__ int log2i(int n) { return __ffs(n) - 1; }
 
+// store(e, load(e)) for e < total over the block, U loads of a thread in
+// flight: one at a time, the copy of 33 KB into the LDS by 128 threads waits 16
+// times on memory
+template <int U, typename V, typename Load, typename Store>
+__device__ __forceinline__ void copy_ahead(int total, Load load, Store store) {
+  const int nt = blockDim.x;
+  for (int e = threadIdx.x; e < total; e += U * nt) {
+    V v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = load(min(e + u * nt, total - 1));
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (e + u * nt < total) store(e + u * nt, v[u]);
+  }
+}
+
 // twiddles exp(-2 pi i t/n), t < n/2, into LDS (no barrier)
 template <typename V>
 __device__ __forceinline__ void load_tw(V* tws, const V* __restrict__ tw, int n) {

@@ -765,7 +765,8 @@ void f64_ibm_setup(Ctx& c) {
       const long i = tgt[r] % gx, j = (tgt[r] / gx) % gy, k = tgt[r] / (gx * gy);
       if (i < 1 || i > g.nx || j < 1 || j > g.ny || k < 1 || k > g.nz) continue;
       int rr[8], ghosts = 0;
-      for (int b = 0; b < 8; b++) {
+      const bool border = i == 1 || i == g.nx || j == 1 || j == g.ny || k == 1 || k == g.nz;
+      for (int b = 0; border && b < 8; b++) {
         const long ii = image(i, g.nx, b & 1), jj = image(j, g.ny, b >> 1 & 1), kk = image(k, g.nz, b >> 2);
         rr[b] = b == 0 ? (int)r : (ii < 0 || jj < 0 || kk < 0 ? -1 : row_of(G(ii, jj, kk)));
         ghosts += b > 0 && rr[b] >= 0;

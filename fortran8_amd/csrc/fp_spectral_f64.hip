@@ -70,7 +70,8 @@ __global__ __launch_bounds__(256) void k_x_forward(Grid g, LineSrc<T> q, int com
   const long plane = (long)g.ny * g.nz, l0 = (long)blockIdx.x << lnl;
   comp += blockIdx.y;
   load_tw(tws, tw, n);
-  for (int e = threadIdx.x; e < nl << L; e += blockDim.x) {
+  const double iy[4] = {1.0 / g.dx, 1.0 / g.dy, 1.0 / g.dz, 1.0 / g.dt};
+  auto value = [&](int e) {
     const int l = e >> L, i = e & (n - 1);
     const long m = (l0 + l) * n + i;
     double v;
@@ -79,9 +80,9 @@ __global__ __launch_bounds__(256) void k_x_forward(Grid g, LineSrc<T> q, int com
     if constexpr (S == Line::Plain) {
       v = q.u[comp * g.n + m];
     } else if constexpr (S == Line::Div) {
-      v = (((-ldbw<WL>(q.u, g, i - 1, j, k, BC_U) + ldbw<WL>(q.u, g, i, j, k, BC_U)) / g.dx
-            + (-ldbw<WL>(q.v, g, i, j - 1, k, BC_V) + ldbw<WL>(q.v, g, i, j, k, BC_V)) / g.dy)
-           + (-ldbw<WL>(q.w, g, i, j, k - 1, BC_W) + ldbw<WL>(q.w, g, i, j, k, BC_W)) / g.dz) / g.dt;
+      v = quot((quot(-ldbw<WL>(q.u, g, i - 1, j, k, BC_U) + ldbw<WL>(q.u, g, i, j, k, BC_U), g.dx, iy[0])
+                + quot(-ldbw<WL>(q.v, g, i, j - 1, k, BC_V) + ldbw<WL>(q.v, g, i, j, k, BC_V), g.dy, iy[1]))
+               + quot(-ldbw<WL>(q.w, g, i, j, k - 1, BC_W) + ldbw<WL>(q.w, g, i, j, k, BC_W), g.dz, iy[2]), g.dt, iy[3]);
     } else {
       const T* f = comp == 0 ? q.u : (comp == 1 ? q.v : q.w);
       const int a = comp == 0, b = comp == 1, c = comp == 2;
@@ -93,8 +94,11 @@ __global__ __launch_bounds__(256) void k_x_forward(Grid g, LineSrc<T> q, int com
       }
       v = (x + y) / 2.0;
     }
-    lds[l * pitch + i] = make_double2(v, 0.0);
-  }
+    return v;
+  };
+  copy_ahead<S == Line::Plain ? 4 : 2, double>(nl << L, value, [&](int e, double v) {
+    lds[(e >> L) * pitch + (e & (n - 1))] = make_double2(v, 0.0);
+  });
   __syncthreads();
   const Lines<double2> f{lds, 1, pitch, lnl, L};
   dif_from_natural<M, false>(f, tws);
@@ -115,13 +119,13 @@ __global__ __launch_bounds__(256) void k_x_inverse(Grid g, const double2* __rest
   const long plane = (long)g.ny * g.nz, l0 = (long)blockIdx.x << lnl;
   load_tw(tws, tw, n);
   const double2* in = spec + blockIdx.y * (plane * g.nxh) + l0;
-  for (int e = threadIdx.x; e < g.nxh << lnl; e += blockDim.x) {
-    const int l = e & (nl - 1), i = e >> lnl;
-    double2 v = in[plane * i + l];
-    if (i == 0 || i == h) v.y = 0.0;
-    lds[l * pitch + i] = v;
-    if (i > 0 && i < h) lds[l * pitch + (n - i)] = make_double2(v.x, -v.y);
-  }
+  copy_ahead<4, double2>(g.nxh << lnl, [&](int e) { return in[plane * (e >> lnl) + (e & (nl - 1))]; },
+                         [&](int e, double2 v) {
+                           const int l = e & (nl - 1), i = e >> lnl;
+                           if (i == 0 || i == h) v.y = 0.0;
+                           lds[l * pitch + i] = v;
+                           if (i > 0 && i < h) lds[l * pitch + (n - i)] = make_double2(v.x, -v.y);
+                         });
   __syncthreads();
   const Lines<double2> f{lds, 1, pitch, lnl, L};
   dif_from_natural<M, true>(f, tws);
@@ -178,55 +182,97 @@ __global__ __launch_bounds__(256) void k_line_pivots(Grid g, int kind, const dou
   }
 }
 
-// One lane's line: its values v[0..ny) (stride vs doubles) in LDS, its P in
-// lp[0..ny) (stride ps); y the pivots (stride ys), read LINE_AHEAD rows ahead.
-constexpr int LINE_AHEAD = 16;
-__device__ __forceinline__ void line_solve(const Grid& g, int kind, double k2, double rn, const double* __restrict__ y,
-                                           int ys, double* v, int vs, double* lp, int ps) {
+// One lane's line: its values v[0..ny) (stride vs doubles) and its pivots
+// lp[0..ny] (stride ps) in LDS; P takes a pivot's place once it is used.  TB rows
+// (ny is a multiple) a batch: their values are read together, the next batch's
+// while this one is computed, so that the recurrences wait on arithmetic only.
+// (With the pivots read from memory 16 rows ahead and the values a row ahead,
+// k_lines_y took 144 us for the three components at 256x128x128, now 110.)
+template <int TB>
+__device__ __forceinline__ void line_solve_by(const Grid& g, int kind, double k2, double rn, double* v, int vs, double* lp,
+                                              int ps) {
   const LineRow lr(g, kind, k2);
   const int ny = g.ny;
   double P = lr.first(), Q = 0.0;
-  double yn[LINE_AHEAD];
+  double yn[TB], vn[TB];
 #pragma unroll
-  for (int u = 0; u < LINE_AHEAD; u++) yn[u] = y[(long)min(u, ny) * ys];
-  double nxt = v[0];
-  for (int r0 = 1; r0 <= ny; r0 += LINE_AHEAD) {
-    double yc[LINE_AHEAD];
+  for (int u = 0; u < TB; u++) {
+    yn[u] = lp[u * ps];
+    vn[u] = v[u * vs];
+  }
+  // all but the last batch: interior rows of every kind
+  const double off = lr.off, diag = lr.diag;
+  int r0 = 1;
+  for (; r0 + TB <= ny; r0 += TB) {
+    double yc[TB], vc[TB];
 #pragma unroll
-    for (int u = 0; u < LINE_AHEAD; u++) {
+    for (int u = 0; u < TB; u++) {
       yc[u] = yn[u];
-      yn[u] = y[(long)min(r0 + LINE_AHEAD - 1 + u, ny) * ys];
+      vc[u] = vn[u];
     }
 #pragma unroll
-    for (int u = 0; u < LINE_AHEAD; u++) {
-      const int r = r0 + u;
-      if (r <= ny) {
-        double a, b, c;
-        bool rhs;
-        lr.row(r, a, b, c, rhs);
-        const double d = rhs ? nxt * rn : 0.0;
-        if (r < ny) nxt = v[r * vs];
-        const double den = a + c * P;
-        Q = quot(d - c * Q, den, yc[u]);
-        P = quot(-b, den, yc[u]);
-        v[(r - 1) * vs] = Q;
-        lp[(r - 1) * ps] = P;   // both lanes of the line: the same value
-      }
+    for (int u = 0; u < TB; u++) {
+      yn[u] = lp[(r0 + TB - 1 + u) * ps];
+      vn[u] = v[(r0 + TB - 1 + u) * vs];
     }
+#pragma unroll
+    for (int u = 0; u < TB; u++) {
+      const double den = diag + off * P;
+      Q = quot(vc[u] * rn - off * Q, den, yc[u]);
+      P = quot(-off, den, yc[u]);
+      v[(r0 - 1 + u) * vs] = Q;
+      lp[(r0 - 1 + u) * ps] = P;   // both lanes of the line: the same value
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < TB; u++) {
+    double a, b, c;
+    bool rhs;
+    lr.row(r0 + u, a, b, c, rhs);
+    const double d = rhs ? vn[u] * rn : 0.0;
+    const double den = a + c * P;
+    Q = quot(d - c * Q, den, yn[u]);
+    P = quot(-b, den, yn[u]);
+    v[(r0 - 1 + u) * vs] = Q;
+    lp[(r0 - 1 + u) * ps] = P;
   }
   {
     double a, b, c;
     bool rhs;
     lr.row(ny + 1, a, b, c, rhs);
-    Q = quot(0.0 - c * Q, a + c * P, y[(long)ny * ys]);
+    Q = quot(0.0 - c * Q, a + c * P, lp[ny * ps]);
   }
-  double x = Q, Pn = lp[(ny - 1) * ps], qn = v[(ny - 1) * vs];
-  for (int r = ny; r >= 1; r--) {
-    const double p = Pn, q = qn;
-    if (r > 1) { Pn = lp[(r - 2) * ps]; qn = v[(r - 2) * vs]; }
-    x = p * x + q;
-    v[(r - 1) * vs] = x;
+  double x = Q, pn[TB], qn[TB];
+#pragma unroll
+  for (int u = 0; u < TB; u++) {
+    pn[u] = lp[(ny - 1 - u) * ps];
+    qn[u] = v[(ny - 1 - u) * vs];
   }
+  for (r0 = ny; r0 >= 1; r0 -= TB) {
+    double pc[TB], qc[TB];
+#pragma unroll
+    for (int u = 0; u < TB; u++) {
+      pc[u] = pn[u];
+      qc[u] = qn[u];
+    }
+    if (r0 > TB) {
+#pragma unroll
+      for (int u = 0; u < TB; u++) {
+        pn[u] = lp[(r0 - TB - 1 - u) * ps];
+        qn[u] = v[(r0 - TB - 1 - u) * vs];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < TB; u++) {
+      x = pc[u] * x + qc[u];
+      v[(r0 - 1 - u) * vs] = x;
+    }
+  }
+}
+__device__ __forceinline__ void line_solve(const Grid& g, int kind, double k2, double rn, double* v, int vs, double* lp,
+                                           int ps) {
+  if (g.ny >= 8) line_solve_by<8>(g, kind, k2, rn, v, vs, lp, ps);
+  else line_solve_by<4>(g, kind, k2, rn, v, vs, lp, ps);
 }
 
 // Line solves of 2^ltl consecutive kz rows of one kx and component per block,
@@ -237,17 +283,20 @@ __global__ __launch_bounds__(128) void k_lines_y(Grid g, double2* __restrict__ s
                                                  const double* __restrict__ kz2, int ltl) {
   extern __shared__ double2 lds[];
   const int ny = g.ny, tl = 1 << ltl, pitch = ny + 1;
-  double* lp = (double*)(lds + tl * pitch);   // [row][line]
+  double* lp = (double*)(lds + tl * pitch);   // pivots, then P, [row][line]
   const int kind = kind0 + blockIdx.y;
   const long b0 = (long)blockIdx.x << ltl;    // first (kx, kz row) line
   const int i = (int)(b0 / g.nz), kr0 = (int)(b0 & (g.nz - 1));
   double2* base = spec + blockIdx.y * ((long)g.nxh * ny * g.nz) + b0 * ny;
-  for (int e = threadIdx.x; e < tl << g.lny; e += blockDim.x) lds[(e >> g.lny) * pitch + (e & (ny - 1))] = base[e];
+  const double* y = table + (kind == 1 ? tstride : (kind == 3 ? 2 * tstride : 0)) + (long)i * (ny + 1) * g.nz + kr0;
+  copy_ahead<8, double>((ny + 1) << ltl, [&](int e) { return y[(e >> ltl) * (long)g.nz + (e & (tl - 1))]; },
+                        [&](int e, double v) { lp[e] = v; });
+  copy_ahead<8, double2>(tl << g.lny, [&](int e) { return base[e]; },
+                         [&](int e, double2 v) { lds[(e >> g.lny) * pitch + (e & (ny - 1))] = v; });
   __syncthreads();
   if (threadIdx.x < 2 * tl) {
     const int l = threadIdx.x >> 1, c = threadIdx.x & 1, kr = kr0 + l;
-    const double* y = table + (kind == 1 ? tstride : (kind == 3 ? 2 * tstride : 0)) + (long)i * (ny + 1) * g.nz + kr;
-    line_solve(g, kind, kx2[i] + kz2[brev(kr, log2i(g.nz))], rn, y, g.nz, (double*)(lds + l * pitch) + c, 2, lp + l, tl);
+    line_solve(g, kind, kx2[i] + kz2[brev(kr, log2i(g.nz))], rn, (double*)(lds + l * pitch) + c, 2, lp + l, tl);
   }
   __syncthreads();
   for (int e = threadIdx.x; e < tl << g.lny; e += blockDim.x) base[e] = lds[(e >> g.lny) * pitch + (e & (ny - 1))];
@@ -268,12 +317,13 @@ __global__ __launch_bounds__(1024) void k_slab(Grid g, double2* __restrict__ spe
   const int ny = g.ny, nz = g.nz, pitch = ny + 1, lnz = log2i(nz);
   double2* tz = lds + nz * pitch;
   double2* ty = tz + nz / 2;                  // periodic
-  double* lp = (double*)ty;                   // between walls: P, [row][kz]
+  double* lp = (double*)ty;                   // between walls: pivots, then P, [row][kz]
   const int i = blockIdx.x, kind = kind0 + blockIdx.y;
   double2* base = spec + (blockIdx.y * (long)g.nxh + i) * ((long)ny * nz);
   load_tw(tz, twz, nz);
   if (!WL) load_tw(ty, twy, ny);
-  for (int e = threadIdx.x; e < ny * nz; e += blockDim.x) lds[(e >> g.lny) * pitch + (e & (ny - 1))] = base[e];
+  copy_ahead<4, double2>(ny * nz, [&](int e) { return base[e]; },
+                         [&](int e, double2 v) { lds[(e >> g.lny) * pitch + (e & (ny - 1))] = v; });
   __syncthreads();
   const Lines<double2> fy{lds, 1, pitch, lnz, g.lny}, fz{lds, pitch, 1, g.lny, lnz};
   if constexpr (!WL) {
@@ -285,11 +335,12 @@ __global__ __launch_bounds__(1024) void k_slab(Grid g, double2* __restrict__ spe
     dif_from_reversed<M>(fz, tz, false);
     dif_from_reversed<M>(fy, ty);
   } else {
+    const double* y = table + (kind == 1 ? tstride : (kind == 3 ? 2 * tstride : 0)) + (long)i * (ny + 1) * nz;
+    copy_ahead<4, double>((ny + 1) * nz, [&](int e) { return y[e]; }, [&](int e, double v) { lp[e] = v; });
     dif_from_natural<M, false>(fz, tz);
     for (int t = threadIdx.x; t < 2 * nz; t += blockDim.x) {
       const int kr = t >> 1, c = t & 1;
-      const double* y = table + (kind == 1 ? tstride : (kind == 3 ? 2 * tstride : 0)) + (long)i * (ny + 1) * nz + kr;
-      line_solve(g, kind, kx2[i] + kz2[brev(kr, lnz)], rn, y, nz, (double*)(lds + kr * pitch) + c, 2, lp + kr, nz);
+      line_solve(g, kind, kx2[i] + kz2[brev(kr, lnz)], rn, (double*)(lds + kr * pitch) + c, 2, lp + kr, nz);
     }
     __syncthreads();
     dif_from_reversed<M>(fz, tz);
@@ -307,7 +358,8 @@ __global__ __launch_bounds__(256) void k_y_lines(Grid g, double2* __restrict__ s
   double2* tws = lds + nl * pitch;
   double2* base = spec + blockIdx.y * ((long)g.nxh * n * g.nz) + ((long)blockIdx.x << (lnl + g.lny));
   load_tw(tws, tw, n);
-  for (int e = threadIdx.x; e < nl << g.lny; e += blockDim.x) lds[(e >> g.lny) * pitch + (e & (n - 1))] = base[e];
+  copy_ahead<4, double2>(nl << g.lny, [&](int e) { return base[e]; },
+                         [&](int e, double2 v) { lds[(e >> g.lny) * pitch + (e & (n - 1))] = v; });
   __syncthreads();
   const Lines<double2> f{lds, 1, pitch, lnl, g.lny};
   if (inv) dif_from_reversed<M>(f, tws);
@@ -328,7 +380,8 @@ __global__ __launch_bounds__(256) void k_z_lines(Grid g, double2* __restrict__ s
   const int i = blockIdx.x >> lt, j0 = (blockIdx.x & ((1 << lt) - 1)) << lnl;
   double2* base = spec + (blockIdx.y * (long)g.nxh + i) * ((long)g.ny * n) + j0;
   load_tw(tws, tw, n);
-  for (int e = threadIdx.x; e < n << lnl; e += blockDim.x) lds[e] = base[((long)(e >> lnl) << g.lny) + (e & (nl - 1))];
+  copy_ahead<4, double2>(n << lnl, [&](int e) { return base[((long)(e >> lnl) << g.lny) + (e & (nl - 1))]; },
+                         [&](int e, double2 v) { lds[e] = v; });
   __syncthreads();
   const Lines<double2> f{lds, nl, 1, lnl, L};
   if (mode == 0) {
@@ -350,10 +403,10 @@ namespace {
 
 size_t lds_slab64(const Grid& g) {
   size_t w = sizeof(double2) * ((size_t)g.nz * (g.ny + 1) + g.nz / 2);
-  return w + (g.walls ? sizeof(double) * (size_t)g.ny * g.nz : sizeof(double2) * (g.ny / 2));
+  return w + (g.walls ? sizeof(double) * (size_t)(g.ny + 1) * g.nz : sizeof(double2) * (g.ny / 2));
 }
 constexpr int LNL_Y = 4;   // lines per block of k_lines_y (log2)
-size_t lds_lines_y(int ny, int ltl) { return (sizeof(double2) * (ny + 1) + sizeof(double) * ny) << ltl; }
+size_t lds_lines_y(int ny, int ltl) { return (sizeof(double2) + sizeof(double)) * (ny + 1) << ltl; }
 
 template <typename F>
 void allow_lds(F* f, int bytes) {
