@@ -361,12 +361,21 @@ __device__ __forceinline__ void solve6(double (&a)[6][6], double (&b)[6]) {
 #pragma unroll
     for (int r = c + 1; r < 6; r++)
       if (fabs(a[r][c]) > mv) { mv = fabs(a[r][c]); p = r; }
+    // by selects, where any lane swaps: a branch per row leaves the matrix in
+    // scratch memory (k_adj_newton at 64x64x32 19 us with it, 11 without)
+    if (__any(p != c)) {
 #pragma unroll
-    for (int r = c + 1; r < 6; r++) {
-      if (r == p) {
+      for (int r = c + 1; r < 6; r++) {
+        const bool here = r == p;
 #pragma unroll
-        for (int q = 0; q < 6; q++) { const double t = a[c][q]; a[c][q] = a[r][q]; a[r][q] = t; }
-        const double t = b[c]; b[c] = b[r]; b[r] = t;
+        for (int q = 0; q < 6; q++) {
+          const double t = a[c][q], u = a[r][q];
+          a[c][q] = here ? u : t;
+          a[r][q] = here ? t : u;
+        }
+        const double t = b[c], u = b[r];
+        b[c] = here ? u : t;
+        b[r] = here ? t : u;
       }
     }
     const double inv = 1.0 / a[c][c];
@@ -433,9 +442,12 @@ __global__ __launch_bounds__(256) void k_adj_newton(Grid g, const double* __rest
                              {0.5 * xb[1], xb[3], 0.5 * xb[4]},
                              {0.5 * xb[2], 0.5 * xb[4], xb[5]}};
     const double Xm[3][3] = {{x[0], x[1], x[2]}, {x[1], x[3], x[4]}, {x[2], x[4], x[5]}};
+#pragma unroll
     for (int r = 0; r < 3; r++)
+#pragma unroll
       for (int c = 0; c < 3; c++) {
         double s = 0.0;
+#pragma unroll
         for (int q = 0; q < 3; q++) s += Lm[r][q] * Xm[q][c];
         Mb[(r + 3 * c) * n + m] = -2.0 * s;
       }
@@ -642,6 +654,23 @@ __global__ __launch_bounds__(256) void k_gather(double* __restrict__ dst, Gather
     dst[e] = gt.src[q][off];
   }
 }
+// the reverse: one range into up to eight arrays
+struct Scatter {
+  double* dst[8];
+  long len[8];
+  int count;
+};
+__global__ __launch_bounds__(256) void k_scatter(const double* __restrict__ src, Scatter sc, long total) {
+  for (long e = blockIdx.x * 256L + threadIdx.x; e < total; e += (long)gridDim.x * 256) {
+    long off = e;
+    int q = 0;
+    while (q < sc.count - 1 && off >= sc.len[q]) {
+      off -= sc.len[q];
+      q++;
+    }
+    sc.dst[q][off] = src[e];
+  }
+}
 void gather(Ctx& c, double* dst, std::initializer_list<std::pair<const double*, long>> parts) {
   Gather gt{};
   long total = 0;
@@ -674,29 +703,19 @@ void ensure_tape(Adj& a, int every, long n) {
   if ((int)a.tape_first.size() != every) a.tape_first.assign(every, 0);
 }
 
+// a checkpoint: the state and the histories, eight arrays in one launch (64x64x32:
+// eight copies of 5 us each way before)
 void save_state(Ctx& c, double* dst) {
   const long n = c.g.n;
-  d2d(c, dst, c.U, sizeof(double) * n);
-  d2d(c, dst + n, c.V, sizeof(double) * n);
-  d2d(c, dst + 2 * n, c.W, sizeof(double) * n);
-  d2d(c, dst + 3 * n, c.P, sizeof(double) * n);
-  d2d(c, dst + 4 * n, c.C[c.cur], sizeof(double) * 6 * n);
-  d2d(c, dst + 10 * n, c.A0, sizeof(double) * 3 * n);
-  d2d(c, dst + 13 * n, c.T0, sizeof(double) * 3 * n);
-  d2d(c, dst + 16 * n, c.B0, sizeof(double) * 3 * n);
+  gather(c, dst, {{c.U, n}, {c.V, n}, {c.W, n}, {c.P, n}, {c.C[c.cur], 6 * n}, {c.A0, 3 * n}, {c.T0, 3 * n}, {c.B0, 3 * n}});
 }
 
 void load_state(Ctx& c, const double* src) {
   const long n = c.g.n;
   if (c.mixed) mixed_settle_history(c);
-  d2d(c, c.U, src, sizeof(double) * n);
-  d2d(c, c.V, src + n, sizeof(double) * n);
-  d2d(c, c.W, src + 2 * n, sizeof(double) * n);
-  d2d(c, c.P, src + 3 * n, sizeof(double) * n);
-  d2d(c, c.C[c.cur], src + 4 * n, sizeof(double) * 6 * n);
-  d2d(c, c.A0, src + 10 * n, sizeof(double) * 3 * n);
-  d2d(c, c.T0, src + 13 * n, sizeof(double) * 3 * n);
-  d2d(c, c.B0, src + 16 * n, sizeof(double) * 3 * n);
+  const Scatter sc{{c.U, c.V, c.W, c.P, c.C[c.cur], c.A0, c.T0, c.B0}, {n, n, n, n, 6 * n, 3 * n, 3 * n, 3 * n}, 8};
+  const long nb = std::min((long)nblk(CK_WORDS * n, 256), 2048L);
+  hipLaunchKernelGGL(k_scatter, dim3((unsigned)nb), dim3(256), 0, c.stream, src, sc, CK_WORDS * n);
 }
 
 void check_supported(Ctx& c) {
