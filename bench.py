@@ -246,8 +246,8 @@ def main():
     # the selection streamed along z where a block holds whole x-rows
     streamed = case.params.nx in (64, 128, 256)
     kernel_names = {"fenep_select": "fp::m_select%s<%s>" % ("_z" if streamed else "", "float" if prec else "double"),
-                    "fenep_cstar_newton": "fp::m_cstar_newton" if prec else "fp::k_cstar_newton<%s>" % walls,
-                    "predictor": mixed_pred if prec else "fp::k_predictor<%s>" % walls}
+                    "fenep_cstar_newton": "fp::m_cstar_newton" if prec else "fp::k_cstar_newton<%s, false>" % walls,
+                    "predictor": mixed_pred if prec else "fp::k_predictor_z<%s>" % walls}
     out = {
         "metric": "Mcell-steps/s 256x128x128 FENE-P+IBM",
         "value": round(value, 3),
