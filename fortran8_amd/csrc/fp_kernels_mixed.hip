@@ -47,7 +47,6 @@ struct Mixed {
   float* Up = nullptr;            // Helmholtz increment d: u* = u^n + d
   float* F = nullptr;
   float2* spec = nullptr;
-  float* thp = nullptr;
   float2 *twx = nullptr, *twy = nullptr, *twz = nullptr;
   float *kx2 = nullptr, *ky2 = nullptr, *kz2 = nullptr;
   double *phi = nullptr, *b = nullptr;
@@ -80,7 +79,6 @@ struct Mixed {
   float* uc = nullptr;            // target velocities, 3 planes
   float* mf = nullptr;            // marker forces, 3 planes
   double* mf64 = nullptr;
-  float* ftmp = nullptr;          // 3 ghosted raw spread arrays
   float* sw[3] = {nullptr, nullptr, nullptr};  // CSR entry weights
   // spreading folded onto interior targets (all three components)
   int* fr_row = nullptr;          // sliced ELL: offset of each 64-row slice
@@ -3402,7 +3400,6 @@ void mixed_create(Ctx& c) {
   dalloc(&X->AT[0], 6 * n); dalloc(&X->AT[1], 6 * n);
   dalloc(&X->Q, 3 * n); dalloc(&X->Up, 3 * n);
   dalloc(&X->spec, (size_t)g.nxh * g.sy * g.nz);
-  if (g.walls) dalloc(&X->thp, (size_t)(g.ny + 2) * g.nxh * g.nz);
   dalloc(&X->phi, n); dalloc(&X->b, n); dalloc(&X->r32, n);
   if (c.p.poisson_variant == FP_POISSON_SOR) {
     const SorPlan<float> p = sor_plan<float>(g);
@@ -3476,7 +3473,7 @@ void mixed_destroy(Ctx& c) {
   if (X->side) (void)hipStreamDestroy(X->side);
   dfree(X->U); dfree(X->V); dfree(X->W); dfree(X->P); dfree(X->C[0]); dfree(X->C[1]); dfree(X->f);
   dfree(X->AT[0]); dfree(X->AT[1]); dfree(X->Q); dfree(X->Up); dfree(X->F);
-  dfree(X->spec); dfree(X->thp); dfree(X->twx); dfree(X->twy); dfree(X->twz);
+  dfree(X->spec); dfree(X->twx); dfree(X->twy); dfree(X->twz);
   dfree(X->kx2); dfree(X->ky2); dfree(X->kz2);
   dfree(X->phi); dfree(X->b); dfree(X->r32); dfree(X->red); dfree(X->part); dfree(X->skip);
   dfree(X->e32); dfree(X->sor_pb); dfree(X->sor_flag); dfree(X->sor_part);
@@ -3489,7 +3486,7 @@ void mixed_destroy(Ctx& c) {
   if (X->dc_host) (void)hipHostFree(X->dc_host);
   dfree(X->X2); dfree(X->amb); dfree(X->amb_list); dfree(X->chk);
   dfree(X->amb_idx); dfree(X->amb_data);
-  dfree(X->wi); dfree(X->org); dfree(X->uc); dfree(X->mf); dfree(X->mf64); dfree(X->ftmp);
+  dfree(X->wi); dfree(X->org); dfree(X->uc); dfree(X->mf); dfree(X->mf64);
   for (int k = 0; k < 3; k++) dfree(X->sw[k]);
   dfree(X->fr_row); dfree(X->fr_len); dfree(X->fr_tgt); dfree(X->fr_ent); dfree(X->fr_w);
   dfree(X->zi_w); dfree(X->zi_org);
@@ -3607,7 +3604,7 @@ void mixed_set_force(Ctx& c) {
 void mixed_set_markers(Ctx& c) {
   Mixed& X = MX(c);
   const Grid& g = c.g;
-  dfree(X.wi); dfree(X.org); dfree(X.uc); dfree(X.mf); dfree(X.mf64); dfree(X.ftmp);
+  dfree(X.wi); dfree(X.org); dfree(X.uc); dfree(X.mf); dfree(X.mf64);
   dalloc(&X.wi, (size_t)c.nmk * 81); dalloc(&X.org, (size_t)c.nmk * 3); dalloc(&X.uc, 3 * c.nmk);
   dalloc(&X.mf, 3 * c.nmk); dalloc(&X.mf64, 3 * c.nmk);
   hipLaunchKernelGGL(m_ibm_setup_interp, dim3(nblk(c.nmk, 128)), dim3(128), 0, c.stream, g, c.nmk, c.nc, c.nl, c.mk, X.wi,
