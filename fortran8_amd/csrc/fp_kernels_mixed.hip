@@ -1839,7 +1839,7 @@ __global__ __launch_bounds__(256) void m_fft_yz(Grid g, float2* __restrict__ spe
 // odd nx / 2 + 1.
 // The kernel moves its spectrum once, 16 B a point; m_fft_yz, a barrier and two
 // LDS passes a stage and its index arithmetic: the three launches of 64^3 23 us
-// there and 17 here, a step of 256^3 240 us less.
+// there and 14 here, of 256^3 300 and 110.
 // cmul_f with the fusions that m_fft_yz is compiled to written out (after the
 // divide the other product of each pair is rounded first); the functions below
 // contract nothing else, so that no product joins a sum of the next stage

@@ -23,7 +23,7 @@
 // division, y, x), 24 of the step's launches.  Small grids are bound by those
 // launches: the Newtonian 32^3 step took 127 us and takes 49, the FENE-P step
 // at 64^3 340 and 228 us.  At 256 x 128 x 128 between walls the four solves
-// went from 1.16 to 0.46 ms; there the line solves' serial recurrence and the
+// went from 1.16 to 0.43 ms; there the line solves' serial recurrence and the
 // LDS passes bound them.
 #include "fp_fft.h"
 #include <algorithm>
