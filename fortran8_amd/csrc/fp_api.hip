@@ -489,6 +489,7 @@ int fp_step(void* vc, int nsteps, int sync) {
 // `scratch` (diag_scratch_words(c.g) doubles of device memory).
 static void diagnostics_into(Ctx& c, fp_diag* d, double* scratch) {
   std::memset(d, 0, sizeof(*d));
+  if (c.mixed) mixed_mark_copy_out(c);
   f64_diag(c, d, scratch);
   d->sor_itr = c.sor_itr;
   d->n_dc = c.mixed ? mixed_last_ndc(c) : 0.0;
@@ -681,6 +682,7 @@ int fp_time_stats(void* vc, double* out) {
   if (!c || !out) return FP_E_ARG;
   if (!c->state_set) return fail(c, FP_E_STATE, "state not set");
   try {
+    if (c->mixed) mixed_mark_copy_out(*c);
     f64_time_stats(*c, out);
   } catch (const std::string& e) {
     return fail(c, FP_E_HIP, e);
@@ -694,6 +696,7 @@ int fp_energy_spectrum(void* vc, double* E, int nbins) {
   if (c->g.walls) return fail(c, FP_E_ARG, "the shell spectrum needs a periodic grid");
   if (!c->state_set) return fail(c, FP_E_STATE, "state not set");
   try {
+    if (c->mixed) mixed_mark_copy_out(*c);
     f64_energy_spectrum(*c, E, nbins);
   } catch (const std::string& e) {
     return fail(c, FP_E_HIP, e);
@@ -706,6 +709,7 @@ int fp_time_stats_map(void* vc, int ncyl, const double* xy, double diameter, dou
   if (!c || ncyl < 0 || (ncyl > 0 && !xy) || !(diameter >= 0.0) || (!map18 && !out13)) return fail(c, FP_E_ARG, "bad arguments");
   if (!c->state_set) return fail(c, FP_E_STATE, "state not set");
   try {
+    if (c->mixed) mixed_mark_copy_out(*c);
     if (f64_time_stats_map(*c, ncyl, xy, diameter, map18, out13)) return fail(c, FP_E_ARG, "the mask covers the whole plane");
   } catch (const std::string& e) {
     return fail(c, FP_E_HIP, e);
@@ -718,6 +722,7 @@ int fp_energy_spectrum_z(void* vc, int ncyl, const double* xy, double diameter, 
   if (!c || ncyl < 0 || (ncyl > 0 && !xy) || !(diameter >= 0.0) || (!Emask && !Efirst)) return fail(c, FP_E_ARG, "bad arguments");
   if (!c->state_set) return fail(c, FP_E_STATE, "state not set");
   try {
+    if (c->mixed) mixed_mark_copy_out(*c);
     if (f64_energy_spectrum_z(*c, ncyl, xy, diameter, Emask, Efirst)) return fail(c, FP_E_ARG, "the mask covers the whole plane");
   } catch (const std::string& e) {
     return fail(c, FP_E_HIP, e);

@@ -38,7 +38,8 @@ struct Mixed {
   int cur = 0;
   float* f = nullptr;
   // histories A0 (3 planes) and T0 (3 planes): AT[h] holds the context's, and
-  // AT[hs] those of the last copy-out (hs < 0: c.A0 and c.T0 do).  A step
+  // AT[hs] those of the last copy-out (hs < 0: c.A0 and c.T0 do; diagnostics and
+  // statistics count as one).  A step
   // whose histories are both writes the other buffer, so a copy-out of the
   // state moves no history.
   float* AT[2] = {nullptr, nullptr};
@@ -3512,6 +3513,9 @@ void mixed_settle_history(Ctx& c) {
   X.hs = -1;
 }
 
+// (nothing moves: the next step writes the other buffer)
+void mixed_mark_copy_out(Ctx& c) { MX(c).hs = MX(c).h; }
+
 // a selection made ahead still reads the old C; it no longer applies
 static void drop_selection(Mixed& X, hipStream_t s) {
   if (X.sel_ready) FP_HIP_CHECK(hipStreamWaitEvent(s, X.sel_done, 0));
@@ -3569,7 +3573,7 @@ void mixed_get_to_device(Ctx& c, double* const* dst, hipStream_t s) {
   const float* src[4] = {X.U, X.V, X.W, X.P};
   for (int q = 0; q < 10; q++) out.src[q] = q < 4 ? src[q] : X.C[X.cur] + (q - 4) * n;
   hipLaunchKernelGGL(m_state_out, dim3(nblk(n, 1024), 10), dim3(256), 0, s, n, out);
-  X.hs = X.h;
+  mixed_mark_copy_out(c);
 }
 
 void mixed_phi_to_f64(Ctx& c) {

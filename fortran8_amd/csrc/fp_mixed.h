@@ -12,6 +12,7 @@ void mixed_store_to_f64(Ctx& c);    // mixed state -> FP64 state buffers
 void mixed_set_from_device(Ctx& c, const double* const* src5, int keep_phi, hipStream_t s);
 void mixed_get_to_device(Ctx& c, double* const* dst5, hipStream_t s);
 void mixed_settle_history(Ctx& c);  // before c.A0 and c.T0 are written
+void mixed_mark_copy_out(Ctx& c);   // the present histories become those of the last copy-out
 void mixed_phi_to_f64(Ctx& c);      // the FP64 potential only
 void mixed_set_force(Ctx& c);
 void mixed_set_markers(Ctx& c);

@@ -170,7 +170,12 @@ int fp_diagnostics_static(void* ctx, fp_diag* d);
  * context's own stream.  has_history of fp_set_state_device: 0 and 1 as in
  * fp_set_state (the potential Phi starts from 0, as after init,
  * fenep.f90:95); 2 as 1 and Phi kept, for a state that continues the
- * context's own run (the SOR variant's sweeps start from Phi). */
+ * context's own run (the SOR variant's sweeps start from Phi).  With 1 and 2 an
+ * FP64 context keeps the histories of its last step.  A mixed context takes
+ * those it had when its state was last read out: by fp_get_state,
+ * fp_get_state_device, fp_get_phi, fp_diagnostics, fp_diagnostics_static,
+ * fp_time_stats, fp_time_stats_map, fp_energy_spectrum, fp_energy_spectrum_z or
+ * fp_adj_record (before the first of these, those of fp_set_state). */
 int fp_set_state_device(void* ctx, const double* U, const double* V,
                         const double* W, const double* P, const double* C6,
                         int has_history, void* stream);
