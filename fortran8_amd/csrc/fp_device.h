@@ -102,17 +102,24 @@ __device__ __forceinline__ void band_cell(const Grid& g, long L, long& m, int& i
 }
 
 
-// n / d correctly rounded, from y = 1/d correctly rounded: two residual
-// corrections (P. W. Markstein, "Computation of elementary functions on the
-// IBM RISC System/6000 processor", 1990: with q within an ulp of n/d and
-// y = RN(1/d), q + (n - d q) y rounds to RN(n/d)).  The first correction
-// brings n y, whose error can exceed an ulp, within one; the residuals are
-// exact unless |n| is below 2^-960.  Five dependent operations instead of about twelve with a
-// quarter-rate reciprocal among them.  y = 0 gives 0.
-__device__ __forceinline__ double quot(double n, double d, double y) {
+// n / d correctly rounded for finite n and d != 0, from y = 1/d correctly
+// rounded: two residual corrections (P. W. Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990: with q
+// within an ulp of n/d and y = RN(1/d), q + (n - d q) y rounds to RN(n/d)).
+// The first correction brings n y, whose error can exceed an ulp, within one;
+// the residuals are exact unless |n| is below 2^-960, and the quotient must not
+// overflow.  Five dependent operations instead of about twelve with a
+// quarter-rate reciprocal among them.  An infinite n gives NaN, a zero n a
+// zero of either sign, y = 0 gives 0.
+__device__ __forceinline__ double quot_finite(double n, double d, double y) {
   double q = n * y;
   q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
   return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+// the same, an infinite, NaN or zero n or d as in the division n / d (one more
+// operation, the last one of the hardware's division)
+__device__ __forceinline__ double quot(double n, double d, double y) {
+  return __builtin_amdgcn_div_fixup(quot_finite(n, d, y), d, n);
 }
 
 // ---- FENE-P algebra (FP64) ------------------------------------------------
@@ -196,7 +203,7 @@ struct CstarConst {
 // the diagonal shift dg = (1 + f dt / wi) / 2
 __device__ __forceinline__ double lyap_shift_d(const CstarConst& K, double dt, double x0, double x3, double x5) {
   const double f = K.L2m3 / (((K.L2 - x0) - x3) - x5);
-  return (1.0 + quot(f * dt, K.wi, K.iwi)) / 2.0;
+  return (1.0 + quot_finite(f * dt, K.wi, K.iwi)) / 2.0;
 }
 __device__ __forceinline__ void lyap_func_d(const double* A0, const double* b, const double* x, double dg, double* l) {
   double a11 = A0[0] + dg, a22 = A0[4] + dg, a33 = A0[8] + dg;
@@ -242,7 +249,7 @@ __device__ __forceinline__ void gauss6_d(double (&Ah)[6][7], double* x) {
     const double piv = Ah[k][k], y = 1.0 / piv;
     zero = zero || piv == 0.0;
 #pragma unroll
-    for (int c = k + 1; c < 7; c++) Ah[k][c] = quot(Ah[k][c], piv, y);
+    for (int c = k + 1; c < 7; c++) Ah[k][c] = quot_finite(Ah[k][c], piv, y);
 #pragma unroll
     for (int r = 0; r < 6; r++) {
       if (r != k) {
@@ -257,6 +264,9 @@ __device__ __forceinline__ void gauss6_d(double (&Ah)[6][7], double* x) {
 }
 
 // Newton of Lyapunov (fenep.f90:554-578) with the central-difference Jacobian.
+// Its quotients are quot_finite's: an infinity in the iterate, the gradient or
+// the right-hand side is a difference of infinities in the Jacobian, so the six
+// components end as NaN as they do with divisions.
 // Only the diagonal entries of the iterate move the shift: 7 values of it per
 // iteration, not 13; the entries of the Jacobian that no term of a row makes
 // are the zero differences they were.
@@ -279,7 +289,7 @@ __device__ __forceinline__ int newton_d(const CstarConst& K, const double* A0, c
 #pragma unroll
       for (int row = 0; row < 6; row++) {
         const bool none = (col == 1 && row == 5) || (col == 2 && row == 3) || (col == 4 && row == 0);
-        Ah[row][col] = none ? 0.0 : quot(l1[row] - l2[row], K.dc2, K.idc2);
+        Ah[row][col] = none ? 0.0 : quot_finite(l1[row] - l2[row], K.dc2, K.idc2);
       }
     }
     double l[6], r[6];

@@ -31,7 +31,8 @@ __device__ __forceinline__ int wrapped(int a, int d, int n, int ls) { return (in
 
 // Coefficients of the candidate faces (cand_p, cand_n) as fma(cp, c, fma(cm,
 // a, z b)): halves and quarters multiply exactly, (3 z)/2 rounds as 1.5 z, and a
-// term that a candidate lacks adds zero, so the value is cand_p's, bit for bit.
+// term that a candidate lacks adds zero, so the value is cand_p's, bit for bit,
+// where that term is finite.
 struct FaceCoef {
   double a, b, c;
   __device__ __forceinline__ double operator()(double cm, double z, double cp) const {
@@ -81,10 +82,10 @@ __global__ __launch_bounds__(128) void k_cstar_newton(Grid g, CstarConst K, cons
     else if (d == 1) { v1 = wlo ? 0.0 : LD(V, ym); v2 = whi ? 0.0 : LD(V, 0); }   // V_kabe
     else { v1 = LD(W, zm); v2 = LD(W, 0); }
     const double h2 = K.h2[d], ih2 = K.ih2[d];
-    const double s1 = quot((-v2 + fabs(v2)) * dt, h2, ih2);
-    const double s2 = 1.0 / 6.0 + quot((-v2 - fabs(v2)) * dt, h2, ih2);
-    const double s3 = 1.0 / 6.0 + quot((v1 - fabs(v1)) * dt, h2, ih2);
-    const double s4 = quot((v1 + fabs(v1)) * dt, h2, ih2);
+    const double s1 = quot_finite((-v2 + fabs(v2)) * dt, h2, ih2);
+    const double s2 = 1.0 / 6.0 + quot_finite((-v2 - fabs(v2)) * dt, h2, ih2);
+    const double s3 = 1.0 / 6.0 + quot_finite((v1 - fabs(v1)) * dt, h2, ih2);
+    const double s4 = quot_finite((v1 + fabs(v1)) * dt, h2, ih2);
     const int a = d == 0 ? i : (d == 1 ? j : k), na = d == 0 ? g.nx : (d == 1 ? g.ny : g.nz);
     const int ls = d == 0 ? 0 : (d == 1 ? g.lnx : lz);
     const int om = wrapped(a, -1, na, ls), op = wrapped(a, 1, na, ls);
@@ -110,14 +111,42 @@ __global__ __launch_bounds__(128) void k_cstar_newton(Grid g, CstarConst K, cons
         v[q][4] = h0 ? v[q][2] : (h1 ? 2.0 * v[q][3] - v[q][2] : v[q][4]);
       }
     }
+    double sum[6];
+    bool odd = false;
 #pragma unroll
     for (int q = 0; q < 6; q++) {
       double acc = cx[q] + s3 * pl(v[q][1], v[q][2], v[q][3]);   // Cp(a-1): own left face
       acc = acc + s1 * pr(v[q][2], v[q][3], v[q][4]);            // Cp(a): left face of a+1
       acc = acc + s4 * nl(v[q][0], v[q][1], v[q][2]);            // Cn(a-1): right face of a-1
       acc = acc + s2 * nr(v[q][1], v[q][2], v[q][3]);            // Cn(a): own right face
-      cx[q] = acc;
+      sum[q] = acc;
+      odd = odd || !(fabs(acc) < INFINITY);
     }
+    // a coefficient of zero times an infinity or NaN: again, with the terms
+    // that the faces have
+    if (__any(odd)) {
+#pragma unroll 1
+      for (int q = 0; q < 6; q++) {
+        double w[5];
+#pragma unroll
+        for (int o = 0; o < 5; o++) w[o] = v[0][o];
+#pragma unroll
+        for (int u = 1; u < 6; u++)
+#pragma unroll
+          for (int o = 0; o < 5; o++) w[o] = u == q ? v[u][o] : w[o];
+        double acc = cx[0];
+#pragma unroll
+        for (int u = 1; u < 6; u++) acc = u == q ? cx[u] : acc;
+        acc = acc + s3 * cand_p(l0, w[1], w[2], w[3]);
+        acc = acc + s1 * cand_p(lp, w[2], w[3], w[4]);
+        acc = acc + s4 * cand_n(lm, w[0], w[1], w[2]);
+        acc = acc + s2 * cand_n(l0, w[1], w[2], w[3]);
+#pragma unroll
+        for (int u = 0; u < 6; u++) sum[u] = u == q ? acc : sum[u];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 6; q++) cx[q] = sum[q];
   }
   // Lyapunov
   double b[6];
@@ -140,15 +169,15 @@ __global__ __launch_bounds__(128) void k_cstar_newton(Grid g, CstarConst K, cons
     const double x = LD(V, a + row(B) + c);
     return (B < 0 && wlo) || (B == 0 && whi) ? 0.0 : x;
   };
-  double a11 = -quot(dt * (-UL(xm, 0, 0) + UL(0, 0, 0)), K.h[0], K.ih[0]);
-  double a12 = -quot(dt * (((-VL(xm, -1, 0) + VL(xp, -1, 0)) - VL(xm, 0, 0)) + VL(xp, 0, 0)), K.h4[0], K.ih4[0]);
-  double a13 = -quot(dt * (((-WV(xm, 0, zm) + WV(xp, 0, zm)) - WV(xm, 0, 0)) + WV(xp, 0, 0)), K.h4[0], K.ih4[0]);
-  double a21 = -quot(dt * (((-UL(xm, -1, 0) - UL(0, -1, 0)) + UL(xm, 1, 0)) + UL(0, 1, 0)), K.h4[1], K.ih4[1]);
-  double a22 = -quot(dt * (-VL(0, -1, 0) + VL(0, 0, 0)), K.h[1], K.ih[1]);
-  double a23 = -quot(dt * (((-WV(0, -1, zm) + WV(0, 1, zm)) - WV(0, -1, 0)) + WV(0, 1, 0)), K.h4[1], K.ih4[1]);
-  double a31 = -quot(dt * (((-UL(xm, 0, zm) - UL(0, 0, zm)) + UL(xm, 0, zp)) + UL(0, 0, zp)), K.h4[2], K.ih4[2]);
-  double a32 = -quot(dt * (((-VL(0, -1, zm) - VL(0, 0, zm)) + VL(0, -1, zp)) + VL(0, 0, zp)), K.h4[2], K.ih4[2]);
-  double a33 = -quot(dt * (-WV(0, 0, zm) + WV(0, 0, 0)), K.h[2], K.ih[2]);
+  double a11 = -quot_finite(dt * (-UL(xm, 0, 0) + UL(0, 0, 0)), K.h[0], K.ih[0]);
+  double a12 = -quot_finite(dt * (((-VL(xm, -1, 0) + VL(xp, -1, 0)) - VL(xm, 0, 0)) + VL(xp, 0, 0)), K.h4[0], K.ih4[0]);
+  double a13 = -quot_finite(dt * (((-WV(xm, 0, zm) + WV(xp, 0, zm)) - WV(xm, 0, 0)) + WV(xp, 0, 0)), K.h4[0], K.ih4[0]);
+  double a21 = -quot_finite(dt * (((-UL(xm, -1, 0) - UL(0, -1, 0)) + UL(xm, 1, 0)) + UL(0, 1, 0)), K.h4[1], K.ih4[1]);
+  double a22 = -quot_finite(dt * (-VL(0, -1, 0) + VL(0, 0, 0)), K.h[1], K.ih[1]);
+  double a23 = -quot_finite(dt * (((-WV(0, -1, zm) + WV(0, 1, zm)) - WV(0, -1, 0)) + WV(0, 1, 0)), K.h4[1], K.ih4[1]);
+  double a31 = -quot_finite(dt * (((-UL(xm, 0, zm) - UL(0, 0, zm)) + UL(xm, 0, zp)) + UL(0, 0, zp)), K.h4[2], K.ih4[2]);
+  double a32 = -quot_finite(dt * (((-VL(0, -1, zm) - VL(0, 0, zm)) + VL(0, -1, zp)) + VL(0, 0, zp)), K.h4[2], K.ih4[2]);
+  double a33 = -quot_finite(dt * (-WV(0, 0, zm) + WV(0, 0, 0)), K.h[2], K.ih[2]);
 #undef UL
 #undef VL
 #undef WV

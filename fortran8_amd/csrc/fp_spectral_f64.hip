@@ -3,7 +3,9 @@
 // fft_*_kabe, fenep_2d.f90:1179-1342) and the pressure Poisson equation
 // (fft_poisson, fenep.f90:1529-1560; fft_poisson_kabe and tdma,
 // fenep_2d.f90:1145-1342).  Compiled with -ffp-contract=off; fused
-// multiply-adds appear only where they are written out (quot, below).
+// multiply-adds appear only where they are written out (quot, quot_finite).
+// The quotients of spectrum values are quot_finite's: an infinity on the grid
+// is NaN in every spectrum value.
 //
 // The transforms are radix-2 decimations in frequency: the butterflies, their
 // twiddles and their operand order are those of the CPU restatement's Stockham
@@ -43,7 +45,7 @@ struct Divide {
     const double lhs = kind == 3 ? -k2 : 1.0 + coef * k2;
     if (fabs(lhs) < 1.0e-16) return make_double2(0.0, 0.0);
     const double y = 1.0 / lhs;
-    return make_double2(quot(s.x * rn, lhs, y), quot(s.y * rn, lhs, y));
+    return make_double2(quot_finite(s.x * rn, lhs, y), quot_finite(s.y * rn, lhs, y));
   }
 };
 
@@ -218,8 +220,8 @@ __device__ __forceinline__ void line_solve_by(const Grid& g, int kind, double k2
 #pragma unroll
     for (int u = 0; u < TB; u++) {
       const double den = diag + off * P;
-      Q = quot(vc[u] * rn - off * Q, den, yc[u]);
-      P = quot(-off, den, yc[u]);
+      Q = quot_finite(vc[u] * rn - off * Q, den, yc[u]);
+      P = quot_finite(-off, den, yc[u]);
       v[(r0 - 1 + u) * vs] = Q;
       lp[(r0 - 1 + u) * ps] = P;   // both lanes of the line: the same value
     }
@@ -231,8 +233,8 @@ __device__ __forceinline__ void line_solve_by(const Grid& g, int kind, double k2
     lr.row(r0 + u, a, b, c, rhs);
     const double d = rhs ? vn[u] * rn : 0.0;
     const double den = a + c * P;
-    Q = quot(d - c * Q, den, yn[u]);
-    P = quot(-b, den, yn[u]);
+    Q = quot_finite(d - c * Q, den, yn[u]);
+    P = quot_finite(-b, den, yn[u]);
     v[(r0 - 1 + u) * vs] = Q;
     lp[(r0 - 1 + u) * ps] = P;
   }
@@ -240,7 +242,7 @@ __device__ __forceinline__ void line_solve_by(const Grid& g, int kind, double k2
     double a, b, c;
     bool rhs;
     lr.row(ny + 1, a, b, c, rhs);
-    Q = quot(0.0 - c * Q, a + c * P, lp[ny * ps]);
+    Q = quot_finite(0.0 - c * Q, a + c * P, lp[ny * ps]);
   }
   double x = Q, pn[TB], qn[TB];
 #pragma unroll
