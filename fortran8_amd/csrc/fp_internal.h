@@ -52,7 +52,7 @@ struct Ctx {
   int nspec = 1;                      // components it holds
   bool slab64 = false;                // a kx slab fits in LDS
   double* piv = nullptr;              // walls: pivots of the y line solves (three kinds)
-  double piv_beta = 0.0;              // the beta they were built with
+  double piv_beta = NAN;              // the beta they were built with
   double2 *twx = nullptr, *twy = nullptr, *twz = nullptr;
   double *kx2 = nullptr, *ky2 = nullptr, *kz2 = nullptr;
   double* red = nullptr;              // reduction scratch

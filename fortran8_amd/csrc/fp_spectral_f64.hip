@@ -421,10 +421,11 @@ int lnl_lines_y(const Grid& g) {
   return l;
 }
 
+// words of one kind's table of pivots
+long piv_words(const Grid& g) { return (long)g.nxh * (g.ny + 1) * g.nz; }
 void line_pivots(Ctx& c) {
   const Grid& g = c.g;
-  const long stride = (long)g.nxh * (g.ny + 1) * g.nz;
-  if (!c.piv) FP_HIP_CHECK(hipMalloc((void**)&c.piv, sizeof(double) * 3 * stride));
+  const long stride = piv_words(g);
   const int kinds[3] = {0, 1, 3};   // U and W share a table
   for (int t = 0; t < 3; t++)
     hipLaunchKernelGGL(k_line_pivots, dim3((unsigned)(((long)g.nxh * g.nz + 255) / 256)), dim3(256), 0, c.stream, g, kinds[t],
@@ -479,8 +480,8 @@ void solve(Ctx& c, int kind0, int comps, const double* q, double* x, bool div) {
   else if (g.walls) x_forward<Line::Div, true>(c, 0, comps, src);
   else x_forward<Line::Div, false>(c, 0, comps, src);
   const double rn = 1.0 / (double)(g.walls ? (long)g.nx * g.nz : g.n);
-  const long tstride = (long)g.nxh * (g.ny + 1) * g.nz;
-  if (g.walls && (!c.piv || c.piv_beta != g.beta)) line_pivots(c);
+  const long tstride = piv_words(g);
+  if (g.walls && c.piv_beta != g.beta) line_pivots(c);
   if (c.slab64) {
     const int threads = std::max(64, std::min(1024, g.ny * g.nz / 4));
     // three stages a pass where both axes divide into them: 64^3's step of 80 us
@@ -513,6 +514,9 @@ void f64_spectral_create(Ctx& c) {
   const size_t per = (size_t)g.nxh * g.ny * g.nz;
   c.nspec = per <= ((size_t)1 << 24) ? 3 : 1;
   FP_HIP_CHECK(hipMalloc((void**)&c.spec, sizeof(double2) * per * c.nspec));
+  // the pivots' tables: only the FP64 step solves between walls; filled by
+  // the first solve and when beta has changed
+  if (g.walls && c.p.precision == FP_PREC_F64) FP_HIP_CHECK(hipMalloc((void**)&c.piv, sizeof(double) * 3 * piv_words(g)));
   int lds_max = 0, dev = 0;
   FP_HIP_CHECK(hipGetDevice(&dev));
   FP_HIP_CHECK(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
