@@ -801,6 +801,7 @@ void adj_record(Ctx& c, int nsteps, int every, int replay, double* drag_out) {
   if (nsteps < 1 || every < 1) throw std::string("E_ARG:nsteps and every must be >= 1");
   if (c.p.method == FP_METHOD_IBM && c.nmk == 0) throw std::string("E_STATE:IBM method without markers");
   Adj& a = adj_of(c);
+  f64_spectral_reserve(c);
   const long n = c.g.n;
   const int polymer = c.p.beta != 1.0;
   if (replay && c.mixed) throw std::string("E_ARG:replay of recorded selections runs on the FP64 path");

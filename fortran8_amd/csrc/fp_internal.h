@@ -126,6 +126,7 @@ void f64_fill_f(Ctx& c);     // Peterlin factor of the current C
 void f64_spread_add(Ctx& c, const double* mfield, double* out);  // out += spread of marker values
 // ---- spectral solves (fp_spectral_f64.hip)
 void f64_spectral_create(Ctx& c);
+void f64_spectral_reserve(Ctx& c);   // a spectrum of as many components as the solves take at once
 void f64_solve(Ctx& c, int kind, const double* q, double* x);   // kind 0..2 Helmholtz, 3 Poisson
 void f64_helmholtz(Ctx& c, const double* q, double* x);         // the three components
 void f64_poisson(Ctx& c, const double* up, double* x);          // lap x = div up / dt

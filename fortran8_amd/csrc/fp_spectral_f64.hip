@@ -508,12 +508,30 @@ void solve(Ctx& c, int kind0, int comps, const double* q, double* x, bool div) {
 
 // The spectrum holds three components where that is small beside the state
 // (their solves then share launches); one above it, where a component alone
-// fills the device.
+// fills the device, and in a mixed context, whose step makes no FP64 solve
+// (its shell spectrum goes a component at a time) until it records for the
+// adjoint.
+static int solve_components(const Grid& g) { return (size_t)g.nxh * g.ny * g.nz <= ((size_t)1 << 24) ? 3 : 1; }
+static size_t spectrum_bytes(const Grid& g, int comps) { return sizeof(double2) * (size_t)g.nxh * g.ny * g.nz * comps; }
+
+void f64_spectral_reserve(Ctx& c) {
+  const int comps = solve_components(c.g);
+  if (c.nspec >= comps) return;
+  double2* more = nullptr;
+  if (hipMalloc((void**)&more, spectrum_bytes(c.g, comps)) != hipSuccess) {
+    (void)hipGetLastError();   // the solves go on one component at a time
+    return;
+  }
+  FP_HIP_CHECK(hipStreamSynchronize(c.stream));
+  (void)hipFree(c.spec);
+  c.spec = more;
+  c.nspec = comps;
+}
+
 void f64_spectral_create(Ctx& c) {
   const Grid& g = c.g;
-  const size_t per = (size_t)g.nxh * g.ny * g.nz;
-  c.nspec = per <= ((size_t)1 << 24) ? 3 : 1;
-  FP_HIP_CHECK(hipMalloc((void**)&c.spec, sizeof(double2) * per * c.nspec));
+  c.nspec = c.p.precision == FP_PREC_F64 ? solve_components(g) : 1;
+  FP_HIP_CHECK(hipMalloc((void**)&c.spec, spectrum_bytes(g, c.nspec)));
   // the pivots' tables: only the FP64 step solves between walls; filled by
   // the first solve and when beta has changed
   if (g.walls && c.p.precision == FP_PREC_F64) FP_HIP_CHECK(hipMalloc((void**)&c.piv, sizeof(double) * 3 * piv_words(g)));

@@ -29,3 +29,17 @@ def test_steps_allocate_nothing(case):
     g.step(2)
     assert free_bytes() == before
     g.close()
+
+
+def test_a_mixed_context_holds_one_component_of_the_fp64_spectrum():
+    """256^3: 264 B a cell of FP64 planes, 9 of selections and iteration counts,
+    214 of the mixed step, 8 of the FP64 spectrum's one component; two more
+    would be 16"""
+    p = configs.kolmogorov(n=16, precision=1).params
+    p.nx = p.ny = p.nz = 256
+    api.FenepGPU(p).close()
+    before = free_bytes()
+    g = api.FenepGPU(p)
+    used = (before - free_bytes()) / 256 ** 3
+    g.close()
+    assert 264 + 9 + 214 < used < 264 + 9 + 214 + 8 + 8
