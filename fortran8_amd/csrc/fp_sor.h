@@ -63,7 +63,11 @@ __global__ __launch_bounds__(1024) void k_sor_tile(Grid g, SorCoef<T> co, const 
   // wait a memory latency on its own
   const int th = LN ? THREADS : (int)blockDim.x;
   constexpr int NE = LN ? (WY * WZ * (1 << (LN - 1)) + THREADS - 1) / THREADS : 8;
-  constexpr int NQ = LN ? (QY * QZ * (1 << (LN - 1)) + THREADS - 1) / THREADS : 4;
+  // (a trip loads NE and NQ pairs a thread: as many of the right-hand side, in
+  // proportion, as of the iterate, whose count ends the loop)
+  constexpr int NQ = LN ? (QY * QZ * (1 << (LN - 1)) + THREADS - 1) / THREADS : (NE * QY * QZ + WY * WZ - 1) / (WY * WZ);
+  static_assert((LN ? WY * WZ * (1 << (LN - 1)) <= NE * THREADS && QY * QZ * (1 << (LN - 1)) <= NQ * THREADS
+                    : NQ * WY * WZ >= NE * QY * QZ), "every row of the right-hand side is loaded");
   for (int e0 = threadIdx.x, q0 = threadIdx.x; e0 < (WY * WZ) << lh; e0 += NE * th, q0 += NQ * th) {
     Pair pe[NE], pq[NQ];
 #pragma unroll
