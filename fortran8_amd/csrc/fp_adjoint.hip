@@ -614,6 +614,7 @@ struct Adj {
   double *ABT = nullptr, *Xb = nullptr, *lam = nullptr, *Mb = nullptr, *gm = nullptr, *Fb = nullptr;
   double *acc = nullptr, *part = nullptr;
   int tape_every = 0, ck_count = 0;
+  long gm_markers = 0;             // markers that gm holds
 };
 
 template <typename T>
@@ -888,8 +889,14 @@ void adj_backward(Ctx& c, const double* weights, const double* bar_final, double
     alloc0(&a.bar, (size_t)BAR_WORDS * n);
     alloc0(&a.ubs, 3 * n); alloc0(&a.phib, n); alloc0(&a.bb, n); alloc0(&a.Rb, 3 * n); alloc0(&a.Qb, 3 * n);
     alloc0(&a.ABT, 9 * n); alloc0(&a.Xb, 6 * n); alloc0(&a.lam, 6 * n); alloc0(&a.Mb, 9 * n);
-    alloc0(&a.gm, 3 * (c.nmk > 0 ? c.nmk : 1)); alloc0(&a.Fb, 3 * n);
+    alloc0(&a.Fb, 3 * n);
     alloc0(&a.acc, NACC); alloc0(&a.part, (size_t)NACC * nblk(n, 256));
+  }
+  if (a.gm_markers < c.nmk) {   // (the markers may have been set anew since the last sweep)
+    free0(a.gm);
+    a.gm_markers = 0;
+    alloc0(&a.gm, 3 * c.nmk);
+    a.gm_markers = c.nmk;
   }
   hipStream_t st = c.stream;
   if (c.mixed) mixed_join(c);   // no selection made ahead still writes c.sel
