@@ -23,6 +23,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", "--offload-arch=" + ARCH,
           "-Wno-unused-command-line-argument"]
 UNITS = [
     ("fp_kernels_f64.hip", ["-ffp-contract=off"]),
+    ("fp_select_f64.hip", ["-ffp-contract=off"]),
     ("fp_spectral_f64.hip", ["-ffp-contract=off"]),
     ("fp_stats.hip", ["-ffp-contract=off"]),
     ("fp_kernels_mixed.hip", ["-ffp-contract=fast-honor-pragmas"]),

@@ -165,6 +165,7 @@ void fp::step_f64(Ctx& c) {
     if (c.sel_replay) {
       FP_HIP_CHECK(hipMemcpyAsync(c.sel, c.sel_replay, g.n, hipMemcpyDeviceToDevice, c.stream));
     } else {
+      Timer t(c, "fenep_select");
       f64_select(c);
     }
     { Timer t(c, "fenep_cstar_newton"); f64_cstar_newton(c); }
@@ -244,9 +245,7 @@ int fp_create(const fp_params* p, void** out) {
     dalloc(&c->C[0], 6 * n); dalloc(&c->C[1], 6 * n);
     dalloc(&c->fC, n); dalloc(&c->sel, n); dalloc(&c->nitr, n);
     dalloc(&c->A0, 3 * n); dalloc(&c->T0, 3 * n); dalloc(&c->B0, 3 * n);
-    // (Q also holds the lists of the selection: 1536 words per 256 cells)
-    dalloc(&c->Q, std::max<long>(3 * n, 768)); dalloc(&c->Up, 3 * n);
-    dalloc(&c->sel_count, 1);
+    dalloc(&c->Q, 3 * n); dalloc(&c->Up, 3 * n);
     f64_spectral_create(*c);
     dalloc(&c->red, 64);
     dalloc(&c->part, (size_t)(g.n / 256 + 1024));
@@ -285,7 +284,7 @@ int fp_destroy(void* vc) {
   adj_free(*c);
   f64_sor_destroy(*c);
   dfree(c->U); dfree(c->V); dfree(c->W); dfree(c->P); dfree(c->Phi);
-  dfree(c->C[0]); dfree(c->C[1]); dfree(c->fC); dfree(c->sel); dfree(c->sel_count); dfree(c->nitr);
+  dfree(c->C[0]); dfree(c->C[1]); dfree(c->fC); dfree(c->sel); dfree(c->nitr);
   dfree(c->A0); dfree(c->T0); dfree(c->B0); dfree(c->Q); dfree(c->Up); dfree(c->F);
   dfree(c->spec); dfree(c->piv); dfree(c->red); dfree(c->part);
   dfree(c->twx); dfree(c->twy); dfree(c->twz); dfree(c->kx2); dfree(c->ky2); dfree(c->kz2);

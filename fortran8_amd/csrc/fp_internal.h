@@ -43,7 +43,6 @@ struct Ctx {
   int cur = 0;
   double *fC = nullptr;               // Peterlin factor of the current C
   uint8_t* sel = nullptr;
-  unsigned* sel_count = nullptr;      // FP64 step: selections left to FP64
   double *A0 = nullptr, *T0 = nullptr, *B0 = nullptr;  // 3 planes each
   double *Q = nullptr;                // 3 planes: predictor RHS / Ua
   double *Up = nullptr;               // 3 planes: u*
@@ -101,7 +100,7 @@ struct Ctx {
   size_t stat_words = 0;
 };
 
-// ---- launchers (fp_kernels_f64.hip; f64_select: fp_kernels_mixed.hip)
+// ---- launchers (fp_kernels_f64.hip; f64_select: fp_select_f64.hip)
 void f64_select(Ctx& c);
 void f64_cstar_newton(Ctx& c);
 void f64_predictor(Ctx& c);

@@ -58,10 +58,8 @@ template <bool WL, bool BIG>
 __global__ __launch_bounds__(128) void k_cstar_newton(Grid g, CstarConst K, const double* __restrict__ C,
                                                       const uint8_t* __restrict__ sel, const double* __restrict__ U,
                                                       const double* __restrict__ V, const double* __restrict__ W,
-                                                      double* __restrict__ Cn, double* __restrict__ fC, int* __restrict__ nitr,
-                                                      unsigned* __restrict__ sel_count) {
+                                                      double* __restrict__ Cn, double* __restrict__ fC, int* __restrict__ nitr) {
   const long L = xcd_cell();
-  if (L == 0) *sel_count = 0u;   // for the next step's selection
   if (L >= g.n) return;
   long m;
   int i, j, k;
@@ -990,7 +988,7 @@ void f64_cstar_newton(Ctx& c) {
   auto kern = g.walls ? (big ? k_cstar_newton<true, true> : k_cstar_newton<true, false>)
                       : (big ? k_cstar_newton<false, true> : k_cstar_newton<false, false>);
   hipLaunchKernelGGL(kern, dim3(nblk(g.n, 128)), dim3(128), 0, c.stream, g, K, c.C[c.cur], c.sel, c.U, c.V, c.W,
-                     c.C[1 - c.cur], c.fC, c.nitr, c.sel_count);
+                     c.C[1 - c.cur], c.fC, c.nitr);
   c.cur = 1 - c.cur;
 }
 

@@ -142,17 +142,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t brsrc(const void* base, unsign
 }
 template <typename V>
 __device__ __forceinline__ V ldu(const V* base, long n, unsigned e) {
-  static_assert(sizeof(V) == 8 || sizeof(V) == 4 || sizeof(V) == 1, "8-, 4- or 1-byte elements");
-  // FP64 planes may exceed what 32-bit byte offsets reach
-  if constexpr (sizeof(V) == 8) {
-    return base[e];
-  } else {
-    const __amdgpu_buffer_rsrc_t r = brsrc(base, (unsigned)n * (unsigned)sizeof(V));
-    if constexpr (sizeof(V) == 4)
-      return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, (int)(e * 4u), 0, 0));
-    else
-      return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b8(r, (int)e, 0, 0));
-  }
+  static_assert(sizeof(V) == 4 || sizeof(V) == 1, "4-byte or 1-byte elements");
+  const __amdgpu_buffer_rsrc_t r = brsrc(base, (unsigned)n * (unsigned)sizeof(V));
+  if constexpr (sizeof(V) == 4)
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, (int)(e * 4u), 0, 0));
+  else
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b8(r, (int)e, 0, 0));
 }
 template <typename V>
 __device__ __forceinline__ void stu(V* base, long n, unsigned e, V v) {
@@ -215,12 +210,9 @@ __device__ __forceinline__ int woff32(int a, int d, int n, int s) {
 #define SEL_K3E 7.10542736e-15f    /* 64 eps64 */
 #define SEL_KME 4.76837158e-07f    /* 8 eps32 */
 #define SEL_KCE 4.76837158e-07f    /* 8 eps32 */
-// FP64 fields are rounded to FP32 for the candidates: the entries' rounding
-// moves an eigenvalue by up to 2 eps32 Smax more (|1.5| + |0.5| of the cells'
-// entries), and the angle of a nearly double root by so much over r.  A matrix
-// that the reference takes for its sentinel may so leave the flagged zone by
-// 3 (4 eps32 Smax / r)^2 in arg: the candidate is flagged as well where that is
-// not below its delta, (12 eps32 Smax)^2 > 2 delta r^2.
+// (cells held in FP64 and rounded to FP32 would take 12: the entries' rounding
+// moves an eigenvalue by up to 2 eps32 Smax more, half of it either way.  The FP64
+// step decides in FP64, fp_select_f64.hip; the model test of the bound reads this.)
 #define SEL_KCE64 7.15255737e-07f  /* 12 eps32 */
 
 // lambda_min of one candidate and the half-width of its interval without
@@ -231,9 +223,7 @@ struct Lmin {
   bool amb;   // near the sentinel boundary (or degenerate): decide in FP64
 };
 
-// F64: of a field stored in FP64, ein its entry term
-template <bool F64 = false>
-__device__ __forceinline__ Lmin lmin32(const float* a, float ein = 0.0f) {
+__device__ __forceinline__ Lmin lmin32(const float* a) {
   const float third = 1.0f / 3.0f;
   const float m = ((a[0] + a[3]) + a[5]) * third;
   const float b11 = a[0] - m, b22 = a[3] - m, b33 = a[5] - m;
@@ -273,7 +263,6 @@ __device__ __forceinline__ Lmin lmin32(const float* a, float ein = 0.0f) {
   o.lam = fmaf(r, ps, m);
   // written so that a NaN arg counts as ambiguous
   o.amb = !(fabsf(arg) <= fmaf(-2.0f, d, 1.0f));
-  if (F64) o.amb = o.amb || !(ein * ein <= 2.0f * (d * r2));
   o.e0 = r * fmaf(d, v, SEL_KME * rho);
   return o;
 }
@@ -281,11 +270,6 @@ __device__ __forceinline__ Lmin lmin32(const float* a, float ein = 0.0f) {
 // bound on the entries of one cell's C: |diag| + 2 |offdiag| summed
 __device__ __forceinline__ float entry_bound(const float* c) {
   return (fabsf(c[0]) + fabsf(c[3]) + fabsf(c[5])) + 2.0f * ((fabsf(c[1]) + fabsf(c[2])) + fabsf(c[4]));
-}
-
-template <typename T>
-__device__ __forceinline__ float entry_term(float eba, float ebb, float ebc) {
-  return (sizeof(T) == 8 ? SEL_KCE64 : SEL_KCE) * fmaxf(fmaxf(eba, ebb), ebc);
 }
 
 // candidate face values (fenep.f90:179-184) in FP32, each with at most two
@@ -303,12 +287,11 @@ __device__ __forceinline__ float cand_nf(int l, float cm, float c, float cp) {
   return fmaf(cm, -0.25f, fmaf(cp, 0.25f, c));
 }
 // the six candidates of one axis line (cm, c, cp) evaluated
-template <bool F64 = false>
-__device__ __forceinline__ Lmin cand_lmin(bool right, int l, const float (&v)[3][6], float ein = 0.0f) {
+__device__ __forceinline__ Lmin cand_lmin(bool right, int l, const float (&v)[3][6]) {
   float a[6];
 #pragma unroll
   for (int q = 0; q < 6; q++) a[q] = right ? cand_nf(l, v[0][q], v[1][q], v[2][q]) : cand_pf(l, v[0][q], v[1][q], v[2][q]);
-  return lmin32<F64>(a, ein);
+  return lmin32(a);
 }
 
 // maxloc over {v_0, v_1, v_2, 0} of v_l = min(lambda(Cp_l), lambda(Cn_l))
@@ -341,9 +324,9 @@ __device__ __forceinline__ int sel_decide(const Lmin (&P)[3], const Lmin (&N)[3]
 // takes the linear extrapolation 2 C_0 - C_1 of the two nearest rows
 // (C_kabe), and a point beyond it the centre (it only feeds faces whose
 // upwind weight is exactly zero); the wrapped rows loaded there are replaced.
-template <int R, typename T>
-__device__ __forceinline__ void load_line(const T* __restrict__ C, const Grid& g, long m, int i, int j, int k, int d,
-                                          T (&v)[2 * R + 1][6]) {
+template <int R>
+__device__ __forceinline__ void load_line(const float* __restrict__ C, const Grid& g, long m, int i, int j, int k, int d,
+                                          float (&v)[2 * R + 1][6]) {
   // 32-bit cell indices from the plane bases (n <= 2^30 cells)
   unsigned e[2 * R + 1];
 #pragma unroll
@@ -357,29 +340,27 @@ __device__ __forceinline__ void load_line(const T* __restrict__ C, const Grid& g
 #pragma unroll
   for (int o = 0; o < 2 * R + 1; o++)
 #pragma unroll
-    for (int q = 0; q < 6; q++) v[o][q] = ldu<T>(C + q * g.n, g.n, e[o]);
+    for (int q = 0; q < 6; q++) v[o][q] = ldu(C + q * g.n, g.n, e[o]);
   // (the lanes of a wavefront share their row in the callers' cell orders,
   // so the interior rows branch past the patches)
   if (R == 1 && d == 1 && g.walls && (j == 0 || j == g.ny - 1)) {
     const bool lo = j == 0, hi = j == g.ny - 1;
 #pragma unroll
     for (int q = 0; q < 6; q++) {
-      v[0][q] = lo ? T(2) * v[1][q] - v[2][q] : v[0][q];
-      v[2][q] = hi ? T(2) * v[1][q] - v[0][q] : v[2][q];
+      v[0][q] = lo ? 2.0f * v[1][q] - v[2][q] : v[0][q];
+      v[2][q] = hi ? 2.0f * v[1][q] - v[0][q] : v[2][q];
     }
   }
-  if constexpr (R == 2) {
-    if (d == 1 && g.walls && (j < 2 || j >= g.ny - 2)) {
-      // rows 0, 1 at the low wall and ny-2, ny-1 at the high wall; each
-      // replacement reads only entries that no earlier one changes
-      const bool l0 = j == 0, l1 = j == 1, h1 = j == g.ny - 2, h0 = j == g.ny - 1;
+  if (R == 2 && d == 1 && g.walls && (j < 2 || j >= g.ny - 2)) {
+    // rows 0, 1 at the low wall and ny-2, ny-1 at the high wall; each
+    // replacement reads only entries that no earlier one changes
+    const bool l0 = j == 0, l1 = j == 1, h1 = j == g.ny - 2, h0 = j == g.ny - 1;
 #pragma unroll
-      for (int q = 0; q < 6; q++) {
-        v[1][q] = l0 ? T(2) * v[2][q] - v[3][q] : v[1][q];
-        v[0][q] = l0 ? v[2][q] : (l1 ? T(2) * v[1][q] - v[2][q] : v[0][q]);
-        v[3][q] = h0 ? T(2) * v[2][q] - v[1][q] : v[3][q];
-        v[4][q] = h0 ? v[2][q] : (h1 ? T(2) * v[3][q] - v[2][q] : v[4][q]);
-      }
+    for (int q = 0; q < 6; q++) {
+      v[1][q] = l0 ? 2.0f * v[2][q] - v[3][q] : v[1][q];
+      v[0][q] = l0 ? v[2][q] : (l1 ? 2.0f * v[1][q] - v[2][q] : v[0][q]);
+      v[3][q] = h0 ? 2.0f * v[2][q] - v[1][q] : v[3][q];
+      v[4][q] = h0 ? v[2][q] : (h1 ? 2.0f * v[3][q] - v[2][q] : v[4][q]);
     }
   }
 }
@@ -423,10 +404,7 @@ __device__ __forceinline__ bool row_cell(const Grid& g, long& m, int& i, int& j,
 #define SEL_STAGE 64
 
 // one LDS atomic per wavefront: the first unsure lane reserves the slots.
-// Called by every lane of the wavefront.  STAGE: FP32 fields (the re-decision
-// of an FP64 field gathers its values: staging them would hold 18 FP64 values
-// in registers through the evaluations).
-template <bool STAGE>
+// Called by every lane of the wavefront.
 __device__ __forceinline__ void sel_record(bool unsure, unsigned entry, const float (&v)[3][6], unsigned* s_cnt,
                                            unsigned* __restrict__ region, float* __restrict__ stage, unsigned cap) {
   const unsigned long long ball = __ballot(unsure);
@@ -439,7 +417,7 @@ __device__ __forceinline__ void sel_record(bool unsure, unsigned entry, const fl
     if (unsure) {
       const unsigned slot = base + (unsigned)__popcll(ball & ((1ull << lane) - 1ull));
       region[slot] = entry;
-      if (STAGE && slot < cap) {
+      if (slot < cap) {
 #pragma unroll
         for (int o = 0; o < 3; o++)
 #pragma unroll
@@ -465,11 +443,9 @@ __device__ __forceinline__ void sel_publish(unsigned* s_cnt, unsigned* s_base, l
 }
 
 // One cell per thread, any grid shape.
-template <typename T>
-__global__ __launch_bounds__(SEL_BLOCK) void m_select(Grid g, const T* __restrict__ C, uint8_t* __restrict__ sel,
+__global__ __launch_bounds__(SEL_BLOCK) void m_select(Grid g, const float* __restrict__ C, uint8_t* __restrict__ sel,
                                                       unsigned* __restrict__ total, unsigned* __restrict__ amb_idx,
                                                       unsigned* __restrict__ amb_list, float* __restrict__ amb_data) {
-  constexpr bool F64 = sizeof(T) == 8;
   __shared__ unsigned s_cnt, s_base;
   if (threadIdx.x == 0) s_cnt = 0u;
   __syncthreads();
@@ -485,19 +461,14 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select(Grid g, const T* __restric
     int idx = 0;
     float v[3][6];
     if (valid) {
-      T w[3][6];
-      load_line<1, T>(C, g, m, i, j, k, d, w);
-#pragma unroll
-      for (int o = 0; o < 3; o++)
-#pragma unroll
-        for (int q = 0; q < 6; q++) v[o][q] = (float)w[o][q];
-      const float ein = entry_term<T>(entry_bound(v[0]), entry_bound(v[1]), entry_bound(v[2]));
+      load_line<1>(C, g, m, i, j, k, d, v);
+      const float ein = SEL_KCE * fmaxf(fmaxf(entry_bound(v[0]), entry_bound(v[1])), entry_bound(v[2]));
       Lmin P[3], N[3];
 #pragma unroll
-      for (int l = 0; l < 3; l++) { P[l] = cand_lmin<F64>(false, l, v, ein); N[l] = cand_lmin<F64>(true, l, v, ein); }
+      for (int l = 0; l < 3; l++) { P[l] = cand_lmin(false, l, v); N[l] = cand_lmin(true, l, v); }
       idx = sel_decide(P, N, ein, unsure);
     }
-    sel_record<!F64>(unsure, (unsigned)(m * 3 + d), v, &s_cnt, region, stage, SEL_STAGE);
+    sel_record(unsure, (unsigned)(m * 3 + d), v, &s_cnt, region, stage, SEL_STAGE);
     s |= (uint8_t)(idx << (2 * d));
   }
   if (valid) sel[m] = s;
@@ -505,8 +476,8 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select(Grid g, const T* __restric
 }
 
 // The selection streamed along z, for nx = 64, 128 or 256 and nz a multiple
-// of KC: a block of 256 threads holds 256/nx whole x-rows and walks KC planes
-// (select_planes).  The midpoint candidate of a face, C_a/2 + C_{a+1}/2, is the right
+// of SZ_K: a block of 256 threads holds 256/nx whole x-rows and walks SZ_K
+// planes.  The midpoint candidate of a face, C_a/2 + C_{a+1}/2, is the right
 // face's candidate of level 0 for cell a and the left face's of level 1 for
 // cell a+1 (fenep.f90:179-184), bit for bit.  Along x a thread evaluates it
 // for its right face and hands it to its neighbour through LDS (the rows are
@@ -514,25 +485,24 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select(Grid g, const T* __restric
 // to the next plane in registers.  16 of the 18 eigenvalue evaluations of a
 // cell remain, plus one per column for its first plane, and the z line is
 // loaded one plane per step.
-template <typename T, int KC>
-__global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const T* __restrict__ C, uint8_t* __restrict__ sel,
+#define SZ_K 4
+__global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const float* __restrict__ C, uint8_t* __restrict__ sel,
                                                         unsigned* __restrict__ total, unsigned* __restrict__ amb_idx,
                                                         unsigned* __restrict__ amb_list, float* __restrict__ amb_data) {
-  constexpr bool F64 = sizeof(T) == 8;
   __shared__ unsigned s_cnt, s_base;
   __shared__ float s_lam[2][SEL_BLOCK], s_e0[2][SEL_BLOCK];
   __shared__ int s_amb[2][SEL_BLOCK];
   const int t = threadIdx.x;
   if (t == 0) s_cnt = 0u;
   const long xb = xcd_block();
-  const int nkg = g.nz / KC;
+  const int nkg = g.nz / SZ_K;
   const int kg = (int)(xb % nkg), jg = (int)(xb / nkg);
   const int i = t & (g.nx - 1);
   const int j = (jg << (8 - g.lnx)) + (t >> g.lnx);
   const int tl = (t & ~(g.nx - 1)) | ((i - 1) & (g.nx - 1));   // the x neighbour on the left
-  const int k0 = kg * KC;
-  const unsigned cap = SEL_STAGE * KC;
-  unsigned* region = amb_list + (size_t)blockIdx.x * (SEL_REGION * KC);
+  const int k0 = kg * SZ_K;
+  const unsigned cap = SEL_STAGE * SZ_K;
+  unsigned* region = amb_list + (size_t)blockIdx.x * (SEL_REGION * SZ_K);
   float* stage = amb_data + (size_t)blockIdx.x * 18 * cap;
   const long n = g.n;
   const int sz = g.nx * g.ny;
@@ -546,54 +516,53 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const T* __restr
     const unsigned e = m + (unsigned)woff32(k0, -1, g.nz, sz);
 #pragma unroll
     for (int q = 0; q < 6; q++) {
-      z[0][q] = (float)ldu(C + q * n, n, e);
-      z[1][q] = (float)ldu(C + q * n, n, m);
+      z[0][q] = ldu(C + q * n, n, e);
+      z[1][q] = ldu(C + q * n, n, m);
     }
   }
   float ebm = entry_bound(z[0]), ebc = entry_bound(z[1]);
   // Cp_1 along z of the first plane; later planes take the previous Cn_0
-  Lmin zl = cand_lmin<F64>(false, 1, z, entry_term<T>(ebm, ebc, 0.0f));
+  Lmin zl = cand_lmin(false, 1, z);
   __syncthreads();
-  for (int kk = 0; kk < KC; kk++) {
+  for (int kk = 0; kk < SZ_K; kk++) {
     const int par = kk & 1;
     {
       const unsigned e = m + (unsigned)woff32(k0 + kk, 1, g.nz, sz);
 #pragma unroll
-      for (int q = 0; q < 6; q++) z[2][q] = (float)ldu(C + q * n, n, e);
+      for (int q = 0; q < 6; q++) z[2][q] = ldu(C + q * n, n, e);
     }
     const float ebp = entry_bound(z[2]);
     // x: the right-face midpoint first, for the neighbour
     float x[3][6];
 #pragma unroll
     for (int q = 0; q < 6; q++) {
-      x[0][q] = (float)ldu(C + q * n, n, m + (unsigned)exm);
+      x[0][q] = ldu(C + q * n, n, m + (unsigned)exm);
       x[1][q] = z[1][q];
-      x[2][q] = (float)ldu(C + q * n, n, m + (unsigned)exp);
+      x[2][q] = ldu(C + q * n, n, m + (unsigned)exp);
     }
-    const float einx = entry_term<T>(entry_bound(x[0]), ebc, entry_bound(x[2]));
     Lmin XP[3], XN[3];
-    XN[0] = cand_lmin<F64>(true, 0, x, einx);
+    XN[0] = cand_lmin(true, 0, x);
     s_lam[par][t] = XN[0].lam;
     s_e0[par][t] = XN[0].e0;
     s_amb[par][t] = XN[0].amb;
-    XP[0] = cand_lmin<F64>(false, 0, x, einx);
-    XN[1] = cand_lmin<F64>(true, 1, x, einx);
-    XP[2] = cand_lmin<F64>(false, 2, x, einx);
-    XN[2] = cand_lmin<F64>(true, 2, x, einx);
+    XP[0] = cand_lmin(false, 0, x);
+    XN[1] = cand_lmin(true, 1, x);
+    XP[2] = cand_lmin(false, 2, x);
+    XN[2] = cand_lmin(true, 2, x);
+    const float einx = SEL_KCE * fmaxf(fmaxf(entry_bound(x[0]), ebc), entry_bound(x[2]));
     uint8_t sb = 0;
     // z: Cp_1 carried in
     {
-      const float einz = entry_term<T>(ebm, ebc, ebp);
       Lmin P[3], N[3];
       P[1] = zl;
-      P[0] = cand_lmin<F64>(false, 0, z, einz);
-      N[0] = cand_lmin<F64>(true, 0, z, einz);
-      N[1] = cand_lmin<F64>(true, 1, z, einz);
-      P[2] = cand_lmin<F64>(false, 2, z, einz);
-      N[2] = cand_lmin<F64>(true, 2, z, einz);
+      P[0] = cand_lmin(false, 0, z);
+      N[0] = cand_lmin(true, 0, z);
+      N[1] = cand_lmin(true, 1, z);
+      P[2] = cand_lmin(false, 2, z);
+      N[2] = cand_lmin(true, 2, z);
       bool unsure = false;
-      const int idx = sel_decide(P, N, einz, unsure);
-      sel_record<!F64>(unsure, m * 3u + 2u, z, &s_cnt, region, stage, cap);
+      const int idx = sel_decide(P, N, SEL_KCE * fmaxf(fmaxf(ebm, ebc), ebp), unsure);
+      sel_record(unsure, m * 3u + 2u, z, &s_cnt, region, stage, cap);
       sb |= (uint8_t)(idx << 4);
       zl = N[0];
     }
@@ -602,32 +571,23 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const T* __restr
       float y[3][6];
 #pragma unroll
       for (int q = 0; q < 6; q++) {
-        y[0][q] = (float)ldu(C + q * n, n, m + (unsigned)eym);
+        y[0][q] = ldu(C + q * n, n, m + (unsigned)eym);
         y[1][q] = z[1][q];
-        y[2][q] = (float)ldu(C + q * n, n, m + (unsigned)eyp);
+        y[2][q] = ldu(C + q * n, n, m + (unsigned)eyp);
       }
       if (ylo || yhi) {   // a wavefront holds one row: interior rows skip this
 #pragma unroll
         for (int q = 0; q < 6; q++) {
-          if constexpr (F64) {
-            // (in the stored type: the ghost is what the reference holds)
-            const T yc = ldu(C + q * n, n, m), yn = ldu(C + q * n, n, m + (unsigned)(ylo ? eyp : eym));
-            const float gh = (float)(T(2) * yc - yn);
-            y[0][q] = ylo ? gh : y[0][q];
-            y[2][q] = yhi ? gh : y[2][q];
-          } else {
-            y[0][q] = ylo ? 2.0f * y[1][q] - y[2][q] : y[0][q];
-            y[2][q] = yhi ? 2.0f * y[1][q] - y[0][q] : y[2][q];
-          }
+          y[0][q] = ylo ? 2.0f * y[1][q] - y[2][q] : y[0][q];
+          y[2][q] = yhi ? 2.0f * y[1][q] - y[0][q] : y[2][q];
         }
       }
-      const float einy = entry_term<T>(entry_bound(y[0]), ebc, entry_bound(y[2]));
       Lmin P[3], N[3];
 #pragma unroll
-      for (int l = 0; l < 3; l++) { P[l] = cand_lmin<F64>(false, l, y, einy); N[l] = cand_lmin<F64>(true, l, y, einy); }
+      for (int l = 0; l < 3; l++) { P[l] = cand_lmin(false, l, y); N[l] = cand_lmin(true, l, y); }
       bool unsure = false;
-      const int idx = sel_decide(P, N, einy, unsure);
-      sel_record<!F64>(unsure, m * 3u + 1u, y, &s_cnt, region, stage, cap);
+      const int idx = sel_decide(P, N, SEL_KCE * fmaxf(fmaxf(entry_bound(y[0]), ebc), entry_bound(y[2])), unsure);
+      sel_record(unsure, m * 3u + 1u, y, &s_cnt, region, stage, cap);
       sb |= (uint8_t)(idx << 2);
     }
     __syncthreads();
@@ -637,7 +597,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const T* __restr
     {
       bool unsure = false;
       const int idx = sel_decide(XP, XN, einx, unsure);
-      sel_record<!F64>(unsure, m * 3u, x, &s_cnt, region, stage, cap);
+      sel_record(unsure, m * 3u, x, &s_cnt, region, stage, cap);
       sb |= (uint8_t)idx;
     }
     sel[m] = sb;
@@ -650,7 +610,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const T* __restr
     ebc = ebp;
     m += (unsigned)sz;
   }
-  sel_publish(&s_cnt, &s_base, blockIdx.x, SEL_REGION * KC, total, amb_idx);
+  sel_publish(&s_cnt, &s_base, blockIdx.x, SEL_REGION * SZ_K, total, amb_idx);
 }
 
 // the reference's selection (select_d, evaluated as written) of one (cell,
@@ -682,27 +642,23 @@ __device__ __forceinline__ int select_ref(const Grid& g, const float* __restrict
 // (2.4 of 6 on average in the throughput case), one reference Vieta per trip.
 // The three cells of (cell m, axis d), wall ghosts by the C_kabe rule (the
 // values m_select reads through load_line).
-template <bool WL, typename T>
-__device__ __forceinline__ void sel_cells(const Grid& g, const T* __restrict__ C, long m, int d, T (&fm)[6],
-                                          T (&fc)[6], T (&fp)[6]) {
+template <bool WL>
+__device__ __forceinline__ void sel_cells(const Grid& g, const float* __restrict__ C, long m, int d, float (&fm)[6],
+                                          float (&fc)[6], float (&fp)[6]) {
   int i, j, k;
   cell_ijk(g, m, i, j, k);
   const int di = d == 0, dj = d == 1, dk = d == 2;
 #pragma unroll
   for (int q = 0; q < 6; q++) {
-    const T* Cq = C + q * g.n;
+    const float* Cq = C + q * g.n;
     fm[q] = ldbw<WL>(Cq, g, i - di, j - dj, k - dk, BC_C);
     fc[q] = Cq[m];
     fp[q] = ldbw<WL>(Cq, g, i + di, j + dj, k + dk, BC_C);
   }
 }
 
-template <typename T>
-__device__ __forceinline__ int select_pruned(const T (&tm)[6], const T (&tc)[6], const T (&tp)[6]) {
-  float fm[6], fc[6], fp[6];
-#pragma unroll
-  for (int q = 0; q < 6; q++) { fm[q] = (float)tm[q]; fc[q] = (float)tc[q]; fp[q] = (float)tp[q]; }
-  const float ein = entry_term<T>(entry_bound(fm), entry_bound(fc), entry_bound(fp));
+__device__ __forceinline__ int select_pruned(const float (&fm)[6], const float (&fc)[6], const float (&fp)[6]) {
+  const float ein = SEL_KCE * fmaxf(fmaxf(entry_bound(fm), entry_bound(fc)), entry_bound(fp));
   // one level per trip (a rolled loop keeps the register count, and so the
   // occupancy that hides the FP64 latencies, down)
   float lam[6], err[6];
@@ -712,7 +668,7 @@ __device__ __forceinline__ int select_pruned(const T (&tm)[6], const T (&tc)[6],
     float ap[6], an[6];
 #pragma unroll
     for (int q = 0; q < 6; q++) { ap[q] = cand_pf(l, fm[q], fc[q], fp[q]); an[q] = cand_nf(l, fm[q], fc[q], fp[q]); }
-    const Lmin P = lmin32<sizeof(T) == 8>(ap, ein), N = lmin32<sizeof(T) == 8>(an, ein);
+    const Lmin P = lmin32(ap), N = lmin32(an);
 #pragma unroll
     for (int u = 0; u < 3; u++)
       if (u == l) {
@@ -761,9 +717,9 @@ __device__ __forceinline__ int select_pruned(const T (&tm)[6], const T (&tc)[6],
 #pragma unroll
     for (int q = 0; q < 6; q++) {
 #pragma clang fp contract(off)
-      const double cq = (double)tc[q];
-      const double A = (wa * (a_c ? cq : (double)tm[q])) * sh;
-      const double Cc = (wc * (c_c ? cq : (double)tp[q])) * sh;
+      const double cq = (double)fc[q];
+      const double A = (wa * (a_c ? cq : (double)fm[q])) * sh;
+      const double Cc = (wc * (c_c ? cq : (double)fp[q])) * sh;
       a[q] = (A + (three ? cq : -0.0)) + Cc;
     }
     const double v = vieta_d(a);
@@ -782,10 +738,10 @@ __device__ __forceinline__ int select_pruned(const T (&tm)[6], const T (&tc)[6],
 
 // FP64 re-decision of the uncertified selections: grid-stride over the
 // packed list; an entry's 18 input values come from its select block's
-// staging area for the block's first `cap` entries (FP32 fields) and are
-// gathered for the rest
-template <bool WL, typename T>
-__global__ __launch_bounds__(64) void m_select_fix(Grid g, const T* __restrict__ C, uint8_t* __restrict__ sel,
+// staging area for the block's first `cap` entries and are gathered for the
+// rest
+template <bool WL>
+__global__ __launch_bounds__(64) void m_select_fix(Grid g, const float* __restrict__ C, uint8_t* __restrict__ sel,
                                                     const unsigned* __restrict__ total,
                                                     const unsigned* __restrict__ amb_idx,
                                                     const unsigned* __restrict__ amb_list,
@@ -793,26 +749,23 @@ __global__ __launch_bounds__(64) void m_select_fix(Grid g, const T* __restrict__
   const long cnt = (long)*total;
   for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < cnt; t += (long)gridDim.x * blockDim.x) {
     const unsigned at = amb_idx[t];
+    const unsigned blk = at / region, slot = at - blk * region;
     const unsigned e = amb_list[at];
     const long m = (long)(e / 3u);
     const int d = (int)(e % 3u);
-    T fm[6], fc[6], fp[6];
-    bool staged = false;
-    if constexpr (sizeof(T) == 4) {
-      const unsigned blk = at / region, slot = at - blk * region;
-      staged = slot < cap;
-      if (staged) {
-        const float* src = amb_data + (size_t)blk * 18 * cap + slot;
+    float fm[6], fc[6], fp[6];
+    if (slot < cap) {
+      const float* src = amb_data + (size_t)blk * 18 * cap + slot;
 #pragma unroll
-        for (int q = 0; q < 6; q++) {
-          fm[q] = src[q * cap];
-          fc[q] = src[(6 + q) * cap];
-          fp[q] = src[(12 + q) * cap];
-        }
+      for (int q = 0; q < 6; q++) {
+        fm[q] = src[q * cap];
+        fc[q] = src[(6 + q) * cap];
+        fp[q] = src[(12 + q) * cap];
       }
+    } else {
+      sel_cells<WL>(g, C, m, d, fm, fc, fp);
     }
-    if (!staged) sel_cells<WL, T>(g, C, m, d, fm, fc, fp);
-    const int idx = select_pruned<T>(fm, fc, fp);
+    const int idx = select_pruned(fm, fc, fp);
     // the byte holds three axes: update only this axis
     unsigned* word = (unsigned*)((size_t)(sel + m) & ~(size_t)3);
     const int sh = 8 * (int)((size_t)(sel + m) & 3) + 2 * d;
@@ -976,7 +929,7 @@ __device__ __forceinline__ void cstar_newton_cell(const Grid& g, const float* __
     const T w3 = s3 * gp_ + s2 * gn + s1 * bq;
     const T w4 = s1 * gq;
     float v[5][6];
-    load_line<2, float>(C, g, m, i, j, k, d, v);
+    load_line<2>(C, g, m, i, j, k, d, v);
 #pragma unroll
     for (int q = 0; q < 6; q++)
       cx[q] += w0 * (T)v[0][q] + w1 * (T)v[1][q] + w2 * (T)v[2][q] + w3 * (T)v[3][q] + w4 * (T)v[4][q];
@@ -3987,66 +3940,38 @@ static void dc_record(Ctx& c) {
   X.dc_pending = true;
 }
 
-// Planes a block of the z-streamed selection walks (0: the per-cell kernel):
-// whole x-rows in a block of 256 threads.  Four planes where it runs beside
-// other kernels (the mixed step): more, shorter blocks take issue slots from
-// them (64^3: 155 us a step with four, 167 with one).  On its own (the FP64
-// step) as many, up to four, as leave eight blocks per CU: the midpoint handed
-// along z saves one evaluation in 17, an idle SIMD costs more.
-static int select_planes(const Grid& g, bool beside) {
-  if (g.nx != 64 && g.nx != 128 && g.nx != 256) return 0;
-  int kc = 4;
-  while (!beside && kc > 1 && g.n / (SEL_BLOCK * kc) < 2048) kc >>= 1;
-  return kc;   // (nz is a power of two, at least 4)
-}
+// the z-streamed selection's shapes: whole x-rows in a block of 256 threads
+// (nz is a power of two, at least 4).  More, shorter blocks take issue slots from
+// the kernels beside it: 64^3 155 us a step with four planes a block, 167 with one.
+static bool select_streamed(const Grid& g) { return g.nx == 64 || g.nx == 128 || g.nx == 256; }
 
-// The selection of the field C (FP32 or FP64) into c.sel: certified FP32
-// decisions, then the listed rest in FP64.  total: the count of the list, zero on
-// entry; idx, list: 3 entries per cell of each 256-cell block; data: the
-// staging area of FP32 fields.
-template <typename T>
-static void select_launch(Ctx& c, const T* C, unsigned* total, unsigned* idx, unsigned* list, float* data, int tm,
-                          hipStream_t s) {
+// cleared: X.amb is zero
+static void select_fenep(Ctx& c, int tm, hipStream_t s, bool cleared) {
+  Mixed& X = MX(c);
   const Grid& g = c.g;
   const long nb = nblk(g.n, SEL_BLOCK);
   // select blocks, and each block's region and staging entries (the same
   // totals either way: 3 n entries, 18 n / 4 staged values)
-  const int kc = select_planes(g, sizeof(T) == 4);
-  const unsigned region = SEL_REGION * std::max(1, kc), cap = SEL_STAGE * std::max(1, kc);
+  const bool zs = select_streamed(g);
+  const long nbs = zs ? g.n / (SEL_BLOCK * SZ_K) : nb;
+  const unsigned region = zs ? SEL_REGION * SZ_K : SEL_REGION, cap = zs ? SEL_STAGE * SZ_K : SEL_STAGE;
+  if (!cleared) zero_words(X.amb, 1, s);
   {
     MTimer t(c, tm ? "fenep_select" : nullptr, s);
-    if (kc) {
-      auto streamed = kc == 4 ? m_select_z<T, 4> : (kc == 2 ? m_select_z<T, 2> : m_select_z<T, 1>);
-      hipLaunchKernelGGL(streamed, dim3(g.n / (SEL_BLOCK * kc)), dim3(SEL_BLOCK), 0, s, g, C, c.sel, total, idx, list, data);
-    } else
-      hipLaunchKernelGGL(m_select<T>, dim3(nb), dim3(SEL_BLOCK), 0, s, g, C, c.sel, total, idx, list, data);
+    if (zs)
+      hipLaunchKernelGGL(m_select_z, dim3(nbs), dim3(SEL_BLOCK), 0, s, g, X.C[X.cur], c.sel, X.amb, X.amb_idx,
+                         X.amb_list, X.amb_data);
+    else
+      hipLaunchKernelGGL(m_select, dim3(nb), dim3(SEL_BLOCK), 0, s, g, X.C[X.cur], c.sel, X.amb, X.amb_idx,
+                         X.amb_list, X.amb_data);
   }
   {
     MTimer t(c, tm ? "fenep_select_fp64_fix" : nullptr, s);
     // n / 4 threads, one wavefront per block: 16 per SIMD at 256x128x128,
     // enough to hide the FP64 latencies
-    auto fix = g.walls ? m_select_fix<true, T> : m_select_fix<false, T>;
-    hipLaunchKernelGGL(fix, dim3(nb), dim3(64), 0, s, g, C, c.sel, total, idx, list, data, region, cap);
+    hipLaunchKernelGGL(g.walls ? m_select_fix<true> : m_select_fix<false>, dim3(nb), dim3(64), 0, s, g, X.C[X.cur], c.sel,
+                       X.amb, X.amb_idx, X.amb_list, X.amb_data, region, cap);
   }
-}
-
-// cleared: X.amb is zero
-static void select_fenep(Ctx& c, int tm, hipStream_t s, bool cleared) {
-  Mixed& X = MX(c);
-  if (!cleared) zero_words(X.amb, 1, s);
-  select_launch<float>(c, X.C[X.cur], X.amb, X.amb_idx, X.amb_list, X.amb_data, tm, s);
-}
-
-// The FP64 step's selection.  The reference formula in FP64 for every
-// candidate (18 arc cosines and cosines a cell, 4.0e8 VALU instructions at
-// 256x128x128) took 853 us; the certified FP32 decisions and the FP64 of the
-// few per cent that stay open make the same selection.  The lists live in the
-// predictor's output c.Q, which the step writes later; c.sel_count is zero on entry
-// (k_cstar_newton clears it).
-void f64_select(Ctx& c) {
-  unsigned* list = (unsigned*)c.Q;
-  const long words = (long)nblk(c.g.n, SEL_BLOCK) * SEL_REGION;
-  select_launch<double>(c, c.C[c.cur], c.sel_count, list, list + words, nullptr, 1, c.stream);
 }
 
 // Start the selection of the C this step produced on the side stream: it
