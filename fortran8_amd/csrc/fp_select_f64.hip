@@ -10,13 +10,13 @@
 // formula in FP64 (vieta_d), at the levels whose intervals can hold the maximum.
 //
 // Bound by FP64 issue: 1449 VALU operations a cell and plane, 1174 of them FP64
-// (168 of 240 us at 256x128x128; three wavefronts per SIMD and the packed
-// formula's latency the rest).  256x128x128 between walls, us, by what is left
-// to the formula, against 780-806 for the formula at every candidate in any
-// state: nothing (smooth, with or without noise) 240-265, 0.25 % (noise of 1e-3
-// on C = I) 306, a third (uniform in z) 450, all (C = I) 790.  64^3, against
-// 58-66: 22, 36, 38 and 64.  (Intervals from FP32 arithmetic and a second kernel
-// over a list took 178-190, 250, 715 and 2740, and 40, 45, 108 and 322.)
+// (168 of 240 us at 256x128x128; three wavefronts per SIMD).  256x128x128
+// between walls, us, by what is left to the formula, against 780-806 for the
+// formula at every candidate in any state: nothing (smooth, with or without
+// noise) 240-260, 0.25 % (noise of 1e-3 on C = I) 264 (304 without the short
+// lists' own path), a third (uniform in z) 434, all (C = I) 783.  64^3, against
+// 58-66: 22, 27 (39), 38 and 63.  (Intervals from FP32 arithmetic and a second
+// kernel over a list took 178-190, 250, 715 and 2740, and 40, 45, 108 and 322.)
 #include "fp_device.h"
 #include <algorithm>
 
@@ -116,6 +116,15 @@ __device__ __forceinline__ int decide(const Lam& a, const Lam& b, const Lam& c) 
 
 }  // namespace
 
+// the first maximum of the levels taken, or the zero slope (select_d)
+struct Best {
+  double v = 0.0;
+  int idx = -1;
+  __device__ __forceinline__ void take(int l, double x) {
+    if (!isnan(x) && (idx < 0 || x > v)) { idx = l; v = x; }
+  }
+  __device__ __forceinline__ int option() const { return idx < 0 || 0.0 > v ? 3 : idx; }
+};
 // The reference's selection among the levels `need` of the cells cm, c, cp.
 // Where the three are the same, levels 0 and 1 have the same two faces.
 __device__ __forceinline__ int formula(int need, const double (&cm)[6], const double (&c)[6], const double (&cp)[6]) {
@@ -126,8 +135,7 @@ __device__ __forceinline__ int formula(int need, const double (&cm)[6], const do
     diff |= (x ^ __builtin_bit_cast(unsigned long long, cm[q])) | (x ^ __builtin_bit_cast(unsigned long long, cp[q]));
   }
   if (diff == 0 && (need & 1)) need &= ~2;
-  double best = 0.0;
-  int idx = -1;
+  Best best;
 #pragma unroll 1
   for (int l = 0; l < 3; l++) {
     if (!(need >> l & 1)) continue;
@@ -137,10 +145,9 @@ __device__ __forceinline__ int formula(int need, const double (&cm)[6], const do
       ap[q] = cand_p(l, cm[q], c[q], cp[q]);
       an[q] = cand_n(l, cm[q], c[q], cp[q]);
     }
-    const double v = minval2_d(vieta_d(ap), vieta_d(an));
-    if (!isnan(v) && (idx < 0 || v > best)) { idx = l; best = v; }
+    best.take(l, minval2_d(vieta_d(ap), vieta_d(an)));
   }
-  return idx < 0 || 0.0 > best ? 3 : idx;
+  return best.option();
 }
 
 // A block holds 256 consecutive cells (whole x-rows where XS: nx <= 256) and
@@ -246,13 +253,12 @@ __global__ __launch_bounds__(256, 3) void k_select(Grid g, const double* __restr
   }
   __syncthreads();
   const unsigned cnt = s_cnt;
-  for (unsigned e = t; e < cnt; e += 256) {
-    const unsigned what = s_list[e];
+  // the cells of a pair and its place in the block
+  auto pair_cells = [&](unsigned what, double (&cm)[6], double (&c)[6], double (&cp)[6]) {
     const int cell = (int)(what & 1023u), d = (int)(what >> 10 & 3u);
     const long mc = m0 + (cell & 255) + (long)(cell >> 8) * plane;
     int ci, cj, ck;
     cell_ijk(g, mc, ci, cj, ck);
-    double cm[6], c[6], cp[6];
 #pragma unroll
     for (int q = 0; q < 6; q++) {
       const double* Cq = C + q * n;
@@ -260,8 +266,41 @@ __global__ __launch_bounds__(256, 3) void k_select(Grid g, const double* __restr
       c[q] = Cq[mc];
       cp[q] = ldb(Cq, g, ci + (d == 0), cj + (d == 1), ck + (d == 2), BC_C);
     }
-    const unsigned idx = (unsigned)formula((int)(what >> 12), cm, c, cp);
+  };
+  auto settle = [&](unsigned what, unsigned idx) {
+    const int cell = (int)(what & 1023u), d = (int)(what >> 10 & 3u);
     atomicOr(&s_sel[cell >> 2], idx << (8 * (cell & 3) + 2 * d));
+  };
+  if (cnt <= 42) {
+    // a short list: a lane per pair and face, one formula's latency instead of
+    // that of all its faces.  (A long one would idle the lanes of the faces
+    // that are not needed.)
+    double* res = (double*)s_mid;
+    const unsigned e = t / 6, l = t % 6 >> 1;
+    if (e < cnt) {
+      const unsigned what = s_list[e];
+      if (what >> (12 + l) & 1u) {
+        double cm[6], c[6], cp[6], a[6];
+        pair_cells(what, cm, c, cp);
+#pragma unroll
+        for (int q = 0; q < 6; q++) a[q] = t & 1 ? cand_n(l, cm[q], c[q], cp[q]) : cand_p(l, cm[q], c[q], cp[q]);
+        res[t] = vieta_d(a);
+      }
+    }
+    __syncthreads();
+    if ((unsigned)t < cnt) {
+      Best best;
+      for (int q = 0; q < 3; q++)
+        if (s_list[t] >> (12 + q) & 1u) best.take(q, minval2_d(res[6 * t + 2 * q], res[6 * t + 2 * q + 1]));
+      settle(s_list[t], best.option());
+    }
+  } else {
+    for (unsigned e = t; e < cnt; e += 256) {
+      const unsigned what = s_list[e];
+      double cm[6], c[6], cp[6];
+      pair_cells(what, cm, c, cp);
+      settle(what, (unsigned)formula((int)(what >> 12), cm, c, cp));
+    }
   }
   __syncthreads();
   const int words = (int)std::min<long>(64, (n - m0) >> 2);

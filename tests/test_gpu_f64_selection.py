@@ -19,8 +19,8 @@ def state(kind, c, rng):
     eye = np.broadcast_to(np.array([1.0, 0, 0, 1, 0, 1]), c.shape).copy()
     if kind == "at rest":
         return eye
-    if kind == "noise 1e-15":
-        return eye + 1e-15 * rng.standard_normal(c.shape)
+    if kind.startswith("noise"):         # 1e-4: a few pairs a block
+        return eye + float(kind.split()[1]) * rng.standard_normal(c.shape)
     if kind == "small":
         return 1e-60 * c
     c = np.broadcast_to(c[:1], c.shape).copy()
@@ -31,7 +31,7 @@ def state(kind, c, rng):
     return c
 
 
-KINDS = ["at rest", "noise 1e-15", "small", "uniform in z", "uniform in y and z", "half uniform"]
+KINDS = ["at rest", "noise 1e-15", "noise 1e-4", "small", "uniform in z", "uniform in y and z", "half uniform"]
 
 
 @pytest.mark.parametrize("kind", KINDS)
