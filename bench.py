@@ -245,7 +245,7 @@ def main():
     mixed_pred = "fp::m_predictor<false>" if "predictor_walls" in kt else "fp::m_predictor_z<%s>" % walls
     # the selection streamed along z where a block holds whole x-rows
     streamed = case.params.nx in (64, 128, 256)
-    kernel_names = {"fenep_select": "fp::m_select%s<%s>" % ("_z" if streamed else "", "float" if prec else "double"),
+    kernel_names = {"fenep_select": ("fp::m_select_z" if streamed else "fp::m_select") if prec else "fp::k_select",
                     "fenep_cstar_newton": "fp::m_cstar_newton" if prec else "fp::k_cstar_newton<%s, false>" % walls,
                     "predictor": mixed_pred if prec else "fp::k_predictor_z<%s>" % walls}
     out = {

@@ -51,9 +51,9 @@ __device__ __forceinline__ FaceCoef face_n(int l) {
 // The four faces of a cell and axis come from one line of five cells (30 loads an
 // axis; each face with its own loads took 72).  Bound by FP64 issue: the
 // Newton's 6 x 6 elimination and its central-difference Jacobian.  256x128x128
-// between walls: 1420 -> 549 us (quotients by a shared divisor through its
+// between walls: 1420 -> 500-540 us (quotients by a shared divisor through its
 // reciprocal, row swaps only where a wavefront needs one, 7 shifts a Newton
-// iteration instead of 13, the shared line); 64^3: 85 -> 42 us.
+// iteration instead of 13, the shared line); 64^3: 85 -> 41 us.
 template <bool WL, bool BIG>
 __global__ __launch_bounds__(128) void k_cstar_newton(Grid g, CstarConst K, const double* __restrict__ C,
                                                       const uint8_t* __restrict__ sel, const double* __restrict__ U,
@@ -206,12 +206,7 @@ __device__ __forceinline__ double c0_at(const Grid& g, const double* __restrict_
   return fC[m] * C[q * g.n + m] - E;
 }
 
-// One cell of the predictor over a stencil accessor S (v(c, ..): velocity
-// component c, c0(q, ..): C0, at an offset from the cell): convection (fenep.f90:694-734), viscous (736-770), polymer_stress
-// (645-691) and the predictor right-hand side of navier (803-826),
-// fft_navier (1466-1511) or ibm_preliminary (1994-2013), with the history
-// updates A0=A, T0=T, B0=B done in place.
-// the cell's own inputs, read where they are used
+// the predictor's own inputs of a cell, read where they are used
 template <bool WL>
 struct PredAt {
   const Grid& g;
@@ -255,6 +250,12 @@ struct PredConst {
   double dx, dy, dz, dxx, dyy, dzz, dx4, dy4, dz4;
   double idx, idy, idz, idxx, idyy, idzz, idx4, idy4, idz4;
 };
+// One cell of the predictor over a stencil accessor S (v(c, ..): velocity
+// component c, c0(q, ..): C0, at an offset from the cell) and the cell's own inputs
+// `in`: convection (fenep.f90:694-734), viscous (736-770), polymer_stress
+// (645-691) and the predictor right-hand side of navier (803-826),
+// fft_navier (1466-1511) or ibm_preliminary (1994-2013), with the history
+// updates A0=A, T0=T, B0=B done in place.
 template <bool WL, class Acc, class In>
 __device__ __forceinline__ void pred_cell(const Grid& g, const PredConst& K, const Acc& S, const In& in, int method,
                                           int first, int polymer, int i, int j, int k, long m, double* A0, double* T0,
@@ -730,8 +731,9 @@ void f64_ibm(Ctx& c) {
 
 // Host-side construction of the spreading CSR: for each ghosted target the
 // contributing (marker, stencil slot) pairs in the order of the reference's
-// loops (markers n, m, l; then k, j, i), extended by every point the ghost
-// folds write to, so that one gather pass per step rewrites all of them.
+// loops (markers n, m, l; then k, j, i), and the points that the ghost folds
+// add to; the forced cells are the interior ones among them, each with the rows
+// that it gathers (k_ibm_spread).
 void f64_ibm_setup(Ctx& c) {
   const Grid& g = c.g;
   std::vector<double> mk(6 * c.nmk);

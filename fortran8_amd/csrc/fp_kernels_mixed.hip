@@ -3771,8 +3771,8 @@ double mixed_last_ndc(Ctx& c) {
 }
 
 // C+- selection of the current stored field: certified FP32 decisions, the
-// per-block list counts scanned, the rest re-decided in FP64.  tm != 0 times
-// the two phases.
+// rest, whose places the blocks append to one packed list, re-decided in FP64.
+// tm != 0 times the two phases.
 static void select_fenep(Ctx& c, int tm, hipStream_t s, bool cleared = false);
 
 // Selection of the current stored field as the step makes it (certified FP32

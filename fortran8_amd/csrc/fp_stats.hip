@@ -3,7 +3,9 @@
 // fields) and compute in FP64; a mixed state is not widened in memory first.
 // Sums: registers over a thread's cells, shuffles over a wavefront, one
 // partial per block and a second kernel over the partials, always in the same
-// order.  Compiled with -ffp-contract=off.
+// order; the shell spectrum alone adds into a block's bins with LDS atomics, so
+// its last bits depend on the order in which wavefronts arrive.  Compiled with
+// -ffp-contract=off.
 #include "fp_fft.h"
 #include "fp_mixed.h"
 #include <algorithm>
