@@ -540,6 +540,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const float* __r
       x[1][q] = z[1][q];
       x[2][q] = ldu(C + q * n, n, m + (unsigned)exp);
     }
+    const float einx = SEL_KCE * fmaxf(fmaxf(entry_bound(x[0]), ebc), entry_bound(x[2]));
     Lmin XP[3], XN[3];
     XN[0] = cand_lmin(true, 0, x);
     s_lam[par][t] = XN[0].lam;
@@ -549,10 +550,10 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const float* __r
     XN[1] = cand_lmin(true, 1, x);
     XP[2] = cand_lmin(false, 2, x);
     XN[2] = cand_lmin(true, 2, x);
-    const float einx = SEL_KCE * fmaxf(fmaxf(entry_bound(x[0]), ebc), entry_bound(x[2]));
     uint8_t sb = 0;
     // z: Cp_1 carried in
     {
+      const float einz = SEL_KCE * fmaxf(fmaxf(ebm, ebc), ebp);
       Lmin P[3], N[3];
       P[1] = zl;
       P[0] = cand_lmin(false, 0, z);
@@ -561,7 +562,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const float* __r
       P[2] = cand_lmin(false, 2, z);
       N[2] = cand_lmin(true, 2, z);
       bool unsure = false;
-      const int idx = sel_decide(P, N, SEL_KCE * fmaxf(fmaxf(ebm, ebc), ebp), unsure);
+      const int idx = sel_decide(P, N, einz, unsure);
       sel_record(unsure, m * 3u + 2u, z, &s_cnt, region, stage, cap);
       sb |= (uint8_t)(idx << 4);
       zl = N[0];
@@ -582,11 +583,12 @@ __global__ __launch_bounds__(SEL_BLOCK) void m_select_z(Grid g, const float* __r
           y[2][q] = yhi ? 2.0f * y[1][q] - y[0][q] : y[2][q];
         }
       }
+      const float einy = SEL_KCE * fmaxf(fmaxf(entry_bound(y[0]), ebc), entry_bound(y[2]));
       Lmin P[3], N[3];
 #pragma unroll
       for (int l = 0; l < 3; l++) { P[l] = cand_lmin(false, l, y); N[l] = cand_lmin(true, l, y); }
       bool unsure = false;
-      const int idx = sel_decide(P, N, SEL_KCE * fmaxf(fmaxf(entry_bound(y[0]), ebc), entry_bound(y[2])), unsure);
+      const int idx = sel_decide(P, N, einy, unsure);
       sel_record(unsure, m * 3u + 1u, y, &s_cnt, region, stage, cap);
       sb |= (uint8_t)(idx << 2);
     }
