@@ -22,7 +22,7 @@
 // Three launches serve the three Helmholtz problems and three the Poisson
 // equation (its right-hand side formed in the x transform) where a kx slab
 // fits in LDS, five otherwise.  Before: five per component (x, y, z with the
-// division, y, x), 24 of the step's launches.  Small grids are bound by those
+// division, y, x), 20 of the step's 24 launches.  Small grids are bound by those
 // launches: the Newtonian 32^3 step took 127 us and takes 49, the FENE-P step
 // at 64^3 340 and 228 us.  At 256 x 128 x 128 between walls the four solves
 // went from 1.16 to 0.43 ms; there the line solves' serial recurrence and the
