@@ -44,8 +44,8 @@ __device__ constexpr double PSI[11] = {-0.5000000000704921,    -0.40824827798859
 //              34 u rho^2 r beside what arg's error makes
 //  this value  B's diagonal 4 u S: det 48 u r^2 S and 144 u r^3 of rounding, r^2
 //              8 u r S: arg 36 u rho + 90 u, and 3 times the reciprocal square
-//              root's error: that of v_rsq_f64 (2^-23) is 1.5 2^-46 after one
-//              Newton step, 4.5 2^-46 = 576 u; r is off by 4 u S + 192 u r
+//              root's error: that of v_rsq_f64 (2^-23; 2^-24.2 is the largest of 6.7e7
+//              measured) is 1.5 2^-46 after one Newton step, 4.5 2^-46 = 576 u; r is off by 4 u S + 192 u r
 //  lambda'     |d lambda / d arg| <= 0.41 r / sqrt(1 - arg), and 0.58 r /
 //              sqrt(1 - arg) over an interval of half-width d where 1 - arg >= 2 d
 // d = 1.43e-14 rho^3 + 1e-12, 128 u rho^3 + 9000 u, is above both errors of arg together.  Where |arg| <= 1
